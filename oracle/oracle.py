@@ -30,10 +30,10 @@ class Counters(C.Structure):
 
 
 def build(reference: bool | None = None) -> None:
-    """Compiles liboracle.so, and _ref/libphxref.so when the reference tree is present."""
+    """Compiles liboracle.so, and _ref/libphxref.so when the reference's sources are present."""
     subprocess.run(["make", "-s", "-B", "-C", str(HERE), "liboracle.so"], check=True)
     if reference is None:
-        reference = REFERENCE_ROOT.exists()
+        reference = (REFERENCE_ROOT / "source").is_dir()
     if reference:
         subprocess.run(["make", "-s", "-B", "-C", str(HERE), "ref", "asship"], check=True)
 
