@@ -57,6 +57,7 @@ phx_status uploadArray(PhxContext* ctx, T*& dst, const T* src, size_t count, siz
 void freeScene(PhxScene* s)
 {
 	hipFree(s->nodes);
+	hipFree(s->wide);
 	hipFree(s->tris);
 	hipFree(s->datas);
 	hipFree(s->materials);
@@ -569,6 +570,12 @@ static phx_status phx_scene_upload_impl(PhxContext* ctx, const PhxBVHNode* nodes
 		st = uploadArray(ctx, s->nodes, laid.data(), numNodes, s->bytes);
 		if (st == PHX_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
 			st = fail(PHX_ERR_HIP, "phx_scene_upload: node upload failed");
+	}
+	if (st == PHX_OK) {
+		const std::vector<WideNode> wide = buildWide(nodes, numNodes, kTopCap / 2u);
+		st = uploadArray(ctx, s->wide, wide.data(), wide.size(), s->bytes);
+		if (st == PHX_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
+			st = fail(PHX_ERR_HIP, "phx_scene_upload: wide node upload failed");
 	}
 	if (st == PHX_OK) {
 		std::vector<PhxTriangleVertices> pre = pretransform(triangles, numTriangles);

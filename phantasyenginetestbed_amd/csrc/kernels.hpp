@@ -6,6 +6,7 @@
 #include <cstdint>
 
 #include "../../include/phx.h"
+#include "wide_nodes.hpp"
 
 namespace phx {
 
@@ -16,6 +17,7 @@ struct SceneView {
 	const PhxTriangleVertices* trisPre;
 	uint32_t numNodes;
 	uint32_t numTris;
+	const WideNode* wide;   // four-wide nodes (wide_nodes.hpp), or null: binary traversal only
 	uint32_t finiteBounds;  // every node bound within +-2^126 (enables the NaN-free slab path)
 	uint32_t topCount;      // nodes [0, topCount) are the top levels in breadth-first order
 };

@@ -105,6 +105,7 @@ struct PhxPlan {
 struct PhxScene {
 	PhxContext* ctx = nullptr;
 	PhxBVHNode* nodes = nullptr;
+	phx::WideNode* wide = nullptr;  // four-wide nodes, null if the tree cannot have them
 	PhxTriangleVertices* tris = nullptr;
 	PhxTriangleData* datas = nullptr;
 	PhxMaterial* materials = nullptr;
@@ -166,7 +167,7 @@ void dropContext(PhxContext* ctx);
 
 inline SceneView view(const PhxScene* s)
 {
-	return SceneView{s->nodes, s->tris, s->numNodes, s->numTris, s->finiteBounds, s->topCount};
+	return SceneView{s->nodes, s->tris, s->numNodes, s->numTris, s->wide, s->finiteBounds, s->topCount};
 }
 
 inline TraceLaunch traceLaunch(const PhxContext* ctx, uint32_t flags, bool anyhit)

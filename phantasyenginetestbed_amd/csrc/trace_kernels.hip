@@ -17,6 +17,7 @@
 
 #include "kernels.hpp"
 #include "trace_device.hpp"
+#include "wide_nodes.hpp"
 
 namespace phx {
 namespace {
@@ -121,12 +122,14 @@ constexpr int kSimpleStack = 72;
 // castRay<144> of one ray (BVHTraversal.hpp:37-128) into `c` (which holds the miss result on
 // entry): pop, decide both children, left first; a visited leaf is tested at once, a visited
 // inner node pushed.
-// castRay's pending stack for one lane: its first kLds entries in the lane's LDS column (entry e
-// at col[e * kBlock], one 4-B word per lane per row, so a wave's accesses are conflict-free), the
-// rest in private memory. A pop is on the path to the next node's load, and an LDS pop returns
-// sooner than a private (scratch) one.
+// Pending stack of one lane: its first words in the lane's LDS column (word e at col[e * kBlock], one
+// 4-B word per lane per row, so a wave's accesses are conflict-free), the rest in private memory. A
+// pop is on the path to the next node's load, and an LDS pop returns sooner than a private (scratch)
+// one. Binary traversals keep 4-B entries (put / get), wide ones 8-B entries of a reference and its
+// entry distance (put2 / get2): 72 of the former take as many words as kWideMaxPending of the latter.
 template <int kLds>
 struct ColumnStack {
+	static_assert(kLds % 2 == 0 && kSimpleStack == 2 * int(kWideMaxPending), "entry sizes");
 	uint32_t* col;
 	uint32_t deep[kSimpleStack - kLds];
 	__device__ __forceinline__ void put(int e, uint32_t v)
@@ -140,9 +143,29 @@ struct ColumnStack {
 	{
 		return e < kLds ? col[e * kBlock] : deep[e - kLds];
 	}
+	__device__ __forceinline__ void put2(int e, uint32_t ref, float tIn)
+	{
+		if (2 * e < kLds) {
+			col[2 * e * kBlock] = ref;
+			col[(2 * e + 1) * kBlock] = __float_as_uint(tIn);
+		} else {
+			deep[2 * e - kLds] = ref;
+			deep[2 * e + 1 - kLds] = __float_as_uint(tIn);
+		}
+	}
+	__device__ __forceinline__ void get2(int e, uint32_t& ref, float& tIn) const
+	{
+		if (2 * e < kLds) {
+			ref = col[2 * e * kBlock];
+			tIn = __uint_as_float(col[(2 * e + 1) * kBlock]);
+		} else {
+			ref = deep[2 * e - kLds];
+			tIn = __uint_as_float(deep[2 * e + 1 - kLds]);
+		}
+	}
 };
 
-// LDS stack entries per lane: 24 for one-ray-per-lane casts (24 KB per 256-thread block); 12 each
+// LDS stack words per lane: 24 for one-ray-per-lane casts (24 KB per 256-thread block); 12 each
 // for an instance cast's top-tree stack and its entered instance's castRay stack (24 KB, so the
 // five blocks per CU of its launch fit). Larger splits lower the blocks a CU holds and measured
 // slower.
@@ -243,11 +266,184 @@ __device__ __forceinline__ bool anyhit_one(const float4* __restrict__ nodes,
 	return occluded;
 }
 
+// ---- four-wide nodes ---------------------------------------------------------------------------
+//
+// wide_nodes.hpp says what they are and why taking their slots in order, with each slot's entry
+// distance compared again when it is taken, gives castRay's hits bit for bit for every ray whose
+// slab values cannot be NaN (dev::Ray::nanFree). The other rays walk the binary nodes.
+// A traversal is bound by its chain of dependent steps; on 1,004,000 triangles a bounce ray takes
+// 9.8 wide node visits where it takes 21.6 binary ones (random triangles: 32 for 65).
+
+struct WideWords {
+	float4 w0, w1, w2, w3, w4, w5;  // boxes of slots 0-3, (min.xyz, max.xyz) each
+	uint4 ref;
+};
+
+__device__ __forceinline__ WideWords load_wide(const float4* __restrict__ wide, uint32_t i)
+{
+	WideWords n;
+	const float4* p = wide + 8u * size_t(i);
+	n.w0 = p[0];
+	n.w1 = p[1];
+	n.w2 = p[2];
+	n.w3 = p[3];
+	n.w4 = p[4];
+	n.w5 = p[5];
+	n.ref = reinterpret_cast<const uint4*>(p)[6];
+	return n;
+}
+
+// Entry distance and box predicate of the four slots against tCurrMax (BVHTraversal.hpp:59-64;
+// any-hit: tMax).
+struct WideVisit {
+	float tIn[4];
+	bool pass[4];
+};
+
+__device__ __forceinline__ WideVisit decide_wide(const dev::Ray& r, const float4 w0, const float4 w1,
+                                                 const float4 w2, const float4 w3, const float4 w4,
+                                                 const float4 w5, float tCurrMax)
+{
+	WideVisit v;
+	float out[4];
+	dev::slab_fast(r, w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, v.tIn[0], out[0]);
+	dev::slab_fast(r, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w, v.tIn[1], out[1]);
+	dev::slab_fast(r, w3.x, w3.y, w3.z, w3.w, w4.x, w4.y, v.tIn[2], out[2]);
+	dev::slab_fast(r, w4.z, w4.w, w5.x, w5.y, w5.z, w5.w, v.tIn[3], out[3]);
+#pragma unroll
+	for (int i = 0; i < 4; i++)
+		v.pass[i] = (out[i] >= v.tIn[i]) && out[i] > r.tMin && v.tIn[i] < tCurrMax;
+	return v;
+}
+
+// One triangle, with the fast reciprocal: true iff castRay's test passes; t, u, v are its outputs.
+__device__ __forceinline__ bool triangle_fast(const dev::Ray& r, const float4 p0, const float4 e1,
+                                              const float4 e2, float& t, float& u, float& v)
+{
+	const dev::TriDet d = dev::tri_det(r, e1, e2);
+	float f = dev::recip_newton(d.a);
+	if (!dev::recip_newton_ok(d.a)) f = 1.0f / d.a;
+	return dev::tri_finish(r, d, f, p0, e1, e2, t, u, v);
+}
+
+// The triangles of a leaf from `first` to its end marker (p0.w < 0, BVHTraversal.hpp:78-93).
+__device__ __forceinline__ void closest_leaf_marked(const dev::Ray& r, const float4* __restrict__ tris,
+                                                    uint32_t first, Closest& c)
+{
+	for (uint32_t j = first;; j++) {
+		const float4* p = tris + 3u * size_t(j);
+		const float4 p0 = p[0], e1 = p[1], e2 = p[2];
+		float t, u, v;
+		const bool acc = triangle_fast(r, p0, e1, e2, t, u, v) && t < c.t && r.tMin <= t && t <= r.tMax;
+		c.tri = acc ? j : c.tri;
+		c.t = acc ? t : c.t;
+		c.u = acc ? u : c.u;
+		c.v = acc ? v : c.v;
+		if (p0.w < 0.0f) break;
+	}
+}
+
+__device__ __forceinline__ bool anyhit_leaf_marked(const dev::Ray& r, const float4* __restrict__ tris,
+                                                   uint32_t first)
+{
+	for (uint32_t j = first;; j++) {
+		const float4* p = tris + 3u * size_t(j);
+		const float4 p0 = p[0];
+		float t, u, v;
+		if (triangle_fast(r, p0, p[1], p[2], t, u, v) && r.tMin <= t && t < r.tMax) return true;
+		if (p0.w < 0.0f) return false;
+	}
+}
+
+// castRay of one NaN-free ray over the wide nodes into `c` (the miss result on entry); any hit:
+// returns whether a triangle was hit, in any order, and leaves `c` alone. A leaf that a node leaves
+// as its next slot is tested in the same iteration.
+template <bool kAnyHit, class Stack>
+__device__ __forceinline__ bool wide_one(const float4* __restrict__ wide,
+                                         const float4* __restrict__ tris, const dev::Ray& r,
+                                         Closest& c, Stack& st)
+{
+	uint32_t ref = 0u;
+	float tIn = -INFINITY;
+	int sp = 0;
+	while (true) {
+		bool have = true;
+		float lim = kAnyHit ? r.tMax : dev::min_first(r.tMax, c.t);
+		if (!(ref & kWideLeaf)) {
+			const WideWords n = load_wide(wide, ref);
+			const WideVisit v = decide_wide(r, n.w0, n.w1, n.w2, n.w3, n.w4, n.w5, lim);
+			const uint32_t refs[4] = {n.ref.x, n.ref.y, n.ref.z, n.ref.w};
+			// Last slot first, so that the first passing slot is what remains to be taken. A leaf
+			// pair stays one only if both leaves pass.
+			have = false;
+#pragma unroll
+			for (int i = 3; i >= 0; i--) {
+				if (v.pass[i]) {
+					if (have) st.put2(sp++, ref, tIn);
+					ref = refs[i];
+					if (!kAnyHit && i < 3 && !v.pass[i + 1]) ref &= ~kWidePair;
+					tIn = v.tIn[i];
+					have = true;
+				}
+			}
+		}
+		if (have && (ref & kWideLeaf)) {
+			have = false;
+			const uint32_t first = ref & kWideIndex;
+			if (kAnyHit) {
+				if (anyhit_leaf_marked(r, tris, first)) return true;
+			} else if (tIn < lim) {
+				if (ref & kWidePair) {
+					// The sibling leaf (the top entry) is decided now too.
+					uint32_t sib;
+					float sIn;
+					st.get2(sp - 1, sib, sIn);
+					st.put2(sp - 1, sib, sIn < lim ? -INFINITY : INFINITY);
+				}
+				closest_leaf_marked(r, tris, first, c);
+				lim = dev::min_first(r.tMax, c.t);
+			}
+		}
+		while (!have) {
+			if (sp == 0) return false;
+			st.get2(--sp, ref, tIn);
+			have = kAnyHit || tIn < lim;
+		}
+	}
+}
+
+// castRay of any ray: over the wide nodes where the scene has them (wide != nullptr) and the ray
+// is NaN-free, else over the binary ones.
+template <class Stack>
+__device__ __forceinline__ void closest_any(const float4* __restrict__ wide,
+                                            const float4* __restrict__ nodes,
+                                            const float4* __restrict__ tris, const dev::Ray& r,
+                                            Closest& c, Stack& st)
+{
+	Counts none;
+	if (wide && r.nanFree)
+		wide_one<false>(wide, tris, r, c, st);
+	else
+		closest_one<false>(nodes, tris, r, c, none, st);
+}
+template <class Stack>
+__device__ __forceinline__ bool anyhit_any(const float4* __restrict__ wide,
+                                           const float4* __restrict__ nodes,
+                                           const float4* __restrict__ tris, const dev::Ray& r,
+                                           Stack& st)
+{
+	Counts none;
+	Closest c;
+	if (wide && r.nanFree) return wide_one<true>(wide, tris, r, c, st);
+	return anyhit_one<false>(nodes, tris, r, none, st);
+}
+
+// kCount: castDebugRay's counters, which count binary nodes, so every ray walks those.
 template <bool kCount>
 __global__ __launch_bounds__(kBlock) void k_closest_simple(
-	const float4* __restrict__ nodes, const float4* __restrict__ tris,
-	const float4* __restrict__ rays, uint4* __restrict__ hits, uint32_t n,
-	unsigned long long* __restrict__ counters)
+	const float4* __restrict__ wide, const float4* __restrict__ nodes,
+	const float4* __restrict__ tris, const float4* __restrict__ rays, uint4* __restrict__ hits,
+	uint32_t n, unsigned long long* __restrict__ counters)
 {
 	__shared__ uint32_t stackLds[kSimpleLds * kBlock];
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -257,17 +453,19 @@ __global__ __launch_bounds__(kBlock) void k_closest_simple(
 	Counts k;
 	ColumnStack<kSimpleLds> st;
 	st.col = stackLds + threadIdx.x;
-	closest_one<kCount>(nodes, tris, r, c, k, st);
+	if (kCount)
+		closest_one<true>(nodes, tris, r, c, k, st);
+	else
+		closest_any(wide, nodes, tris, r, c, st);
 	hits[i] = make_uint4(c.tri, __float_as_uint(c.t), __float_as_uint(c.u), __float_as_uint(c.v));
 	if (kCount) add_counts(counters, k);
 }
 
 template <bool kCount>
-__global__ __launch_bounds__(kBlock) void k_anyhit_simple(const float4* __restrict__ nodes,
-                                                          const float4* __restrict__ tris,
-                                                          const float4* __restrict__ rays,
-                                                          uint8_t* __restrict__ inLight, uint32_t n,
-                                                          unsigned long long* __restrict__ counters)
+__global__ __launch_bounds__(kBlock) void k_anyhit_simple(
+	const float4* __restrict__ wide, const float4* __restrict__ nodes,
+	const float4* __restrict__ tris, const float4* __restrict__ rays,
+	uint8_t* __restrict__ inLight, uint32_t n, unsigned long long* __restrict__ counters)
 {
 	__shared__ uint32_t stackLds[kSimpleLds * kBlock];
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -276,7 +474,9 @@ __global__ __launch_bounds__(kBlock) void k_anyhit_simple(const float4* __restri
 	Counts k;
 	ColumnStack<kSimpleLds> st;
 	st.col = stackLds + threadIdx.x;
-	inLight[i] = anyhit_one<kCount>(nodes, tris, r, k, st) ? 0 : 1;
+	const bool occluded =
+		kCount ? anyhit_one<true>(nodes, tris, r, k, st) : anyhit_any(wide, nodes, tris, r, st);
+	inLight[i] = occluded ? 0 : 1;
 	if (kCount) add_counts(counters, k);
 }
 
@@ -629,38 +829,47 @@ __host__ __device__ __forceinline__ uint32_t persistent_lds_bytes(uint32_t block
 //
 // For coherent rays -- camera rays in 8x8-tile order, shadow rays towards one light -- a wave traces
 // 64 consecutive rays together over one shared stack of (node, lane mask) entries. Each node is
-// loaded once for the wave (every lane reads the same address); each lane decides both child boxes
-// with its own ray and closest hit, and tests a visited leaf's triangles only where it decided to.
-// Per lane, the nodes expanded and the triangles tested, in their order, are exactly castRay's
-// (BVHTraversal.hpp:37-128): both child boxes are decided before either child is used, a visited
-// leaf's triangles are tested at once, left child first, and inner children are pushed left then
-// right, so the right subtree is expanded first; a lane takes part only in the entries it pushed.
-// The wave expands the union of its lanes' nodes, which for coherent rays is close to one ray's,
-// and every step does the same kind of work. Stack entry e lives in lane e % 64 of the register
-// triple e / 64 (node, mask low, mask high); trees are at most 64 levels deep (checked at upload),
-// and the stack holds at most one pending left child per level.
+// loaded once for the wave (every lane reads the same address, a scalar load); each lane decides the
+// boxes with its own ray and closest hit, and tests a visited leaf's triangles only where it decided
+// to. A lane takes part only in the entries it pushed, and per lane their order is castRay's
+// (BVHTraversal.hpp:37-128), so its hits are too. The wave expands the union of its lanes' nodes,
+// which for coherent rays is close to one ray's, and every step does the same kind of work. Stack
+// entry e lives in lane e % 64 of a few registers.
+//
+// A step is bound by the latency of its dependent node load and the launch by its longest packets
+// (2 waves per SIMD in flight on average), so packets of NaN-free rays walk the four-wide nodes: half
+// the steps, for twice the box tests each. 2,073,600 tiled camera rays on 1,004,000 triangles,
+// generation included: 0.522 ms with binary nodes and IEEE divisions, 0.472 ms with wide nodes and
+// the fast reciprocal.
 
 constexpr uint32_t kPacketBlock = 256;
 
+__device__ __forceinline__ uint32_t lane_get(uint32_t v, int l)
+{
+	return uint32_t(__builtin_amdgcn_readlane(int(v), l));
+}
+// v_writelane_b32 (clang has no builtin for this intrinsic).
+extern "C" __device__ int amdgcn_writelane(int v, int l, int old) __asm("llvm.amdgcn.writelane.i32");
+__device__ __forceinline__ uint32_t lane_set(uint32_t old, uint32_t v, int l)
+{
+	return uint32_t(amdgcn_writelane(int(v), l, int(old)));
+}
+__device__ __forceinline__ uint32_t uniform(uint32_t v)
+{
+	return uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
+}
+
+// The binary nodes, for packets with a ray whose slab values may be NaN and for scenes without
+// wide nodes. Both child boxes are decided before either child is used, a visited leaf's triangles
+// are tested at once, left child first, and inner children are pushed left then right. The stack
+// holds at most one pending left child per level (64, checked at upload).
 template <bool kAnyHit>
-__global__ __launch_bounds__(kPacketBlock) void k_packet(const float4* __restrict__ nodes,
-                                                         const float4* __restrict__ tris,
-                                                         const float4* __restrict__ rays,
-                                                         void* __restrict__ out, uint32_t n,
-                                                         uint32_t finiteBounds)
+__device__ __forceinline__ void packet_binary(const float4* __restrict__ nodes,
+                                              const float4* __restrict__ tris, const dev::Ray& r,
+                                              bool active, Closest& c, bool& occluded)
 {
 	const uint32_t lane = __lane_id();
-	const uint32_t first = blockIdx.x * kPacketBlock + (threadIdx.x & ~63u);
-	if (first >= n) return;  // whole wave
-	const uint32_t i = first + lane;
-	const bool active = i < n;
-	const uint32_t ri = active ? i : first;  // lanes past the end read a valid ray, never used
-	const dev::Ray r = dev::make_ray(rays[2 * size_t(ri)], rays[2 * size_t(ri) + 1]);
-	// The NaN-free slab path only when every active lane may take it (the decision is uniform).
-	const bool fast = __ballot(active && !(finiteBounds != 0u && r.nanFree)) == 0ull;
-	Closest c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
 	Counts none;
-	bool occluded = false;
 	uint32_t sN0 = 0u, sL0 = 0u, sH0 = 0u, sN1 = 0u, sL1 = 0u, sH1 = 0u;
 	int sp = 0;
 	auto push = [&](uint32_t node, uint64_t m) {
@@ -686,7 +895,7 @@ __global__ __launch_bounds__(kPacketBlock) void k_packet(const float4* __restric
 		const int32_t rCnt = __builtin_amdgcn_readfirstlane(nd.w3.w);
 		const float tCurrMax = kAnyHit ? r.tMax : dev::min_first(r.tMax, c.t);
 		bool visitL, visitR;
-		decide(r, fast, nd, tCurrMax, visitL, visitR);
+		decide(r, false, nd, tCurrMax, visitL, visitR);
 		visitL = visitL && in;
 		visitR = visitR && in;
 		uint64_t pushL = 0ull, pushR = 0ull;
@@ -710,13 +919,166 @@ __global__ __launch_bounds__(kPacketBlock) void k_packet(const float4* __restric
 			sp--;
 			const bool low = sp < 64;
 			const int l = low ? sp : sp - 64;
-			cur = uint32_t(__builtin_amdgcn_readlane(int(low ? sN0 : sN1), l));
-			const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(low ? sL0 : sL1), l));
-			const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(low ? sH0 : sH1), l));
+			cur = lane_get(low ? sN0 : sN1, l);
+			const uint32_t lo = lane_get(low ? sL0 : sL1, l);
+			const uint32_t hi = lane_get(low ? sH0 : sH1, l);
 			mask = ((uint64_t(hi) << 32) | lo) & ~done;
 		}
 		if (mask == 0ull) break;
 	}
+}
+
+// A leaf's triangles (uniform addresses: scalar loads) for the lanes in `on`.
+template <bool kAnyHit>
+__device__ __forceinline__ void packet_leaf(const float4* __restrict__ tris, uint32_t first,
+                                            const dev::Ray& r, bool on, Closest& c, bool& occluded)
+{
+	for (uint32_t j = first;; j++) {
+		const float4* p = tris + 3u * size_t(j);
+		const float4 p0 = p[0], e1 = p[1], e2 = p[2];
+		const dev::TriDet d = dev::tri_det(r, e1, e2);
+		float f = dev::recip_newton(d.a);
+		if (__ballot(on && !dev::recip_newton_ok(d.a)) != 0ull) f = 1.0f / d.a;
+		float t, u, v;
+		const bool hit = dev::tri_finish(r, d, f, p0, e1, e2, t, u, v);
+		if (kAnyHit) {
+			occluded = occluded || (on && hit && r.tMin <= t && t < r.tMax);
+		} else {
+			const bool acc = on && hit && t < c.t && r.tMin <= t && t <= r.tMax;
+			c.tri = acc ? j : c.tri;
+			c.t = acc ? t : c.t;
+			c.u = acc ? u : c.u;
+			c.v = acc ? v : c.v;
+		}
+		if (p0.w < 0.0f) break;
+	}
+}
+
+// The wide nodes. Slots are taken in order: leaf slots are tested at once as long as no inner slot
+// comes before them; the first inner slot is the next node, and the slots after it are pushed. A
+// leaf slot that was pushed is decided again when it is taken, from its box in the node (closest
+// hit; entry word 1 names node and slot). Any hit does not depend on order: all its leaf slots are
+// tested at once.
+template <bool kAnyHit>
+__device__ __forceinline__ void packet_wide(const float4* __restrict__ wide,
+                                            const float4* __restrict__ tris, const dev::Ray& r,
+                                            bool active, Closest& c, bool& occluded)
+{
+	const uint32_t lane = __lane_id();
+	uint32_t sR = 0u, sB = 0u, sL = 0u, sH = 0u;  // reference, node and slot, mask
+	int sp = 0;
+	uint32_t cur = 0u;
+	uint64_t mask = __ballot(active);
+	while (true) {
+		const bool in = ((mask >> lane) & 1ull) != 0;
+		const WideWords n = load_wide(wide, cur);
+		const float lim = kAnyHit ? r.tMax : dev::min_first(r.tMax, c.t);
+		WideVisit v = decide_wide(r, n.w0, n.w1, n.w2, n.w3, n.w4, n.w5, lim);
+		const uint32_t refs[4] = {uniform(n.ref.x), uniform(n.ref.y), uniform(n.ref.z),
+		                          uniform(n.ref.w)};
+		uint64_t m[4];
+#pragma unroll
+		for (int i = 0; i < 4; i++) {
+			v.pass[i] = v.pass[i] && in;
+			m[i] = __ballot(v.pass[i]);
+		}
+		bool sibling[4] = {false, false, false, false};  // a pair's second leaf: decided with the first
+		int next = -1;
+#pragma unroll
+		for (int i = 0; i < 4; i++) {
+			if (m[i] == 0ull) continue;
+			if (!(refs[i] & kWideLeaf)) {
+				if (next < 0) next = i;
+				continue;
+			}
+			if (!kAnyHit && next >= 0) continue;  // pushed below
+			if (kAnyHit) {
+				packet_leaf<true>(tris, refs[i] & kWideIndex, r, v.pass[i] && !occluded, c, occluded);
+			} else {
+				const float cm = dev::min_first(r.tMax, c.t);
+				const bool on = v.pass[i] && (sibling[i] || v.tIn[i] < cm);
+				if (i < 3 && (refs[i] & kWidePair)) {
+					v.pass[i + 1] = v.pass[i + 1] && v.tIn[i + 1] < cm;
+					sibling[i + 1] = true;
+				}
+				packet_leaf<false>(tris, refs[i] & kWideIndex, r, on, c, occluded);
+			}
+		}
+		const uint64_t done = kAnyHit ? __ballot(occluded) : 0ull;
+#pragma unroll
+		for (int i = 3; i >= 1; i--) {
+			const uint64_t mi = m[i] & ~done;
+			if (i <= next || next < 0 || mi == 0ull) continue;
+			if (kAnyHit && (refs[i] & kWideLeaf)) continue;
+			uint32_t ref = refs[i];
+			if (i == 3 || m[i < 3 ? i + 1 : 3] == 0ull) ref &= ~kWidePair;
+			sR = lane_set(sR, ref, sp);
+			sB = lane_set(sB, cur * 4u + uint32_t(i), sp);
+			sL = lane_set(sL, uint32_t(mi), sp);
+			sH = lane_set(sH, uint32_t(mi >> 32), sp);
+			sp++;
+		}
+		mask = 0ull;
+		if (next >= 0) {
+#pragma unroll
+			for (int i = 0; i < 4; i++)
+				if (next == i) {
+					mask = m[i] & ~done;
+					cur = refs[i];
+				}
+		}
+		while (mask == 0ull && sp > 0) {
+			sp--;
+			const uint32_t ref = lane_get(sR, sp);
+			const uint64_t me = ((uint64_t(lane_get(sH, sp)) << 32) | lane_get(sL, sp)) & ~done;
+			if (kAnyHit || !(ref & kWideLeaf)) {
+				mask = me;
+				cur = ref;
+				continue;
+			}
+			auto decided = [&](int e, uint64_t who) {
+				const uint32_t at = lane_get(sB, e);
+				const float* b = reinterpret_cast<const float*>(wide + 8u * size_t(at >> 2)) + 6u * (at & 3u);
+				float tIn, tOut;
+				dev::slab_fast(r, b[0], b[1], b[2], b[3], b[4], b[5], tIn, tOut);
+				return ((who >> lane) & 1ull) != 0 && tIn < dev::min_first(r.tMax, c.t);
+			};
+			const bool on = decided(sp, me);
+			bool on2 = false;
+			uint32_t ref2 = 0u;
+			if (ref & kWidePair) {
+				sp--;
+				ref2 = lane_get(sR, sp);
+				on2 = decided(sp, (uint64_t(lane_get(sH, sp)) << 32) | lane_get(sL, sp));
+			}
+			if (__ballot(on) != 0ull) packet_leaf<false>(tris, ref & kWideIndex, r, on, c, occluded);
+			if (__ballot(on2) != 0ull) packet_leaf<false>(tris, ref2 & kWideIndex, r, on2, c, occluded);
+		}
+		if (mask == 0ull) break;
+	}
+}
+
+template <bool kAnyHit>
+__global__ __launch_bounds__(kPacketBlock) void k_packet(const float4* __restrict__ wide,
+                                                         const float4* __restrict__ nodes,
+                                                         const float4* __restrict__ tris,
+                                                         const float4* __restrict__ rays,
+                                                         void* __restrict__ out, uint32_t n)
+{
+	const uint32_t lane = __lane_id();
+	const uint32_t first = blockIdx.x * kPacketBlock + (threadIdx.x & ~63u);
+	if (first >= n) return;  // whole wave
+	const uint32_t i = first + lane;
+	const bool active = i < n;
+	const uint32_t ri = active ? i : first;  // lanes past the end read a valid ray, never used
+	const dev::Ray r = dev::make_ray(rays[2 * size_t(ri)], rays[2 * size_t(ri) + 1]);
+	Closest c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
+	bool occluded = false;
+	// The wide nodes only when every active lane may walk them (the decision is uniform).
+	if (wide && __ballot(active && !r.nanFree) == 0ull)
+		packet_wide<kAnyHit>(wide, tris, r, active, c, occluded);
+	else
+		packet_binary<kAnyHit>(nodes, tris, r, active, c, occluded);
 	if (active) {
 		if (kAnyHit)
 			static_cast<uint8_t*>(out)[i] = occluded ? 0 : 1;
@@ -1960,22 +2322,23 @@ hipError_t launchClosest(const SceneView& s, const PhxRayIn* rays, uint32_t n, P
                          const TraceLaunch& L, unsigned long long* counters, hipStream_t stream)
 {
 	if (n == 0) return hipSuccess;
+	const float4* wide = reinterpret_cast<const float4*>(s.wide);
 	const float4* nodes = reinterpret_cast<const float4*>(s.nodes);
 	const float4* tris = reinterpret_cast<const float4*>(s.trisPre);
 	const float4* r4 = reinterpret_cast<const float4*>(rays);
 	uint4* h4 = reinterpret_cast<uint4*>(hits);
 	if (L.kernel == TraceKernel::Packet && !counters) {
 		hipLaunchKernelGGL(k_packet<false>, dim3(gridFor(n, kPacketBlock)), dim3(kPacketBlock), 0,
-		                   stream, nodes, tris, r4, static_cast<void*>(h4), n, s.finiteBounds);
+		                   stream, wide, nodes, tris, r4, static_cast<void*>(h4), n);
 		return hipGetLastError();
 	}
 	if (L.kernel != TraceKernel::Persistent || n > 0x7FFFFFFFu) {
 		if (counters)
 			hipLaunchKernelGGL(k_closest_simple<true>, dim3(gridFor(n, kBlock)), dim3(kBlock), 0,
-			                   stream, nodes, tris, r4, h4, n, counters);
+			                   stream, wide, nodes, tris, r4, h4, n, counters);
 		else
 			hipLaunchKernelGGL(k_closest_simple<false>, dim3(gridFor(n, kBlock)), dim3(kBlock), 0,
-			                   stream, nodes, tris, r4, h4, n, counters);
+			                   stream, wide, nodes, tris, r4, h4, n, counters);
 		return hipGetLastError();
 	}
 	uint32_t grid, block, top, lds;
@@ -2012,7 +2375,7 @@ hipError_t launchAnyHitCounted(const SceneView& s, const PhxRayIn* rays, uint32_
 {
 	if (n == 0) return hipSuccess;
 	hipLaunchKernelGGL(k_anyhit_simple<true>, dim3(gridFor(n, kBlock)), dim3(kBlock), 0, stream,
-	                   reinterpret_cast<const float4*>(s.nodes),
+	                   nullptr, reinterpret_cast<const float4*>(s.nodes),
 	                   reinterpret_cast<const float4*>(s.trisPre),
 	                   reinterpret_cast<const float4*>(rays), inLight, n, counters);
 	return hipGetLastError();
@@ -2044,17 +2407,18 @@ hipError_t launchAnyHit(const SceneView& s, const PhxRayIn* rays, uint32_t n, ui
                         const TraceLaunch& L, hipStream_t stream)
 {
 	if (n == 0) return hipSuccess;
+	const float4* wide = reinterpret_cast<const float4*>(s.wide);
 	const float4* nodes = reinterpret_cast<const float4*>(s.nodes);
 	const float4* tris = reinterpret_cast<const float4*>(s.trisPre);
 	const float4* r4 = reinterpret_cast<const float4*>(rays);
 	if (L.kernel == TraceKernel::Packet) {
 		hipLaunchKernelGGL(k_packet<true>, dim3(gridFor(n, kPacketBlock)), dim3(kPacketBlock), 0,
-		                   stream, nodes, tris, r4, static_cast<void*>(inLight), n, s.finiteBounds);
+		                   stream, wide, nodes, tris, r4, static_cast<void*>(inLight), n);
 		return hipGetLastError();
 	}
 	if (L.kernel == TraceKernel::Simple || n > 0x7FFFFFFFu) {
 		hipLaunchKernelGGL(k_anyhit_simple<false>, dim3(gridFor(n, kBlock)), dim3(kBlock), 0,
-		                   stream, nodes, tris, r4, inLight, n, nullptr);
+		                   stream, wide, nodes, tris, r4, inLight, n, nullptr);
 		return hipGetLastError();
 	}
 	uint32_t grid, block, top, lds;

@@ -1,0 +1,190 @@
+// Collapses an SBVH into four-wide nodes; see wide_nodes.hpp.
+#include "wide_nodes.hpp"
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <limits>
+
+namespace phx {
+namespace {
+
+// True if the conditions of wide_nodes.hpp on the boxes hold for every node.
+bool eligible(const PhxBVHNode* nodes, uint32_t n)
+{
+	for (uint32_t i = 0; i < n; i++) {
+		const PhxBVHNode& nd = nodes[i];
+		for (int c = 0; c < 2; c++) {
+			const float* b = nd.fData + 6 * c;
+			bool good = true;  // false for NaN too
+			for (int k = 0; k < 3; k++)
+				good &= std::fabs(b[k]) <= 0x1p126f && std::fabs(b[k + 3]) <= 0x1p126f && b[k] <= b[k + 3];
+			if (good && nd.iData[2 + c] == 0) {
+				const float* f = nodes[nd.iData[c]].fData;
+				for (int k = 0; k < 3; k++)
+					good &= f[k] >= b[k] && f[k + 6] >= b[k] && f[k + 3] <= b[k + 3] && f[k + 9] <= b[k + 3];
+			}
+			if (!good) return false;
+		}
+	}
+	return true;
+}
+
+// One slot while a wide node is put together: a leaf, or an inner binary node.
+struct Slot {
+	const float* box;
+	uint32_t ref;    // leaf: the finished reference; inner: the binary node's index
+	bool leaf;
+	float area;      // half surface area, of inner slots
+};
+
+float halfArea(const float* b)
+{
+	const float x = b[3] - b[0], y = b[4] - b[1], z = b[5] - b[2];
+	return x * y + y * z + z * x;
+}
+
+// The slots of binary node `node` in castRay's order (see wide_nodes.hpp); returns how many (2).
+int expand(const PhxBVHNode* nodes, uint32_t node, Slot out[2])
+{
+	const PhxBVHNode& nd = nodes[node];
+	int k = 0;
+	for (int c = 0; c < 2; c++)
+		if (nd.iData[2 + c] != 0) {
+			const uint32_t cnt = uint32_t(nd.iData[2 + c]);
+			uint32_t ref = kWideLeaf | uint32_t(~nd.iData[c]) | ((cnt <= 3u ? cnt : 0u) << kWideCountShift);
+			if (c == 0 && nd.iData[3] != 0) ref |= kWidePair;
+			out[k++] = Slot{nd.fData + 6 * c, ref, true, 0.0f};
+		}
+	for (int c = 1; c >= 0; c--)
+		if (nd.iData[2 + c] == 0) {
+			const float* b = nd.fData + 6 * c;
+			out[k++] = Slot{b, uint32_t(nd.iData[c]), false, halfArea(b)};
+		}
+	return k;
+}
+
+// A wide node's slots: binary node `root` with the inner slots of largest area opened in place
+// until four are used.
+int collapse(const PhxBVHNode* nodes, uint32_t root, Slot s[4])
+{
+	int k = expand(nodes, root, s);
+	while (k < 4) {
+		int best = -1;
+		for (int i = 0; i < k; i++)
+			if (!s[i].leaf && (best < 0 || s[i].area > s[best].area)) best = i;
+		if (best < 0) break;
+		Slot two[2];
+		expand(nodes, s[best].ref, two);
+		for (int i = k; i > best + 1; i--) s[i] = s[i - 1];
+		s[best] = two[0];
+		s[best + 1] = two[1];
+		k++;
+	}
+	return k;
+}
+
+WideNode emptyNode()
+{
+	WideNode w;
+	const float nan = std::numeric_limits<float>::quiet_NaN();
+	for (int i = 0; i < 4; i++) {
+		for (int k = 0; k < 6; k++) w.box[i][k] = nan;
+		w.ref[i] = 0u;
+		w.pad[i] = 0u;
+	}
+	return w;
+}
+
+}  // namespace
+
+std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint32_t topCap)
+{
+	std::vector<WideNode> out;
+	if (!eligible(nodes, numNodes)) return out;
+
+	// A node to fill: the binary node whose subtree it covers and the slots pending beside it.
+	struct Item {
+		uint32_t at, node, pending;
+	};
+	std::vector<Item> queue;  // breadth first up to topCap nodes, then a stack
+	out.reserve(size_t(numNodes) / 2 + 8);
+	out.push_back(emptyNode());
+	uint32_t maxPending = 0;
+
+	// The root: its slots become nodes 1..k. Leaves get a node that holds just them.
+	Slot s[4];
+	const int rootSlots = collapse(nodes, 0, s);
+	struct RootSlot {
+		int first, count;  // range of s
+	};
+	RootSlot rs[4];
+	int numRoot = 0;
+	for (int i = 0; i < rootSlots; i++) {
+		const int count = s[i].leaf && (s[i].ref & kWidePair) ? 2 : 1;
+		rs[numRoot++] = RootSlot{i, count};
+		i += count - 1;
+	}
+	for (int j = 0; j < numRoot; j++) {
+		const Slot& a = s[rs[j].first];
+		std::memcpy(out[0].box[j], a.box, sizeof(out[0].box[j]));
+		if (rs[j].count == 2) {
+			const Slot& b = s[rs[j].first + 1];
+			for (int k = 0; k < 3; k++) {
+				out[0].box[j][k] = std::min(a.box[k], b.box[k]);
+				out[0].box[j][k + 3] = std::max(a.box[k + 3], b.box[k + 3]);
+			}
+		}
+		out[0].ref[j] = uint32_t(j + 1);
+		out.push_back(emptyNode());
+		const uint32_t pending = uint32_t(numRoot - 1 - j);
+		if (a.leaf) {
+			for (int i = 0; i < rs[j].count; i++) {
+				std::memcpy(out[size_t(j) + 1].box[i], s[rs[j].first + i].box, 24);
+				out[size_t(j) + 1].ref[i] = s[rs[j].first + i].ref;
+			}
+			maxPending = std::max(maxPending, pending + 1u);
+		} else {
+			queue.push_back(Item{uint32_t(j + 1), a.ref, pending});
+		}
+	}
+	maxPending = std::max(maxPending, uint32_t(numRoot - 1));
+
+	// Fills node it.at; its inner slots get the next indices and are appended to `next`.
+	auto fill = [&](const Item& it, std::vector<Item>& next) {
+		Slot t[4];
+		const int k = collapse(nodes, it.node, t);
+		maxPending = std::max(maxPending, it.pending + uint32_t(k - 1));
+		for (int i = 0; i < k; i++) {
+			std::memcpy(out[it.at].box[i], t[i].box, 24);
+			if (t[i].leaf) {
+				out[it.at].ref[i] = t[i].ref;
+			} else {
+				const uint32_t child = uint32_t(out.size());
+				out[it.at].ref[i] = child;
+				out.push_back(emptyNode());
+				next.push_back(Item{child, t[i].ref, it.pending + uint32_t(k - 1 - i)});
+			}
+		}
+	};
+	size_t head = 0;
+	while (head < queue.size() && out.size() < topCap) {
+		const Item it = queue[head++];
+		fill(it, queue);
+	}
+	// The rest depth first: a node's children are numbered when it is filled (siblings side by
+	// side), the first slot's subtree before the next one's.
+	std::vector<Item> stack(queue.rbegin(), queue.rend() - ptrdiff_t(head));
+	std::vector<Item> kids;
+	while (!stack.empty()) {
+		const Item it = stack.back();
+		stack.pop_back();
+		kids.clear();
+		fill(it, kids);
+		stack.insert(stack.end(), kids.rbegin(), kids.rend());
+	}
+	if (maxPending > kWideMaxPending || out.size() > kWideIndex) out.clear();
+	return out;
+}
+
+}  // namespace phx

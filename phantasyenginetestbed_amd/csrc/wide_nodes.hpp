@@ -1,0 +1,54 @@
+// Four-wide nodes of an SBVH: the device-side form of the tree that the traversal kernels walk.
+//
+// A wide node merges a binary node with up to two of its descendants, so one 112-B record decides
+// four boxes where castRay's binary nodes take three dependent loads. Hits stay castRay's bit for
+// bit because
+//   - castRay's order does not depend on the ray: at a node, the leaf children are tested (left,
+//     then right), then the right inner child's subtree, then the left one's. The slots of a wide
+//     node are kept in that order, so taking the slots in order is castRay's order;
+//   - every child box lies inside its parent's (checked here). For a ray without NaN slab values
+//     rounding is monotonic, so a child that passes the box predicate at some closest t implies
+//     that its ancestors passed theirs at the larger t of that earlier moment: the binary node
+//     decisions that a wide node leaves out can never have been negative;
+//   - a leaf is decided with the closest t it would be decided with by castRay: its entry distance
+//     is kept with the pending slot and compared when the slot is taken. Two leaves of one parent
+//     are decided together, before either is tested (kWidePair).
+// Trees where this does not hold (bounds outside +-2^126 or NaN, child boxes that are inverted or
+// stick out of their parent, more than kWideMaxPending slots pending at once) get no wide nodes
+// and are traversed binary, as rays with NaN slab values are.
+#pragma once
+
+#include <cstdint>
+#include <vector>
+
+#include "../../include/phx.h"
+
+namespace phx {
+
+// One slot's reference: an inner slot holds the wide node's index; a leaf slot holds kWideLeaf,
+// its first triangle and (bits 28-29) its triangle count if that is 1 to 3, else 0 -- the
+// end marker of the triangle array ends it then. kWidePair: the next slot is the sibling leaf.
+constexpr uint32_t kWideLeaf = 0x80000000u;
+constexpr uint32_t kWidePair = 0x40000000u;
+constexpr uint32_t kWideIndex = 0x0FFFFFFFu;
+constexpr uint32_t kWideCountShift = 28u;
+
+// Pending slots a traversal may hold (the kernels' stacks hold this many 8-byte entries).
+constexpr uint32_t kWideMaxPending = 36u;
+
+// 128 B, so that a record is one cache line: boxes as (min.xyz, max.xyz) per slot, then the
+// references. Empty slots have NaN boxes, which no ray passes.
+struct WideNode {
+	float box[4][6];
+	uint32_t ref[4];
+	uint32_t pad[4];
+};
+static_assert(sizeof(WideNode) == 128, "WideNode is one 128-B line");
+
+// Wide nodes of a validated SBVH (validateBVH), or an empty vector if the tree cannot have them.
+// Node 0 is the root and all its slots are inner: slot i refers to node i + 1 (a leaf or leaf pair
+// of the root gets a node of its own), so a kernel needs only the root's boxes. The first
+// `topCap` nodes are in breadth-first order, the rest depth first in slot order.
+std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint32_t topCap);
+
+}  // namespace phx

@@ -1,0 +1,96 @@
+// CPU walk of the four-wide nodes (csrc/wide_nodes.hpp) in the order the kernels take their slots,
+// for tests/test_wide_nodes.py to compare with the oracle's binary castRay.
+#include <cfloat>
+#include <cmath>
+#include <cstring>
+#include <limits>
+
+#include "../../oracle/oracle.h"
+#include "../../phantasyenginetestbed_amd/csrc/wide_nodes.hpp"
+
+using namespace phx;
+
+namespace {
+
+struct Entry {
+	float tIn;
+	uint32_t ref;
+};
+
+// Closest hit of one ray, or (any hit) whether a triangle lies in [tMin, tMax). `deepest` is raised
+// to the most entries the stack held.
+bool walk(const std::vector<WideNode>& wide, const OrTri* tris, const OrRay& r, bool any, OrHit& c,
+          uint32_t& deepest)
+{
+	const float inf = std::numeric_limits<float>::infinity();
+	c = {0xFFFFFFFFu, FLT_MAX, FLT_MAX, FLT_MAX};
+	Entry stack[64];
+	uint32_t sp = 0;
+	Entry cur = {-inf, 0u};
+	while (true) {
+		const float lim = any ? r.tMax : (c.t < r.tMax ? c.t : r.tMax);
+		bool have = false;
+		if (!(cur.ref & kWideLeaf)) {
+			const WideNode& n = wide[cur.ref];
+			float tIn[4];
+			bool pass[4];
+			for (int i = 0; i < 4; i++) {
+				float tOut;
+				const float* b = n.box[i];
+				const bool hit = oracle_aabb(r.o, r.d, b, b + 3, &tIn[i], &tOut) != 0;
+				pass[i] = hit && tOut > r.tMin && tIn[i] < lim;
+			}
+			for (int i = 3; i >= 0; i--)
+				if (pass[i]) {
+					if (have) stack[sp++] = cur;
+					cur = {tIn[i], n.ref[i]};
+					if (cur.ref & kWidePair && !(i < 3 && pass[i + 1])) cur.ref &= ~kWidePair;
+					have = true;
+				}
+			if (sp > deepest) deepest = sp;
+		} else {
+			if (any || cur.tIn < lim) {
+				if (!any && (cur.ref & kWidePair)) stack[sp - 1].tIn = stack[sp - 1].tIn < lim ? -inf : inf;
+				const uint32_t first = cur.ref & kWideIndex;
+				const uint32_t count = (cur.ref >> kWideCountShift) & 3u;
+				for (uint32_t j = first;; j++) {
+					float t, u, v;
+					const float(*p)[4] = tris[j].v;
+					if (oracle_triangle(p[0], p[1], p[2], r.o, r.d, &t, &u, &v)) {
+						if (any && r.tMin <= t && t < r.tMax) return true;
+						if (!any && t < c.t && r.tMin <= t && t <= r.tMax) c = {j, t, u, v};
+					}
+					const bool last = p[0][3] < 0.0f;
+					if (count && last != (j + 1u == first + count)) return true;  // wrong count code
+					if (last) break;
+				}
+			}
+		}
+		while (!have) {
+			if (sp == 0) return false;
+			cur = stack[--sp];
+			have = any || cur.tIn < (c.t < r.tMax ? c.t : r.tMax);
+		}
+	}
+}
+
+}  // namespace
+
+// Returns the wide nodes' number (0: the tree has none) and writes closest hits and in-light flags.
+extern "C" uint32_t wide_check(const PhxBVHNode* nodes, uint32_t numNodes, const OrTri* tris,
+                               const OrRay* rays, uint32_t n, uint32_t topCap, OrHit* hits,
+                               uint8_t* inLight, uint32_t* deepest)
+{
+	const std::vector<WideNode> wide = buildWide(nodes, numNodes, topCap);
+	*deepest = 0;
+	if (wide.empty()) return 0;
+	// The root's slots refer to nodes 1, 2, ... in order.
+	for (uint32_t i = 0; i < 4; i++)
+		if (wide[0].box[i][0] == wide[0].box[i][0] && wide[0].ref[i] != i + 1u) return 0;
+	OrHit unused;
+	for (uint32_t i = 0; i < n; i++) {
+		walk(wide, tris, rays[i], false, hits[i], *deepest);
+		inLight[i] = walk(wide, tris, rays[i], true, unused, *deepest) ? 0 : 1;
+	}
+	return uint32_t(wide.size());
+}
