@@ -32,8 +32,10 @@ phx_status growStage(void*& buf, size_t& have, size_t need)
 	return PHX_OK;
 }
 
-// Device copy of `count` records followed by `padBytes` zero bytes (kernels that read whole
-// 64-B words may touch up to 64 B past the last triangle).
+// Zero bytes after the triangles: kernels read four triangles at a time.
+constexpr size_t kTrianglePad = 3 * sizeof(PhxTriangleVertices);
+
+// Device copy of `count` records followed by `padBytes` zero bytes.
 template <class T>
 phx_status uploadArray(PhxContext* ctx, T*& dst, const T* src, size_t count, size_t& total,
                        size_t padBytes = 0)
@@ -115,35 +117,21 @@ phx_status castCommon(PhxContext* ctx, const PhxRayIn* rays, uint32_t n, void* o
 	return ok();
 }
 
-// Most node visits of incoherent rays happen in the top levels of the tree, which the persistent
-// kernels keep in LDS. The device copy therefore starts with the first kTopCap nodes in
-// breadth-first order (the root stays node 0) followed by the remaining nodes in their original
-// depth-first order; inner-child indices are remapped, leaf (triangle) indices are unchanged, so
-// every traversal decision -- and every hit -- is the same.
+// Largest treelet of a launch shape, in 64-B units.
 constexpr uint32_t kTopCap = 2048;
+// Wide nodes kept in breadth-first order.
+constexpr uint32_t kWideTop = 1024;
 
-std::vector<PhxBVHNode> relayoutTop(const PhxBVHNode* nodes, uint32_t n, uint32_t* topCount)
+// Blocks per CU of a launch shape, by the LDS and registers it stands for: a stack split of `depth`
+// words per lane, the treelet, 1,440 B a wave for handed-over rays, and, for a plan, its batch
+// table; 20 waves per CU for single casts, 16 for a plan. A shape that does not fit is refused.
+uint32_t shapeBlocksPerCU(const PhxPlan* plan, uint32_t block, uint32_t top, uint32_t helpers,
+                          uint32_t depth)
 {
-	std::vector<uint32_t> bfs;
-	bfs.reserve(std::min(n, kTopCap));
-	bfs.push_back(0);
-	for (size_t h = 0; h < bfs.size() && bfs.size() < kTopCap; h++)
-		for (int side = 0; side < 2 && bfs.size() < kTopCap; side++)
-			if (nodes[bfs[h]].iData[2 + side] == 0) bfs.push_back(uint32_t(nodes[bfs[h]].iData[side]));
-	std::vector<uint32_t> newIndex(n, 0xFFFFFFFFu);
-	for (uint32_t i = 0; i < bfs.size(); i++) newIndex[bfs[i]] = i;
-	uint32_t next = uint32_t(bfs.size());
-	for (uint32_t i = 0; i < n; i++)
-		if (newIndex[i] == 0xFFFFFFFFu) newIndex[i] = next++;
-	std::vector<PhxBVHNode> out(n);
-	for (uint32_t i = 0; i < n; i++) {
-		PhxBVHNode nd = nodes[i];
-		for (int side = 0; side < 2; side++)
-			if (nd.iData[2 + side] == 0) nd.iData[side] = int32_t(newIndex[uint32_t(nd.iData[side])]);
-		out[newIndex[i]] = nd;
-	}
-	*topCount = uint32_t(bfs.size());
-	return out;
+	const uint32_t waves = block / 64u, all = waves + helpers;
+	uint32_t lds = waves * (depth + 1u) * 256u + top * 64u + 16u + waves * 1440u;
+	if (plan) lds += (plan->numBatches + 1u) * 4u + (plan->clock ? plan->numBatches * 12u : 0u);
+	return std::min(163840u / lds, (plan ? 16u : 20u) / std::max(all, 1u));
 }
 
 // Triangles as (p0, e1 = p1 - p0, e2 = p2 - p0); p0.w keeps the end marker. The subtractions are
@@ -282,20 +270,15 @@ phx_status phx_create(int device, PhxContext** outCtx)
 		delete ctx;
 		return hipFail(e, "hipStreamCreate");
 	}
-	// Default shape: one block of 512 threads per CU, no treelet, refill at 8 idle lanes -- the
-	// fastest or close to it for incoherent closest-hit and any-hit casts on MI355X;
-	// phx_autotune refines it per scene and ray mix.
-	uint32_t bpc = 0;
-	e = persistentBlocksPerCU(ctx->blockThreads, ctx->topNodes, 0, ctx->ldsDepth, &bpc);
-	if (e == hipSuccess && bpc == 0) e = hipErrorInvalidConfiguration;
+	// Default shape: one block of 512 threads per CU, 512 rays in flight per CU, which is what the
+	// traversal kernels hold at full occupancy; refill at 8 idle lanes.
 	ctx->gridClosest = ctx->numCUs;
 	ctx->gridAnyhit = ctx->numCUs;
-	// The spill area covers every lane the device can hold (2048 per CU).
 	ctx->spillLanes = ctx->numCUs * 2048u;
-	if (e == hipSuccess) e = hipMalloc(&ctx->work, 64);
-	if (e == hipSuccess) e = hipMemset(ctx->work, 0, 64);
+	e = hipMalloc(&ctx->work, kRayCounterWords * 4u);
+	if (e == hipSuccess) e = hipMemset(ctx->work, 0, kRayCounterWords * 4u);
 	if (e == hipSuccess)
-		e = hipMalloc(&ctx->spill, size_t(persistentSpillWords(ctx->spillLanes)) * sizeof(uint32_t));
+		e = hipMalloc(&ctx->spill, size_t(ctx->numCUs) * kRaysPerCu * kSpillWordsPerRay * 4u);
 	if (e != hipSuccess) {
 		hipFree(ctx->work);
 		hipFree(ctx->spill);
@@ -391,8 +374,8 @@ phx_status phx_get_launch_params(PhxContext* ctx, PhxLaunchParams* out)
 	out->refillMin = ctx->refillMin;
 	out->blockThreads = ctx->blockThreads;
 	out->topNodes = ctx->topNodes;
-	uint32_t bpc = 0;
-	persistentBlocksPerCU(ctx->blockThreads, ctx->topNodes, ctx->helperWaves, ctx->ldsDepth, &bpc);
+	const uint32_t bpc =
+		shapeBlocksPerCU(nullptr, ctx->blockThreads, ctx->topNodes, ctx->helperWaves, ctx->ldsDepth);
 	out->residentGridBlocks = ctx->numCUs * bpc;
 	out->helperWaves = ctx->helperWaves;
 	out->raysPerFetch = ctx->window;
@@ -418,14 +401,13 @@ phx_status phx_set_launch_params(PhxContext* ctx, const PhxLaunchParams* p)
 		return fail(PHX_ERR_INVALID_ARGUMENT,
 		            "phx_set_launch_params: %u threads and %u helper waves exceed 1024 threads",
 		            block, helpers);
-	if (!validLdsDepth(depth))
+	if (depth < 4u || depth > 32u)
 		return fail(PHX_ERR_INVALID_ARGUMENT, "phx_set_launch_params: stackLdsEntries %u outside 4..32",
 		            depth);
 	if (window < 8u || window > 4096u)
 		return fail(PHX_ERR_INVALID_ARGUMENT, "phx_set_launch_params: raysPerFetch %u outside 8..4096",
 		            window);
-	uint32_t bpc = 0;
-	persistentBlocksPerCU(block, top, helpers, depth, &bpc);
+	const uint32_t bpc = shapeBlocksPerCU(nullptr, block, top, helpers, depth);
 	if (bpc == 0)
 		return fail(PHX_ERR_INVALID_ARGUMENT,
 		            "phx_set_launch_params: %u threads (+%u helper waves) with a %u-node treelet and "
@@ -549,7 +531,6 @@ static phx_status phx_scene_upload_impl(PhxContext* ctx, const PhxBVHNode* nodes
 	s->numMaterials = numMaterials;
 	s->numLights = numLights;
 	s->depth = depth;
-	s->finiteBounds = 1;
 	for (int k = 0; k < 3; k++) {  // root box: union of node 0's child boxes (fData layout)
 		const float* f = nodes[0].fData;
 		const float lmn[3] = {f[0], f[1], f[2]}, lmx[3] = {f[3], f[4], f[5]};
@@ -557,29 +538,16 @@ static phx_status phx_scene_upload_impl(PhxContext* ctx, const PhxBVHNode* nodes
 		s->rootMin[k] = std::min(lmn[k], rmn[k]);
 		s->rootMax[k] = std::max(lmx[k], rmx[k]);
 	}
-	// Bounds within +-2^126 (false for inf and NaN) keep every b - o of a ray whose origin is in the
-	// same range finite: the condition of the kernels' NaN-free slab test.
-	for (uint32_t i = 0; i < numNodes && s->finiteBounds; i++)
-		for (int k = 0; k < 12; k++)
-			if (!(std::fabs(nodes[i].fData[k]) <= 0x1p126f)) {
-				s->finiteBounds = 0;
-				break;
-			}
-	{
-		std::vector<PhxBVHNode> laid = relayoutTop(nodes, numNodes, &s->topCount);
-		st = uploadArray(ctx, s->nodes, laid.data(), numNodes, s->bytes);
-		if (st == PHX_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
-			st = fail(PHX_ERR_HIP, "phx_scene_upload: node upload failed");
-	}
+	st = uploadArray(ctx, s->nodes, nodes, numNodes, s->bytes);
 	if (st == PHX_OK) {
-		const std::vector<WideNode> wide = buildWide(nodes, numNodes, kTopCap / 2u);
+		const std::vector<WideNode> wide = buildWide(nodes, numNodes, kWideTop);
 		st = uploadArray(ctx, s->wide, wide.data(), wide.size(), s->bytes);
 		if (st == PHX_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
 			st = fail(PHX_ERR_HIP, "phx_scene_upload: wide node upload failed");
 	}
 	if (st == PHX_OK) {
 		std::vector<PhxTriangleVertices> pre = pretransform(triangles, numTriangles);
-		st = uploadArray(ctx, s->tris, pre.data(), numTriangles, s->bytes, 64);
+		st = uploadArray(ctx, s->tris, pre.data(), numTriangles, s->bytes, kTrianglePad);
 		if (st == PHX_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
 			st = fail(PHX_ERR_HIP, "phx_scene_upload: triangle upload failed");
 	}
@@ -815,24 +783,12 @@ phx_status phx_cast_closest_noalloc(PhxContext* ctx, const PhxScene* scene, cons
 	if (!rays || !hits) return fail(PHX_ERR_INVALID_ARGUMENT, "phx_cast_closest_noalloc: NULL");
 	char* base = static_cast<char*>(noAllocScratch(ctx->device));
 	if (!base) return fail(PHX_ERR_HIP, "phx_cast_closest_noalloc: scratch not set up");
-	// The context's shape, with the largest LDS stack split that fits (the fewest spilled
-	// entries) and the grid capped so its spill columns fit the scratch.
+	// The context's shape, with as many rays in flight as the scratch has spill columns for.
 	TraceLaunch L = traceLaunch(ctx, 0, false);
-	uint32_t bpc = 0;
-	if (persistentBlocksPerCU(L.blockThreads, L.topNodes, L.helperWaves, 32, &bpc) ==
-	        hipSuccess && bpc > 0)
-		L.ldsDepth = 32;
-	const uint32_t perLane = kPersistentStackEntries - L.ldsDepth;
-	const uint32_t maxGrid = kNoAllocSpillWords / (perLane * L.blockThreads);
-	if (maxGrid == 0)
-		return fail(PHX_ERR_INVALID_ARGUMENT, "phx_cast_closest_noalloc: a block of %u threads "
-		            "needs more stack spill than the %u-word scratch holds", L.blockThreads,
-		            kNoAllocSpillWords);
-	L.gridBlocks = std::min(L.gridBlocks, maxGrid);
-	L.spillLanes = L.gridBlocks * L.blockThreads;
+	L.spillColumns = std::min(L.spillColumns, kNoAllocSpillWords / kSpillWordsPerRay);
 	L.work = reinterpret_cast<uint32_t*>(base);
 	L.spill = reinterpret_cast<uint32_t*>(base + kNoAllocCounterBytes);
-	PHX_HIP(launchZeroWords(L.work, 2u, ctx->stream), "phx_cast_closest_noalloc");
+	PHX_HIP(launchZeroWords(L.work, kRayCounterWords, ctx->stream), "phx_cast_closest_noalloc");
 	PHX_HIP(launchClosest(view(scene), rays, numRays, hits, L, nullptr, ctx->stream),
 	        "phx_cast_closest_noalloc");
 	if (!(flags & PHX_ASYNC))
@@ -1002,8 +958,6 @@ static phx_status phx_plan_create_impl(PhxContext* ctx, const PhxBatch* batches,
 	std::vector<BatchDesc> descs(numBatches);
 	std::vector<uint32_t> offsets(numBatches + 1, 0);
 	uint64_t total = 0;
-	const PhxScene* firstScene = batches[0].scene;
-	bool oneScene = true;
 	for (uint32_t b = 0; b < numBatches; b++) {
 		const PhxBatch& in = batches[b];
 		st = checkScene(ctx, in.scene);
@@ -1012,15 +966,11 @@ static phx_status phx_plan_create_impl(PhxContext* ctx, const PhxBatch* batches,
 			return fail(PHX_ERR_INVALID_ARGUMENT, "phx_plan_create: batch %u kind %u", b, in.kind);
 		if (in.numRays && (!in.rays || !in.out))
 			return fail(PHX_ERR_INVALID_ARGUMENT, "phx_plan_create: batch %u null pointer", b);
-		descs[b] = BatchDesc{reinterpret_cast<const float4*>(in.scene->nodes),
-		                     reinterpret_cast<const float4*>(in.scene->tris),
-		                     reinterpret_cast<const float4*>(in.rays), in.out, in.numRays, in.kind,
-		                     in.scene->finiteBounds, 0u};
+		descs[b] = batchDesc(in.scene, in.rays, in.out, in.numRays, in.kind);
 		offsets[b] = uint32_t(total);
 		total += in.numRays;
 		if (total > 0x7FFFFFFFull)
 			return fail(PHX_ERR_INVALID_ARGUMENT, "phx_plan_create: more than 2^31 rays in a plan");
-		oneScene = oneScene && in.scene == firstScene;
 	}
 	offsets[numBatches] = uint32_t(total);
 	PhxPlan* p = new (std::nothrow) PhxPlan();
@@ -1028,26 +978,10 @@ static phx_status phx_plan_create_impl(PhxContext* ctx, const PhxBatch* batches,
 	p->ctx = ctx;
 	p->numBatches = numBatches;
 	p->total = uint32_t(total);
-	// A fused launch is throughput bound: default to the resident grid of the fused kernel without
-	// a treelet or helper waves.
+	// A fused launch is throughput bound: as many rays in flight as the device holds.
 	p->launch = traceLaunch(ctx, 0, false);
-	p->launch.topNodes = 0;
-	uint32_t bpc = 0;
-	p->launch.helperWaves = 0;
-	batchBlocksPerCU(p->launch.blockThreads, 0, 0, p->launch.ldsDepth, numBatches,
-	                 (flags & PHX_PLAN_TRACK_COMPLETION) != 0, &bpc);
-	if (bpc == 0) {  // the context's stack split does not fit this kernel: use the default split
-		p->launch.ldsDepth = 16;
-		batchBlocksPerCU(p->launch.blockThreads, 0, 0, 16, numBatches,
-		                 (flags & PHX_PLAN_TRACK_COMPLETION) != 0, &bpc);
-	}
-	p->launch.gridBlocks = std::max(1u, std::min(ctx->numCUs * std::max(bpc, 1u),
-	                                             ctx->spillLanes / p->launch.blockThreads));
+	p->launch.raysInFlight = p->launch.spillColumns;
 	p->hostDescs = descs;
-	if (oneScene) {
-		p->treeletNodes = reinterpret_cast<const float4*>(firstScene->nodes);
-		p->treeletCount = firstScene->topCount;
-	}
 	size_t dummy = 0;
 	st = uploadArray(ctx, p->descs, descs.data(), numBatches, dummy);
 	if (st == PHX_OK) st = uploadArray(ctx, p->offsets, offsets.data(), numBatches + 1, dummy);
@@ -1094,7 +1028,7 @@ phx_status phx_plan_launch(PhxContext* ctx, PhxPlan* plan, uint32_t flags)
 	const TraceLaunch L = plan->launch;
 	auto launch = [&]() {
 		return launchBatches(plan->descs, plan->offsets, plan->numBatches, plan->total, L,
-		                     plan->treeletNodes, plan->treeletCount, plan->clock, ctx->stream);
+		                     plan->clock, ctx->stream);
 	};
 	if (flags & PHX_PLAN_USE_GRAPH) {
 		if (!plan->graphExec) {
@@ -1148,21 +1082,7 @@ phx_status phx_plan_batch_times(PhxContext* ctx, PhxPlan* plan, float* msSinceSt
 
 namespace {
 
-// Checks a launch shape against the device (block size, LDS, spill area); fills `L`.
-// Blocks per CU of the kernel a shape launches: the persistent kernel for single casts, the fused
-// kernel -- with the plan's batch count and completion tracking -- for a plan.
-uint32_t blocksPerCU(const PhxPlan* plan, uint32_t block, uint32_t top, uint32_t helpers,
-                     uint32_t depth)
-{
-	uint32_t bpc = 0;
-	if (plan)
-		batchBlocksPerCU(block, std::min(top, plan->treeletCount), helpers, depth, plan->numBatches,
-		                 plan->clock != nullptr, &bpc);
-	else
-		persistentBlocksPerCU(block, top, helpers, depth, &bpc);
-	return bpc;
-}
-
+// Checks a launch shape (block size, LDS, grid); fills `L`.
 phx_status shapeFor(PhxContext* ctx, const PhxLaunchParams& p, TraceLaunch& L,
                     const PhxPlan* plan)
 {
@@ -1177,11 +1097,11 @@ phx_status shapeFor(PhxContext* ctx, const PhxLaunchParams& p, TraceLaunch& L,
 	if (helpers > 16u || block + 64u * helpers > 1024u)
 		return fail(PHX_ERR_INVALID_ARGUMENT, "launch params: %u threads and %u helper waves",
 		            block, helpers);
-	if (!validLdsDepth(depth))
+	if (depth < 4u || depth > 32u)
 		return fail(PHX_ERR_INVALID_ARGUMENT, "launch params: stackLdsEntries %u outside 4..32", depth);
 	if (window < 8u || window > 4096u)
 		return fail(PHX_ERR_INVALID_ARGUMENT, "launch params: raysPerFetch %u outside 8..4096", window);
-	if (blocksPerCU(plan, block, p.topNodes, helpers, depth) == 0)
+	if (shapeBlocksPerCU(plan, block, p.topNodes, helpers, depth) == 0)
 		return fail(PHX_ERR_INVALID_ARGUMENT, "launch params: shape does not fit a CU");
 	const uint32_t maxGrid = ctx->spillLanes / block;
 	const uint32_t grid = p.gridBlocksClosest;
@@ -1189,16 +1109,10 @@ phx_status shapeFor(PhxContext* ctx, const PhxLaunchParams& p, TraceLaunch& L,
 		return fail(PHX_ERR_INVALID_ARGUMENT, "launch params: grid %u outside 1..%u", grid, maxGrid);
 	if (p.refillMin == 0 || p.refillMin > 64)
 		return fail(PHX_ERR_INVALID_ARGUMENT, "launch params: refillMin %u", p.refillMin);
-	L.blockThreads = block;
-	L.topNodes = p.topNodes;
-	L.helperWaves = helpers;
-	L.ldsDepth = depth;
+	L = traceLaunch(ctx, 0, false);
+	L.raysInFlight = grid * block;
 	L.window = window;
-	L.gridBlocks = grid;
 	L.refillMin = p.refillMin;
-	L.spillLanes = ctx->spillLanes;
-	L.work = ctx->work;
-	L.spill = ctx->spill;
 	return PHX_OK;
 }
 
@@ -1208,29 +1122,19 @@ struct Candidate {
 	float ms = 0.0f;
 };
 
-// Candidate shapes: block 256/512, treelet 0/512/1024 nodes, a quarter, half or all of the
-// resident grid, refill threshold 8 or 32, and for single batches 0 or 4 helper waves -- plus the
-// one-ray-per-lane kernel for single batches.
+// Candidate shapes: a quarter, half or all of the rays in flight that the device holds, refill
+// threshold 8 or 32 -- plus the one-ray-per-lane and packet kernels for single batches.
 std::vector<Candidate> candidates(PhxContext* ctx, const PhxPlan* plan)
 {
 	std::vector<Candidate> out;
-	for (uint32_t helpers : {0u, 4u}) {
-		if (plan && helpers) continue;
-		for (uint32_t block : {256u, 512u})
-			for (uint32_t top : {0u, 512u, 1024u}) {
-				const uint32_t bpc = blocksPerCU(plan, block, top, helpers, 16u);
-				if (bpc == 0) continue;
-				const uint32_t resident = std::min(ctx->numCUs * bpc, ctx->spillLanes / block);
-				for (uint32_t div : {4u, 2u, 1u})
-					for (uint32_t refill : {8u, 32u}) {
-						Candidate c;
-						c.params = PhxLaunchParams{std::max(1u, resident / div),
-						                           std::max(1u, resident / div), refill, block, top,
-						                           resident, helpers, 64u, 16u};
-						if (shapeFor(ctx, c.params, c.launch, plan) == PHX_OK) out.push_back(c);
-					}
-			}
-	}
+	const uint32_t block = 512u, resident = ctx->numCUs * kRaysPerCu / block;
+	for (uint32_t div : {4u, 2u, 1u})
+		for (uint32_t refill : {8u, 32u}) {
+			Candidate c;
+			c.params = PhxLaunchParams{std::max(1u, resident / div), std::max(1u, resident / div),
+			                           refill, block, 0u, resident, 0u, 64u, 16u};
+			if (shapeFor(ctx, c.params, c.launch, plan) == PHX_OK) out.push_back(c);
+		}
 	if (!plan) {
 		Candidate c;
 		c.launch.kernel = TraceKernel::Simple;
@@ -1285,39 +1189,19 @@ phx_status tune(PhxContext* ctx, std::vector<Candidate>& cands, int reps, Launch
 	return ok();
 }
 
-// Second stage for a persistent winner: rays per fetch, then the stack split, one at a time around
-// `best` (coordinate descent; the current value stays a candidate so `best` only improves). A
-// split that lowers the blocks a CU holds caps the grid at the new resident grid.
+// Second stage for a persistent winner: rays per fetch around `best` (the current value stays a
+// candidate, so `best` only improves).
 template <class Launch>
 phx_status refine(PhxContext* ctx, const PhxPlan* plan, int reps, Launch launch, Candidate& best)
 {
 	if (best.launch.kernel != TraceKernel::Persistent) return PHX_OK;
-	for (int stage = 0; stage < 2; stage++) {
-		std::vector<Candidate> cands{best};
-		for (uint32_t v : stage == 0 ? std::vector<uint32_t>{16u, 32u, 64u, 128u, 256u}
-		                             : std::vector<uint32_t>{8u, 16u, 24u, 32u}) {
-			Candidate c = best;
-			if (stage == 0) {
-				if (v == best.params.raysPerFetch) continue;
-				c.params.raysPerFetch = v;
-			} else {
-				if (v == best.params.stackLdsEntries) continue;
-				c.params.stackLdsEntries = v;
-				const uint32_t bpc = blocksPerCU(plan, c.params.blockThreads, c.params.topNodes,
-				                                 c.params.helperWaves, v);
-				const uint32_t resident =
-					std::min(ctx->numCUs * bpc, ctx->spillLanes / c.params.blockThreads);
-				if (resident == 0) continue;
-				c.params.gridBlocksClosest = std::min(c.params.gridBlocksClosest, resident);
-				c.params.gridBlocksAnyhit = std::min(c.params.gridBlocksAnyhit, resident);
-				c.params.residentGridBlocks = resident;
-			}
-			if (shapeFor(ctx, c.params, c.launch, plan) == PHX_OK) cands.push_back(c);
-		}
-		phx_status st = tune(ctx, cands, reps, launch, best);
-		if (st != PHX_OK) return st;
+	std::vector<Candidate> cands{best};
+	for (uint32_t v : {16u, 32u}) {
+		Candidate c = best;
+		c.params.raysPerFetch = v;
+		if (shapeFor(ctx, c.params, c.launch, plan) == PHX_OK) cands.push_back(c);
 	}
-	return PHX_OK;
+	return tune(ctx, cands, reps, launch, best);
 }
 
 }  // namespace
@@ -1352,16 +1236,16 @@ static phx_status phx_autotune_impl(PhxContext* ctx, const PhxScene* scene, cons
 	// Apply: the one-ray-per-lane and packet kernels are selected per call by flag; record the
 	// persistent shape.
 	if (best.launch.kernel == TraceKernel::Persistent) {
-		ctx->blockThreads = best.launch.blockThreads;
-		ctx->topNodes = best.launch.topNodes;
+		ctx->blockThreads = best.params.blockThreads;
+		ctx->topNodes = best.params.topNodes;
 		if (anyhit)
-			ctx->gridAnyhit = best.launch.gridBlocks;
+			ctx->gridAnyhit = best.params.gridBlocksAnyhit;
 		else
-			ctx->gridClosest = best.launch.gridBlocks;
-		ctx->refillMin = best.launch.refillMin;
-		ctx->helperWaves = best.launch.helperWaves;
-		ctx->ldsDepth = best.launch.ldsDepth;
-		ctx->window = best.launch.window;
+			ctx->gridClosest = best.params.gridBlocksClosest;
+		ctx->refillMin = best.params.refillMin;
+		ctx->helperWaves = best.params.helperWaves;
+		ctx->ldsDepth = best.params.stackLdsEntries;
+		ctx->window = best.params.raysPerFetch;
 	}
 	if (chosen) {
 		*chosen = best.params;
@@ -1411,7 +1295,7 @@ static phx_status phx_plan_autotune_impl(PhxContext* ctx, PhxPlan* plan, PhxLaun
 	// Timed as the plan launches: with its completion tracking, whose LDS can change residency.
 	auto run = [&](const TraceLaunch& L) {
 		return launchBatches(plan->descs, plan->offsets, plan->numBatches, plan->total, L,
-		                     plan->treeletNodes, plan->treeletCount, plan->clock, ctx->stream);
+		                     plan->clock, ctx->stream);
 	};
 	st = tune(ctx, cands, 3, run, best);
 	if (st == PHX_OK) st = refine(ctx, plan, 5, run, best);

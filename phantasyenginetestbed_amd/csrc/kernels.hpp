@@ -18,8 +18,6 @@ struct SceneView {
 	uint32_t numNodes;
 	uint32_t numTris;
 	const WideNode* wide;   // four-wide nodes (wide_nodes.hpp), or null: binary traversal only
-	uint32_t finiteBounds;  // every node bound within +-2^126 (enables the NaN-free slab path)
-	uint32_t topCount;      // nodes [0, topCount) are the top levels in breadth-first order
 };
 
 // Material textures of a scene: one device arena holding the linearisation table, the
@@ -38,51 +36,41 @@ struct TexSet {
 	uint32_t count = 0;
 };
 
-enum class TraceKernel { Persistent, Simple, Packet };
+// Persistent: four lanes per ray. Lane: also persistent, one ray per lane, the last ones four lanes
+// each. Simple: one ray per lane, no persistence. Packet: 64 rays walk together.
+enum class TraceKernel { Persistent, Lane, Simple, Packet };
 
-// Launch parameters of the traversal kernels. `work` points at two zeroed uint32 words owned by
-// the launching stream (the persistent kernels leave them zeroed); `spill` holds
-// persistentSpillWords(gridBlocks) words.
+// Words of a launch's ray counters, and words of stack spill per ray in flight.
+constexpr uint32_t kRayCounterWords = 1024;
+constexpr uint32_t kSpillWordsPerRay = 100;
+// Most rays in flight per CU: 16 waves of 64 rays, one per lane (28 of 16 rays, four lanes each).
+constexpr uint32_t kRaysPerCu = 1024;
+
+// Launch parameters of the traversal kernels. `work` points at kRayCounterWords zeroed words owned
+// by the launching stream (the persistent kernels leave them zeroed); `spill` holds
+// kSpillWordsPerRay words for each of spillColumns rays.
 struct TraceLaunch {
 	TraceKernel kernel = TraceKernel::Persistent;
-	uint32_t gridBlocks = 0;     // persistent grid
-	uint32_t blockThreads = 256; // persistent block size (multiple of 64, <= 1024)
-	uint32_t topNodes = 0;       // treelet nodes held in LDS (capped by the scene's topCount)
+	uint32_t raysInFlight = 0;
+	uint32_t cus = 0;
+	uint32_t spillColumns = 0;
 	uint32_t refillMin = 8;      // refill a wave once this many of its lanes are idle
-	uint32_t spillLanes = 0;     // lanes the spill area is sized for
-	uint32_t helperWaves = 0;    // extra waves per block that only trace offered rays solo
-	uint32_t ldsDepth = 16;      // stack entries per lane held in LDS (the rest spill to HBM)
-	uint32_t window = 64;        // rays a wave claims per fetch from the shared counter
+	uint32_t window = 64;        // most rays a wave claims per fetch from a ray counter
 	uint32_t* work = nullptr;
 	uint32_t* spill = nullptr;
 };
 
-// Words of the stack spill area for `lanes` resident lanes.
-uint32_t persistentSpillWords(uint32_t lanes);
-// Stack entries per lane of the persistent kernels (LDS part + spill part).
-constexpr uint32_t kPersistentStackEntries = 72;
-
 // Scratch of the allocation-free closest-hit cast: a static device array per GPU holding the
-// persistent launch's ray counters (first kNoAllocCounterBytes) and its stack spill area
-// (kNoAllocSpillWords words: 40 spilled entries for 131,072 lanes, 20 MiB).
-constexpr size_t kNoAllocCounterBytes = 256;
-constexpr uint32_t kNoAllocSpillWords = 40u * 131072u;
+// launch's ray counters (first kNoAllocCounterBytes) and its stack spill area (37.5 MiB: 98,304 rays).
+constexpr size_t kNoAllocCounterBytes = kRayCounterWords * 4u;
+constexpr uint32_t kNoAllocSpillWords = 98304u * kSpillWordsPerRay;
 constexpr int kNoAllocMaxDevices = 64;
 // Looks up the scratch array's address on `device` (which must be current) once; phx_create
 // calls it. noAllocScratch returns the address found (nullptr before).
 hipError_t noAllocScratchInit(int device);
 void* noAllocScratch(int device);
-// Zeroes n <= 64 words with a one-block kernel (graph-capturable, allocates nothing).
+// Zeroes n <= 1024 words with a one-block kernel (graph-capturable, allocates nothing).
 hipError_t launchZeroWords(uint32_t* p, uint32_t n, hipStream_t stream);
-// Dynamic LDS bytes of a persistent block.
-uint32_t persistentLdsBytes(uint32_t blockThreads, uint32_t topNodes, uint32_t ldsDepth);
-// True if `depth` LDS stack entries per lane is a supported split (4..32).
-bool validLdsDepth(uint32_t depth);
-// Resident persistent blocks per CU for a block size, treelet size, helper waves and LDS stack
-// depth (0 if it does not fit).
-hipError_t persistentBlocksPerCU(uint32_t blockThreads, uint32_t topNodes, uint32_t helperWaves,
-                                 uint32_t ldsDepth, uint32_t* blocks);
-
 // One instance of a two-level scene on the device: its SBVH (the mesh scene's node and
 // pre-transformed triangle arrays) and the world-to-object affine transform, rows (A | b).
 struct DevInstance {
@@ -132,14 +120,13 @@ hipError_t launchAnyHit(const SceneView& s, const PhxRayIn* rays, uint32_t n, ui
 
 // Device descriptor of one batch of a fused launch (48 B).
 struct BatchDesc {
+	const float4* wide;       // the scene's wide nodes, or `tris` if it has none
 	const float4* nodes;
 	const float4* tris;       // pre-transformed triangles
 	const float4* rays;
 	void* out;                // PhxRayHit* (closest) or uint8_t* (any hit)
 	uint32_t count;
 	uint32_t kind;            // 0 closest hit, 1 any hit
-	uint32_t finiteBounds;
-	uint32_t pad;
 };
 static_assert(sizeof(BatchDesc) == 48, "BatchDesc layout");
 
@@ -153,19 +140,11 @@ struct BatchClock {
 
 constexpr uint32_t kMaxFusedBatches = 1024;
 
-uint32_t batchLdsBytes(uint32_t blockThreads, uint32_t topNodes, uint32_t numBatches,
-                       bool tracked, uint32_t ldsDepth);
-// Resident blocks per CU of the fused kernel for a shape and batch count, with or without
-// completion tracking (0 if it does not fit).
-hipError_t batchBlocksPerCU(uint32_t blockThreads, uint32_t topNodes, uint32_t helperWaves,
-                            uint32_t ldsDepth, uint32_t numBatches, bool tracked,
-                            uint32_t* blocks);
-
 // One persistent launch over `numBatches` batches; offsets[b] = first ray of batch b in the fused
 // index space, offsets[numBatches] = total. `clock` may be null (no completion tracking).
 hipError_t launchBatches(const BatchDesc* descs, const uint32_t* offsets, uint32_t numBatches,
-                         uint32_t total, const TraceLaunch& launch, const float4* treeletNodes,
-                         uint32_t treeletCount, BatchClock* clock, hipStream_t stream);
+                         uint32_t total, const TraceLaunch& launch, BatchClock* clock,
+                         hipStream_t stream);
 
 // Per-frame values of the wavefront frame. Its kernels read them from device memory, so the
 // frame's launches are the same for every frame and can be captured once and replayed as a

@@ -73,7 +73,7 @@ struct PhxContext {
 	uint32_t helperWaves = 0;
 	uint32_t ldsDepth = 16;   // stack entries per lane kept in LDS
 	uint32_t window = 64;     // rays per fetch
-	uint32_t spillLanes = 0;
+	uint32_t spillLanes = 0;  // lanes the device can hold: the limit of grid x block
 	// Staging buffers for calls that pass host pointers, grown on demand.
 	void* stageIn = nullptr;
 	size_t stageInBytes = 0;
@@ -94,8 +94,6 @@ struct PhxPlan {
 	phx::BatchDesc* descs = nullptr;
 	uint32_t* offsets = nullptr;
 	phx::BatchClock* clock = nullptr;
-	const float4* treeletNodes = nullptr;
-	uint32_t treeletCount = 0;
 	hipGraph_t graph = nullptr;
 	hipGraphExec_t graphExec = nullptr;
 	std::vector<phx::BatchDesc> hostDescs;
@@ -112,9 +110,7 @@ struct PhxScene {
 	PhxSphereLight* lights = nullptr;
 	uint32_t numNodes = 0, numTris = 0, numMaterials = 0, numLights = 0;
 	uint32_t depth = 0;
-	uint32_t finiteBounds = 0;
 	float rootMin[3] = {0, 0, 0}, rootMax[3] = {0, 0, 0};  // union of the root's child boxes
-	uint32_t topCount = 0;
 	size_t bytes = 0;
 	void* texArena = nullptr;  // material textures (phx_scene_set_textures)
 	size_t texBytes = 0;
@@ -167,7 +163,17 @@ void dropContext(PhxContext* ctx);
 
 inline SceneView view(const PhxScene* s)
 {
-	return SceneView{s->nodes, s->tris, s->numNodes, s->numTris, s->wide, s->finiteBounds, s->topCount};
+	return SceneView{s->nodes, s->tris, s->numNodes, s->numTris, s->wide};
+}
+
+// One batch of a fused launch on scene `s`.
+inline BatchDesc batchDesc(const PhxScene* s, const PhxRayIn* rays, void* out, uint32_t count,
+                           uint32_t kind)
+{
+	const float4* tris = reinterpret_cast<const float4*>(s->tris);
+	return BatchDesc{s->wide ? reinterpret_cast<const float4*>(s->wide) : tris,
+	                 reinterpret_cast<const float4*>(s->nodes), tris,
+	                 reinterpret_cast<const float4*>(rays), out, count, kind};
 }
 
 inline TraceLaunch traceLaunch(const PhxContext* ctx, uint32_t flags, bool anyhit)
@@ -176,13 +182,10 @@ inline TraceLaunch traceLaunch(const PhxContext* ctx, uint32_t flags, bool anyhi
 	L.kernel = (flags & PHX_KERNEL_ONE_RAY_PER_LANE) ? TraceKernel::Simple
 	           : (flags & PHX_KERNEL_PACKET)        ? TraceKernel::Packet
 	                                                : TraceKernel::Persistent;
-	L.gridBlocks = anyhit ? ctx->gridAnyhit : ctx->gridClosest;
-	L.blockThreads = ctx->blockThreads;
-	L.topNodes = ctx->topNodes;
+	L.raysInFlight = (anyhit ? ctx->gridAnyhit : ctx->gridClosest) * ctx->blockThreads;
+	L.cus = ctx->numCUs;
+	L.spillColumns = ctx->numCUs * kRaysPerCu;
 	L.refillMin = ctx->refillMin;
-	L.spillLanes = ctx->spillLanes;
-	L.helperWaves = ctx->helperWaves;
-	L.ldsDepth = ctx->ldsDepth;
 	L.window = ctx->window;
 	L.work = ctx->work;
 	L.spill = ctx->spill;

@@ -209,11 +209,7 @@ hipError_t launchSlot(PhxServer* s, Slot& slot)
 		if (!(r->req.flags & PHX_MEM_DEVICE) && r->req.numRays)
 			e = hipMemcpyAsync(const_cast<PhxRayIn*>(r->devRays), r->req.rays, r->rayBytes,
 			                   hipMemcpyHostToDevice, slot.stream);
-		const PhxScene* sc = r->req.scene;
-		slot.hostDescs[b] = BatchDesc{reinterpret_cast<const float4*>(sc->nodes),
-		                              reinterpret_cast<const float4*>(sc->tris),
-		                              reinterpret_cast<const float4*>(r->devRays), r->devOut,
-		                              r->req.numRays, r->req.kind, sc->finiteBounds, 0u};
+		slot.hostDescs[b] = batchDesc(r->req.scene, r->devRays, r->devOut, r->req.numRays, r->req.kind);
 		slot.hostOffsets[b] = off;
 		off += r->req.numRays;
 	}
@@ -241,8 +237,7 @@ hipError_t launchSlot(PhxServer* s, Slot& slot)
 		L.work = slot.work;
 		L.spill = slot.spill;
 		if (e == hipSuccess)
-			e = launchBatches(slot.descs, slot.offsets, nb, off, L, nullptr, 0u, nullptr,
-			                  slot.stream);
+			e = launchBatches(slot.descs, slot.offsets, nb, off, L, nullptr, slot.stream);
 	}
 	for (uint32_t b = 0; b < nb && e == hipSuccess; b++) {
 		Request* r = slot.reqs[b];
@@ -367,18 +362,10 @@ static phx_status phx_server_create_impl(PhxContext* ctx, uint64_t budgetBytes, 
 	s->flags = flags;
 	s->budget = budgetBytes;
 	s->shape = traceLaunch(ctx, 0, false);
-	// Continuous batching keeps every block busy: the resident grid of lane-mode blocks of the
-	// fused kernel at its largest batch count, no treelet, no helper waves (which would cut the
-	// blocks a CU holds), the default stack split and rays per fetch (a context's tuned values
-	// are for its single casts).
-	s->shape.topNodes = 0;
-	s->shape.helperWaves = 0;
-	s->shape.ldsDepth = 16;
+	// Continuous batching keeps the device full: as many rays in flight as it holds, and the default
+	// rays per fetch (a context's tuned values are for its single casts).
+	s->shape.raysInFlight = s->shape.spillColumns;
 	s->shape.window = 64;
-	uint32_t bpc = 0;
-	batchBlocksPerCU(s->shape.blockThreads, 0, 0, 16, kMaxFusedBatches, false, &bpc);
-	s->shape.gridBlocks = std::max(1u, ctx->numCUs * bpc);
-	s->shape.spillLanes = s->shape.gridBlocks * s->shape.blockThreads;
 	s->slots.resize(numSlots);
 	hipError_t e = hipSuccess;
 	// Slot 0 launches on the context's stream, the others on streams of their own. HIP maps a
@@ -393,11 +380,11 @@ static phx_status phx_server_create_impl(PhxContext* ctx, uint64_t budgetBytes, 
 			e = hipStreamCreateWithFlags(&slot.stream, hipStreamNonBlocking);
 			slot.ownStream = e == hipSuccess;
 		}
-		if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&slot.work), 64);
-		if (e == hipSuccess) e = hipMemset(slot.work, 0, 64);
+		if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&slot.work), kRayCounterWords * 4u);
+		if (e == hipSuccess) e = hipMemset(slot.work, 0, kRayCounterWords * 4u);
 		if (e == hipSuccess)
 			e = hipMalloc(reinterpret_cast<void**>(&slot.spill),
-			              size_t(persistentSpillWords(s->shape.spillLanes)) * 4u);
+			              size_t(s->shape.spillColumns) * kSpillWordsPerRay * 4u);
 		if (e == hipSuccess)
 			e = hipMalloc(reinterpret_cast<void**>(&slot.descs), sizeof(BatchDesc) * kMaxFusedBatches);
 		if (e == hipSuccess)

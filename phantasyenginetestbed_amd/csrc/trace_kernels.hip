@@ -28,18 +28,24 @@ constexpr int kBlock = 256;
 // Address-space views: records are loaded through pointers the compiler knows to be global (or
 // LDS), so the loads are global_load / ds_read rather than flat loads, whose latency is higher
 // and which wait on both the vector-memory and LDS counters.
+typedef uint32_t U32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t U32x4 __attribute__((ext_vector_type(4)));
 #if defined(__HIP_DEVICE_COMPILE__)
 typedef const float4 __attribute__((address_space(1))) GlobalF4;
-typedef const float __attribute__((address_space(1))) GlobalF1;
-typedef const float4 __attribute__((address_space(3))) LdsF4;
+typedef U32x2 __attribute__((address_space(1))) GlobalU2;
+typedef U32x4 __attribute__((address_space(1))) GlobalU4;
+typedef uint8_t __attribute__((address_space(1))) GlobalU8;
+typedef U32x2 __attribute__((address_space(3))) LdsU2;
+typedef uint32_t __attribute__((address_space(3))) LdsU1;
 #else  // the host pass only needs the declarations to parse
 typedef const float4 GlobalF4;
-typedef const float GlobalF1;
-typedef const float4 LdsF4;
+typedef U32x2 GlobalU2;
+typedef U32x4 GlobalU4;
+typedef uint8_t GlobalU8;
+typedef U32x2 LdsU2;
+typedef uint32_t LdsU1;
 #endif
 __device__ __forceinline__ GlobalF4* as_global(const float4* p) { return (GlobalF4*)(p); }
-__device__ __forceinline__ GlobalF1* as_global(const float* p) { return (GlobalF1*)(p); }
-__device__ __forceinline__ LdsF4* as_lds(const float4* p) { return (LdsF4*)(p); }
 
 struct NodeWords {
 	float4 w0, w1, w2;
@@ -118,6 +124,9 @@ __device__ __forceinline__ void add_counts(unsigned long long* counters, const C
 // Deepest castRay stack for a tree of depth <= 64 (enforced at upload): one pending entry per
 // level plus the two children of the node being expanded.
 constexpr int kSimpleStack = 72;
+// Words that hold such a stack, or a wide walk's pending entries.
+constexpr int kStackWords =
+	kSimpleStack > 2 * int(kWideMaxPending) ? kSimpleStack : 2 * int(kWideMaxPending);
 
 // castRay<144> of one ray (BVHTraversal.hpp:37-128) into `c` (which holds the miss result on
 // entry): pop, decide both children, left first; a visited leaf is tested at once, a visited
@@ -126,12 +135,12 @@ constexpr int kSimpleStack = 72;
 // 4-B word per lane per row, so a wave's accesses are conflict-free), the rest in private memory. A
 // pop is on the path to the next node's load, and an LDS pop returns sooner than a private (scratch)
 // one. Binary traversals keep 4-B entries (put / get), wide ones 8-B entries of a reference and its
-// entry distance (put2 / get2): 72 of the former take as many words as kWideMaxPending of the latter.
+// entry distance (put2 / get2).
 template <int kLds>
 struct ColumnStack {
-	static_assert(kLds % 2 == 0 && kSimpleStack == 2 * int(kWideMaxPending), "entry sizes");
+	static_assert(kLds % 2 == 0, "an 8-B entry is in one place");
 	uint32_t* col;
-	uint32_t deep[kSimpleStack - kLds];
+	uint32_t deep[kStackWords - kLds];
 	__device__ __forceinline__ void put(int e, uint32_t v)
 	{
 		if (e < kLds)
@@ -275,21 +284,15 @@ __device__ __forceinline__ bool anyhit_one(const float4* __restrict__ nodes,
 // 9.8 wide node visits where it takes 21.6 binary ones (random triangles: 32 for 65).
 
 struct WideWords {
-	float4 w0, w1, w2, w3, w4, w5;  // boxes of slots 0-3, (min.xyz, max.xyz) each
-	uint4 ref;
+	float4 w[8];  // slot i: (min.xyz, reference) in word 2i, (max.xyz, -) in word 2i + 1
 };
 
 __device__ __forceinline__ WideWords load_wide(const float4* __restrict__ wide, uint32_t i)
 {
 	WideWords n;
 	const float4* p = wide + 8u * size_t(i);
-	n.w0 = p[0];
-	n.w1 = p[1];
-	n.w2 = p[2];
-	n.w3 = p[3];
-	n.w4 = p[4];
-	n.w5 = p[5];
-	n.ref = reinterpret_cast<const uint4*>(p)[6];
+#pragma unroll
+	for (int k = 0; k < 8; k++) n.w[k] = p[k];
 	return n;
 }
 
@@ -300,19 +303,20 @@ struct WideVisit {
 	bool pass[4];
 };
 
-__device__ __forceinline__ WideVisit decide_wide(const dev::Ray& r, const float4 w0, const float4 w1,
-                                                 const float4 w2, const float4 w3, const float4 w4,
-                                                 const float4 w5, float tCurrMax)
+__device__ __forceinline__ bool decide_slot(const dev::Ray& r, const float4 lo, const float4 hi,
+                                            float tCurrMax, float& tIn)
+{
+	float tOut;
+	dev::slab_fast(r, lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, tIn, tOut);
+	return (tOut >= tIn) && tOut > r.tMin && tIn < tCurrMax;
+}
+
+__device__ __forceinline__ WideVisit decide_wide(const dev::Ray& r, const WideWords& n, float tCurrMax)
 {
 	WideVisit v;
-	float out[4];
-	dev::slab_fast(r, w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, v.tIn[0], out[0]);
-	dev::slab_fast(r, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w, v.tIn[1], out[1]);
-	dev::slab_fast(r, w3.x, w3.y, w3.z, w3.w, w4.x, w4.y, v.tIn[2], out[2]);
-	dev::slab_fast(r, w4.z, w4.w, w5.x, w5.y, w5.z, w5.w, v.tIn[3], out[3]);
 #pragma unroll
 	for (int i = 0; i < 4; i++)
-		v.pass[i] = (out[i] >= v.tIn[i]) && out[i] > r.tMin && v.tIn[i] < tCurrMax;
+		v.pass[i] = decide_slot(r, n.w[2 * i], n.w[2 * i + 1], tCurrMax, v.tIn[i]);
 	return v;
 }
 
@@ -371,8 +375,9 @@ __device__ __forceinline__ bool wide_one(const float4* __restrict__ wide,
 		float lim = kAnyHit ? r.tMax : dev::min_first(r.tMax, c.t);
 		if (!(ref & kWideLeaf)) {
 			const WideWords n = load_wide(wide, ref);
-			const WideVisit v = decide_wide(r, n.w0, n.w1, n.w2, n.w3, n.w4, n.w5, lim);
-			const uint32_t refs[4] = {n.ref.x, n.ref.y, n.ref.z, n.ref.w};
+			const WideVisit v = decide_wide(r, n, lim);
+			const uint32_t refs[4] = {__float_as_uint(n.w[0].w), __float_as_uint(n.w[2].w),
+			                          __float_as_uint(n.w[4].w), __float_as_uint(n.w[6].w)};
 			// Last slot first, so that the first passing slot is what remains to be taken. A leaf
 			// pair stays one only if both leaves pass.
 			have = false;
@@ -671,158 +676,15 @@ __global__ __launch_bounds__(kBlock) void k_trace_instances(
 	}
 }
 
-// ---- persistent wavefronts ----------------------------------------------------------------------
-//
-// A fixed grid of waves pulls rays from a shared counter, one atomic per wavefront for a window
-// of `window` rays (rays per fetch, a launch parameter). Every iteration, lanes without a ray are
-// refilled from the window when at least `refillMin` of the wave's 64 lanes are idle (always when
-// all are). The last wave to finish resets the counter, so every launch starts from zero without a
-// memset.
-//
-// LDS (dynamic) holds, per block:
-//   - castRay's pending stack, [wave][entry][lane] (one 4-B column per lane, so each push/pop is a
-//     conflict-free 256-B row), `depth` entries deep (the stack split, a launch parameter) plus
-//     one row that lanes without a push write to; deeper entries spill to a global array laid out
-//     [entry][lane] (coalesced). Trees are at most 64 levels deep (checked at upload), so the
-//     pending stack never exceeds kPersistentStack entries;
-//   - the top treelet: nodes [0, topCount) of the device node array, which the upload lays out in
-//     breadth-first order so they are the top levels of the tree -- where most node visits of
-//     incoherent rays happen. They are copied once per block and read from LDS afterwards.
-
-constexpr int kMinLdsDepth = 4;    // smallest stack split; the spill area is sized for it
-constexpr int kMaxLdsDepth = 32;
-constexpr int kPersistentStack = 72;
-constexpr int kMaxBlock = 1024;
-
-struct WaveQueue {
-	uint32_t base = 0;   // next unclaimed ray of this wave's window
-	uint32_t left = 0;   // rays left in the window
-	uint32_t start = 0;  // first ray of the window
-	bool exhausted = false;
-};
-
-// Assigns ray indices to the idle lanes of the wave (`idle` = ballot of idle lanes). Returns the
-// lane's new ray index, or kInvalid. Wave-uniform state lives in `q`.
-__device__ __forceinline__ uint32_t refill(WaveQueue& q, uint64_t idle, uint32_t* work,
-                                           uint32_t n, bool isIdle, uint32_t window)
-{
-	const uint32_t need = uint32_t(__popcll(idle));
-	const uint32_t take1 = need < q.left ? need : q.left;
-	const uint32_t base1 = q.base;
-	q.base += take1;
-	q.left -= take1;
-	uint32_t take2 = 0, base2 = 0;
-	if (need > take1) {
-		const int leader = __ffsll((unsigned long long)idle) - 1;
-		uint32_t b = 0;
-		if (int(__lane_id()) == leader) b = atomicAdd(work, window);
-		b = __shfl(b, leader);
-		if (b >= n) {
-			q.exhausted = true;
-			q.left = 0;
-		} else {
-			const uint32_t avail = (n - b) < window ? (n - b) : window;
-			take2 = (need - take1) < avail ? (need - take1) : avail;
-			base2 = b;
-			q.start = b;
-			q.base = b + take2;
-			q.left = avail - take2;
-		}
-	}
-	if (!isIdle) return kInvalid;
-	const uint32_t rank = uint32_t(__popcll(idle & __lanemask_lt()));
-	if (rank < take1) return base1 + rank;
-	if (rank < take1 + take2) return base2 + (rank - take1);
-	return kInvalid;
-}
-
-// Called by every wave as it exits: the last one resets the shared counters to zero.
-__device__ __forceinline__ void retire_wave(uint32_t* work)
-{
-	if (__lane_id() == 0) {
-		__threadfence();
-		const uint32_t totalWaves = gridDim.x * (blockDim.x / 64u);
-		if (atomicAdd(&work[1], 1u) == totalWaves - 1u) {
-			atomicExch(&work[0], 0u);
-			atomicExch(&work[1], 0u);
-		}
-	}
-}
-
-struct LaneStack {
-	uint32_t* lds;    // this wave's [entry][lane] block: depth + 1 rows
-	uint32_t* spill;  // this lane's spill column
-	uint32_t stride;  // spill row stride (lanes in the grid)
-	uint32_t lane;
-	int depth;        // entries kept in LDS
-	int sp;
-
-	// Pushes v if doPush. Lanes that do not push (or whose entry spills) store to the extra row, so
-	// the LDS store needs no branch; only a spilling entry takes one.
-	__device__ __forceinline__ void push_if(bool doPush, uint32_t v)
-	{
-		const bool toLds = doPush && sp < depth;
-		lds[(toLds ? sp : depth) * 64 + int(lane)] = v;
-		if (doPush && sp >= depth && sp < kPersistentStack)
-			spill[size_t(sp - depth) * stride] = v;
-		sp += doPush ? 1 : 0;
-	}
-	// Pops if doPop (the value is meaningless otherwise): every lane reads one LDS word -- lanes
-	// that do not pop, or whose entry spilled, read the extra row -- and only a spilled entry
-	// takes a branch.
-	__device__ __forceinline__ uint32_t pop_if(bool doPop)
-	{
-		sp -= doPop ? 1 : 0;
-		uint32_t v = lds[(doPop && sp < depth ? sp : depth) * 64 + int(lane)];
-		if (doPop && sp >= depth)
-			v = sp < kPersistentStack ? spill[size_t(sp - depth) * stride] : 0u;
-		return v;
-	}
-};
-
-// Visit decision of both children of a node (BVHTraversal.hpp:59-64; any-hit: tCurrMax = tMax).
-__device__ __forceinline__ void decide(const dev::Ray& r, bool fastSlab, const NodeWords& nd,
-                                       float tCurrMax, bool& visitL, bool& visitR)
+// Visit decision of both children of a binary node (BVHTraversal.hpp:59-64; any-hit: tMax).
+__device__ __forceinline__ void decide(const dev::Ray& r, const NodeWords& nd, float tCurrMax,
+                                       bool& visitL, bool& visitR)
 {
 	float inL, outL, inR, outR;
-	if (fastSlab) {
-		dev::slab_fast(r, nd.w0.x, nd.w0.y, nd.w0.z, nd.w0.w, nd.w1.x, nd.w1.y, inL, outL);
-		dev::slab_fast(r, nd.w1.z, nd.w1.w, nd.w2.x, nd.w2.y, nd.w2.z, nd.w2.w, inR, outR);
-	} else {
-		dev::slab(r, nd.w0.x, nd.w0.y, nd.w0.z, nd.w0.w, nd.w1.x, nd.w1.y, inL, outL);
-		dev::slab(r, nd.w1.z, nd.w1.w, nd.w2.x, nd.w2.y, nd.w2.z, nd.w2.w, inR, outR);
-	}
+	dev::slab(r, nd.w0.x, nd.w0.y, nd.w0.z, nd.w0.w, nd.w1.x, nd.w1.y, inL, outL);
+	dev::slab(r, nd.w1.z, nd.w1.w, nd.w2.x, nd.w2.y, nd.w2.z, nd.w2.w, inR, outR);
 	visitL = (outL >= inL) && outL > r.tMin && inL < tCurrMax;
 	visitR = (outR >= inR) && outR > r.tMin && inR < tCurrMax;
-}
-
-// A triangle step tests up to kTriBatch consecutive triangles of the current leaf range, all
-// loaded by the same step, in castRay's order (BVHTraversal.hpp:78-93). Leaves on the paths of
-// costly incoherent rays hold about five triangles, so this shortens their chains of dependent
-// steps. The words of a second triangle past a leaf's last one lie in the next triangle or in the
-// 64 B of padding after the array.
-constexpr uint32_t kTriBatch = 2;
-
-// Per-lane traversal state of the persistent kernels. Every iteration a lane does one unit of
-// work in castRay's per-ray order: expand a node (decide both children, queue the triangles of
-// visited leaf children -- left, then right -- and pick the next node), or test up to kTriBatch
-// queued triangles. Nodes are expanded only once the queued triangles are done, so each box
-// decision sees the closest.t that castRay would see.
-struct LaneTrace {
-	uint32_t triCur, triEnd;    // triangles being tested
-	uint32_t pendCur, pendEnd;  // right-leaf triangles queued behind them
-	int32_t next;               // node castRay pops next, or -1
-};
-
-__host__ __device__ __forceinline__ uint32_t handoff_bytes(uint32_t blockThreads);
-
-// LDS bytes of a persistent launch: the stacks of every wave, the treelet, the handoff area.
-__host__ __device__ __forceinline__ uint32_t persistent_lds_bytes(uint32_t blockThreads,
-                                                                  uint32_t topCount,
-                                                                  uint32_t depth)
-{
-	return (blockThreads / 64u) * (depth + 1u) * 64u * 4u + topCount * 64u +
-	       handoff_bytes(blockThreads);
 }
 
 // ---- packet traversal (coherent rays) ------------------------------------------------------------
@@ -895,7 +757,7 @@ __device__ __forceinline__ void packet_binary(const float4* __restrict__ nodes,
 		const int32_t rCnt = __builtin_amdgcn_readfirstlane(nd.w3.w);
 		const float tCurrMax = kAnyHit ? r.tMax : dev::min_first(r.tMax, c.t);
 		bool visitL, visitR;
-		decide(r, false, nd, tCurrMax, visitL, visitR);
+		decide(r, nd, tCurrMax, visitL, visitR);
 		visitL = visitL && in;
 		visitR = visitR && in;
 		uint64_t pushL = 0ull, pushR = 0ull;
@@ -973,9 +835,10 @@ __device__ __forceinline__ void packet_wide(const float4* __restrict__ wide,
 		const bool in = ((mask >> lane) & 1ull) != 0;
 		const WideWords n = load_wide(wide, cur);
 		const float lim = kAnyHit ? r.tMax : dev::min_first(r.tMax, c.t);
-		WideVisit v = decide_wide(r, n.w0, n.w1, n.w2, n.w3, n.w4, n.w5, lim);
-		const uint32_t refs[4] = {uniform(n.ref.x), uniform(n.ref.y), uniform(n.ref.z),
-		                          uniform(n.ref.w)};
+		WideVisit v = decide_wide(r, n, lim);
+		const uint32_t refs[4] = {
+			uniform(__float_as_uint(n.w[0].w)), uniform(__float_as_uint(n.w[2].w)),
+			uniform(__float_as_uint(n.w[4].w)), uniform(__float_as_uint(n.w[6].w))};
 		uint64_t m[4];
 #pragma unroll
 		for (int i = 0; i < 4; i++) {
@@ -1038,10 +901,10 @@ __device__ __forceinline__ void packet_wide(const float4* __restrict__ wide,
 			}
 			auto decided = [&](int e, uint64_t who) {
 				const uint32_t at = lane_get(sB, e);
-				const float* b = reinterpret_cast<const float*>(wide + 8u * size_t(at >> 2)) + 6u * (at & 3u);
-				float tIn, tOut;
-				dev::slab_fast(r, b[0], b[1], b[2], b[3], b[4], b[5], tIn, tOut);
-				return ((who >> lane) & 1ull) != 0 && tIn < dev::min_first(r.tMax, c.t);
+				const float4* b = wide + 2u * size_t(at);
+				float tIn;
+				const bool pass = decide_slot(r, b[0], b[1], dev::min_first(r.tMax, c.t), tIn);
+				return ((who >> lane) & 1ull) != 0 && pass;
 			};
 			const bool on = decided(sp, me);
 			bool on2 = false;
@@ -1088,771 +951,6 @@ __global__ __launch_bounds__(kPacketBlock) void k_packet(const float4* __restric
 	}
 }
 
-// ---- software-pipelined persistent loop -------------------------------------------------------
-//
-// Each iteration of a lane consumes the record it loaded in the previous iteration and issues the
-// load of the next one as soon as its address is known: right after a node's expansion, and for
-// a triangle step before the triangles are tested, so the test arithmetic runs while the next
-// record is in flight. The loop body is instantiated twice with the two record buffers swapped
-// (A -> B, then B -> A), so no record is ever copied between registers -- a copy would wait for
-// the load it copies. A new ray is loaded together with the root node and its first iteration
-// expands the root, so a ray costs one iteration less than a node of its own would.
-
-constexpr uint32_t kRecIdle = 0, kRecRay = 1, kRecTri = 2, kRecNode = 3;
-
-// s_waitcnt immediate (gfx9 encoding) that waits for vmcnt = 0 only: expcnt 7 and lgkmcnt 15 are
-// the "no wait" values of those fields.
-constexpr int kWaitVmcntZero = (0x7 << 4) | (0xF << 8);
-
-// One record's six 16-B words: a node (words 0-3), a triangle pair (p0, e1, e2 of the first
-// triangle, then of the second), or the root node (words 0-3) with a new ray (words 4-5).
-struct Rec {
-	float4 w0, w1, w2, w3, w4, w5;
-};
-
-struct PipeArgs {
-	const float4* nodes;
-	const float4* tris;
-	const float4* rays;
-	uint4* hits;
-	uint8_t* inLight;
-	uint32_t n;
-	uint32_t* work;
-	uint32_t refillMin;
-	uint32_t topCount;
-	bool finiteBounds;
-	const float4* treelet;  // LDS copy of nodes [0, topCount)
-	const uint32_t* handoff;  // the block's handoff area (LDS)
-	uint32_t window;          // rays per fetch
-	unsigned long long* clock;  // completion clock per ray (completion-clock launches only)
-};
-
-// Loop-carried state of one lane.
-struct Tracer {
-	dev::Ray r;
-	Closest c;
-	LaneTrace s;
-	uint32_t rayIdx;   // ray being traced
-	uint32_t doneIdx;  // ray that ended in the previous step, its result still to be written
-	uint32_t kind;    // record in flight (kRec*)
-	bool fastSlab;
-};
-
-// Writes a ray's result: its closest hit, or (any hit) 0 if occluded -- c.tri == 0 marks a hit
-// there -- and 1 if not.
-template <bool kAnyHit>
-__device__ __forceinline__ void store_result(void* out, uint32_t idx, const Closest& c)
-{
-	if (kAnyHit)
-		static_cast<uint8_t*>(out)[idx] = c.tri == 0u ? 0 : 1;
-	else
-		static_cast<uint4*>(out)[idx] = make_uint4(c.tri, __float_as_uint(c.t),
-		                                           __float_as_uint(c.u), __float_as_uint(c.v));
-}
-template <bool kAnyHit>
-__device__ __forceinline__ void store_result(const PipeArgs& P, uint32_t idx, const Closest& c)
-{
-	store_result<kAnyHit>(kAnyHit ? static_cast<void*>(P.inLight) : static_cast<void*>(P.hits),
-	                      idx, c);
-}
-
-// Both triangles of a pair, branch-free, accepted in castRay's order (BVHTraversal.hpp:78-93).
-// The second is skipped when the pair holds one triangle (its words are the next triangle's or
-// the array's padding).
-template <bool kCount>
-__device__ __forceinline__ void test_pair_closest(const dev::Ray& r, const Rec& A, uint32_t cnt,
-                                                  uint32_t first, Closest& c, Counts& k)
-{
-	const dev::TriDet d0 = dev::tri_det(r, A.w1, A.w2);
-	const dev::TriDet d1 = dev::tri_det(r, A.w4, A.w5);
-	float f0 = dev::recip_newton(d0.a), f1 = dev::recip_newton(d1.a);
-	if (!(dev::recip_newton_ok(d0.a) && dev::recip_newton_ok(d1.a))) {
-		f0 = 1.0f / d0.a;
-		f1 = 1.0f / d1.a;
-	}
-	float t0, u0, v0, t1, u1, v1;
-	const bool h0 = dev::tri_finish(r, d0, f0, A.w0, A.w1, A.w2, t0, u0, v0);
-	const bool h1 = dev::tri_finish(r, d1, f1, A.w3, A.w4, A.w5, t1, u1, v1) && cnt > 1u;
-	const bool acc0 = h0 && t0 < c.t && r.tMin <= t0 && t0 <= r.tMax;
-	c.tri = acc0 ? first : c.tri;
-	c.t = acc0 ? t0 : c.t;
-	c.u = acc0 ? u0 : c.u;
-	c.v = acc0 ? v0 : c.v;
-	const bool acc1 = h1 && t1 < c.t && r.tMin <= t1 && t1 <= r.tMax;
-	c.tri = acc1 ? first + 1u : c.tri;
-	c.t = acc1 ? t1 : c.t;
-	c.u = acc1 ? u1 : c.u;
-	c.v = acc1 ? v1 : c.v;
-	if (kCount) {
-		k.accepted += uint32_t(acc0) + uint32_t(acc1);
-		k.triTests += cnt;
-	}
-}
-
-// Any-hit pair: true iff one of the triangles has tMin <= t < tMax (RayCastKernel.cu:759-765).
-__device__ __forceinline__ bool test_pair_any(const dev::Ray& r, const Rec& A, uint32_t cnt)
-{
-	const dev::TriDet d0 = dev::tri_det(r, A.w1, A.w2);
-	const dev::TriDet d1 = dev::tri_det(r, A.w4, A.w5);
-	float f0 = dev::recip_newton(d0.a), f1 = dev::recip_newton(d1.a);
-	if (!(dev::recip_newton_ok(d0.a) && dev::recip_newton_ok(d1.a))) {
-		f0 = 1.0f / d0.a;
-		f1 = 1.0f / d1.a;
-	}
-	float t0, u0, v0, t1, u1, v1;
-	const bool h0 = dev::tri_finish(r, d0, f0, A.w0, A.w1, A.w2, t0, u0, v0);
-	const bool h1 = dev::tri_finish(r, d1, f1, A.w3, A.w4, A.w5, t1, u1, v1) && cnt > 1u;
-	return (h0 && r.tMin <= t0 && t0 < r.tMax) || (h1 && r.tMin <= t1 && t1 < r.tMax);
-}
-
-// Node expansion (selects, not branches): visited leaf children become the triangle range (left
-// first, the right one queued behind it), the right inner child is castRay's next pop, a left
-// inner child with it is pushed, and with no inner child the stack is popped -- one LDS read for
-// every lane (lanes that do not pop read the spare row); only a spilled entry takes a branch.
-__device__ __forceinline__ void expand_pipe(const NodeWords& nd, bool visitL, bool visitR,
-                                            LaneTrace& s, LaneStack& st)
-{
-	const bool innerL = visitL && nd.w3.z == 0;
-	const bool innerR = visitR && nd.w3.w == 0;
-	const bool leafL = visitL && !innerL;
-	const bool leafR = visitR && !innerR;
-	const uint32_t lFirst = child_index(nd.w3.x), rFirst = child_index(nd.w3.y);
-	const uint32_t lEnd = lFirst + uint32_t(nd.w3.z), rEnd = rFirst + uint32_t(nd.w3.w);
-	s.triCur = leafL ? lFirst : leafR ? rFirst : s.triCur;
-	s.triEnd = leafL ? lEnd : leafR ? rEnd : s.triEnd;
-	const bool both = leafL && leafR;
-	s.pendCur = both ? rFirst : s.pendCur;
-	s.pendEnd = both ? rEnd : s.pendEnd;
-	st.push_if(innerL && innerR, lFirst);
-	const bool doPop = !innerL && !innerR && st.sp > 0;
-	const uint32_t popped = st.pop_if(doPop);
-	s.next = innerR ? int32_t(rFirst) : innerL ? int32_t(lFirst) : doPop ? int32_t(popped) : -1;
-}
-
-// What the wave does after a step: go on, stop (no ray left), or trace its last few rays solo.
-constexpr int kStepGo = 0, kStepDone = 1, kStepSolo = 2;
-
-// Rays left in a wave, once the ray queue is empty, at or below which the wave goes solo: it traces
-// them one at a time with all 64 lanes instead of one lane each, keeping one and offering the
-// others to the block's other waves (below). While waves of the block are idle, the threshold is
-// one more than their number, up to kMaxSoloRays, so each idle wave can take a ray at once.
-constexpr uint32_t kSoloRays = 6;
-constexpr uint32_t kMaxSoloRays = 16;
-__device__ __forceinline__ uint32_t solo_threshold(const uint32_t* handoff);
-
-// One iteration: consume record A, issue the load of the lane's next record into B, test A's
-// triangles, retire finished rays and refill lanes. Every path a lone lane can take is kept short
-// -- once few rays are left, a wave's time per step is the number of instructions it issues --
-// so work that only some lanes need sits in the branch of those lanes. kExitCheck: whether this
-// step tests if the wave is done or should go solo (kStepGo otherwise); the loop runs two steps
-// per turn and checks after the second.
-template <bool kAnyHit, bool kCount, bool kTreelet, bool kExitCheck, bool kClock = false>
-__device__ __forceinline__ int pipe_step(const PipeArgs& P, Tracer& L, LaneStack& st,
-                                          WaveQueue& q, const Rec& A, Rec& B, Counts& k)
-{
-	// Wait for A -- and for the stores of the previous step -- here, before anything else. The
-	// compiler's own waits treat the vector-memory counter as unordered while a store is pending
-	// among loads and then wait for everything, B's loads included; with nothing outstanding at
-	// the top of the step, the only loads in flight during the triangle tests are B's.
-	__builtin_amdgcn_s_waitcnt(kWaitVmcntZero);
-	const uint32_t kind = L.kind;
-	// The result of a ray that ended in the previous step is still in L.c until a new ray starts.
-	const Closest ended = L.c;
-	uint32_t triFirst = 0u, triCnt = 0u;
-	bool anyHit = false;
-	if (kind == kRecTri) {
-		// Up to kTriBatch triangles of the current range; when the range is used up, the right
-		// leaf's range queued behind it (if any) becomes current.
-		triFirst = L.s.triCur;
-		const uint32_t left = L.s.triEnd - triFirst;
-		triCnt = left < kTriBatch ? left : kTriBatch;
-		const bool rangeDone = left <= kTriBatch;
-		L.s.triCur = rangeDone ? L.s.pendCur : triFirst + kTriBatch;
-		L.s.triEnd = rangeDone ? L.s.pendEnd : L.s.triEnd;
-		L.s.pendCur = rangeDone ? 0u : L.s.pendCur;
-		L.s.pendEnd = rangeDone ? 0u : L.s.pendEnd;
-		if (kAnyHit) anyHit = test_pair_any(L.r, A, triCnt);
-	} else if (kind != kRecIdle) {
-		if (kind == kRecRay) {
-			L.r = dev::make_ray(A.w4, A.w5);
-			L.fastSlab = P.finiteBounds && L.r.nanFree;
-			L.c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
-			st.sp = 0;
-			L.s = {0u, 0u, 0u, 0u, -1};
-		}
-		NodeWords nd;
-		nd.w0 = A.w0;
-		nd.w1 = A.w1;
-		nd.w2 = A.w2;
-		nd.w3 = make_int4(__float_as_int(A.w3.x), __float_as_int(A.w3.y), __float_as_int(A.w3.z),
-		                  __float_as_int(A.w3.w));
-		const float tCurrMax = kAnyHit ? L.r.tMax : dev::min_first(L.r.tMax, L.c.t);
-		bool visitL, visitR;
-		decide(L.r, L.fastSlab, nd, tCurrMax, visitL, visitR);
-		if (kCount) {
-			k.nodes++;
-			k.boxHits += uint32_t(visitL) + uint32_t(visitR);
-		}
-		expand_pipe(nd, visitL, visitR, L.s, st);
-	}
-
-	// Next record: more of this ray, or (for lanes whose ray ends here, and idle lanes) a new ray.
-	const bool more = kind != kRecIdle && !anyHit && (L.s.triCur < L.s.triEnd || L.s.next >= 0);
-	uint32_t fresh = kInvalid;
-	if (!q.exhausted) {
-		const uint64_t freeLanes = __ballot(!more);
-		if (freeLanes != 0 && (uint32_t(__popcll(freeLanes)) >= P.refillMin || freeLanes == ~0ull))
-			fresh = refill(q, freeLanes, P.work, P.n, !more, P.window);
-	}
-	const bool tri = more && L.s.triCur < L.s.triEnd;
-	const bool node = more && !tri;
-	const bool ray = fresh != kInvalid;
-	const uint32_t nextKind = tri ? kRecTri : node ? kRecNode : ray ? kRecRay : kRecIdle;
-	// The ended ray's result is written just before the loads, after the waits of this step (the
-	// stack pop's, the refill's), so its latency overlaps the triangle tests, not a wait.
-	if (L.doneIdx != kInvalid) {
-		store_result<kAnyHit>(P, L.doneIdx, ended);
-		if (kClock) P.clock[L.doneIdx] = wall_clock64();
-	}
-	// Every lane issues the same six loads: a node (words 0-3), a triangle pair (words 0-5), or
-	// the root node and a new ray's 32 B; idle lanes and words 4-5 of a node read the root node
-	// (always cached). Offsets are in 16-B words: 4 per node, 3 per triangle.
-	const uint32_t idx = tri ? L.s.triCur : node ? uint32_t(L.s.next) : 0u;
-	const uint32_t word = tri ? idx + (idx << 1) : idx << 2;
-	const float4* rec = (tri ? P.tris : P.nodes) + word;
-	const float4* src45 = tri ? rec + 4 : ray ? P.rays + 2u * size_t(ray ? fresh : 0u) : P.nodes;
-	if (kTreelet && !tri && idx < P.topCount) {
-		const LdsF4* t = as_lds(P.treelet) + 4u * idx;
-		B.w0 = t[0];
-		B.w1 = t[1];
-		B.w2 = t[2];
-		B.w3 = t[3];
-	} else {
-		B.w0 = as_global(rec)[0];
-		B.w1 = as_global(rec)[1];
-		B.w2 = as_global(rec)[2];
-		B.w3 = as_global(rec)[3];
-	}
-	B.w4 = as_global(src45)[0];
-	B.w5 = as_global(src45)[1];
-
-	if (!kAnyHit && kind == kRecTri) test_pair_closest<kCount>(L.r, A, triCnt, triFirst, L.c, k);
-
-	if (kAnyHit && anyHit) L.c.tri = 0u;
-	L.doneIdx = kind != kRecIdle && !more ? L.rayIdx : kInvalid;
-	if (!more) L.rayIdx = fresh;
-	L.kind = nextKind;
-	if (!kExitCheck || !q.exhausted) return kStepGo;
-	const uint64_t busy = __ballot(nextKind != kRecIdle);
-	if (busy == 0) return kStepDone;
-	return !kCount && uint32_t(__popcll(busy)) <= solo_threshold(P.handoff) ? kStepSolo : kStepGo;
-}
-
-// ---- solo mode: one ray per wave ---------------------------------------------------------------
-//
-// Once the ray queue is empty, a wave's last rays are the costliest ones, and a wave with one busy
-// lane still issues every instruction of a step. A wave with at most kSoloRays rays left therefore
-// traces them one after the other with all 64 lanes: a node's twelve slab planes are computed by
-// lanes 0-11 at once and combined across lanes (DPP), the triangles of visited leaves are tested
-// one per lane in a single pass, and the traversal state -- the ray, the closest hit, the stack
-// (entry e in lane e of two registers) -- is uniform, so every decision is a scalar branch.
-// Visiting order and arithmetic are castRay's: the same slab operations with std::min/max
-// semantics, the same triangle test, and a leaf pass accepts candidates in castRay's order
-// (ascending lane = ascending position in the left-then-right leaf sequence), each against the
-// closest hit so far.
-
-__device__ __forceinline__ uint32_t lane_u(uint32_t v, uint32_t l)
-{
-	return uint32_t(__builtin_amdgcn_readlane(int(v), int(l)));
-}
-__device__ __forceinline__ float lane_f(float v, uint32_t l)
-{
-	return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), int(l)));
-}
-// The value of lane (this lane + k) of the same 16-lane row (DPP row_shl:k).
-template <int k>
-__device__ __forceinline__ float from_lane_plus(float v)
-{
-	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x100 | k, 0xF, 0xF, false));
-}
-
-struct SoloHit {
-	uint32_t tri;
-	float t, u, v;
-	bool any;  // any hit found (any-hit traversal)
-};
-
-// Tests the n1 triangles from a1 and then the n2 from a2 -- castRay's order -- one per lane, 64 per
-// pass. Closest hit: each candidate (hit, t < closest t on entry, tMin <= t <= tMax) is accepted
-// in order if t is still below the closest t, exactly as the sequential loop does. Any hit:
-// records a hit with tMin <= t < tMax.
-template <bool kAnyHit>
-__device__ __forceinline__ void solo_tris(const float4* tris, const dev::Ray& r, uint32_t a1,
-                                          uint32_t n1, uint32_t a2, uint32_t n2, SoloHit& c)
-{
-	const uint32_t lane = __lane_id();
-	for (uint32_t base = 0; base < n1 + n2; base += 64u) {
-		const uint32_t j = base + lane;
-		const bool have = j < n1 + n2;
-		const uint32_t tri = j < n1 ? a1 + j : a2 + (j - n1);
-		float t = 0.0f, u = 0.0f, v = 0.0f;
-		bool hit = false;
-		if (have) {
-			const float4* p = tris + 3u * tri;
-			const float4 p0 = as_global(p)[0], e1 = as_global(p)[1], e2 = as_global(p)[2];
-			const dev::TriDet d = dev::tri_det(r, e1, e2);
-			float f = dev::recip_newton(d.a);
-			if (!dev::recip_newton_ok(d.a)) f = 1.0f / d.a;
-			hit = dev::tri_finish(r, d, f, p0, e1, e2, t, u, v);
-		}
-		if (kAnyHit) {
-			if (__ballot(have && hit && r.tMin <= t && t < r.tMax) != 0) {
-				c.any = true;
-				return;
-			}
-		} else {
-			uint64_t cand = __ballot(have && hit && t < c.t && r.tMin <= t && t <= r.tMax);
-			while (cand != 0) {
-				const uint32_t w = uint32_t(__builtin_ctzll(cand));
-				cand &= cand - 1u;
-				const float tw = lane_f(t, w);
-				if (tw < c.t) {
-					c.t = tw;
-					c.u = lane_f(u, w);
-					c.v = lane_f(v, w);
-					c.tri = lane_u(tri, w);
-				}
-			}
-		}
-	}
-}
-
-// The scene and output of a solo ray (uniform).
-struct SoloScene {
-	const float4* nodes;
-	const float4* tris;
-	const float4* rays;
-	void* out;  // uint4 hits (closest hit) or uint8_t (any hit), indexed by the ray's index
-	unsigned long long* clock = nullptr;  // completion clock per ray (completion-clock launches)
-};
-
-// Where a solo ray starts: the state the pipelined loop left for it (the record in flight is
-// loaded again). Uniform values.
-struct SoloStart {
-	float4 oMin, dMax;            // origin and tMin, direction and tMax (1/dir is recomputed)
-	Closest c;                    // closest hit so far
-	uint32_t triCur, triEnd, pendCur, pendEnd;  // queued triangle ranges
-	int32_t next;                 // node to expand next, or -1
-	int sp;                       // stack entries
-	uint32_t rayIdx;
-	uint32_t kind;                // kRecRay: the ray is not set up yet (load it from rays[rayIdx])
-	const uint32_t* ldsCol;       // the owner lane's LDS stack column (entry e at ldsCol[64 e])
-	const uint32_t* spillCol;     // its spill column (entry e >= depth at [(e - depth) stride])
-	uint32_t stride;
-	int depth;
-};
-
-// The start state of lane lsel of this wave.
-__device__ __forceinline__ SoloStart solo_start_lane(const Tracer& L, const LaneStack& st,
-                                                     uint32_t lsel)
-{
-	SoloStart S;
-	S.oMin = make_float4(lane_f(L.r.ox, lsel), lane_f(L.r.oy, lsel), lane_f(L.r.oz, lsel),
-	                     lane_f(L.r.tMin, lsel));
-	S.dMax = make_float4(lane_f(L.r.dx, lsel), lane_f(L.r.dy, lsel), lane_f(L.r.dz, lsel),
-	                     lane_f(L.r.tMax, lsel));
-	S.c = {lane_u(L.c.tri, lsel), lane_f(L.c.t, lsel), lane_f(L.c.u, lsel), lane_f(L.c.v, lsel)};
-	S.triCur = lane_u(L.s.triCur, lsel);
-	S.triEnd = lane_u(L.s.triEnd, lsel);
-	S.pendCur = lane_u(L.s.pendCur, lsel);
-	S.pendEnd = lane_u(L.s.pendEnd, lsel);
-	S.next = int32_t(lane_u(uint32_t(L.s.next), lsel));
-	S.sp = int(lane_u(uint32_t(st.sp), lsel));
-	S.rayIdx = lane_u(L.rayIdx, lsel);
-	S.kind = lane_u(L.kind, lsel);
-	S.ldsCol = st.lds + lsel;
-	S.spillCol = st.spill - __lane_id() + lsel;
-	S.stride = st.stride;
-	S.depth = st.depth;
-	return S;
-}
-
-// Traces a ray to its end from S and writes its result.
-template <bool kAnyHit, bool kClock = false>
-__device__ __forceinline__ void solo_run(const SoloScene& P, const SoloStart& S)
-{
-	const uint32_t lane = __lane_id();
-	const uint32_t rayIdx = S.rayIdx;
-	dev::Ray r;
-	SoloHit c;
-	uint32_t triCur, triEnd, pendCur, pendEnd;
-	int32_t cur;
-	int sp;
-	if (S.kind == kRecRay) {
-		const float4* src = P.rays + 2u * size_t(rayIdx);
-		const float4 a = as_global(src)[0], b = as_global(src)[1];
-		r = dev::make_ray(make_float4(lane_f(a.x, 0), lane_f(a.y, 0), lane_f(a.z, 0), lane_f(a.w, 0)),
-		                  make_float4(lane_f(b.x, 0), lane_f(b.y, 0), lane_f(b.z, 0), lane_f(b.w, 0)));
-		c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX, false};
-		triCur = triEnd = pendCur = pendEnd = 0u;
-		cur = 0;
-		sp = 0;
-	} else {
-		r = dev::make_ray(S.oMin, S.dMax);
-		c = {S.c.tri, S.c.t, S.c.u, S.c.v, false};
-		triCur = S.triCur, triEnd = S.triEnd, pendCur = S.pendCur, pendEnd = S.pendEnd;
-		cur = S.next;
-		sp = S.sp;
-	}
-	// The owner's stack (LDS column, then spill column) into two registers: entry e in lane e of
-	// stk0 (e < 64) or of stk1.
-	uint32_t stk0 = 0u, stk1 = 0u;
-	for (int e = int(lane), h = 0; h < 2; h++, e += 64) {
-		uint32_t v = 0u;
-		if (e < sp)
-			v = e < S.depth ? S.ldsCol[e * 64] : S.spillCol[size_t(e - S.depth) * S.stride];
-		if (h == 0)
-			stk0 = v;
-		else
-			stk1 = v;
-	}
-	// Slab lanes: lane i < 12 holds plane i of a node -- lc.min.xyz, lc.max.xyz, rc.min.xyz,
-	// rc.max.xyz -- whose axis is i mod 3.
-	const uint32_t axis = lane % 3u;
-	const float oA = axis == 0u ? r.ox : axis == 1u ? r.oy : r.oz;
-	const float iA = axis == 0u ? r.ix : axis == 1u ? r.iy : r.iz;
-	const float* nodeWords = reinterpret_cast<const float*>(P.nodes);
-
-	// Triangles queued when the loop handed over (a leaf pair's ranges), then the nodes.
-	solo_tris<kAnyHit>(P.tris, r, triCur, triEnd - triCur, pendCur, pendEnd - pendCur, c);
-	while (!(kAnyHit && c.any)) {
-		if (cur < 0) {
-			if (sp == 0) break;
-			sp--;
-			cur = int32_t(sp < 64 ? lane_u(stk0, uint32_t(sp)) : lane_u(stk1, uint32_t(sp - 64)));
-		}
-		const float w = as_global(nodeWords)[16u * uint32_t(cur) + (lane & 15u)];
-		// t of plane i (lane i), and of plane i + 3 (the max plane of the same axis and box).
-		const float t1 = (w - oA) * iA;
-		const float t2 = from_lane_plus<3>(t1);
-		// min/max with std::min/std::max semantics (BVHTraversal via Intersection.hpp:77-90).
-		const float lo = dev::min_first(t1, t2), hi = dev::max_first(t1, t2);
-		// lanes 0 (left box) and 6 (right box): combine the x, y, z slabs.
-		const float tIn = dev::max_first(dev::max_first(lo, from_lane_plus<1>(lo)), from_lane_plus<2>(lo));
-		const float tOut = dev::min_first(dev::min_first(hi, from_lane_plus<1>(hi)), from_lane_plus<2>(hi));
-		const float tCurrMax = kAnyHit ? r.tMax : dev::min_first(r.tMax, c.t);
-		const uint64_t vis = __ballot((tOut >= tIn) && tOut > r.tMin && tIn < tCurrMax);
-		const bool visitL = (vis & 1ull) != 0, visitR = (vis & (1ull << 6)) != 0;
-		const int32_t lRaw = int32_t(lane_u(__float_as_uint(w), 12u));
-		const int32_t rRaw = int32_t(lane_u(__float_as_uint(w), 13u));
-		const uint32_t lCnt = lane_u(__float_as_uint(w), 14u);
-		const uint32_t rCnt = lane_u(__float_as_uint(w), 15u);
-		const uint32_t lFirst = child_index(lRaw), rFirst = child_index(rRaw);
-		const bool innerL = visitL && lCnt == 0u, innerR = visitR && rCnt == 0u;
-		if (innerL && innerR) {
-			stk0 = int(lane) == sp ? lFirst : stk0;
-			stk1 = int(lane) + 64 == sp ? lFirst : stk1;
-			sp++;
-		}
-		cur = innerR ? int32_t(rFirst) : innerL ? int32_t(lFirst) : -1;
-		const bool leafL = visitL && !innerL, leafR = visitR && !innerR;
-		if (leafL || leafR)
-			solo_tris<kAnyHit>(P.tris, r, lFirst, leafL ? lCnt : 0u, rFirst, leafR ? rCnt : 0u, c);
-	}
-	if (lane == 0u) {
-		const Closest res = {kAnyHit ? (c.any ? 0u : kInvalid) : c.tri, c.t, c.u, c.v};
-		store_result<kAnyHit>(P.out, rayIdx, res);
-		if (kClock) P.clock[rayIdx] = wall_clock64();
-	}
-}
-
-// ---- handing solo rays to the block's other waves ------------------------------------------------
-//
-// A wave that goes solo keeps one ray and offers the others in LDS slots; waves of the block that
-// have nothing left -- and the block's helper waves, which trace nothing else -- claim them and
-// trace them solo, so a wave's last rays run side by side instead of one after another. The stack of an offered ray stays where it is (its owner's LDS
-// column and spill column, which the owner no longer writes). Area layout (32-bit words):
-// [0] slots allocated, [1] slots claimed, [2] waves that may still offer, [3] waves waiting to
-// claim, then
-// kSlotWords per slot. A claimed slot index is below the allocated count, and its owner marks it
-// ready right after writing it, so a claimant's wait ends; the last claim attempts end once no
-// wave may offer and every slot is claimed.
-
-constexpr uint32_t kHandoffPerWave = kMaxSoloRays - 1u;  // a wave offers at most this many rays
-constexpr uint32_t kSlotWords = 24;
-
-// `laneThreads`: the block's lane-mode threads (helper waves offer nothing).
-__host__ __device__ __forceinline__ uint32_t handoff_bytes(uint32_t laneThreads)
-{
-	return 16u + (laneThreads / 64u) * kHandoffPerWave * kSlotWords * 4u;
-}
-
-__device__ __forceinline__ uint32_t lds_load(const uint32_t* p)
-{
-	return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
-// The solo threshold of a wave of the block (see kSoloRays).
-__device__ __forceinline__ uint32_t solo_threshold(const uint32_t* H)
-{
-	const uint32_t idle = __builtin_amdgcn_readfirstlane(lds_load(&H[3]));
-	return idle + 1u > kSoloRays ? (idle + 1u < kMaxSoloRays ? idle + 1u : kMaxSoloRays) : kSoloRays;
-}
-
-// Every thread of the block calls this before the block's first barrier: resets the counters and
-// every slot's ready word (LDS holds whatever an earlier block left there, and a stale ready word
-// would let a claimant read a slot before its owner writes it). `laneWaves`: the waves that run
-// the lane-mode loop and may offer rays.
-__device__ __forceinline__ void handoff_init(uint32_t* H, uint32_t laneWaves)
-{
-	if (threadIdx.x == 0) {
-		H[0] = 0u;
-		H[1] = 0u;
-		H[2] = laneWaves;
-		H[3] = 0u;
-	}
-	const uint32_t slots = laneWaves * kHandoffPerWave;
-	for (uint32_t i = threadIdx.x; i < slots; i += blockDim.x) H[4u + i * kSlotWords + 22u] = 0u;
-}
-
-// Offers the rays of the lanes in `offer` (each lane writes its own slot), then retires this wave
-// as a producer.
-__device__ __forceinline__ void handoff_offer(uint32_t* H, uint64_t offer, const Tracer& L,
-                                              const LaneStack& st, uint32_t batch)
-{
-	const uint32_t lane = __lane_id();
-	const uint32_t n = uint32_t(__popcll(offer));
-	if (n != 0u) {
-		uint32_t base = 0u;
-		if (lane == 0u) base = atomicAdd(&H[0], n);
-		base = lane_u(base, 0u);
-		const bool mine = ((offer >> lane) & 1ull) != 0;
-		uint32_t* w = H + 4u + (base + uint32_t(__popcll(offer & __lanemask_lt()))) * kSlotWords;
-		if (mine) {
-			w[0] = __float_as_uint(L.r.ox);
-			w[1] = __float_as_uint(L.r.oy);
-			w[2] = __float_as_uint(L.r.oz);
-			w[3] = __float_as_uint(L.r.tMin);
-			w[4] = __float_as_uint(L.r.dx);
-			w[5] = __float_as_uint(L.r.dy);
-			w[6] = __float_as_uint(L.r.dz);
-			w[7] = __float_as_uint(L.r.tMax);
-			w[8] = L.c.tri;
-			w[9] = __float_as_uint(L.c.t);
-			w[10] = __float_as_uint(L.c.u);
-			w[11] = __float_as_uint(L.c.v);
-			w[12] = L.s.triCur;
-			w[13] = L.s.triEnd;
-			w[14] = L.s.pendCur;
-			w[15] = L.s.pendEnd;
-			w[16] = uint32_t(L.s.next);
-			w[17] = uint32_t(st.sp);
-			w[18] = L.rayIdx;
-			w[19] = L.kind;
-			w[20] = ((threadIdx.x >> 6) << 6) | lane;  // owner: wave in block, lane
-			w[21] = batch;
-		}
-		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-		if (mine) __hip_atomic_store(&w[22], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-	}
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-	if (lane == 0u) atomicSub(&H[2], 1u);
-}
-
-// Claims an offered ray: its slot, or kInvalid once none is left and no wave can offer more.
-__device__ __forceinline__ uint32_t handoff_claim(uint32_t* H)
-{
-	uint32_t got = kInvalid;
-	if (__lane_id() == 0u) {
-		atomicAdd(&H[3], 1u);
-		while (true) {
-			const uint32_t c = lds_load(&H[1]);
-			if (c < lds_load(&H[0])) {
-				if (atomicCAS(&H[1], c, c + 1u) == c) {
-					got = c;
-					break;
-				}
-				continue;
-			}
-			if (lds_load(&H[2]) == 0u && lds_load(&H[1]) >= lds_load(&H[0])) break;
-			__builtin_amdgcn_s_sleep(2);
-		}
-		atomicSub(&H[3], 1u);
-	}
-	return lane_u(got, 0u);
-}
-
-// The start state in a claimed slot (waits for its owner to mark it ready).
-__device__ __forceinline__ SoloStart solo_start_slot(const uint32_t* H, uint32_t slot,
-                                                     const uint32_t* ldsStacks,
-                                                     const uint32_t* spill, uint32_t stride,
-                                                     int depth, uint32_t& batch)
-{
-	const uint32_t* w = H + 4u + slot * kSlotWords;
-	while (lane_u(lds_load(&w[22]), 0u) == 0u) __builtin_amdgcn_s_sleep(1);
-	uint32_t v[22];
-#pragma unroll
-	for (int i = 0; i < 22; i++) v[i] = __builtin_amdgcn_readfirstlane(w[i]);
-	SoloStart S;
-	S.oMin = make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
-	                     __uint_as_float(v[3]));
-	S.dMax = make_float4(__uint_as_float(v[4]), __uint_as_float(v[5]), __uint_as_float(v[6]),
-	                     __uint_as_float(v[7]));
-	S.c = {v[8], __uint_as_float(v[9]), __uint_as_float(v[10]), __uint_as_float(v[11])};
-	S.triCur = v[12];
-	S.triEnd = v[13];
-	S.pendCur = v[14];
-	S.pendEnd = v[15];
-	S.next = int32_t(v[16]);
-	S.sp = int(v[17]);
-	S.rayIdx = v[18];
-	S.kind = v[19];
-	const uint32_t wave = v[20] >> 6, lane = v[20] & 63u;
-	S.ldsCol = ldsStacks + wave * (uint32_t(depth) + 1u) * 64u + lane;
-	// Spill columns are numbered over the grid's lane-mode threads (`stride` of them).
-	S.spillCol = spill + (blockIdx.x * (stride / gridDim.x) + wave * 64u + lane);
-	S.stride = stride;
-	S.depth = depth;
-	batch = v[21];
-	return S;
-}
-
-// The block's last `helpers` waves (helper waves) run no lane-mode loop: they wait for offered rays
-// and trace them solo, at raised priority so that the waves still in lane mode on their SIMD delay
-// them little. A block with helpers has more waves for a solo tail than waves in lane mode.
-__device__ __forceinline__ bool is_helper(uint32_t helpers)
-{
-	return (threadIdx.x >> 6) >= blockDim.x / 64u - helpers;
-}
-
-// Shared skeleton of the persistent closest-hit (kAnyHit = false) and any-hit kernels. Without a
-// treelet (kTreelet false) every record comes from global memory and no LDS path is compiled.
-// LDS stacks and spill columns belong to the lane-mode threads only.
-// kClock: `counters` is instead a completion clock of n + 1 words: each ray's device clock
-// (wall_clock64) when its result is written, and in word n the earliest block start.
-template <bool kAnyHit, bool kCount, bool kTreelet, bool kClock = false>
-__device__ __forceinline__ void persistent_trace(
-	const float4* __restrict__ nodes, const float4* __restrict__ tris,
-	const float4* __restrict__ rays, uint4* __restrict__ hits, uint8_t* __restrict__ inLight,
-	uint32_t n, uint32_t* __restrict__ work, uint32_t* __restrict__ spill, uint32_t refillMin,
-	bool finiteBounds, uint32_t topCount, uint32_t helpers, int depth, uint32_t window,
-	unsigned long long* __restrict__ counters)
-{
-	extern __shared__ float4 ldsRaw[];
-	const uint32_t laneWaves = blockDim.x / 64u - helpers;
-	const uint32_t laneThreads = laneWaves * 64u;
-	uint32_t* ldsStacks = reinterpret_cast<uint32_t*>(ldsRaw);
-	float4* treelet = ldsRaw + laneWaves * (uint32_t(depth) + 1u) * 64u / 4u;
-	uint32_t* handoff = reinterpret_cast<uint32_t*>(treelet + 4u * topCount);
-	if (kClock && threadIdx.x == 0) atomicMin(&counters[n], wall_clock64());
-	if (kTreelet)
-		for (uint32_t i = threadIdx.x; i < 4u * topCount; i += blockDim.x) treelet[i] = nodes[i];
-	handoff_init(handoff, laneWaves);
-	__syncthreads();
-
-	const SoloScene S = {nodes, tris, rays,
-	                     kAnyHit ? static_cast<void*>(inLight) : static_cast<void*>(hits),
-	                     kClock ? counters : nullptr};
-	const uint32_t stride = gridDim.x * laneThreads;
-	if (!kCount && is_helper(helpers)) {
-		__builtin_amdgcn_s_setprio(3);
-		for (uint32_t slot = handoff_claim(handoff); slot != kInvalid; slot = handoff_claim(handoff)) {
-			uint32_t batch;
-			solo_run<kAnyHit, kClock>(S, solo_start_slot(handoff, slot, ldsStacks, spill, stride, depth,
-			                                     batch));
-		}
-		retire_wave(work);
-		return;
-	}
-
-	LaneStack st;
-	st.lds = ldsStacks + (threadIdx.x >> 6) * (uint32_t(depth) + 1u) * 64u;
-	st.depth = depth;
-	st.stride = stride;
-	st.spill = spill + (blockIdx.x * laneThreads + threadIdx.x);
-	st.lane = __lane_id();
-	st.sp = 0;
-
-	const PipeArgs P = {nodes, tris, rays, hits, inLight, n, work, refillMin,
-	                    kTreelet ? topCount : 0u, finiteBounds, treelet, handoff, window,
-	                    kClock ? counters : nullptr};
-	WaveQueue q;
-	Tracer L;
-	L.c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
-	L.s = {0u, 0u, 0u, 0u, -1};
-	L.rayIdx = kInvalid;
-	L.doneIdx = kInvalid;
-	L.kind = kRecIdle;
-	L.fastSlab = false;
-	L.r = dev::make_ray(make_float4(0.f, 0.f, 0.f, 0.f), make_float4(1.f, 1.f, 1.f, 0.f));
-	const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-	Rec A = {z, z, z, z, z, z}, B = A;
-	Counts k;
-	int next = kStepGo;
-	while (next == kStepGo) {
-		pipe_step<kAnyHit, kCount, kTreelet, false, kClock>(P, L, st, q, A, B, k);
-		next = pipe_step<kAnyHit, kCount, kTreelet, true, kClock>(P, L, st, q, B, A, k);
-	}
-	if (L.doneIdx != kInvalid) {
-		store_result<kAnyHit>(P, L.doneIdx, L.c);
-		if (kClock) P.clock[L.doneIdx] = wall_clock64();
-	}
-	if (!kCount) {
-		// Solo: keep the first busy lane's ray, offer the others to the block, then trace offered
-		// rays until none is left (the loads still in flight land in A, which is not read again).
-		const uint64_t busy = next == kStepSolo ? __ballot(L.kind != kRecIdle) : 0ull;
-		handoff_offer(handoff, busy & (busy - 1u), L, st, 0u);
-		if (busy != 0)
-			solo_run<kAnyHit, kClock>(S, solo_start_lane(L, st, uint32_t(__builtin_ctzll(busy))));
-		for (uint32_t slot = handoff_claim(handoff); slot != kInvalid; slot = handoff_claim(handoff)) {
-			uint32_t batch;
-			solo_run<kAnyHit, kClock>(S, solo_start_slot(handoff, slot, ldsStacks, spill, st.stride, depth,
-			                                     batch));
-		}
-	}
-	if (kCount) add_counts(counters, k);
-	retire_wave(work);
-}
-template <bool kCount, bool kTreelet, bool kClock = false>
-__global__ __launch_bounds__(kMaxBlock) void k_closest_persistent(
-	const float4* __restrict__ nodes, const float4* __restrict__ tris,
-	const float4* __restrict__ rays, uint4* __restrict__ hits, uint32_t n,
-	uint32_t* __restrict__ work, uint32_t* __restrict__ spill, uint32_t refillMin,
-	uint32_t finiteBounds, uint32_t topCount, uint32_t helpers, uint32_t depth, uint32_t window,
-	unsigned long long* __restrict__ counters)
-{
-	persistent_trace<false, kCount, kTreelet, kClock>(nodes, tris, rays, hits, nullptr, n, work,
-	                                                  spill, refillMin, finiteBounds != 0,
-	                                                  topCount, helpers, int(depth), window,
-	                                                  counters);
-}
-
-template <bool kTreelet>
-__global__ __launch_bounds__(kMaxBlock) void k_anyhit_persistent(
-	const float4* __restrict__ nodes, const float4* __restrict__ tris,
-	const float4* __restrict__ rays, uint8_t* __restrict__ inLight, uint32_t n,
-	uint32_t* __restrict__ work, uint32_t* __restrict__ spill, uint32_t refillMin,
-	uint32_t finiteBounds, uint32_t topCount, uint32_t helpers, uint32_t depth, uint32_t window)
-{
-	persistent_trace<true, false, kTreelet>(nodes, tris, rays, nullptr, inLight, n, work, spill,
-	                                        refillMin, finiteBounds != 0, topCount, helpers,
-	                                        int(depth), window, nullptr);
-}
-
-// ---- fused multi-batch launch ---------------------------------------------------------------------
-//
-// One persistent launch over many ray batches (closest-hit or any-hit, on one or several scenes):
-// the batches' rays form one index space [0, total) pulled from the shared counter as above; a
-// lane maps its ray index to (batch, local index) by binary search over the batch offsets held in
-// LDS. The treelet, if any, belongs to one scene (`treeletNodes`); lanes on other scenes read
-// every node from global memory. With completion tracking on, the lanes completing rays in the
-// block count completions and the latest completion time per batch in LDS, and every block adds
-// them to the batch table with one global atomic per batch when it retires, so each batch's
-// latency inside the launch is known (the clock only grows, so completion times need no reset
-// between launches). The last wave to retire resets the counters for the next launch.
-
-constexpr uint32_t kMaxBatches = 1024;
-
 __device__ __forceinline__ uint32_t find_batch(const uint32_t* offsets, uint32_t numBatches,
                                                uint32_t g)
 {
@@ -1868,327 +966,826 @@ __device__ __forceinline__ uint32_t find_batch(const uint32_t* offsets, uint32_t
 	return lo;
 }
 
-// The batch of each new ray of a refill, without a search per lane: a wave's windows come in
-// increasing order, so the wave keeps the batch of its current window's first ray (`cur`) and of the
-// window before it (`prev`, whose last rays a refill may still hand out). A lane starts from its
-// window's batch and steps over the batch ends below its index -- usually none or one, since a
-// window (at most 4096 rays) is mostly shorter than a batch; after four steps it searches.
-struct BatchCursor {
-	uint32_t start = 0;  // first ray of the window
-	uint32_t batch = 0;  // its batch
-};
+// ---- four lanes per ray ---------------------------------------------------------------------------
+//
+// Single casts of incoherent rays (k_quad). Four lanes trace a ray: one box of a wide node each, or one
+// triangle of a leaf each, combined across the four (DPP and 4 bits of a ballot). A wave holds 16
+// rays, its stacks are in LDS, and it runs at eight waves per SIMD. An iteration loads and consumes a
+// leaf and the node to be taken after it together: the node's slots are decided after the leaf's
+// triangles, with its entry distance compared again, so the order is castRay's. See wide_nodes.hpp
+// for why the hits are too.
+//
+// With one lane per ray and binary nodes (64 rays a wave, two or three waves per SIMD, a software
+// pipeline and a one-ray-per-wave mode for a wave's last rays) a launch was bound by its chains of
+// steps: 25 a bounce ray on 1,004,000 triangles, half of the time spent on the last 1% of the rays,
+// and 15,600 fetches from and 2,048 retirements to one address at 10 ns each. Before and now:
+//   998,029 bounce rays, closest hit   0.567 ms   0.466 ms
+//   their 998,029 shadow rays, any hit  0.254 ms   0.122 ms
+//   65,536 random rays, 100,000 random triangles  0.243 ms   0.125 ms
+// Many rays at once are bound by VALU issue (a wave instruction serves 16 rays), the rest by the
+// chain of the costliest rays: about 450 iterations of 0.9 us, the time a wave takes to issue one.
 
-__device__ __forceinline__ uint32_t batch_from(const uint32_t* offsets, uint32_t numBatches,
-                                               uint32_t from, uint32_t g)
+constexpr uint32_t kQuadBlock = 512;  // largest block of the persistent kernels
+constexpr uint32_t kQuadWavesPerSimd = 7;  // (72 registers)
+
+// Stacks of a wave: kCols columns of kRows entries (8 B) in LDS, with three rows below the bottom, so
+// that the top three can be read at any depth. Deeper entries spill to memory, kSpillEntries a
+// column, one after another.
+constexpr int kQuadRows = 20;  // (pending stacks of 20 are rare)
+constexpr int kLaneRows = 16;  // (9.5 KB a wave: 16 waves per CU)
+// Idle lanes of a one-ray-per-lane wave before it takes new rays: 64 batches of 3.2 million rays take
+// 1.79 ms with 4, 1.73 with 8 and 32, 1.70 with 16.
+constexpr uint32_t kLaneRefill = 16;
+constexpr uint32_t kSpillEntries = kSpillWordsPerRay / 2u;
+constexpr int kMaxPending = 66;     // of a binary walk (64 levels)
+static_assert(int(kWideMaxPending) <= kMaxPending, "pending slots of a wide walk");
+static_assert(kLaneRows + int(kSpillEntries) >= kMaxPending, "stack entries of a ray");
+static_assert(kQuadRows + int(kSpillEntries) >= kMaxPending, "stack entries of a ray");
+
+template <int kRows, uint32_t kCols>
+__host__ __device__ constexpr uint32_t wave_stack_entries() { return (uint32_t(kRows) + 3u) * kCols; }
+
+// LDS entry of the bottom of column `col` of the block's wave `wave`.
+template <int kRows, uint32_t kCols>
+__device__ __forceinline__ uint32_t stack_base(uint32_t wave, uint32_t col)
 {
-	uint32_t b = from;
-	for (int k = 0; k < 4; k++) {
-		if (offsets[b + 1u] > g) return b;
-		b++;
-	}
-	return find_batch(offsets, numBatches, g);
+	return wave * wave_stack_entries<kRows, kCols>() + 3u * kCols + col;
+}
+template <int kRows, uint32_t kCols>
+__device__ __forceinline__ GlobalU2* spill_entry(U32x2* spill, uint32_t base, int at)
+{
+	const uint32_t b = base - 3u * kCols, wave = b / wave_stack_entries<kRows, kCols>();
+	const uint32_t col = b - wave * wave_stack_entries<kRows, kCols>();
+	const size_t column = size_t(blockIdx.x * (blockDim.x / 64u) + wave) * kCols + col;
+	return (GlobalU2*)(spill) + column * kSpillEntries + uint32_t(at - kRows);
 }
 
-// Launch-wide arguments of the fused kernel.
-struct MultiArgs {
-	const BatchDesc* descs;
-	const uint32_t* offsets;  // LDS copy: offsets[b] = first global ray index of batch b
-	uint32_t numBatches;
-	uint32_t total;
-	uint32_t* work;
-	uint32_t refillMin;
-	uint32_t topCount;
-	const float4* treeletNodes;  // the scene whose top nodes are in the LDS treelet
-	const float4* treelet;       // LDS
-	unsigned long long* blockFinish;  // LDS, per batch (completion tracking)
-	uint32_t* blockDone;              // LDS, per batch
-	const uint32_t* handoff;          // the block's handoff area (LDS)
-	uint32_t window;                  // rays per fetch
-};
+// Ray counters of a launch, one 128-B line each: 8 that hand out windows, 8 + 1 that count blocks
+// as they end.
+constexpr uint32_t kCounters = 8;
+constexpr uint32_t kCounterStride = 32;
 
-// Per-lane state of the fused kernel: the pipelined loop's, plus the scene, output and kind of
-// the lane's batch.
-struct MultiTracer {
-	Tracer t;
+__host__ __device__ __forceinline__ uint32_t quad_lds_words(uint32_t waves)
+{
+	return waves * 2u * wave_stack_entries<kQuadRows, 16u>();
+}
+
+// (__ballot takes an int: a select and a compare more.)
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
+// v of another lane of the quad (DPP quad_perm).
+template <int kCtrl>
+__device__ __forceinline__ float quad_perm(float v)
+{
+	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xF, 0xF, true));
+}
+
+// 1/a: the fast reciprocal, or the division where a lane's value is out of its range.
+__device__ __forceinline__ float recip_wave(float a)
+{
+	float f = dev::recip_newton(a);
+	if (__builtin_expect(ballot(!dev::recip_newton_ok(a)) != 0ull, 0)) f = 1.0f / a;
+	return f;
+}
+
+// Sets r up from its record; false if it walks the binary nodes instead: a direction component
+// outside the fast reciprocal's range (zero among them) or an origin beyond 2^126, with which slab
+// values could be NaN.
+__device__ __forceinline__ bool quad_ray(const float4 a, const float4 b, dev::Ray& r)
+{
+	r.ox = a.x, r.oy = a.y, r.oz = a.z, r.tMin = a.w;
+	r.dx = b.x, r.dy = b.y, r.dz = b.z, r.tMax = b.w;
+	r.ix = dev::recip_newton(b.x);
+	r.iy = dev::recip_newton(b.y);
+	r.iz = dev::recip_newton(b.z);
+	auto within = [](float x) { return fabsf(x) >= 0x1p-126f && fabsf(x) < 0x1p126f; };
+	return within(b.x) && within(b.y) && within(b.z) && fabsf(a.x) <= 0x1p126f &&
+	       fabsf(a.y) <= 0x1p126f && fabsf(a.z) <= 0x1p126f;
+}
+
+// What a launch traces. Single casts: one scene, ray array and output. Batches: per ray through its
+// batch's descriptor (offsets in LDS).
+struct QuadArgs {
+	const float4* wide;         // (tris where the scene has no wide nodes)
 	const float4* nodes;
 	const float4* tris;
-	void* out;
-	uint32_t batch;
-	bool anyHit;
-	bool finiteBounds;
-	bool inTreelet;
+	const float4* rays;
+	void* out;                  // uint4 hits or uint8_t inLight flags
+	uint32_t n;                 // rays of the launch
+	uint32_t window;            // rays a wave claims at a time (at most 64)
+	uint32_t refill;       // idle rays of a wave before it takes new ones
+	uint32_t* work;             // kCounters window counters, then the retirement counters
+	U32x2* spill;
+	unsigned long long* clock;  // completion clock per ray, and the earliest block start in word n
+	const BatchDesc* descs;
+	const uint32_t* offsets;    // LDS
+	uint32_t numBatches;
+	unsigned long long* blockFinish;  // LDS, per batch (completion tracking)
+	uint32_t* blockDone;              // LDS, per batch
 };
 
-__device__ __forceinline__ void track_done(const MultiArgs& P, uint32_t batch)
+// One lane's state of its ray.
+struct Quad {
+	dev::Ray r;
+	uint32_t ray = kInvalid;     // index in the launch
+	uint32_t node = kInvalid;    // node to expand next, entered at nodeIn
+	float nodeIn = 0.0f;
+	bool leaf = false;           // triangles to test before it: this lane's is tri
+	uint32_t tri = 0u, triNext = 0u;  // triNext: lane 0's next one if the leaf goes on
+	uint32_t skip = 0u;          // lanes whose end marker is the first leaf's of a pair
+	int sp = 0;
+	uint32_t base = 0u;          // its stack column: LDS entry of the bottom row
+	float best = FLT_MAX, u = FLT_MAX, v = FLT_MAX;  // closest hit; u, v, hit in the lane it is `mine`
+	uint32_t hit = kInvalid;
+	bool mine = false;
+	bool exact = false;          // walks the binary nodes
+	// batches
+	const float4* wide = nullptr;
+	const float4* tris = nullptr;
+	uint32_t batch = 0u;
+	bool any = false;
+};
+
+// Writes a ray's result: its closest hit, or 0 if occluded and 1 if not.
+template <bool kBatch, bool kTrack, bool kClock>
+__device__ __forceinline__ void quad_result(const QuadArgs& P, uint32_t ray, uint32_t batch,
+                                            const Closest& c, bool any, bool occluded)
 {
-	// Block-local LDS atomics; flushed to the batch table when the block retires.
-	atomicAdd(&P.blockDone[batch], 1u);
-	atomicMax(&P.blockFinish[batch], wall_clock64());
+	void* out = P.out;
+	uint32_t at = ray;
+	if (kBatch) {
+		out = P.descs[batch].out;
+		at = ray - P.offsets[batch];
+	}
+	const U32x4 hit = {c.tri, __float_as_uint(c.t), __float_as_uint(c.u), __float_as_uint(c.v)};
+	if (any)
+		((GlobalU8*)(out))[at] = occluded ? 0 : 1;
+	else
+		((GlobalU4*)(out))[at] = hit;
+	if (kClock) P.clock[ray] = wall_clock64();
+	if (kTrack) {
+		atomicAdd(&P.blockDone[batch], 1u);
+		atomicMax(&P.blockFinish[batch], wall_clock64());
+	}
 }
 
-// pipe_step for the fused kernel: the same iteration, with the scene, output and kind taken from
-// each lane's batch (looked up in the batch table when the lane takes a new ray). A lane's result
-// is written with its own batch's output before a new ray's batch replaces it.
-template <bool kTreelet, bool kTrack, bool kExitCheck>
-__device__ __forceinline__ int pipe_step_multi(const MultiArgs& P, MultiTracer& M, LaneStack& st,
-                                               WaveQueue& q, BatchCursor& cur, BatchCursor& prev,
-                                               const Rec& A, Rec& B)
-{
-	__builtin_amdgcn_s_waitcnt(kWaitVmcntZero);
-	Tracer& L = M.t;
-	Counts none;
-	const uint32_t kind = L.kind;
-	uint32_t triFirst = 0u, triCnt = 0u;
-	bool anyHit = false;
-	if (kind == kRecTri) {
-		triFirst = L.s.triCur;
-		const uint32_t left = L.s.triEnd - triFirst;
-		triCnt = left < kTriBatch ? left : kTriBatch;
-		const bool rangeDone = left <= kTriBatch;
-		L.s.triCur = rangeDone ? L.s.pendCur : triFirst + kTriBatch;
-		L.s.triEnd = rangeDone ? L.s.pendEnd : L.s.triEnd;
-		L.s.pendCur = rangeDone ? 0u : L.s.pendCur;
-		L.s.pendEnd = rangeDone ? 0u : L.s.pendEnd;
-		if (M.anyHit) anyHit = test_pair_any(L.r, A, triCnt);
-	} else if (kind != kRecIdle) {
-		if (kind == kRecRay) {
-			L.r = dev::make_ray(A.w4, A.w5);
-			L.fastSlab = M.finiteBounds && L.r.nanFree;
-			L.c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
-			st.sp = 0;
-			L.s = {0u, 0u, 0u, 0u, -1};
-		}
-		NodeWords nd;
-		nd.w0 = A.w0;
-		nd.w1 = A.w1;
-		nd.w2 = A.w2;
-		nd.w3 = make_int4(__float_as_int(A.w3.x), __float_as_int(A.w3.y), __float_as_int(A.w3.z),
-		                  __float_as_int(A.w3.w));
-		const float tCurrMax = M.anyHit ? L.r.tMax : dev::min_first(L.r.tMax, L.c.t);
-		bool visitL, visitR;
-		decide(L.r, L.fastSlab, nd, tCurrMax, visitL, visitR);
-		expand_pipe(nd, visitL, visitR, L.s, st);
+// Rays [next, end) claimed by a wave (uniform). Its first window is its own, so that no launch starts
+// with all waves at one counter; the others come from a counter shared by every eighth block,
+// interleaved, so that costly regions of a ray array are spread over all of them.
+struct RayWindows {
+	uint32_t next = 0u, end = 0u;
+	uint32_t* counter;
+
+	__device__ __forceinline__ RayWindows(const QuadArgs& P, uint32_t waveInBlock)
+		: counter(P.work + blockIdx.x % kCounters * kCounterStride)
+	{
+		set(P, uint64_t(blockIdx.x * (blockDim.x / 64u) + waveInBlock) * P.window);
+	}
+	__device__ __forceinline__ void set(const QuadArgs& P, uint64_t first)
+	{
+		if (first >= P.n) return;
+		next = uint32_t(first);
+		end = P.n - next < P.window ? P.n : next + P.window;
+	}
+	// The next window; false if there is none.
+	__device__ __forceinline__ bool claim(const QuadArgs& P)
+	{
+		const uint32_t waves = gridDim.x * (blockDim.x / 64u);
+		const uint32_t counters = gridDim.x < kCounters ? gridDim.x : kCounters;
+		uint32_t b = 0u;
+		if (__lane_id() == 0u) b = atomicAdd(counter, 1u);
+		const uint64_t first =
+			(uint64_t(waves) + uint64_t(uniform(b)) * counters + blockIdx.x % kCounters) * P.window;
+		if (first >= P.n) return false;
+		set(P, first);
+		return true;
+	}
+};
+
+// kAny: the launch's any-hit rays: 0 none, 1 all, 2 per batch. kBig: a scene's triangles or wide
+// nodes take 4 GB or more, so 32-bit offsets into them do not do.
+template <int kAny, bool kBatch, bool kTrack, bool kClock, bool kBig, int kRows, uint32_t kCols>
+struct QuadTracer {
+	const QuadArgs& P;
+	LdsU2* stacks;       // the block's stack columns
+	uint32_t lane, l;
+	Quad q;
+
+	__device__ __forceinline__ bool isAny() const { return kAny == 1 || (kAny == 2 && q.any); }
+	__device__ __forceinline__ uint32_t nibble(bool p) const
+	{
+		const uint64_t b = ballot(p);
+		return uint32_t(b >> (lane & 60u)) & 15u;
+	}
+	// Entry `at` of the stack column: in LDS, or spilled (at >= kRows).
+	__device__ __forceinline__ LdsU2* row(int at) const { return stacks + (q.base + uint32_t(at) * kCols); }
+	__device__ __forceinline__ GlobalU2* spilled(int at) const
+	{
+		return spill_entry<kRows, kCols>(P.spill, q.base, at);
+	}
+	__device__ __forceinline__ U32x2 entry(int at) const
+	{
+		U32x2 e = {0u, 0u};
+		if (at < kRows) e = *row(at);
+		else e = *spilled(at);
+		return e;
 	}
 
-	const bool more = kind != kRecIdle && !anyHit && (L.s.triCur < L.s.triEnd || L.s.next >= 0);
-	uint32_t fresh = kInvalid;
-	if (!q.exhausted) {
-		const uint64_t freeLanes = __ballot(!more);
-		if (freeLanes != 0 && (uint32_t(__popcll(freeLanes)) >= P.refillMin || freeLanes == ~0ull)) {
-			const uint32_t start = q.start;
-			fresh = refill(q, freeLanes, P.work, P.total, !more, P.window);
-			if (q.start != start && !q.exhausted) {
-				// a new window (uniform): its batch, searched from the current one onwards
-				prev = cur;
-				cur.start = q.start;
-				cur.batch = batch_from(P.offsets, P.numBatches, cur.batch, cur.start);
+	// Sets this quad up for ray `ray`: its record, and if it is new its traversal.
+	__device__ __forceinline__ void start(uint32_t ray, bool fresh)
+	{
+		const float4* rays = P.rays;
+		uint32_t at = ray;
+		bool hasWide = P.wide != P.tris;
+		if (kBatch) {
+			if (fresh) q.batch = find_batch(P.offsets, P.numBatches, ray);
+			at = ray - P.offsets[q.batch];
+			const BatchDesc d = P.descs[q.batch];
+			rays = d.rays;
+			q.wide = d.wide;
+			q.tris = d.tris;
+			q.any = d.kind != 0u;
+			hasWide = d.wide != d.tris;
+		}
+		const float4 a = as_global(rays)[2 * size_t(at)], b = as_global(rays)[2 * size_t(at) + 1];
+		q.exact = !(quad_ray(a, b, q.r) && hasWide);
+		if (__builtin_expect(ballot(q.exact) != 0ull, 0)) {
+			q.r.ix = 1.0f / b.x;
+			q.r.iy = 1.0f / b.y;
+			q.r.iz = 1.0f / b.z;
+		}
+		q.ray = ray;
+		if (fresh) {
+			q.node = 0u;
+			q.nodeIn = -INFINITY;
+			q.leaf = false;
+			q.sp = 0;
+			q.best = q.u = q.v = FLT_MAX;
+			q.hit = kInvalid;
+			q.mine = l == 0u;
+		}
+	}
+
+	// Expands a binary node: lanes 0 and 1 decide its children as castRay does, and what is visited is
+	// pushed in castRay's order (left leaf, right leaf, right subtree, left subtree; decided now).
+	__device__ __forceinline__ void expand_binary(float lim)
+	{
+		const float4* nodes = kBatch ? P.descs[q.batch].nodes : P.nodes;
+		const float* f = reinterpret_cast<const float*>(nodes + 4u * size_t(q.node));
+		const float* box = f + 6u * (l & 1u);
+		const int32_t child = __float_as_int(f[12u + (l & 1u)]);
+		const bool isLeaf = __float_as_int(f[14u + (l & 1u)]) != 0;
+		float tIn, tOut;
+		dev::slab(q.r, box[0], box[1], box[2], box[3], box[4], box[5], tIn, tOut);
+		const bool pass = l < 2u && (tOut >= tIn) && tOut > q.r.tMin && tIn < lim;
+		const uint32_t m = nibble(pass);
+		const bool leftFirst = (nibble(pass && isLeaf) & 1u) != 0u;
+		const int at = q.sp + (m == 3u && (l == 0u) == leftFirst ? 1 : 0);
+		const U32x2 e = {child_index(child) | (isLeaf ? kWideLeaf : 0u), __float_as_uint(-INFINITY)};
+		if (pass) {
+			if (at < kRows) *row(at) = e;
+			else *spilled(at) = e;
+		}
+		q.sp += __popc(m);
+	}
+
+	// One iteration of the wave's rays.
+	__device__ __forceinline__ void step()
+	{
+		const bool active = q.ray != kInvalid;
+		const bool any = isAny();
+		const float4* wide = kBatch ? q.wide : P.wide;
+		const float4* tris = kBatch ? q.tris : P.tris;
+		// Straight-line loads, so that a leaf's and a node's are in flight together (in branches, the
+		// compiler waits for the first to test its end marker); quads without one read the array's
+		// first line. Offsets in bytes: 48 per triangle, 128 per wide node.
+		const uint32_t tri = q.leaf ? q.tri : 0u;
+		const uint32_t node = q.node != kInvalid && !q.exact ? q.node : 0u;
+		const float4* pl;
+		const float4* pn;
+		if (kBig) {
+			pl = tris + 3u * size_t(tri);
+			pn = wide + 8u * size_t(node) + 2u * l;
+		} else {
+			pl = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(tris) + ((tri + 2u * tri) << 4));
+			pn = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(wide) + ((node << 7) + (l << 5)));
+		}
+		const float4 p0 = as_global(pl)[0], e1 = as_global(pl)[1], e2 = as_global(pl)[2];
+		const float4 lo = as_global(pn)[0], hi = as_global(pn)[1];
+		bool more = false, occluded = false;
+		if (q.leaf) {
+			// The leaf's triangles up to its end marker; candidates are accepted in lane order, which
+			// is castRay's: the smallest t, the lowest lane on equal t.
+			const uint32_t ends = nibble(p0.w < 0.0f) & ~q.skip;
+			const bool inLeaf = (ends & ((1u << l) - 1u)) == 0u;
+			const dev::TriDet d = dev::tri_det(q.r, e1, e2);
+			const float f = recip_wave(d.a);
+			float t, u, v;
+			const bool hit = dev::tri_finish(q.r, d, f, p0, e1, e2, t, u, v) && inLeaf && q.r.tMin <= t;
+			if (kAny != 0) occluded = nibble(hit && t < q.r.tMax) != 0u && any;
+			if (kAny != 1 && !any) {
+				const bool cand = hit && t < q.best && t <= q.r.tMax;
+				float tm = cand ? t : INFINITY;
+				tm = fminf(tm, quad_perm<0xB1>(tm));  // lanes 1 0 3 2
+				tm = fminf(tm, quad_perm<0x4E>(tm));  // lanes 2 3 0 1
+				const bool least = cand && t == tm;
+				const uint32_t win = nibble(least);
+				const bool me = least && (win & ((1u << l) - 1u)) == 0u;
+				q.best = me ? t : fminf(q.best, tm);  // (its own t: a zero's sign)
+				q.mine = win != 0u ? me : q.mine;
+				q.u = me ? u : q.u;
+				q.v = me ? v : q.v;
+				q.hit = me ? q.tri : q.hit;
+			}
+			q.leaf = more = ends == 0u;
+			q.tri = q.triNext + l;
+			q.triNext += 4u;
+			q.skip = 0u;
+		}
+		const float lim = any ? q.r.tMax : dev::min_first(q.r.tMax, q.best);
+		if (__builtin_expect(q.exact && q.node != kInvalid && !more, 0)) {
+			expand_binary(lim);
+			q.node = kInvalid;
+		}
+		if (q.node != kInvalid && !more) {
+			// The passing slots are pushed, last slot first; a leaf pair stays one only if both pass.
+			float tIn;
+			const bool pass = decide_slot(q.r, lo, hi, lim, tIn) && (any || q.nodeIn < lim);
+			const uint32_t m = nibble(pass);
+			const uint32_t after = m >> (l + 1u);
+			uint32_t ref = __float_as_uint(lo.w);
+			ref = (after & 1u) ? ref : ref & ~kWidePair;
+			const int at = q.sp + __popc(after);
+			const U32x2 e = {ref, __float_as_uint(tIn)};
+			if (pass && at < kRows) *row(at) = e;
+			if (__builtin_expect(pass && at >= kRows, 0)) *spilled(at) = e;
+			q.sp += __popc(m);
+			q.node = kInvalid;
+		}
+		if (!active) return;
+		bool end = occluded;
+		if (!more && !occluded) {
+			// What comes next: the top entry that the closest hit has not overtaken; if it is a leaf,
+			// also its sibling (decided now, tested with it if the leaf has at most three
+			// triangles) and the entry below, if that is a node.
+			U32x2 x1, x2, x3;
+			if (__builtin_expect(q.sp <= kRows, 1)) {
+				const LdsU2* top = row(q.sp - 3);
+				x3 = top[0];
+				x2 = top[kCols];
+				x1 = top[2u * kCols];
+			} else {
+				x1 = entry(q.sp - 1);
+				x2 = entry(q.sp - 2);
+				x3 = entry(q.sp - 3);
+			}
+			if (!any)
+				while (q.sp > 0 && !(__uint_as_float(x1.y) < lim)) {
+					q.sp--;
+					x1 = x2;
+					x2 = x3;
+					x3 = entry(q.sp - 3);
+				}
+			if (q.sp == 0) {
+				end = true;
+			} else {
+				q.sp--;
+				if (!(x1.x & kWideLeaf)) {
+					q.node = x1.x;
+					q.nodeIn = __uint_as_float(x1.y);
+				} else {
+					const uint32_t first = x1.x & kWideIndex;
+					const uint32_t count = (x1.x >> kWideCountShift) & 3u;
+					q.leaf = true;
+					q.tri = first + l;
+					q.triNext = first + 4u;
+					q.skip = 0u;
+					U32x2 below = x2;
+					if (x1.x & kWidePair) {
+						const bool both = any || __uint_as_float(x2.y) < lim;
+						if (count != 0u) {
+							q.sp--;
+							below = x3;
+							if (both) {
+								const uint32_t at = (x2.x & kWideIndex) - count;
+								q.tri = l < count ? q.tri : at + l;
+								q.triNext = at + 4u;
+								q.skip = (1u << count) - 1u;
+							}
+						} else if (!any) {
+							const U32x2 e = {x2.x, __float_as_uint(both ? -INFINITY : INFINITY)};
+							if (q.sp <= kRows) *row(q.sp - 1) = e;
+							else *spilled(q.sp - 1) = e;
+						}
+					}
+					if (q.sp > 0 && !(below.x & kWideLeaf)) {
+						q.node = below.x;
+						q.nodeIn = __uint_as_float(below.y);
+						q.sp--;
+					}
+				}
 			}
 		}
+		if (end) {
+			const Closest c = {q.hit, q.best, q.u, q.v};
+			if (any ? l == 0u : q.mine)
+				quad_result<kBatch, kTrack, kClock>(P, q.ray, q.batch, c, any, occluded);
+			q.ray = kInvalid;
+			q.node = kInvalid;
+			q.leaf = false;
+		}
 	}
-	const bool tri = more && L.s.triCur < L.s.triEnd;
-	const bool node = more && !tri;
-	const bool ray = fresh != kInvalid;
-	// A new ray's batch: the largest b with offsets[b] <= its global index.
-	uint32_t nb = 0u, local = 0u;
-	BatchDesc nd{};
-	if (ray) {
-		nb = batch_from(P.offsets, P.numBatches, fresh >= cur.start ? cur.batch : prev.batch, fresh);
-		local = fresh - P.offsets[nb];
-		nd = P.descs[nb];
-	}
-	const uint32_t nextKind = tri ? kRecTri : node ? kRecNode : ray ? kRecRay : kRecIdle;
-	// The same six loads for every lane: a node, a triangle pair, or a new ray's root node and
-	// 32 B; idle lanes and words 4-5 of a node read their scene's root.
-	const float4* nodes = ray ? nd.nodes : M.nodes;
-	const uint32_t idx = tri ? L.s.triCur : node ? uint32_t(L.s.next) : 0u;
-	const uint32_t word = tri ? idx + (idx << 1) : idx << 2;
-	const float4* rec = (tri ? M.tris : nodes) + word;
-	const float4* src45 = tri ? rec + 4 : ray ? nd.rays + 2u * size_t(local) : nodes;
-	const bool inTreelet = ray ? nd.nodes == P.treeletNodes : M.inTreelet;
-	if (kTreelet && !tri && inTreelet && idx < P.topCount) {
-		const LdsF4* t = as_lds(P.treelet) + 4u * idx;
-		B.w0 = t[0];
-		B.w1 = t[1];
-		B.w2 = t[2];
-		B.w3 = t[3];
-	} else {
-		B.w0 = as_global(rec)[0];
-		B.w1 = as_global(rec)[1];
-		B.w2 = as_global(rec)[2];
-		B.w3 = as_global(rec)[3];
-	}
-	B.w4 = as_global(src45)[0];
-	B.w5 = as_global(src45)[1];
+};
 
-	if (kind == kRecTri && !M.anyHit) test_pair_closest<false>(L.r, A, triCnt, triFirst, L.c, none);
+template <int kAny, bool kBatch, bool kTrack, bool kClock, bool kBig>
+__device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
+{
+	const uint32_t waveInBlock = uniform(threadIdx.x >> 6), blockWaves = blockDim.x / 64u;
+	QuadTracer<kAny, kBatch, kTrack, kClock, kBig, kQuadRows, 16u> T{P};
+	T.stacks = (LdsU2*)(reinterpret_cast<U32x2*>(lds));
+	T.lane = __lane_id();
+	T.l = T.lane & 3u;
+	T.q.base = stack_base<kQuadRows, 16u>(waveInBlock, T.lane >> 2);
+	if (kClock && threadIdx.x == 0u) atomicMin(&P.clock[P.n], wall_clock64());
+	RayWindows W(P, waveInBlock);
+	while (true) {
+		const uint64_t idle = ballot(T.q.ray == kInvalid);
+		if (idle != 0ull) {
+			if (W.next >= W.end) {
+				if (!W.claim(P)) break;
+							if (W.next >= W.end) continue;
+			}
+			const uint32_t room = uint32_t(__popcll(idle)) / 4u;
+			if (room >= P.refill) {
+				const uint32_t ray = W.next + uint32_t(__popcll(idle & __lanemask_lt())) / 4u;
+				if (T.q.ray == kInvalid && ray < W.end) T.start(ray, true);
+				W.next = W.end - W.next < room ? W.end : W.next + room;
+			}
+		}
+		T.step();
+	}
 
-	if (kind != kRecIdle && !more) {
-		if (M.anyHit)
-			static_cast<uint8_t*>(M.out)[L.rayIdx] = anyHit ? 0 : 1;
-		else
-			static_cast<uint4*>(M.out)[L.rayIdx] = make_uint4(
-				L.c.tri, __float_as_uint(L.c.t), __float_as_uint(L.c.u), __float_as_uint(L.c.v));
-		if (kTrack) track_done(P, M.batch);
-	}
-	if (ray) {
-		M.nodes = nd.nodes;
-		M.tris = nd.tris;
-		M.out = nd.out;
-		M.batch = nb;
-		M.anyHit = nd.kind != 0u;
-		M.finiteBounds = nd.finiteBounds != 0u;
-		M.inTreelet = inTreelet;
-	}
-	if (!more) L.rayIdx = ray ? local : kInvalid;
-	L.kind = nextKind;
-	if (!kExitCheck || !q.exhausted) return kStepGo;
-	const uint64_t busy = __ballot(nextKind != kRecIdle);
-	if (busy == 0) return kStepDone;
-	return uint32_t(__popcll(busy)) <= solo_threshold(P.handoff) ? kStepSolo : kStepGo;
+	// The rays are handed out (a loop of its own: its state is only what step() needs).
+	while (ballot(T.q.ray != kInvalid) != 0ull) T.step();
+	__syncthreads();
 }
 
-template <bool kTreelet, bool kTrack>
-__device__ __forceinline__ void trace_batches(const BatchDesc* __restrict__ descs,
-                                              const uint32_t* __restrict__ offsetsGlobal,
-                                              uint32_t numBatches, uint32_t total,
-                                              uint32_t* __restrict__ work,
-                                              uint32_t* __restrict__ spill, uint32_t refillMin,
-                                              const float4* __restrict__ treeletNodes,
-                                              uint32_t topCount, uint32_t helpers, int depth,
-                                              uint32_t window, BatchClock* __restrict__ clock)
+// ---- one ray per lane, then four lanes per ray -----------------------------------------------------
+//
+// Fused launches, and the frame's bounce rays beside its shadow packets: a wave traces 64 rays, one a
+// lane, and once no rays are left to take and at most 16 are busy, those four lanes each, on the
+// stack columns that they have. A step of one ray per lane issues fewer instructions a ray (a wave
+// instruction serves 64 rays, not 16) but reads 64 lines with each load, takes a leaf and a node in
+// steps of their own and is as slow as its costliest lane, so four lanes per ray are the faster way
+// for a launch by itself (1,048,576 random rays, 4 waves per SIMD: 0.485 ms against 0.468 ms) and one
+// lane is where the device is full: 64 batches of 3.2 million rays on two scenes take 1.66 ms (2.3 ms
+// four lanes each; 1.80 ms with the binary nodes). There the texture data path is busy 85% of the
+// time, the VALUs 63%. Handing the records over in LDS, four lanes to a line, took it to 1.60 ms and
+// single casts from 0.106 to 0.123 ms, so each lane loads its own.
+
+template <int kAny, bool kBatch, bool kTrack, bool kClock>
+struct LaneTracer {
+	const QuadArgs& P;
+	LdsU2* stacks;
+	dev::Ray r;
+	uint32_t ray = kInvalid;
+	uint32_t ref = 0u;     // what the ray takes next: a node, or kWideLeaf and a triangle
+	int sp = 0;
+	uint32_t base = 0u;
+	Closest c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
+	bool exact = false, any = false;
+	uint32_t batch = 0u;
+	const float4* wide = nullptr;
+	const float4* tris = nullptr;
+
+	__device__ __forceinline__ bool isAny() const { return kAny == 1 || (kAny == 2 && any); }
+	__device__ __forceinline__ void put(bool on, int at, uint32_t ref, float tIn)
+	{
+		const U32x2 e = {ref, __float_as_uint(tIn)};
+		if (on && at < kLaneRows) stacks[base + uint32_t(at) * 64u] = e;
+		if (__builtin_expect(on && at >= kLaneRows, 0)) *spill_entry<kLaneRows, 64u>(P.spill, base, at) = e;
+	}
+	__device__ __forceinline__ U32x2 get(int at) const
+	{
+		U32x2 e = stacks[base + uint32_t(at < kLaneRows ? at : 0) * 64u];
+		if (__builtin_expect(at >= kLaneRows, 0)) e = *spill_entry<kLaneRows, 64u>(P.spill, base, at);
+		return e;
+	}
+
+	__device__ __forceinline__ void start(uint32_t index)
+	{
+		const float4* rays = P.rays;
+		uint32_t at = index;
+		bool hasWide = P.wide != P.tris;
+		if (kBatch) {
+			batch = find_batch(P.offsets, P.numBatches, index);
+			at = index - P.offsets[batch];
+			const BatchDesc d = P.descs[batch];
+			rays = d.rays;
+			wide = d.wide;
+			tris = d.tris;
+			any = d.kind != 0u;
+			hasWide = d.wide != d.tris;
+		}
+		const float4 a = as_global(rays)[2 * size_t(at)], b = as_global(rays)[2 * size_t(at) + 1];
+		exact = !(quad_ray(a, b, r) && hasWide);
+		if (__builtin_expect(exact, 0)) {
+			r.ix = 1.0f / b.x;
+			r.iy = 1.0f / b.y;
+			r.iz = 1.0f / b.z;
+		}
+		ray = index;
+		ref = 0u;
+		sp = 0;
+		c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
+	}
+
+	// Decides a binary node's children as castRay does and pushes what is visited in its order.
+	__device__ __forceinline__ void expand_binary(float lim)
+	{
+		const float4* nodes = kBatch ? P.descs[batch].nodes : P.nodes;
+		const NodeWords nd = load_node(nodes, ref);
+		bool visitL, visitR;
+		decide(r, nd, lim, visitL, visitR);
+		const uint32_t refL = child_index(nd.w3.x) | (nd.w3.z != 0 ? kWideLeaf : 0u);
+		const uint32_t refR = child_index(nd.w3.y) | (nd.w3.w != 0 ? kWideLeaf : 0u);
+		const bool leftFirst = visitL && nd.w3.z != 0;
+		put(visitL && visitR, sp, leftFirst ? refR : refL, -INFINITY);
+		put(visitL || visitR, sp + (visitL && visitR ? 1 : 0),
+		    visitL && visitR ? (leftFirst ? refL : refR) : visitL ? refL : refR, -INFINITY);
+		sp += (visitL ? 1 : 0) + (visitR ? 1 : 0);
+	}
+
+	__device__ __forceinline__ void step()
+	{
+		const bool active = ray != kInvalid;
+		const bool any = isAny();
+		const bool leaf = active && (ref & kWideLeaf) != 0u;
+		const bool node = active && !leaf && !exact;
+		const float4* wide = kBatch ? this->wide : P.wide;
+		const float4* tris = kBatch ? this->tris : P.tris;
+		const float4* rec = leaf ? tris + 3u * size_t(ref & kWideIndex) : wide + 8u * size_t(node ? ref : 0u);
+		float4 w[8];
+#pragma unroll
+		for (int i = 0; i < 8; i++) w[i] = as_global(rec)[i];
+		if (!active) return;
+		bool occluded = false, pop = true;
+		if (leaf) {
+			// Up to two triangles, accepted in order.
+			const dev::TriDet d0 = dev::tri_det(r, w[1], w[2]);
+			const dev::TriDet d1 = dev::tri_det(r, w[4], w[5]);
+			const float f0 = recip_wave(d0.a), f1 = recip_wave(d1.a);
+			float t0, u0, v0, t1, u1, v1;
+			const bool last0 = w[0].w < 0.0f;
+			const bool h0 = dev::tri_finish(r, d0, f0, w[0], w[1], w[2], t0, u0, v0) && r.tMin <= t0;
+			const bool h1 = dev::tri_finish(r, d1, f1, w[3], w[4], w[5], t1, u1, v1) && !last0 && r.tMin <= t1;
+			if (kAny != 0) occluded = any && ((h0 && t0 < r.tMax) || (h1 && t1 < r.tMax));
+			if (kAny != 1) {
+				const uint32_t first = ref & kWideIndex;
+				const bool acc0 = h0 && t0 < c.t && t0 <= r.tMax;
+				c.tri = acc0 ? first : c.tri;
+				c.t = acc0 ? t0 : c.t;
+				c.u = acc0 ? u0 : c.u;
+				c.v = acc0 ? v0 : c.v;
+				const bool acc1 = h1 && t1 < c.t && t1 <= r.tMax;
+				c.tri = acc1 ? first + 1u : c.tri;
+				c.t = acc1 ? t1 : c.t;
+				c.u = acc1 ? u1 : c.u;
+				c.v = acc1 ? v1 : c.v;
+			}
+			pop = last0 || w[3].w < 0.0f;
+			ref = kWideLeaf | ((ref & kWideIndex) + 2u);
+		}
+		const float lim = any ? r.tMax : dev::min_first(r.tMax, c.t);
+		float tIn = -INFINITY;
+		if (node) {
+			WideWords n;
+#pragma unroll
+			for (int i = 0; i < 8; i++) n.w[i] = w[i];
+			const WideVisit v = decide_wide(r, n, lim);
+			const bool p0 = v.pass[0], p1 = v.pass[1], p2 = v.pass[2], p3 = v.pass[3];
+			uint32_t r0 = __float_as_uint(w[0].w), r1 = __float_as_uint(w[2].w);
+			uint32_t r2 = __float_as_uint(w[4].w);
+			const uint32_t r3 = __float_as_uint(w[6].w);
+			r0 = p1 ? r0 : r0 & ~kWidePair;
+			r1 = p2 ? r1 : r1 & ~kWidePair;
+			r2 = p3 ? r2 : r2 & ~kWidePair;
+			const bool p01 = p0 || p1, p012 = p01 || p2;
+			const int at2 = sp + (p3 ? 1 : 0), at1 = at2 + (p2 ? 1 : 0);
+			put(p3 && p012, sp, r3, v.tIn[3]);
+			put(p2 && p01, at2, r2, v.tIn[2]);
+			put(p1 && p0, at1, r1, v.tIn[1]);
+			pop = !(p012 || p3);
+			sp = pop ? sp : at1 + (p1 ? 1 : 0) + (p0 ? 1 : 0) - 1;
+			ref = p0 ? r0 : p1 ? r1 : p2 ? r2 : r3;
+		}
+		if (__builtin_expect(exact && !leaf, 0)) expand_binary(lim);
+		bool end = occluded;
+		if (pop && !occluded) {
+			// The top entry that the closest hit has not overtaken.
+			end = true;
+			while (sp > 0) {
+				sp--;
+				const U32x2 e = get(sp);
+				if (any || __uint_as_float(e.y) < lim) {
+					ref = e.x;
+					end = false;
+					break;
+				}
+			}
+		}
+		if (!any && !end && (pop || node) && (ref & (kWideLeaf | kWidePair)) == (kWideLeaf | kWidePair)) {
+			// The sibling of a leaf that is taken is decided with it.
+			const U32x2 e = get(sp - 1);
+			put(true, sp - 1, e.x, __uint_as_float(e.y) < lim ? -INFINITY : INFINITY);
+		}
+		if (end) {
+			quad_result<kBatch, kTrack, kClock>(P, ray, batch, c, any, occluded);
+			ray = kInvalid;
+		}
+	}
+};
+
+template <int kAny, bool kBatch, bool kTrack, bool kClock>
+__device__ __forceinline__ void lane_trace(const QuadArgs& P, uint32_t* lds)
 {
-	extern __shared__ float4 ldsRaw[];
-	const uint32_t laneWaves = blockDim.x / 64u - helpers;
-	const uint32_t laneThreads = laneWaves * 64u;
-	uint32_t* ldsStacks = reinterpret_cast<uint32_t*>(ldsRaw);
-	float4* treelet = ldsRaw + laneWaves * (uint32_t(depth) + 1u) * 64u / 4u;
-	uint32_t* handoff = reinterpret_cast<uint32_t*>(treelet + 4u * topCount);
+	const uint32_t waveInBlock = uniform(threadIdx.x >> 6), lane = __lane_id();
+	LdsU2* stacks = (LdsU2*)(reinterpret_cast<U32x2*>(lds));
+	if (kClock && threadIdx.x == 0u) atomicMin(&P.clock[P.n], wall_clock64());
+	LaneTracer<kAny, kBatch, kTrack, kClock> T{P, stacks};
+	T.base = stack_base<kLaneRows, 64u>(waveInBlock, lane);
+	if (kBatch) {  // read by lanes without a ray
+		T.wide = P.descs[0].wide;
+		T.tris = P.descs[0].tris;
+	}
+	RayWindows W(P, waveInBlock);
+	while (true) {
+		const uint64_t idle = ballot(T.ray == kInvalid);
+		if (idle != 0ull) {
+			if (W.next >= W.end) {
+				if (!W.claim(P)) break;
+							if (W.next >= W.end) continue;
+			}
+			const uint32_t room = uint32_t(__popcll(idle));
+			if (room >= P.refill) {
+				const uint32_t ray = W.next + uint32_t(__popcll(idle & __lanemask_lt()));
+				if (T.ray == kInvalid && ray < W.end) T.start(ray);
+				W.next = W.end - W.next < room ? W.end : W.next + room;
+			}
+		}
+		T.step();
+	}
+	// No more rays: until at most 16 are left.
+	uint64_t busy = ballot(T.ray != kInvalid);
+	while (__popcll(busy) > 16) {
+		T.step();
+		busy = ballot(T.ray != kInvalid);
+	}
+	if (busy == 0ull) return;
+	// The k-th busy lane's ray goes to lanes 4k to 4k + 3.
+	QuadTracer<kAny, kBatch, kTrack, kClock, true, kLaneRows, 64u> Q{P};
+	Q.stacks = stacks;
+	Q.lane = lane;
+	Q.l = lane & 3u;
+	const uint32_t rank = uint32_t(__popcll(busy & __lanemask_lt()));
+	const bool on = T.ray != kInvalid;
+	auto move = [&](uint32_t v) {
+		// Lane 4k reads its source: the busy lanes push to it, all others to a lane that nobody reads.
+		const int to = on ? int(rank * 16u) : 4;
+		const uint32_t at4k = uint32_t(__builtin_amdgcn_ds_permute(to, int(v)));
+		return uint32_t(__builtin_amdgcn_update_dpp(0, int(at4k), 0x00, 0xF, 0xF, true));
+	};
+	const uint32_t ray = move(T.ray), ref = move(T.ref);
+	Q.q.sp = int(move(uint32_t(T.sp)));
+	Q.q.base = move(T.base);
+	const float best = __uint_as_float(move(__float_as_uint(T.c.t)));
+	const float u = __uint_as_float(move(__float_as_uint(T.c.u)));
+	const float v = __uint_as_float(move(__float_as_uint(T.c.v)));
+	const uint32_t hit = move(T.c.tri), batch = kBatch ? move(T.batch) : 0u;
+	if (lane / 4u < uint32_t(__popcll(busy))) {
+		Q.q.batch = batch;
+		Q.start(ray, false);
+		Q.q.best = best;
+		Q.q.u = u;
+		Q.q.v = v;
+		Q.q.hit = hit;
+		Q.q.mine = Q.l == 0u;
+		Q.q.leaf = (ref & kWideLeaf) != 0u;
+		Q.q.tri = (ref & kWideIndex) + Q.l;
+		Q.q.triNext = (ref & kWideIndex) + 4u;
+		Q.q.node = Q.q.leaf ? kInvalid : ref;
+		Q.q.nodeIn = -INFINITY;
+	}
+	if (kBatch && Q.q.ray == kInvalid) {  // read by lanes without a ray
+		Q.q.wide = P.descs[0].wide;
+		Q.q.tris = P.descs[0].tris;
+	}
+	while (ballot(Q.q.ray != kInvalid) != 0ull) Q.step();
+}
+
+// Called by every block as it ends: the last one resets the launch's counters. Counted per group of
+// blocks first, so that no address sees more than an eighth of them.
+__device__ __forceinline__ bool retire_block(uint32_t* work)
+{
+	const uint32_t group = blockIdx.x % kCounters;
+	const uint32_t inGroup = (gridDim.x - group + kCounters - 1u) / kCounters;
+	const uint32_t groups = gridDim.x < kCounters ? gridDim.x : kCounters;
+	__threadfence();
+	if (atomicAdd(&work[(kCounters + group) * kCounterStride], 1u) != inGroup - 1u) return false;
+	if (atomicAdd(&work[2u * kCounters * kCounterStride], 1u) != groups - 1u) return false;
+	for (uint32_t i = 0; i <= 2u * kCounters; i++) atomicExch(&work[i * kCounterStride], 0u);
+	return true;
+}
+
+__host__ __device__ __forceinline__ uint32_t lane_lds_words(uint32_t waves)
+{
+	return waves * 2u * wave_stack_entries<kLaneRows, 64u>();
+}
+
+template <bool kAnyHit, bool kClock, bool kBig>
+__global__ __launch_bounds__(kQuadBlock, kQuadWavesPerSimd) void k_quad(
+	const float4* __restrict__ wide, const float4* __restrict__ nodes,
+	const float4* __restrict__ tris, const float4* __restrict__ rays, void* __restrict__ out,
+	uint32_t n, uint32_t window, uint32_t refill, uint32_t* __restrict__ work,
+	U32x2* __restrict__ spill, unsigned long long* __restrict__ clock)
+{
+	extern __shared__ uint32_t lds[];
+	const QuadArgs P = {wide, nodes, tris, rays, out, n, window, refill, work, spill, clock,
+	                    nullptr, nullptr, 0u, nullptr, nullptr};
+	quad_trace<kAnyHit ? 1 : 0, false, false, kClock, kBig>(P, lds);
+	if (threadIdx.x == 0u) retire_block(work);
+}
+
+template <bool kAnyHit>
+__global__ __launch_bounds__(kQuadBlock, 4) void k_lane(
+	const float4* __restrict__ wide, const float4* __restrict__ nodes,
+	const float4* __restrict__ tris, const float4* __restrict__ rays, void* __restrict__ out,
+	uint32_t n, uint32_t window, uint32_t refillLanes, uint32_t* __restrict__ work,
+	U32x2* __restrict__ spill)
+{
+	extern __shared__ uint32_t lds[];
+	const QuadArgs P = {wide, nodes, tris, rays, out, n, window, refillLanes, work, spill, nullptr,
+	                    nullptr, nullptr, 0u, nullptr, nullptr};
+	lane_trace<kAnyHit ? 1 : 0, false, false, false>(P, lds);
+	__syncthreads();
+	if (threadIdx.x == 0u) retire_block(work);
+}
+
+// ---- fused multi-batch launch ---------------------------------------------------------------------
+//
+// One persistent launch over many ray batches (closest-hit or any-hit, on one or several scenes):
+// the batches' rays form one index space [0, total) handed out as above; a ray's index is mapped to
+// (batch, local index) by binary search over the batch offsets held in LDS, when its quad starts it.
+// With completion tracking on, the quads completing rays in the block count completions and the
+// latest completion time per batch in LDS, and every block adds them to the batch table with one
+// global atomic per batch when it ends, so each batch's latency inside the launch is known (the
+// clock only grows, so completion times need no reset between launches). The last block to end
+// resets the counters for the next launch.
+// Six waves per SIMD: a ray's scene, batch and kind take 70 registers.
+
+__host__ __device__ __forceinline__ uint32_t batch_lds_words(uint32_t waves, uint32_t numBatches,
+                                                             bool tracked)
+{
+	return lane_lds_words(waves) + (tracked ? 3u * numBatches : 0u) + numBatches + 1u;
+}
+
+template <bool kTrack>
+__global__ __launch_bounds__(kQuadBlock, 4) void k_trace_batches(
+	const BatchDesc* __restrict__ descs, const uint32_t* __restrict__ offsetsGlobal,
+	uint32_t numBatches, uint32_t total, uint32_t window, uint32_t refill,
+	uint32_t* __restrict__ work, U32x2* __restrict__ spill, BatchClock* __restrict__ clock)
+{
+	extern __shared__ uint32_t lds[];
+	// (An even number of words precedes the 8-byte finish times.)
 	unsigned long long* blockFinish =
-		reinterpret_cast<unsigned long long*>(handoff + handoff_bytes(laneThreads) / 4u);
+		reinterpret_cast<unsigned long long*>(lds + lane_lds_words(blockDim.x / 64u));
 	uint32_t* blockDone = reinterpret_cast<uint32_t*>(blockFinish + (kTrack ? numBatches : 0u));
 	uint32_t* offsets = blockDone + (kTrack ? numBatches : 0u);
 	if (kTrack && threadIdx.x == 0) atomicMin(&clock->start, wall_clock64());
-	for (uint32_t i = threadIdx.x; i < 4u * topCount; i += blockDim.x) treelet[i] = treeletNodes[i];
 	for (uint32_t i = threadIdx.x; i <= numBatches; i += blockDim.x) offsets[i] = offsetsGlobal[i];
 	if (kTrack)
 		for (uint32_t i = threadIdx.x; i < numBatches; i += blockDim.x) {
 			blockFinish[i] = 0ull;
 			blockDone[i] = 0u;
 		}
-	handoff_init(handoff, laneWaves);
 	__syncthreads();
-
-	const MultiArgs P = {descs, offsets, numBatches, total, work, refillMin,
-	                     kTreelet ? topCount : 0u, treeletNodes, treelet, blockFinish, blockDone,
-	                     handoff, window};
-	const uint32_t stride = gridDim.x * laneThreads;
-	// Traces the ray of a claimed slot solo.
-	auto runSlot = [&](uint32_t slot) {
-		uint32_t b;
-		const SoloStart S0 = solo_start_slot(handoff, slot, ldsStacks, spill, stride, depth, b);
-		const BatchDesc d = descs[b];
-		const SoloScene S = {d.nodes, d.tris, d.rays, d.out};
-		if (d.kind != 0u)
-			solo_run<true>(S, S0);
-		else
-			solo_run<false>(S, S0);
-		if (kTrack && __lane_id() == 0u) track_done(P, b);
-	};
-	const bool helper = is_helper(helpers);
-	if (helper) {
-		__builtin_amdgcn_s_setprio(3);
-		for (uint32_t slot = handoff_claim(handoff); slot != kInvalid; slot = handoff_claim(handoff))
-			runSlot(slot);
-	}
-
-	LaneStack st;
-	st.lds = ldsStacks + (threadIdx.x >> 6) * (uint32_t(depth) + 1u) * 64u;
-	st.depth = depth;
-	st.stride = stride;
-	st.spill = spill + (blockIdx.x * laneThreads + threadIdx.x);
-	st.lane = __lane_id();
-	st.sp = 0;
-	WaveQueue q;
-	BatchCursor cur, prev;
-	MultiTracer M;
-	Tracer& L = M.t;
-	L.c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
-	L.s = {0u, 0u, 0u, 0u, -1};
-	L.rayIdx = kInvalid;
-	L.doneIdx = kInvalid;
-	L.kind = kRecIdle;
-	L.fastSlab = false;
-	L.r = dev::make_ray(make_float4(0.f, 0.f, 0.f, 0.f), make_float4(1.f, 1.f, 1.f, 0.f));
-	// Until a lane takes its first ray, it reads batch 0's root node.
-	M.nodes = descs[0].nodes;
-	M.tris = descs[0].tris;
-	M.out = descs[0].out;
-	M.batch = 0u;
-	M.anyHit = false;
-	M.finiteBounds = false;
-	M.inTreelet = false;
-	const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-	Rec A = {z, z, z, z, z, z}, B = A;
-	int next = helper ? kStepDone : kStepGo;
-	while (next == kStepGo) {
-		pipe_step_multi<kTreelet, kTrack, false>(P, M, st, q, cur, prev, A, B);
-		next = pipe_step_multi<kTreelet, kTrack, true>(P, M, st, q, cur, prev, B, A);
-	}
-	if (!helper) {
-		// Solo: keep the first busy lane's ray, offer the others to the block, then trace offered
-		// rays until none is left.
-		const uint64_t busy = next == kStepSolo ? __ballot(L.kind != kRecIdle) : 0ull;
-		handoff_offer(handoff, busy & (busy - 1u), L, st, M.batch);
-		if (busy != 0) {
-			const uint32_t lsel = uint32_t(__builtin_ctzll(busy));
-			const uint32_t b = lane_u(M.batch, lsel);
-			const SoloStart S0 = solo_start_lane(L, st, lsel);
-			const BatchDesc d = descs[b];
-			const SoloScene S = {d.nodes, d.tris, d.rays, d.out};
-			if (d.kind != 0u)
-				solo_run<true>(S, S0);
-			else
-				solo_run<false>(S, S0);
-			if (kTrack && __lane_id() == 0u) track_done(P, b);
-		}
-		for (uint32_t slot = handoff_claim(handoff); slot != kInvalid; slot = handoff_claim(handoff))
-			runSlot(slot);
-	}
+	const QuadArgs P = {nullptr, nullptr, nullptr, nullptr, nullptr, total, window, refill, work,
+	                    spill, nullptr, descs, offsets, numBatches, blockFinish, blockDone};
+	lane_trace<2, true, kTrack, false>(P, lds);
+	__syncthreads();
 	if (kTrack) {
-		__syncthreads();
 		for (uint32_t b = threadIdx.x; b < numBatches; b += blockDim.x)
 			if (blockDone[b]) {
 				atomicAdd(&clock->done[b], blockDone[b]);
 				atomicMax(&clock->finish[b], blockFinish[b]);
 			}
-	}
-	// The last wave resets the shared counters (and, with tracking, the batch counters).
-	if (__lane_id() == 0) {
 		__threadfence();
-		const uint32_t totalWaves = gridDim.x * (blockDim.x / 64u);
-		const bool last = atomicAdd(&work[1], 1u) == totalWaves - 1u;
-		if (last) {
-			atomicExch(&work[0], 0u);
-			atomicExch(&work[1], 0u);
-			if (kTrack) {
-				for (uint32_t b = 0; b < numBatches; b++) atomicExch(&clock->done[b], 0u);
-				clock->lastStart = clock->start;
-				atomicExch(&clock->start, ~0ull);
-			}
-		}
+		__syncthreads();
 	}
-}
-
-template <bool kTreelet, bool kTrack>
-__global__ __launch_bounds__(kMaxBlock) void k_trace_batches(
-	const BatchDesc* __restrict__ descs, const uint32_t* __restrict__ offsetsGlobal,
-	uint32_t numBatches, uint32_t total, uint32_t* __restrict__ work,
-	uint32_t* __restrict__ spill, uint32_t refillMin, const float4* __restrict__ treeletNodes,
-	uint32_t topCount, uint32_t helpers, uint32_t depth, uint32_t window,
-	BatchClock* __restrict__ clock)
-{
-	trace_batches<kTreelet, kTrack>(descs, offsetsGlobal, numBatches, total, work, spill, refillMin,
-	                                treeletNodes, topCount, helpers, int(depth), window, clock);
+	if (threadIdx.x == 0u && retire_block(work) && kTrack) {
+		for (uint32_t b = 0; b < numBatches; b++) atomicExch(&clock->done[b], 0u);
+		clock->lastStart = atomicExch(&clock->start, ~0ull);
+	}
 }
 
 // ---- device self-check of the fast reciprocal -----------------------------------------------------
@@ -2216,18 +1813,57 @@ __global__ __launch_bounds__(kBlock) void k_check_reciprocal(bool exhaustive, ui
 
 uint32_t gridFor(uint32_t n, uint32_t block) { return n / block + (n % block != 0u); }
 
-// Persistent launch shape: grid capped by the work and by the spill area's lane count (lane-mode
-// threads only); the block is the lane-mode threads plus the helper waves.
-void persistentShape(const TraceLaunch& L, const SceneView& s, uint32_t n, uint32_t& grid,
-                     uint32_t& block, uint32_t& top, uint32_t& ldsBytes)
+// Whether 32-bit byte offsets into the scene's triangles and wide nodes do not do (kBig).
+bool bigScene(const SceneView& s)
 {
-	block = L.blockThreads + 64u * L.helperWaves;
-	top = L.topNodes < s.topCount ? L.topNodes : s.topCount;
-	grid = L.gridBlocks < gridFor(n, L.blockThreads) ? L.gridBlocks : gridFor(n, L.blockThreads);
-	const uint32_t maxGrid = L.spillLanes / L.blockThreads;
-	if (grid > maxGrid) grid = maxGrid;
-	if (grid == 0) grid = 1;
-	ldsBytes = persistent_lds_bytes(L.blockThreads, top, L.ldsDepth);
+	return size_t(s.numTris) * 48u >= (size_t(1) << 32) || size_t(s.numNodes) * 128u >= (size_t(1) << 32);
+}
+
+// Launch shapes of the persistent kernels for n rays. A launch keeps at most L.raysInFlight rays in
+// flight, each on a column of the spill area.
+struct Shape {
+	uint32_t grid, block, window, refill;
+};
+
+Shape shapeOf(uint32_t waves, uint32_t most, uint32_t block)
+{
+	while (block > 64u && block / 64u > most) block /= 2u;
+	const uint32_t perBlock = block / 64u;
+	return Shape{std::max(1u, std::min(gridFor(waves, perBlock), most / perBlock)), block, 0u, 0u};
+}
+
+// Four lanes per ray.
+//   - A launch that fills the device takes windows of 16 to 64 rays, two per wave at least, so that the
+//     last ones even out what the waves have left.
+//   - A launch that does not gives each wave as few rays as about 2,048 waves need (two per SIMD: a
+//     wave's time per iteration grows with the kinds of step its rays are at), up to the 16 it has
+//     lanes for.
+Shape quadShape(const TraceLaunch& L, uint32_t n)
+{
+	const uint32_t most = std::max(
+		1u, std::min(std::min(L.raysInFlight, L.spillColumns) / 16u, L.cus * kQuadWavesPerSimd * 4u));
+	const uint32_t window =
+		n / 16u >= most ? std::min(std::max(16u, n / (2u * most)), std::min(64u, std::max(16u, L.window)))
+		                : std::min(16u, std::max(gridFor(n, 2048u), gridFor(n, most)));
+	const uint32_t waves = std::min(most, gridFor(n, window));
+	Shape s = shapeOf(waves, most, 256u);  // (four waves: a CU holds seven such blocks)
+	s.window = window;
+	s.refill = std::min(16u, std::max(1u, L.refillMin / 4u));
+	return s;
+}
+
+// One ray per lane: windows of 64 rays; blocks small enough that every CU has one.
+Shape laneShape(const TraceLaunch& L, uint32_t n)
+{
+	const uint32_t most =
+		std::max(1u, std::min(std::min(L.raysInFlight, L.spillColumns) / 64u, L.cus * 16u));
+	const uint32_t waves = std::min(most, gridFor(n, 64u));
+	uint32_t block = kQuadBlock;
+	while (block > 64u && waves / (block / 64u) < L.cus) block /= 2u;
+	Shape s = shapeOf(waves, most, block);
+	s.window = 64u;
+	s.refill = kLaneRefill;
+	return s;
 }
 
 }  // namespace
@@ -2240,14 +1876,13 @@ void persistentShape(const TraceLaunch& L, const SceneView& s, uint32_t n, uint3
 // hipGetSymbolAddress returns for the current device, looked up once per device.
 static __device__ __align__(256) uint8_t
 	scratch[kNoAllocCounterBytes + size_t(kNoAllocSpillWords) * 4u];
-static_assert(kPersistentStack == int(kPersistentStackEntries), "stack entries per lane");
 
 namespace {
 
 std::mutex gScratchMu;
 void* gScratchPtr[kNoAllocMaxDevices] = {};
 
-// Zeroes `n` words (n <= 64); a kernel rather than a memset, so a caller may capture it in a graph.
+// Zeroes `n` words (n <= 1024); a kernel rather than a memset, so a caller may capture it in a graph.
 __global__ void k_zero_words(uint32_t* p, uint32_t n)
 {
 	if (threadIdx.x < n) p[threadIdx.x] = 0u;
@@ -2276,37 +1911,11 @@ void* noAllocScratch(int device)
 
 hipError_t launchZeroWords(uint32_t* p, uint32_t n, hipStream_t stream)
 {
-	hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, stream, p, n);
+	hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(1024), 0, stream, p, n);
 	return hipGetLastError();
 }
 
-uint32_t persistentSpillWords(uint32_t lanes)
-{
-	return uint32_t(kPersistentStack - kMinLdsDepth) * lanes;
-}
-
-bool validLdsDepth(uint32_t depth)
-{
-	return depth >= uint32_t(kMinLdsDepth) && depth <= uint32_t(kMaxLdsDepth);
-}
-
-uint32_t persistentLdsBytes(uint32_t blockThreads, uint32_t topNodes, uint32_t ldsDepth)
-{
-	return persistent_lds_bytes(blockThreads, topNodes, ldsDepth);
-}
-
-hipError_t persistentBlocksPerCU(uint32_t blockThreads, uint32_t topNodes, uint32_t helperWaves,
-                                 uint32_t ldsDepth, uint32_t* blocks)
-{
-	int a = 0;
-	const void* fn = topNodes ? reinterpret_cast<const void*>(k_closest_persistent<false, true>)
-	                          : reinterpret_cast<const void*>(k_closest_persistent<false, false>);
-	hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-		&a, fn, int(blockThreads + 64u * helperWaves),
-		persistent_lds_bytes(blockThreads, topNodes, ldsDepth));
-	*blocks = uint32_t(a > 0 ? a : 0);
-	return e;
-}
+static_assert(kRayCounterWords >= (2u * kCounters + 1u) * kCounterStride, "ray counters");
 
 hipError_t launchCheckReciprocal(bool exhaustive, unsigned long long* mismatches, uint64_t* tested,
                                  hipStream_t stream)
@@ -2332,24 +1941,29 @@ hipError_t launchClosest(const SceneView& s, const PhxRayIn* rays, uint32_t n, P
 		                   stream, wide, nodes, tris, r4, static_cast<void*>(h4), n);
 		return hipGetLastError();
 	}
-	if (L.kernel != TraceKernel::Persistent || n > 0x7FFFFFFFu) {
-		if (counters)
-			hipLaunchKernelGGL(k_closest_simple<true>, dim3(gridFor(n, kBlock)), dim3(kBlock), 0,
-			                   stream, wide, nodes, tris, r4, h4, n, counters);
-		else
-			hipLaunchKernelGGL(k_closest_simple<false>, dim3(gridFor(n, kBlock)), dim3(kBlock), 0,
-			                   stream, wide, nodes, tris, r4, h4, n, counters);
+	// Counters count binary node visits, which the one-ray-per-lane kernel makes.
+	if (counters) {
+		hipLaunchKernelGGL(k_closest_simple<true>, dim3(gridFor(n, kBlock)), dim3(kBlock), 0, stream,
+		                   wide, nodes, tris, r4, h4, n, counters);
 		return hipGetLastError();
 	}
-	uint32_t grid, block, top, lds;
-	TraceLaunch shape = L;
-	if (counters) shape.helperWaves = 0;  // the counting variant traces every ray in lane mode
-	persistentShape(shape, s, n, grid, block, top, lds);
-	auto kernel = counters ? (top ? k_closest_persistent<true, true> : k_closest_persistent<true, false>)
-	                       : (top ? k_closest_persistent<false, true> : k_closest_persistent<false, false>);
-	hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), lds, stream, nodes, tris, r4, h4, n,
-	                   L.work, L.spill, L.refillMin, s.finiteBounds, top, shape.helperWaves,
-	                   L.ldsDepth, L.window, counters);
+	if (L.kernel == TraceKernel::Simple || L.kernel == TraceKernel::Packet || n > 0x7FFFFFFFu) {
+		hipLaunchKernelGGL(k_closest_simple<false>, dim3(gridFor(n, kBlock)), dim3(kBlock), 0, stream,
+		                   wide, nodes, tris, r4, h4, n, nullptr);
+		return hipGetLastError();
+	}
+	if (L.kernel == TraceKernel::Lane) {
+		const Shape q = laneShape(L, n);
+		hipLaunchKernelGGL(k_lane<false>, dim3(q.grid), dim3(q.block), lane_lds_words(q.block / 64u) * 4u,
+		                   stream, wide ? wide : tris, nodes, tris, r4, static_cast<void*>(h4), n,
+		                   q.window, q.refill, L.work, reinterpret_cast<U32x2*>(L.spill));
+		return hipGetLastError();
+	}
+	const Shape q = quadShape(L, n);
+	auto kernel = bigScene(s) ? k_quad<false, false, true> : k_quad<false, false, false>;
+	hipLaunchKernelGGL(kernel, dim3(q.grid), dim3(q.block), quad_lds_words(q.block / 64u) * 4u, stream,
+	                   wide ? wide : tris, nodes, tris, r4, static_cast<void*>(h4), n, q.window, q.refill,
+	                   L.work, reinterpret_cast<U32x2*>(L.spill), nullptr);
 	return hipGetLastError();
 }
 
@@ -2358,15 +1972,15 @@ hipError_t launchClosestClock(const SceneView& s, const PhxRayIn* rays, uint32_t
 {
 	if (n == 0) return hipSuccess;
 	if (n > 0x7FFFFFFFu) return hipErrorInvalidValue;
-	uint32_t grid, block, top, lds;
-	persistentShape(L, s, n, grid, block, top, lds);
-	auto kernel = top ? k_closest_persistent<false, true, true> : k_closest_persistent<false, false, true>;
-	hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), lds, stream,
-	                   reinterpret_cast<const float4*>(s.nodes),
-	                   reinterpret_cast<const float4*>(s.trisPre),
-	                   reinterpret_cast<const float4*>(rays), reinterpret_cast<uint4*>(hits), n,
-	                   L.work, L.spill, L.refillMin, s.finiteBounds, top, L.helperWaves, L.ldsDepth,
-	                   L.window, clock);
+	const float4* nodes = reinterpret_cast<const float4*>(s.nodes);
+	const float4* tris = reinterpret_cast<const float4*>(s.trisPre);
+	const float4* wide = s.wide ? reinterpret_cast<const float4*>(s.wide) : tris;
+	const Shape q = quadShape(L, n);
+	auto kernel = k_quad<false, true, true>;
+	hipLaunchKernelGGL(kernel, dim3(q.grid), dim3(q.block), quad_lds_words(q.block / 64u) * 4u, stream,
+	                   wide, nodes, tris, reinterpret_cast<const float4*>(rays),
+	                   static_cast<void*>(hits), n, q.window,
+	                   q.refill, L.work, reinterpret_cast<U32x2*>(L.spill), clock);
 	return hipGetLastError();
 }
 
@@ -2421,54 +2035,30 @@ hipError_t launchAnyHit(const SceneView& s, const PhxRayIn* rays, uint32_t n, ui
 		                   stream, wide, nodes, tris, r4, inLight, n, nullptr);
 		return hipGetLastError();
 	}
-	uint32_t grid, block, top, lds;
-	persistentShape(L, s, n, grid, block, top, lds);
-	hipLaunchKernelGGL(top ? k_anyhit_persistent<true> : k_anyhit_persistent<false>, dim3(grid),
-	                   dim3(block), lds, stream, nodes, tris, r4, inLight, n, L.work, L.spill,
-	                   L.refillMin, s.finiteBounds, top, L.helperWaves, L.ldsDepth, L.window);
+	if (L.kernel == TraceKernel::Lane) {
+		const Shape q = laneShape(L, n);
+		hipLaunchKernelGGL(k_lane<true>, dim3(q.grid), dim3(q.block), lane_lds_words(q.block / 64u) * 4u,
+		                   stream, wide ? wide : tris, nodes, tris, r4, static_cast<void*>(inLight), n,
+		                   q.window, q.refill, L.work, reinterpret_cast<U32x2*>(L.spill));
+		return hipGetLastError();
+	}
+	const Shape q = quadShape(L, n);
+	auto kernel = bigScene(s) ? k_quad<true, false, true> : k_quad<true, false, false>;
+	hipLaunchKernelGGL(kernel, dim3(q.grid), dim3(q.block), quad_lds_words(q.block / 64u) * 4u, stream,
+	                   wide ? wide : tris, nodes, tris, r4, static_cast<void*>(inLight), n, q.window, q.refill,
+	                   L.work, reinterpret_cast<U32x2*>(L.spill), nullptr);
 	return hipGetLastError();
 }
 
-uint32_t batchLdsBytes(uint32_t blockThreads, uint32_t topNodes, uint32_t numBatches,
-                       bool tracked, uint32_t ldsDepth)
-{
-	return persistent_lds_bytes(blockThreads, topNodes, ldsDepth) + (numBatches + 1u) * 4u +
-	       (tracked ? numBatches * 12u : 0u);
-}
-
-hipError_t batchBlocksPerCU(uint32_t blockThreads, uint32_t topNodes, uint32_t helperWaves,
-                            uint32_t ldsDepth, uint32_t numBatches, bool tracked,
-                            uint32_t* blocks)
-{
-	int a = 0;
-	const void* fn =
-		tracked ? (topNodes ? reinterpret_cast<const void*>(k_trace_batches<true, true>)
-		                    : reinterpret_cast<const void*>(k_trace_batches<false, true>))
-		        : (topNodes ? reinterpret_cast<const void*>(k_trace_batches<true, false>)
-		                    : reinterpret_cast<const void*>(k_trace_batches<false, false>));
-	hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-		&a, fn, int(blockThreads + 64u * helperWaves),
-		batchLdsBytes(blockThreads, topNodes, numBatches, tracked, ldsDepth));
-	*blocks = uint32_t(a > 0 ? a : 0);
-	return e;
-}
-
 hipError_t launchBatches(const BatchDesc* descs, const uint32_t* offsets, uint32_t numBatches,
-                         uint32_t total, const TraceLaunch& L, const float4* treeletNodes,
-                         uint32_t treeletCount, BatchClock* clock, hipStream_t stream)
+                         uint32_t total, const TraceLaunch& L, BatchClock* clock, hipStream_t stream)
 {
 	if (total == 0) return hipSuccess;
-	const uint32_t block = L.blockThreads;  // lane-mode threads; helper waves come on top
-	const uint32_t top = L.topNodes < treeletCount ? L.topNodes : treeletCount;
-	uint32_t grid = L.gridBlocks < gridFor(total, block) ? L.gridBlocks : gridFor(total, block);
-	if (grid > L.spillLanes / block) grid = L.spillLanes / block;
-	if (grid == 0) grid = 1;
-	auto kernel = clock ? (top ? k_trace_batches<true, true> : k_trace_batches<false, true>)
-	                    : (top ? k_trace_batches<true, false> : k_trace_batches<false, false>);
-	hipLaunchKernelGGL(kernel, dim3(grid), dim3(block + 64u * L.helperWaves),
-	                   batchLdsBytes(block, top, numBatches, clock != nullptr, L.ldsDepth), stream,
-	                   descs, offsets, numBatches, total, L.work, L.spill, L.refillMin, treeletNodes,
-	                   top, L.helperWaves, L.ldsDepth, L.window, clock);
+	const Shape q = laneShape(L, total);
+	hipLaunchKernelGGL(clock ? k_trace_batches<true> : k_trace_batches<false>, dim3(q.grid),
+	                   dim3(q.block), batch_lds_words(q.block / 64u, numBatches, clock != nullptr) * 4u,
+	                   stream, descs, offsets, numBatches, total, 64u, q.refill, L.work,
+	                   reinterpret_cast<U32x2*>(L.spill), clock);
 	return hipGetLastError();
 }
 

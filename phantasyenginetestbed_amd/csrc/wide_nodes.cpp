@@ -88,12 +88,15 @@ WideNode emptyNode()
 {
 	WideNode w;
 	const float nan = std::numeric_limits<float>::quiet_NaN();
-	for (int i = 0; i < 4; i++) {
-		for (int k = 0; k < 6; k++) w.box[i][k] = nan;
-		w.ref[i] = 0u;
-		w.pad[i] = 0u;
-	}
+	for (WideNode::Slot& s : w.slot) s = WideNode::Slot{{nan, nan, nan}, 0u, {nan, nan, nan}, 0u};
 	return w;
+}
+
+void setSlot(WideNode::Slot& s, const float* box, uint32_t ref)
+{
+	std::memcpy(s.min, box, sizeof(s.min));
+	std::memcpy(s.max, box + 3, sizeof(s.max));
+	s.ref = ref;
 }
 
 }  // namespace
@@ -127,22 +130,19 @@ std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint
 	}
 	for (int j = 0; j < numRoot; j++) {
 		const Slot& a = s[rs[j].first];
-		std::memcpy(out[0].box[j], a.box, sizeof(out[0].box[j]));
+		setSlot(out[0].slot[j], a.box, uint32_t(j + 1));
 		if (rs[j].count == 2) {
 			const Slot& b = s[rs[j].first + 1];
 			for (int k = 0; k < 3; k++) {
-				out[0].box[j][k] = std::min(a.box[k], b.box[k]);
-				out[0].box[j][k + 3] = std::max(a.box[k + 3], b.box[k + 3]);
+				out[0].slot[j].min[k] = std::min(a.box[k], b.box[k]);
+				out[0].slot[j].max[k] = std::max(a.box[k + 3], b.box[k + 3]);
 			}
 		}
-		out[0].ref[j] = uint32_t(j + 1);
 		out.push_back(emptyNode());
 		const uint32_t pending = uint32_t(numRoot - 1 - j);
 		if (a.leaf) {
-			for (int i = 0; i < rs[j].count; i++) {
-				std::memcpy(out[size_t(j) + 1].box[i], s[rs[j].first + i].box, 24);
-				out[size_t(j) + 1].ref[i] = s[rs[j].first + i].ref;
-			}
+			for (int i = 0; i < rs[j].count; i++)
+				setSlot(out[size_t(j) + 1].slot[i], s[rs[j].first + i].box, s[rs[j].first + i].ref);
 			maxPending = std::max(maxPending, pending + 1u);
 		} else {
 			queue.push_back(Item{uint32_t(j + 1), a.ref, pending});
@@ -156,12 +156,11 @@ std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint
 		const int k = collapse(nodes, it.node, t);
 		maxPending = std::max(maxPending, it.pending + uint32_t(k - 1));
 		for (int i = 0; i < k; i++) {
-			std::memcpy(out[it.at].box[i], t[i].box, 24);
 			if (t[i].leaf) {
-				out[it.at].ref[i] = t[i].ref;
+				setSlot(out[it.at].slot[i], t[i].box, t[i].ref);
 			} else {
 				const uint32_t child = uint32_t(out.size());
-				out[it.at].ref[i] = child;
+				setSlot(out[it.at].slot[i], t[i].box, child);
 				out.push_back(emptyNode());
 				next.push_back(Item{child, t[i].ref, it.pending + uint32_t(k - 1 - i)});
 			}

@@ -34,14 +34,17 @@ constexpr uint32_t kWideIndex = 0x0FFFFFFFu;
 constexpr uint32_t kWideCountShift = 28u;
 
 // Pending slots a traversal may hold (the kernels' stacks hold this many 8-byte entries).
-constexpr uint32_t kWideMaxPending = 36u;
+constexpr uint32_t kWideMaxPending = 60u;
 
-// 128 B, so that a record is one cache line: boxes as (min.xyz, max.xyz) per slot, then the
-// references. Empty slots have NaN boxes, which no ray passes.
+// 128 B, one cache line: a 32-B record per slot, so that four lanes read one slot each and one lane
+// reads a slot in two 16-B words. Empty slots have NaN boxes, which no ray passes.
 struct WideNode {
-	float box[4][6];
-	uint32_t ref[4];
-	uint32_t pad[4];
+	struct Slot {
+		float min[3];
+		uint32_t ref;
+		float max[3];
+		uint32_t pad;
+	} slot[4];
 };
 static_assert(sizeof(WideNode) == 128, "WideNode is one 128-B line");
 

@@ -36,14 +36,14 @@ bool walk(const std::vector<WideNode>& wide, const OrTri* tris, const OrRay& r, 
 			bool pass[4];
 			for (int i = 0; i < 4; i++) {
 				float tOut;
-				const float* b = n.box[i];
-				const bool hit = oracle_aabb(r.o, r.d, b, b + 3, &tIn[i], &tOut) != 0;
+				const WideNode::Slot& b = n.slot[i];
+				const bool hit = oracle_aabb(r.o, r.d, b.min, b.max, &tIn[i], &tOut) != 0;
 				pass[i] = hit && tOut > r.tMin && tIn[i] < lim;
 			}
 			for (int i = 3; i >= 0; i--)
 				if (pass[i]) {
 					if (have) stack[sp++] = cur;
-					cur = {tIn[i], n.ref[i]};
+					cur = {tIn[i], n.slot[i].ref};
 					if (cur.ref & kWidePair && !(i < 3 && pass[i + 1])) cur.ref &= ~kWidePair;
 					have = true;
 				}
@@ -86,7 +86,7 @@ extern "C" uint32_t wide_check(const PhxBVHNode* nodes, uint32_t numNodes, const
 	if (wide.empty()) return 0;
 	// The root's slots refer to nodes 1, 2, ... in order.
 	for (uint32_t i = 0; i < 4; i++)
-		if (wide[0].box[i][0] == wide[0].box[i][0] && wide[0].ref[i] != i + 1u) return 0;
+		if (wide[0].slot[i].min[0] == wide[0].slot[i].min[0] && wide[0].slot[i].ref != i + 1u) return 0;
 	OrHit unused;
 	for (uint32_t i = 0; i < n; i++) {
 		walk(wide, tris, rays[i], false, hits[i], *deepest);

@@ -13,7 +13,7 @@ from oracle import oracle as O
 from phantasyenginetestbed_amd import phx
 
 ROOT = Path(__file__).resolve().parents[1]
-CAPACITY = 36
+CAPACITY = 60
 
 
 @pytest.fixture(scope="module")
