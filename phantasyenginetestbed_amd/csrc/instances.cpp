@@ -24,7 +24,8 @@ using namespace phx;
 struct PhxInstanceSet {
 	PhxContext* ctx = nullptr;
 	uint32_t count = 0;
-	PhxBVHNode* top = nullptr;    // device: top tree, one instance per leaf
+	PhxBVHNode* top = nullptr;    // device: top tree, one instance per leaf, 64 B of padding
+	WideNode* topWide = nullptr;  // device: its wide nodes, null if it cannot have them
 	DevInstance* inst = nullptr;  // device: instances in top-tree leaf order
 	DevInstance* byIndex = nullptr;  // device: instances in the caller's order (hit records)
 	std::vector<const PhxScene*> meshes;  // distinct meshes, held until release
@@ -183,6 +184,7 @@ phx_status checkSet(PhxContext* ctx, const PhxInstanceSet* set)
 void freeSet(PhxInstanceSet* s)
 {
 	hipFree(s->top);
+	hipFree(s->topWide);
 	hipFree(s->inst);
 	hipFree(s->byIndex);
 	for (const PhxScene* m : s->meshes) dropScene(m);
@@ -194,6 +196,7 @@ void freeSet(PhxInstanceSet* s)
 namespace phx {
 
 const PhxBVHNode* instanceTop(const PhxInstanceSet* s) { return s->top; }
+const WideNode* instanceTopWide(const PhxInstanceSet* s) { return s->topWide; }
 const DevInstance* instanceArray(const PhxInstanceSet* s) { return s->inst; }
 const DevInstance* instanceByIndex(const PhxInstanceSet* s) { return s->byIndex; }
 uint32_t instanceCount(const PhxInstanceSet* s) { return s->count; }
@@ -226,6 +229,8 @@ static phx_status phx_instances_build_impl(PhxContext* ctx, const PhxInstance* i
 		    !worldBox(in.objectToWorld, in.mesh->rootMin, in.mesh->rootMax, boxes[i]))
 			return fail(PHX_ERR_INVALID_ARGUMENT, "phx_instances_build: instance %u has a singular "
 			            "or non-finite transform", i);
+		d.wide = in.mesh->wide ? reinterpret_cast<const float4*>(in.mesh->wide)
+		                       : reinterpret_cast<const float4*>(in.mesh->tris);
 		d.nodes = reinterpret_cast<const float4*>(in.mesh->nodes);
 		d.tris = reinterpret_cast<const float4*>(in.mesh->tris);
 		d.datas = in.mesh->datas;
@@ -252,9 +257,12 @@ static phx_status phx_instances_build_impl(PhxContext* ctx, const PhxInstance* i
 		}
 		std::vector<DevInstance> laid(count);
 		for (size_t slot = 0; slot < tb.order.size(); slot++) laid[slot] = dev[tb.order[slot]];
+		const std::vector<WideNode> wide = buildWide(tb.nodes.data(), uint32_t(tb.nodes.size()), 0u);
 		size_t bytes = 0;
-		if (hipMalloc(reinterpret_cast<void**>(&s->top), tb.nodes.size() * sizeof(PhxBVHNode)) !=
+		if (hipMalloc(reinterpret_cast<void**>(&s->top), (tb.nodes.size() + 1u) * sizeof(PhxBVHNode)) !=
 		        hipSuccess ||
+		    (!wide.empty() && hipMalloc(reinterpret_cast<void**>(&s->topWide),
+		                                wide.size() * sizeof(WideNode)) != hipSuccess) ||
 		    hipMalloc(reinterpret_cast<void**>(&s->inst), laid.size() * sizeof(DevInstance)) !=
 		        hipSuccess ||
 		    hipMalloc(reinterpret_cast<void**>(&s->byIndex), dev.size() * sizeof(DevInstance)) !=
@@ -265,6 +273,9 @@ static phx_status phx_instances_build_impl(PhxContext* ctx, const PhxInstance* i
 		bytes = tb.nodes.size() * sizeof(PhxBVHNode);
 		hipError_t e = hipMemcpyAsync(s->top, tb.nodes.data(), bytes, hipMemcpyHostToDevice,
 		                              ctx->stream);
+		if (e == hipSuccess && !wide.empty())
+			e = hipMemcpyAsync(s->topWide, wide.data(), wide.size() * sizeof(WideNode),
+			                   hipMemcpyHostToDevice, ctx->stream);
 		if (e == hipSuccess)
 			e = hipMemcpyAsync(s->inst, laid.data(), laid.size() * sizeof(DevInstance),
 			                   hipMemcpyHostToDevice, ctx->stream);
@@ -314,14 +325,14 @@ hipError_t enqueueInstanceCast(PhxContext* ctx, const PhxScene* scene, const Phx
                                uint8_t* inLight)
 {
 	hipError_t e = hipSuccess;
+	const TraceLaunch L = traceLaunch(ctx, 0, inLight != nullptr);
 	if (scene) {
-		const TraceLaunch L = traceLaunch(ctx, 0, inLight != nullptr);
 		e = inLight ? launchAnyHit(view(scene), rays, n, inLight, L, ctx->stream)
 		            : launchClosest(view(scene), rays, n, hits, L, nullptr, ctx->stream);
 	}
 	if (e == hipSuccess)
-		e = launchInstances(set->top, set->inst, set->count, rays, n, hits, ids, inLight,
-		                    scene != nullptr, ctx->stream);
+		e = launchInstances(set->top, set->topWide, set->inst, set->count, rays, n, hits, ids, inLight,
+		                    scene != nullptr, L, ctx->stream);
 	return e;
 }
 

@@ -74,6 +74,7 @@ hipError_t launchZeroWords(uint32_t* p, uint32_t n, hipStream_t stream);
 // One instance of a two-level scene on the device: its SBVH (the mesh scene's node and
 // pre-transformed triangle arrays) and the world-to-object affine transform, rows (A | b).
 struct DevInstance {
+	const float4* wide;            // the mesh's wide nodes, or `tris` if it has none
 	const float4* nodes;
 	const float4* tris;
 	const PhxTriangleData* datas;  // for hit records (may be null)
@@ -84,11 +85,12 @@ struct DevInstance {
 
 // Closest hit (inLight == nullptr; hits and optionally instOut written) or any hit (inLight) of
 // every ray against the instances under the top tree `top` (one instance per leaf; `inst` in
-// top-tree leaf order). `seeded`: hits / inLight hold the static scene's results on entry, which
+// top-tree leaf order; topWide: its wide nodes or null, then `top` has 64 B of padding).
+// L: the ray counters. `seeded`: hits / inLight hold the static scene's results on entry, which
 // win ties (closest) or already occlude (any hit).
-hipError_t launchInstances(const PhxBVHNode* top, const DevInstance* inst, uint32_t numInst,
-                           const PhxRayIn* rays, uint32_t n, PhxRayHit* hits, uint32_t* instOut,
-                           uint8_t* inLight, bool seeded, hipStream_t stream);
+hipError_t launchInstances(const PhxBVHNode* top, const WideNode* topWide, const DevInstance* inst,
+                           uint32_t numInst, const PhxRayIn* rays, uint32_t n, PhxRayHit* hits, uint32_t* instOut,
+                           uint8_t* inLight, bool seeded, const TraceLaunch& L, hipStream_t stream);
 
 // Any hit of every ray (one ray per lane) adding castDebugRay-style counters of the any-hit
 // traversal (trianglesIntersected = rays occluded) to counters[0..4].

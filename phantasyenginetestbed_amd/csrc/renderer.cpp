@@ -38,6 +38,7 @@ struct PhxRenderer {
 	const PhxInstanceSet* instances = nullptr;
 	uint32_t* primInst = nullptr;
 	uint32_t* bounceInst = nullptr;
+	uint32_t* instWork = nullptr;  // ray counters of the instance casts on the frame's stream
 	float4* lastOut = nullptr;
 	FrameParams* params = nullptr;  // per-frame values the frame kernels read (device)
 	// The bounce rays' closest hits run on a side stream beside the primary shadow rays (fork
@@ -79,7 +80,7 @@ void freeRenderer(PhxRenderer* r)
 	void* bufs[] = {r->prim,    r->primHits, r->gbuf,   r->bounce,  r->throughput,
 	                r->bounceHits, r->bounceInfo, r->contrib, r->shadow, r->inLight,
 	                r->color,   r->hist[0],  r->hist[1], r->out,    r->params,
-	                r->vel[0],  r->vel[1], r->primInst, r->bounceInst};
+	                r->vel[0],  r->vel[1], r->primInst, r->bounceInst, r->instWork};
 	for (void* b : bufs) hipFree(b);
 	delete r;
 }
@@ -150,6 +151,10 @@ phx_status enqueueFrame(PhxContext* ctx, PhxRenderer* r, const PhxScene* scene,
 	const PhxInstanceSet* inst = r->instances && instanceCount(r->instances) ? r->instances : nullptr;
 	const uint32_t numInst = inst ? instanceCount(inst) : 0u;
 	const DevInstance* instByIndex = inst ? instanceByIndex(inst) : nullptr;
+	// Instance casts on the frame's stream run beside the bounce cast on r->side, whose ray counters
+	// are the context's: they have their own.
+	TraceLaunch onMain = closest;
+	onMain.work = r->instWork;
 
 	// Primary hits -> hit records -> contributions and shadow rays of every light.
 	PHX_HIP(launchGenPrimaryRays(*cam, r->w, r->h, 0.0f, 0.0f, 1e-4f, FLT_MAX, order, r->prim, s,
@@ -157,8 +162,8 @@ phx_status enqueueFrame(PhxContext* ctx, PhxRenderer* r, const PhxScene* scene,
 	        what);
 	PHX_HIP(launchClosest(sv, r->prim, r->n, r->primHits, primary, nullptr, s), what);
 	if (inst)
-		PHX_HIP(launchInstances(instanceTop(inst), instanceArray(inst), numInst, r->prim, r->n,
-		                        r->primHits, r->primInst, nullptr, true, s),
+		PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst, r->prim, r->n,
+		                        r->primHits, r->primInst, nullptr, true, onMain, s),
 		        what);
 	PHX_HIP(launchInterpret(r->prim, r->primHits, r->n, scene->datas, scene->numTris,
 	                        scene->materials, scene->numMaterials, scene->tex, r->gbuf, s,
@@ -179,15 +184,15 @@ phx_status enqueueFrame(PhxContext* ctx, PhxRenderer* r, const PhxScene* scene,
 		PHX_HIP(hipStreamWaitEvent(r->side, r->fork, 0), what);
 		PHX_HIP(launchClosest(sv, r->bounce, r->m, r->bounceHits, bounce, nullptr, r->side), what);
 		if (inst)
-			PHX_HIP(launchInstances(instanceTop(inst), instanceArray(inst), numInst, r->bounce,
-			                        r->m, r->bounceHits, r->bounceInst, nullptr, true, r->side),
+			PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst, r->bounce,
+			                        r->m, r->bounceHits, r->bounceInst, nullptr, true, closest, r->side),
 			        what);
 		PHX_HIP(hipEventRecord(r->join, r->side), what);
 	}
 	PHX_HIP(launchAnyHit(sv, r->shadow, r->n * L, r->inLight, shadows, s), what);
 	if (inst)
-		PHX_HIP(launchInstances(instanceTop(inst), instanceArray(inst), numInst, r->shadow,
-		                        r->n * L, nullptr, nullptr, r->inLight, true, s),
+		PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst, r->shadow,
+		                        r->n * L, nullptr, nullptr, r->inLight, true, onMain, s),
 		        what);
 	PHX_HIP(launchShadowLogic(r->color, r->w, r->h, 1u, false, r->inLight, r->contrib, L, s), what);
 
@@ -203,8 +208,8 @@ phx_status enqueueFrame(PhxContext* ctx, PhxRenderer* r, const PhxScene* scene,
 		        what);
 		PHX_HIP(launchAnyHit(sv, r->shadow, r->m * L, r->inLight, bounceShadows, s), what);
 		if (inst)
-			PHX_HIP(launchInstances(instanceTop(inst), instanceArray(inst), numInst, r->shadow,
-			                        r->m * L, nullptr, nullptr, r->inLight, true, s),
+			PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst, r->shadow,
+			                        r->m * L, nullptr, nullptr, r->inLight, true, onMain, s),
 			        what);
 		PHX_HIP(launchShadowLogic(r->color, r->w, r->h, 2u, true, r->inLight, r->contrib, L, s),
 		        what);
@@ -264,12 +269,15 @@ phx_status phx_renderer_create(PhxContext* ctx, uint32_t width, uint32_t height,
 	if (st == PHX_OK) st = devAlloc(r->color, r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->hist[0], r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->hist[1], r->n, what);
+	if (st == PHX_OK) st = devAlloc(r->instWork, kRayCounterWords, what);
 	if (st == PHX_OK) st = devAlloc(r->primInst, r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->bounceInst, std::max(r->m, 1u), what);
 	if (st == PHX_OK) st = devAlloc(r->vel[0], r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->vel[1], r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->out, r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->params, 1, what);
+	if (st == PHX_OK && launchZeroWords(r->instWork, kRayCounterWords, ctx->stream) != hipSuccess)
+		st = fail(PHX_ERR_HIP, "%s: clearing the ray counters failed", what);
 	if (st == PHX_OK && (hipStreamCreateWithFlags(&r->side, hipStreamNonBlocking) != hipSuccess ||
 	                     hipEventCreateWithFlags(&r->fork, hipEventDisableTiming) != hipSuccess ||
 	                     hipEventCreateWithFlags(&r->join, hipEventDisableTiming) != hipSuccess))

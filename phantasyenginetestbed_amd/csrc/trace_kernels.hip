@@ -124,9 +124,11 @@ __device__ __forceinline__ void add_counts(unsigned long long* counters, const C
 // Deepest castRay stack for a tree of depth <= 64 (enforced at upload): one pending entry per
 // level plus the two children of the node being expanded.
 constexpr int kSimpleStack = 72;
-// Words that hold such a stack, or a wide walk's pending entries.
-constexpr int kStackWords =
-	kSimpleStack > 2 * int(kWideMaxPending) ? kSimpleStack : 2 * int(kWideMaxPending);
+// Words that hold such a stack, or 8-B entries of either walk.
+constexpr int kMaxPending = 66;  // children of a binary walk (64 levels), or slots of a wide one
+static_assert(int(kWideMaxPending) <= kMaxPending, "pending slots of a wide walk");
+constexpr int kStackWords = 2 * kMaxPending;
+static_assert(kStackWords >= kSimpleStack, "4-B entries");
 
 // castRay<144> of one ray (BVHTraversal.hpp:37-128) into `c` (which holds the miss result on
 // entry): pop, decide both children, left first; a visited leaf is tested at once, a visited
@@ -174,12 +176,9 @@ struct ColumnStack {
 	}
 };
 
-// LDS stack words per lane: 24 for one-ray-per-lane casts (24 KB per 256-thread block); 12 each
-// for an instance cast's top-tree stack and its entered instance's castRay stack (24 KB, so the
-// five blocks per CU of its launch fit). Larger splits lower the blocks a CU holds and measured
-// slower.
+// LDS stack words per lane of the one-ray-per-lane casts (24 KB per 256-thread block). Larger splits
+// lower the blocks a CU holds and measured slower.
 constexpr int kSimpleLds = 24;
-constexpr int kInstanceLds = 12;
 
 template <bool kCount, class Stack>
 __device__ __forceinline__ void closest_one(const float4* __restrict__ nodes,
@@ -483,197 +482,6 @@ __global__ __launch_bounds__(kBlock) void k_anyhit_simple(
 		kCount ? anyhit_one<true>(nodes, tris, r, k, st) : anyhit_any(wide, nodes, tris, r, st);
 	inLight[i] = occluded ? 0 : 1;
 	if (kCount) add_counts(counters, k);
-}
-
-// ---- instances (two-level traversal) ------------------------------------------------------------
-//
-// A top tree over the instances' world boxes (one instance per leaf, PhxBVHNode layout) is walked
-// in castRay's order. An instance is entered iff the ray's slab test on its world box hits with
-// tOut > tMin and tIn <= min(tMax, best t) -- `<=`, so an instance that could tie the best hit is
-// still traced. Each entered instance runs castRay on its own SBVH with the ray moved into object
-// space (o' = A o + b, d' = A d, the same t range; t is the same parameter in both spaces), from a
-// miss, so its result is the one castRay gives for that instance alone. The closest of those
-// results wins, the lower instance index on equal t. With `hits` holding a static-scene result on
-// entry (seeded), that result counts as instance -1: an instance must be strictly closer.
-
-__device__ __forceinline__ dev::Ray object_ray(const DevInstance& in, const dev::Ray& w)
-{
-	const float* A = in.worldToObject;
-	float o[3], d[3];
-	for (int k = 0; k < 3; k++) {
-		float a = A[4 * k] * w.ox + A[4 * k + 1] * w.oy;
-		a = a + A[4 * k + 2] * w.oz;
-		o[k] = a + A[4 * k + 3];
-		float b = A[4 * k] * w.dx + A[4 * k + 1] * w.dy;
-		d[k] = b + A[4 * k + 2] * w.dz;
-	}
-	return dev::make_ray(make_float4(o[0], o[1], o[2], w.tMin), make_float4(d[0], d[1], d[2], w.tMax));
-}
-
-// The kernel is a per-lane state machine: every iteration a lane does one unit of its ray's work
-// -- a top-tree node, entering an instance, or one node of the entered instance's castRay (with
-// that node's leaf triangles) -- and a lane whose ray is done takes the next ray of its wave's
-// range (`raysPerWave` consecutive rays per wave), so the lanes of a wave do not wait for the
-// wave's costliest ray. (Written as nested loops, one ray per lane, the same casts took 3.8x as
-// long for closest hit and 2.7x for any hit on 1M rays into 300 instances.) Per ray, the order is
-// the one above: both children of a top node are decided with the best t on reaching it, inner
-// children are pushed left then right, the visited leaves' instances are entered left leaf
-// first, and each entry's castRay result is merged when its traversal ends.
-template <bool kAnyHit>
-__global__ __launch_bounds__(kBlock) void k_trace_instances(
-	const float4* __restrict__ top, const DevInstance* __restrict__ inst, uint32_t numInst,
-	const float4* __restrict__ rays, uint4* __restrict__ hits, uint32_t* __restrict__ instOut,
-	uint8_t* __restrict__ inLight, uint32_t n, uint32_t seeded, uint32_t raysPerWave)
-{
-	__shared__ uint32_t innerLds[kInstanceLds * kBlock];
-	__shared__ uint32_t topLds[kInstanceLds * kBlock];
-	const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-	uint32_t next = wave * raysPerWave;  // wave-uniform
-	const uint32_t end = next < n ? (n - next < raysPerWave ? n : next + raysPerWave) : next;
-	ColumnStack<kInstanceLds> inner;
-	inner.col = innerLds + threadIdx.x;
-	ColumnStack<kInstanceLds> topStk;
-	topStk.col = topLds + threadIdx.x;
-	uint32_t ray = kInvalid;
-	dev::Ray r = dev::make_ray(make_float4(0.f, 0.f, 0.f, 0.f), make_float4(1.f, 1.f, 1.f, 0.f));
-	dev::Ray o = r;
-	Closest best = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX}, c = best;
-	uint32_t bestInst = kInvalid, curId = 0u;
-	bool seededHit = false, occluded = false, inInner = false;
-	int tsp = 0, isp = 0;
-	uint32_t pend0 = 0u, pend0End = 0u, pend1 = 0u, pend1End = 0u;  // leaf instance ranges
-	const float4* iNodes = nullptr;
-	const float4* iTris = nullptr;
-	Counts none;
-	while (true) {
-		// Lanes without a ray take the next rays of the wave's range, in lane order.
-		const uint64_t idle = __ballot(ray == kInvalid);
-		bool fresh = false;
-		if (idle != 0 && next < end) {
-			const uint32_t rank = __builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32),
-			                                                __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0u));
-			if (ray == kInvalid && next + rank < end) {
-				ray = next + rank;
-				fresh = true;
-			}
-			const uint32_t taken = uint32_t(__popcll(idle));
-			next = end - next < taken ? end : next + taken;
-		}
-		if (__ballot(ray != kInvalid) == 0) break;
-		if (ray == kInvalid) continue;
-		if (fresh) {
-			r = dev::make_ray(rays[2 * size_t(ray)], rays[2 * size_t(ray) + 1]);
-			best = Closest{kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
-			bestInst = kInvalid;
-			seededHit = false;
-			occluded = false;
-			if (!kAnyHit && seeded) {
-				const uint4 h = hits[ray];
-				best = Closest{h.x, __uint_as_float(h.y), __uint_as_float(h.z), __uint_as_float(h.w)};
-				seededHit = h.x != kInvalid;
-			}
-			if (kAnyHit && seeded) occluded = inLight[ray] == 0;
-			tsp = numInst ? 1 : 0;
-			topStk.put(0, 0u);
-			pend0 = pend0End = pend1 = pend1End = 0u;
-			inInner = false;
-		}
-		// A lane may take a top-tree node, enter the instance it leaves pending and take that
-		// instance's first node in one iteration; the order of each ray's work is unchanged.
-		bool done = false;
-		if (!inInner && !occluded && pend0 >= pend0End && pend1 >= pend1End && tsp > 0) {
-			// One top-tree node: decide both children with the best t so far.
-			tsp--;
-			const NodeWords nd = load_node(top, topStk.get(tsp));
-			float inL, outL, inR, outR;
-			dev::slab(r, nd.w0.x, nd.w0.y, nd.w0.z, nd.w0.w, nd.w1.x, nd.w1.y, inL, outL);
-			dev::slab(r, nd.w1.z, nd.w1.w, nd.w2.x, nd.w2.y, nd.w2.z, nd.w2.w, inR, outR);
-			const float lim = kAnyHit ? r.tMax : dev::min_first(r.tMax, best.t);
-			const bool visitL = (outL >= inL) && outL > r.tMin && (kAnyHit ? inL < lim : inL <= lim);
-			const bool visitR = (outR >= inR) && outR > r.tMin && (kAnyHit ? inR < lim : inR <= lim);
-			if (visitL && nd.w3.z == 0 && tsp < kSimpleStack) topStk.put(tsp++, child_index(nd.w3.x));
-			if (visitR && nd.w3.w == 0 && tsp < kSimpleStack) topStk.put(tsp++, child_index(nd.w3.y));
-			if (visitL && nd.w3.z != 0) {
-				pend0 = child_index(nd.w3.x);
-				pend0End = pend0 + uint32_t(nd.w3.z);
-			}
-			if (visitR && nd.w3.w != 0) {
-				pend1 = child_index(nd.w3.y);
-				pend1End = pend1 + uint32_t(nd.w3.w);
-			}
-		}
-		if (!inInner && !occluded && (pend0 < pend0End || pend1 < pend1End)) {
-			// Enter the next instance of the visited leaves (left leaf first).
-			const uint32_t j = pend0 < pend0End ? pend0++ : pend1++;
-			const DevInstance& in = inst[j];
-			curId = in.index;
-			iNodes = in.nodes;
-			iTris = in.tris;
-			o = object_ray(in, r);
-			c = Closest{kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
-			inner.put(0, 0u);
-			isp = 1;
-			inInner = true;
-		}
-		if (inInner) {
-			// One node of the entered instance's castRay (closest_one / anyhit_one's loop body).
-			isp--;
-			const NodeWords nd = load_node(iNodes, inner.get(isp));
-			float inL, outL, inR, outR;
-			dev::slab(o, nd.w0.x, nd.w0.y, nd.w0.z, nd.w0.w, nd.w1.x, nd.w1.y, inL, outL);
-			dev::slab(o, nd.w1.z, nd.w1.w, nd.w2.x, nd.w2.y, nd.w2.z, nd.w2.w, inR, outR);
-			const float lim = kAnyHit ? o.tMax : dev::min_first(o.tMax, c.t);
-			const bool visitL = (outL >= inL) && outL > o.tMin && inL < lim;
-			const bool visitR = (outR >= inR) && outR > o.tMin && inR < lim;
-			bool hitAny = false;
-			if (visitL) {
-				if (nd.w3.z == 0) {
-					if (isp < kSimpleStack) inner.put(isp++, child_index(nd.w3.x));
-				} else if (kAnyHit) {
-					hitAny = anyhit_leaf(o, iTris, child_index(nd.w3.x), nd.w3.z);
-				} else {
-					closest_leaf<false>(o, iTris, child_index(nd.w3.x), nd.w3.z, c, none);
-				}
-			}
-			if (visitR && !hitAny) {
-				if (nd.w3.w == 0) {
-					if (isp < kSimpleStack) inner.put(isp++, child_index(nd.w3.y));
-				} else if (kAnyHit) {
-					hitAny = anyhit_leaf(o, iTris, child_index(nd.w3.y), nd.w3.w);
-				} else {
-					closest_leaf<false>(o, iTris, child_index(nd.w3.y), nd.w3.w, c, none);
-				}
-			}
-			if (kAnyHit && hitAny) {
-				occluded = true;
-				done = true;
-			} else if (isp == 0) {
-				inInner = false;
-				if (!kAnyHit) {
-					const bool tieWins = c.t == best.t && !seededHit &&
-					                     (bestInst == kInvalid || curId < bestInst);
-					if (c.tri != kInvalid && (c.t < best.t || tieWins)) {
-						best = c;
-						bestInst = curId;
-						seededHit = false;
-					}
-				}
-			}
-		}
-		if (!done && !inInner)
-			done = occluded || (pend0 >= pend0End && pend1 >= pend1End && tsp == 0);
-		if (done) {
-			if (kAnyHit) {
-				inLight[ray] = occluded ? 0 : 1;
-			} else {
-				if (bestInst != kInvalid || !seeded)
-					hits[ray] = make_uint4(best.tri, __float_as_uint(best.t), __float_as_uint(best.u),
-					                       __float_as_uint(best.v));
-				if (instOut) instOut[ray] = bestInst;
-			}
-			ray = kInvalid;
-		}
-	}
 }
 
 // Visit decision of both children of a binary node (BVHTraversal.hpp:59-64; any-hit: tMax).
@@ -997,8 +805,6 @@ constexpr int kLaneRows = 16;  // (9.5 KB a wave: 16 waves per CU)
 // 1.79 ms with 4, 1.73 with 8 and 32, 1.70 with 16.
 constexpr uint32_t kLaneRefill = 16;
 constexpr uint32_t kSpillEntries = kSpillWordsPerRay / 2u;
-constexpr int kMaxPending = 66;     // of a binary walk (64 levels)
-static_assert(int(kWideMaxPending) <= kMaxPending, "pending slots of a wide walk");
 static_assert(kLaneRows + int(kSpillEntries) >= kMaxPending, "stack entries of a ray");
 static_assert(kQuadRows + int(kSpillEntries) >= kMaxPending, "stack entries of a ray");
 
@@ -1443,93 +1249,52 @@ __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 // time, the VALUs 63%. Handing the records over in LDS, four lanes to a line, took it to 1.60 ms and
 // single casts from 0.106 to 0.123 ms, so each lane loads its own.
 
-template <int kAny, bool kBatch, bool kTrack, bool kClock>
-struct LaneTracer {
-	const QuadArgs& P;
-	LdsU2* stacks;
+// One lane's castRay over the wide nodes, or the binary ones (exact), one record at a time.
+struct LaneWalk {
 	dev::Ray r;
-	uint32_t ray = kInvalid;
-	uint32_t ref = 0u;     // what the ray takes next: a node, or kWideLeaf and a triangle
+	uint32_t ref = 0u;  // what the ray takes next: a node, or kWideLeaf and a triangle
 	int sp = 0;
-	uint32_t base = 0u;
+	int floor = 0;      // the stack's bottom for this walk
 	Closest c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
-	bool exact = false, any = false;
-	uint32_t batch = 0u;
-	const float4* wide = nullptr;
-	const float4* tris = nullptr;
-
-	__device__ __forceinline__ bool isAny() const { return kAny == 1 || (kAny == 2 && any); }
-	__device__ __forceinline__ void put(bool on, int at, uint32_t ref, float tIn)
-	{
-		const U32x2 e = {ref, __float_as_uint(tIn)};
-		if (on && at < kLaneRows) stacks[base + uint32_t(at) * 64u] = e;
-		if (__builtin_expect(on && at >= kLaneRows, 0)) *spill_entry<kLaneRows, 64u>(P.spill, base, at) = e;
-	}
-	__device__ __forceinline__ U32x2 get(int at) const
-	{
-		U32x2 e = stacks[base + uint32_t(at < kLaneRows ? at : 0) * 64u];
-		if (__builtin_expect(at >= kLaneRows, 0)) e = *spill_entry<kLaneRows, 64u>(P.spill, base, at);
-		return e;
-	}
-
-	__device__ __forceinline__ void start(uint32_t index)
-	{
-		const float4* rays = P.rays;
-		uint32_t at = index;
-		bool hasWide = P.wide != P.tris;
-		if (kBatch) {
-			batch = find_batch(P.offsets, P.numBatches, index);
-			at = index - P.offsets[batch];
-			const BatchDesc d = P.descs[batch];
-			rays = d.rays;
-			wide = d.wide;
-			tris = d.tris;
-			any = d.kind != 0u;
-			hasWide = d.wide != d.tris;
-		}
-		const float4 a = as_global(rays)[2 * size_t(at)], b = as_global(rays)[2 * size_t(at) + 1];
-		exact = !(quad_ray(a, b, r) && hasWide);
-		if (__builtin_expect(exact, 0)) {
-			r.ix = 1.0f / b.x;
-			r.iy = 1.0f / b.y;
-			r.iz = 1.0f / b.z;
-		}
-		ray = index;
-		ref = 0u;
-		sp = 0;
-		c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
-	}
+	bool exact = false;
 
 	// Decides a binary node's children as castRay does and pushes what is visited in its order.
-	__device__ __forceinline__ void expand_binary(float lim)
+	template <class Stack>
+	__device__ __forceinline__ void expand_binary(const float4* nodes, float lim, Stack& st)
 	{
-		const float4* nodes = kBatch ? P.descs[batch].nodes : P.nodes;
 		const NodeWords nd = load_node(nodes, ref);
 		bool visitL, visitR;
 		decide(r, nd, lim, visitL, visitR);
 		const uint32_t refL = child_index(nd.w3.x) | (nd.w3.z != 0 ? kWideLeaf : 0u);
 		const uint32_t refR = child_index(nd.w3.y) | (nd.w3.w != 0 ? kWideLeaf : 0u);
 		const bool leftFirst = visitL && nd.w3.z != 0;
-		put(visitL && visitR, sp, leftFirst ? refR : refL, -INFINITY);
-		put(visitL || visitR, sp + (visitL && visitR ? 1 : 0),
-		    visitL && visitR ? (leftFirst ? refL : refR) : visitL ? refL : refR, -INFINITY);
-		sp += (visitL ? 1 : 0) + (visitR ? 1 : 0);
+		if (visitL && visitR) st.put2(sp++, leftFirst ? refR : refL, -INFINITY);
+		if (visitL || visitR)
+			st.put2(sp++, visitL && visitR ? (leftFirst ? refL : refR) : visitL ? refL : refR, -INFINITY);
 	}
 
-	__device__ __forceinline__ void step()
+	__device__ __forceinline__ bool at_leaf() const { return (ref & kWideLeaf) != 0u; }
+	// The record that advance() consumes: a wide node, or a leaf's next two triangles (the words past
+	// a leaf's last one are the next triangle's or the array's padding). Lanes without one (`on`
+	// false) and exact nodes read the array's first line.
+	__device__ __forceinline__ void load(bool on, const float4* wide, const float4* tris,
+	                                     float4 w[8]) const
 	{
-		const bool active = ray != kInvalid;
-		const bool any = isAny();
-		const bool leaf = active && (ref & kWideLeaf) != 0u;
-		const bool node = active && !leaf && !exact;
-		const float4* wide = kBatch ? this->wide : P.wide;
-		const float4* tris = kBatch ? this->tris : P.tris;
-		const float4* rec = leaf ? tris + 3u * size_t(ref & kWideIndex) : wide + 8u * size_t(node ? ref : 0u);
-		float4 w[8];
+		const float4* rec = on && at_leaf() ? tris + 3u * size_t(ref & kWideIndex)
+		                                    : wide + 8u * size_t(on && !exact ? ref : 0u);
 #pragma unroll
 		for (int i = 0; i < 8; i++) w[i] = as_global(rec)[i];
-		if (!active) return;
-		bool occluded = false, pop = true;
+	}
+
+	// Expands a node or tests up to two triangles of a leaf, and picks what the lane takes next. True
+	// if the traversal has ended (`occluded`: with an any-hit ray's hit).
+	template <int kAny, class Stack>
+	__device__ __forceinline__ bool advance(const float4 w[8], const float4* nodes, bool any, Stack& st,
+	                                        bool& occluded)
+	{
+		const bool leaf = at_leaf(), node = !leaf && !exact;
+		bool pop = true;
+		occluded = false;
 		if (leaf) {
 			// Up to two triangles, accepted in order.
 			const dev::TriDet d0 = dev::tri_det(r, w[1], w[2]);
@@ -1557,7 +1322,6 @@ struct LaneTracer {
 			ref = kWideLeaf | ((ref & kWideIndex) + 2u);
 		}
 		const float lim = any ? r.tMax : dev::min_first(r.tMax, c.t);
-		float tIn = -INFINITY;
 		if (node) {
 			WideWords n;
 #pragma unroll
@@ -1572,35 +1336,115 @@ struct LaneTracer {
 			r2 = p3 ? r2 : r2 & ~kWidePair;
 			const bool p01 = p0 || p1, p012 = p01 || p2;
 			const int at2 = sp + (p3 ? 1 : 0), at1 = at2 + (p2 ? 1 : 0);
-			put(p3 && p012, sp, r3, v.tIn[3]);
-			put(p2 && p01, at2, r2, v.tIn[2]);
-			put(p1 && p0, at1, r1, v.tIn[1]);
+			if (p3 && p012) st.put2(sp, r3, v.tIn[3]);
+			if (p2 && p01) st.put2(at2, r2, v.tIn[2]);
+			if (p1 && p0) st.put2(at1, r1, v.tIn[1]);
 			pop = !(p012 || p3);
 			sp = pop ? sp : at1 + (p1 ? 1 : 0) + (p0 ? 1 : 0) - 1;
 			ref = p0 ? r0 : p1 ? r1 : p2 ? r2 : r3;
 		}
-		if (__builtin_expect(exact && !leaf, 0)) expand_binary(lim);
-		bool end = occluded;
-		if (pop && !occluded) {
-			// The top entry that the closest hit has not overtaken.
-			end = true;
-			while (sp > 0) {
-				sp--;
-				const U32x2 e = get(sp);
-				if (any || __uint_as_float(e.y) < lim) {
-					ref = e.x;
-					end = false;
-					break;
-				}
+		if (__builtin_expect(exact && !leaf, 0)) expand_binary(nodes, lim, st);
+		if (occluded || (pop && !take(lim, any, st))) return true;
+		if (!any && (pop || node)) decide_sibling(lim, st);
+		return false;
+	}
+	// Takes the top entry that the closest hit has not overtaken; false if there is none.
+	template <class Stack>
+	__device__ __forceinline__ bool take(float lim, bool any, Stack& st)
+	{
+		while (sp > floor) {
+			uint32_t at;
+			float tIn;
+			st.get2(--sp, at, tIn);
+			if (any || tIn < lim) {
+				ref = at;
+				return true;
 			}
 		}
-		if (!any && !end && (pop || node) && (ref & (kWideLeaf | kWidePair)) == (kWideLeaf | kWidePair)) {
-			// The sibling of a leaf that is taken is decided with it.
-			const U32x2 e = get(sp - 1);
-			put(true, sp - 1, e.x, __uint_as_float(e.y) < lim ? -INFINITY : INFINITY);
+		return false;
+	}
+	// The sibling of a leaf that is taken is decided with it.
+	template <class Stack>
+	__device__ __forceinline__ void decide_sibling(float lim, Stack& st)
+	{
+		if ((ref & (kWideLeaf | kWidePair)) == (kWideLeaf | kWidePair)) {
+			uint32_t at;
+			float tIn;
+			st.get2(sp - 1, at, tIn);
+			st.put2(sp - 1, at, tIn < lim ? -INFINITY : INFINITY);
 		}
-		if (end) {
-			quad_result<kBatch, kTrack, kClock>(P, ray, batch, c, any, occluded);
+	}
+};
+
+// A lane's stack column: entries in LDS, the deeper ones spilled.
+struct SpillStack {
+	LdsU2* stacks;
+	U32x2* spill;
+	uint32_t base;
+	__device__ __forceinline__ void put2(int at, uint32_t ref, float tIn)
+	{
+		const U32x2 e = {ref, __float_as_uint(tIn)};
+		if (__builtin_expect(at < kLaneRows, 1)) stacks[base + uint32_t(at) * 64u] = e;
+		else *spill_entry<kLaneRows, 64u>(spill, base, at) = e;
+	}
+	__device__ __forceinline__ void get2(int at, uint32_t& ref, float& tIn) const
+	{
+		U32x2 e = stacks[base + uint32_t(at < kLaneRows ? at : 0) * 64u];
+		if (__builtin_expect(at >= kLaneRows, 0)) e = *spill_entry<kLaneRows, 64u>(spill, base, at);
+		ref = e.x;
+		tIn = __uint_as_float(e.y);
+	}
+};
+
+template <int kAny, bool kBatch, bool kTrack, bool kClock>
+struct LaneTracer {
+	const QuadArgs& P;
+	SpillStack stack;
+	LaneWalk t;
+	uint32_t ray = kInvalid;
+	bool any = false;
+	uint32_t batch = 0u;
+	const float4* wide = nullptr;
+	const float4* tris = nullptr;
+
+	__device__ __forceinline__ bool isAny() const { return kAny == 1 || (kAny == 2 && any); }
+	__device__ __forceinline__ void start(uint32_t index)
+	{
+		const float4* rays = P.rays;
+		uint32_t at = index;
+		bool hasWide = P.wide != P.tris;
+		if (kBatch) {
+			batch = find_batch(P.offsets, P.numBatches, index);
+			at = index - P.offsets[batch];
+			const BatchDesc d = P.descs[batch];
+			rays = d.rays;
+			wide = d.wide;
+			tris = d.tris;
+			any = d.kind != 0u;
+			hasWide = d.wide != d.tris;
+		}
+		const float4 a = as_global(rays)[2 * size_t(at)], b = as_global(rays)[2 * size_t(at) + 1];
+		t.exact = !(quad_ray(a, b, t.r) && hasWide);
+		if (__builtin_expect(t.exact, 0)) {
+			t.r.ix = 1.0f / b.x;
+			t.r.iy = 1.0f / b.y;
+			t.r.iz = 1.0f / b.z;
+		}
+		ray = index;
+		t.ref = 0u;
+		t.sp = 0;
+		t.c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
+	}
+
+	__device__ __forceinline__ void step()
+	{
+		const bool active = ray != kInvalid;
+		float4 w[8];
+		t.load(active, kBatch ? wide : P.wide, kBatch ? tris : P.tris, w);
+		if (!active) return;
+		bool occluded;
+		if (t.template advance<kAny>(w, kBatch ? P.descs[batch].nodes : P.nodes, isAny(), stack, occluded)) {
+			quad_result<kBatch, kTrack, kClock>(P, ray, batch, t.c, isAny(), occluded);
 			ray = kInvalid;
 		}
 	}
@@ -1612,8 +1456,8 @@ __device__ __forceinline__ void lane_trace(const QuadArgs& P, uint32_t* lds)
 	const uint32_t waveInBlock = uniform(threadIdx.x >> 6), lane = __lane_id();
 	LdsU2* stacks = (LdsU2*)(reinterpret_cast<U32x2*>(lds));
 	if (kClock && threadIdx.x == 0u) atomicMin(&P.clock[P.n], wall_clock64());
-	LaneTracer<kAny, kBatch, kTrack, kClock> T{P, stacks};
-	T.base = stack_base<kLaneRows, 64u>(waveInBlock, lane);
+	LaneTracer<kAny, kBatch, kTrack, kClock> T{P, {stacks, P.spill, stack_base<kLaneRows, 64u>(waveInBlock, lane)}};
+	T.t.r = {};
 	if (kBatch) {  // read by lanes without a ray
 		T.wide = P.descs[0].wide;
 		T.tris = P.descs[0].tris;
@@ -1655,13 +1499,13 @@ __device__ __forceinline__ void lane_trace(const QuadArgs& P, uint32_t* lds)
 		const uint32_t at4k = uint32_t(__builtin_amdgcn_ds_permute(to, int(v)));
 		return uint32_t(__builtin_amdgcn_update_dpp(0, int(at4k), 0x00, 0xF, 0xF, true));
 	};
-	const uint32_t ray = move(T.ray), ref = move(T.ref);
-	Q.q.sp = int(move(uint32_t(T.sp)));
-	Q.q.base = move(T.base);
-	const float best = __uint_as_float(move(__float_as_uint(T.c.t)));
-	const float u = __uint_as_float(move(__float_as_uint(T.c.u)));
-	const float v = __uint_as_float(move(__float_as_uint(T.c.v)));
-	const uint32_t hit = move(T.c.tri), batch = kBatch ? move(T.batch) : 0u;
+	const uint32_t ray = move(T.ray), ref = move(T.t.ref);
+	Q.q.sp = int(move(uint32_t(T.t.sp)));
+	Q.q.base = move(T.stack.base);
+	const float best = __uint_as_float(move(__float_as_uint(T.t.c.t)));
+	const float u = __uint_as_float(move(__float_as_uint(T.t.c.u)));
+	const float v = __uint_as_float(move(__float_as_uint(T.t.c.v)));
+	const uint32_t hit = move(T.t.c.tri), batch = kBatch ? move(T.batch) : 0u;
 	if (lane / 4u < uint32_t(__popcll(busy))) {
 		Q.q.batch = batch;
 		Q.start(ray, false);
@@ -1700,6 +1544,217 @@ __device__ __forceinline__ bool retire_block(uint32_t* work)
 __host__ __device__ __forceinline__ uint32_t lane_lds_words(uint32_t waves)
 {
 	return waves * 2u * wave_stack_entries<kLaneRows, 64u>();
+}
+
+// ---- instances (two-level traversal) ------------------------------------------------------------
+//
+// A top tree over the instances' world boxes (one instance per leaf, PhxBVHNode layout) is walked
+// in castRay's order. An instance is entered iff the ray's slab test on its world box hits with
+// tOut > tMin and tIn <= min(tMax, best t) -- `<=`, so an instance that could tie the best hit is
+// still traced. Each entered instance runs castRay on its own SBVH with the ray moved into object
+// space (o' = A o + b, d' = A d, the same t range; t is the same parameter in both spaces), from a
+// miss, so its result is the one castRay gives for that instance alone. The closest of those
+// results wins, the lower instance index on equal t. With `hits` holding a static-scene result on
+// entry (seeded), that result counts as instance -1: an instance must be strictly closer.
+
+// Ray (a, b) in an instance's object space; false if it walks the binary nodes (quad_ray).
+__device__ __forceinline__ bool object_ray(const DevInstance& in, const float4 a, const float4 b,
+                                           dev::Ray& r)
+{
+	const float* A = in.worldToObject;
+	float o[3], d[3];
+	for (int k = 0; k < 3; k++) {
+		float p = A[4 * k] * a.x + A[4 * k + 1] * a.y;
+		p = p + A[4 * k + 2] * a.z;
+		o[k] = p + A[4 * k + 3];
+		float q = A[4 * k] * b.x + A[4 * k + 1] * b.y;
+		d[k] = q + A[4 * k + 2] * b.z;
+	}
+	const bool fast = quad_ray(make_float4(o[0], o[1], o[2], a.w), make_float4(d[0], d[1], d[2], b.w), r);
+	if (!fast) {
+		r.ix = 1.0f / d[0];
+		r.iy = 1.0f / d[1];
+		r.iz = 1.0f / d[2];
+	}
+	return fast;
+}
+
+// The kernel is a per-lane state machine over persistent waves. The top tree has wide nodes too, so a
+// lane between instances and a lane inside one take the same kind of step (LaneWalk), each with its
+// own ray; `tIn <= x` is taken as `tIn < next float above x`. A lane that enters or leaves an instance
+// loads the ray of the top tree again (two words for nine registers) and does so at once: collecting
+// such lanes until they are 8 or 16 makes the wave wait longer than their instructions take (3.18 and
+// 3.6 ms instead of 3.0). Rays are handed out as in the other persistent kernels, so lanes do not wait
+// for the wave's costliest ray.
+//
+// Bound by the texture data path, which returns a lane's 16 B a cycle (75% busy), and by VALU issue
+// (65%, with 17 of 64 lanes active on average). On the binary nodes, with exact slabs and divisions, a
+// top-tree step in every iteration and a fixed range of rays per wave, 1,048,576 rays into 300
+// instances took 4.92 ms (closest) and 262,147 any-hit rays into 120 instances and a scene 0.71 ms;
+// now 3.17 and 0.44 ms. (Wide nodes inside the instances alone: 4.14 and 0.49 ms.)
+
+constexpr uint32_t kInstanceRefill = 8;  // idle lanes of a wave before it takes new rays
+constexpr uint32_t kInstanceWaves = 20;  // per CU: 5 per SIMD (96 registers)
+
+// A lane's stack column: 14 entries in LDS (28 KB a block, 5 blocks a CU), the deeper ones in private
+// memory. (The LDS part through an LDS pointer and read in any case: a choice between the two would be
+// made of flat loads.)
+struct InstanceStack {
+	static constexpr int kRows = 14;
+	LdsU2* col;
+	U32x2 (&deep)[2 * kMaxPending - kRows];
+	__device__ __forceinline__ void put2(int at, uint32_t ref, float tIn)
+	{
+		const U32x2 e = {ref, __float_as_uint(tIn)};
+		if (__builtin_expect(at < kRows, 1)) col[at * kBlock] = e;
+		else deep[at - kRows] = e;
+	}
+	__device__ __forceinline__ void get2(int at, uint32_t& ref, float& tIn) const
+	{
+		U32x2 e = col[(at < kRows ? at : 0) * kBlock];
+		if (__builtin_expect(ballot(at >= kRows) != 0ull, 0))
+			if (at >= kRows) e = deep[at - kRows];
+		ref = e.x;
+		tIn = __uint_as_float(e.y);
+	}
+};
+
+// The next float above x, so that t < next_up(x) is t <= x.
+__device__ __forceinline__ float next_up(float x)
+{
+	const float y = x + 0.0f;  // (-0 to 0)
+	if (!(fabsf(y) < INFINITY)) return y;
+	return __uint_as_float(y >= 0.0f ? __float_as_uint(y) + 1u : __float_as_uint(y) - 1u);
+}
+
+template <bool kAnyHit>
+__global__ __launch_bounds__(kBlock, 5) void k_trace_instances(
+	const float4* __restrict__ top, const float4* __restrict__ topWide,
+	const DevInstance* __restrict__ inst, uint32_t numInst, const float4* __restrict__ rays,
+	uint4* __restrict__ hits, uint32_t* __restrict__ instOut, uint8_t* __restrict__ inLight,
+	uint32_t n, uint32_t seeded, uint32_t* __restrict__ work)
+{
+	__shared__ U32x2 stackLds[InstanceStack::kRows * kBlock];
+	U32x2 deep[2 * kMaxPending - InstanceStack::kRows];
+	InstanceStack stack = {(LdsU2*)(stackLds) + threadIdx.x, deep};  // the top tree's entries, an instance's above
+	QuadArgs P = {};
+	P.n = n;
+	P.window = 64u;
+	P.work = work;
+	RayWindows W(P, uniform(threadIdx.x >> 6));
+
+	LaneWalk t;  // in the top tree, or the entered instance's castRay
+	t.r = {};
+	Closest best = t.c;
+	uint32_t ray = kInvalid, bestInst = kInvalid, id = 0u;
+	bool inside = false;   // t walks an instance
+	bool leave = false;    // that walk has ended (or the ray is new)
+	bool seededHit = false, fresh = false, handedOut = false;
+	const float4* wide = topWide;
+	const float4* tris = nullptr;
+	const float4* nodes = top;
+	while (true) {
+		const uint64_t idle = ballot(ray == kInvalid);
+		if (!handedOut && uint32_t(__popcll(idle)) >= kInstanceRefill) {
+			if (W.next >= W.end && !W.claim(P)) {
+				handedOut = true;
+			} else {
+				const uint32_t mine = W.next + uint32_t(__popcll(idle & __lanemask_lt()));
+				if (ray == kInvalid && mine < W.end) {
+					ray = mine;
+					best = t.c = Closest{kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
+					bestInst = kInvalid;
+					seededHit = false;
+					leave = fresh = true;
+					if (!kAnyHit && seeded) {
+						const uint4 h = hits[ray];
+						best = Closest{h.x, __uint_as_float(h.y), __uint_as_float(h.z), __uint_as_float(h.w)};
+						seededHit = h.x != kInvalid;
+					}
+					if (kAnyHit && seeded && inLight[ray] == 0) ray = kInvalid;  // (stays 0)
+				}
+				const uint32_t taken = uint32_t(__popcll(idle));
+				W.next = W.end - W.next < taken ? W.end : W.next + taken;
+			}
+		}
+		const bool busy = ray != kInvalid;
+		if (ballot(busy) == 0ull) {
+			if (handedOut) break;
+			continue;
+		}
+		if (busy && (leave || (!inside && t.at_leaf()))) {
+			const float4 a = as_global(rays)[2 * size_t(ray)], b = as_global(rays)[2 * size_t(ray) + 1];
+			if (leave) {
+				leave = inside = false;
+				// The closer result, the lower index on equal t.
+				if (!kAnyHit && t.c.tri != kInvalid) {
+					const bool tieWins = t.c.t == best.t && !seededHit && (bestInst == kInvalid || id < bestInst);
+					if (t.c.t < best.t || tieWins) {
+						best = t.c;
+						bestInst = id;
+						seededHit = false;
+					}
+				}
+				t.exact = !(quad_ray(a, b, t.r) && topWide != top);
+				if (__builtin_expect(t.exact, 0)) {
+					t.r.ix = 1.0f / b.x;
+					t.r.iy = 1.0f / b.y;
+					t.r.iz = 1.0f / b.z;
+				}
+				if (!kAnyHit) t.r.tMax = next_up(t.r.tMax);
+				t.c = Closest{kInvalid, kAnyHit ? FLT_MAX : next_up(best.t), FLT_MAX, FLT_MAX};
+				t.floor = 0;
+				wide = topWide;
+				nodes = top;
+				const float lim = kAnyHit ? t.r.tMax : dev::min_first(t.r.tMax, t.c.t);
+				if (fresh) {
+					t.ref = 0u;
+					t.sp = 0;
+				}
+				if (fresh ? numInst == 0u : !t.take(lim, kAnyHit, stack)) {
+					if (kAnyHit) {
+						inLight[ray] = 1;
+					} else {
+						if (bestInst != kInvalid || !seeded)
+							hits[ray] = make_uint4(best.tri, __float_as_uint(best.t), __float_as_uint(best.u),
+							                       __float_as_uint(best.v));
+						if (instOut) instOut[ray] = bestInst;
+					}
+					ray = kInvalid;
+				} else if (!kAnyHit && !fresh) {
+					t.decide_sibling(lim, stack);
+				}
+				fresh = false;
+			}
+			if (ray != kInvalid && (t.ref & kWideLeaf)) {
+				const DevInstance& in = inst[t.ref & kWideIndex];
+				id = in.index;
+				nodes = in.nodes;
+				tris = in.tris;
+				wide = in.wide;
+				t.exact = !(object_ray(in, a, b, t.r) && wide != tris);
+				t.ref = 0u;
+				t.floor = t.sp;
+				t.c = Closest{kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
+				inside = true;
+			}
+		}
+		const bool walks = ray != kInvalid && !leave && (inside || !t.at_leaf());
+		if (ballot(walks) == 0ull) continue;
+		float4 w[8];
+		t.load(walks, wide, tris, w);
+		bool occluded;
+		if (walks && t.template advance<kAnyHit ? 1 : 0>(w, nodes, kAnyHit, stack, occluded)) {
+			leave = true;
+			if (kAnyHit && occluded) {
+				inLight[ray] = 0;
+				ray = kInvalid;
+				leave = inside = false;
+			}
+		}
+	}
+	__syncthreads();
+	if (threadIdx.x == 0u) retire_block(work);
 }
 
 template <bool kAnyHit, bool kClock, bool kBig>
@@ -1995,25 +2050,23 @@ hipError_t launchAnyHitCounted(const SceneView& s, const PhxRayIn* rays, uint32_
 	return hipGetLastError();
 }
 
-hipError_t launchInstances(const PhxBVHNode* top, const DevInstance* inst, uint32_t numInst,
+hipError_t launchInstances(const PhxBVHNode* top, const WideNode* topWide, const DevInstance* inst, uint32_t numInst,
                           const PhxRayIn* rays, uint32_t n, PhxRayHit* hits, uint32_t* instOut,
-                          uint8_t* inLight, bool seeded, hipStream_t stream)
+                          uint8_t* inLight, bool seeded, const TraceLaunch& L, hipStream_t stream)
 {
 	if (n == 0) return hipSuccess;
 	const float4* t4 = reinterpret_cast<const float4*>(top);
+	const float4* w4 = topWide ? reinterpret_cast<const float4*>(topWide) : t4;
 	const float4* r4 = reinterpret_cast<const float4*>(rays);
-	// Rays per wave: enough waves to fill the device (about 5,120: five per SIMD, the most the
-	// kernel's registers allow), at least one ray per lane.
-	const uint32_t perWave = std::max<uint32_t>(64u, std::min<uint32_t>(1024u, (n + 5119u) / 5120u));
-	const uint32_t waves = (n + perWave - 1u) / perWave;
-	const dim3 grid((waves + kBlock / 64u - 1u) / (kBlock / 64u));
+	const uint32_t waves = std::min(L.cus * kInstanceWaves, gridFor(n, 64u));
+	const dim3 grid(gridFor(waves, kBlock / 64u));
 	if (inLight)
-		hipLaunchKernelGGL(k_trace_instances<true>, grid, dim3(kBlock), 0, stream, t4, inst,
-		                   numInst, r4, nullptr, nullptr, inLight, n, uint32_t(seeded), perWave);
+		hipLaunchKernelGGL(k_trace_instances<true>, grid, dim3(kBlock), 0, stream, t4, w4, inst,
+		                   numInst, r4, nullptr, nullptr, inLight, n, uint32_t(seeded), L.work);
 	else
-		hipLaunchKernelGGL(k_trace_instances<false>, grid, dim3(kBlock), 0, stream, t4, inst,
+		hipLaunchKernelGGL(k_trace_instances<false>, grid, dim3(kBlock), 0, stream, t4, w4, inst,
 		                   numInst, r4, reinterpret_cast<uint4*>(hits), instOut, nullptr, n,
-		                   uint32_t(seeded), perWave);
+		                   uint32_t(seeded), L.work);
 	return hipGetLastError();
 }
 
