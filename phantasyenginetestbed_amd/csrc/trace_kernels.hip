@@ -506,13 +506,17 @@ __device__ __forceinline__ void decide(const dev::Ray& r, const NodeWords& nd, f
 // which for coherent rays is close to one ray's, and every step does the same kind of work. Stack
 // entry e lives in lane e % 64 of a few registers.
 //
-// A step is bound by the latency of its dependent node load and the launch by its longest packets
-// (2 waves per SIMD in flight on average), so packets of NaN-free rays walk the four-wide nodes: half
-// the steps, for twice the box tests each. 2,073,600 tiled camera rays on 1,004,000 triangles,
-// generation included: 0.522 ms with binary nodes and IEEE divisions, 0.472 ms with wide nodes and
-// the fast reciprocal.
+// A step is bound by the instructions that one wave can issue (loading the next node before the leaves
+// are tested gains nothing) and the launch by its longest packets (2 waves per SIMD in flight on
+// average), so packets of NaN-free rays walk the four-wide nodes: half the steps, for twice the box
+// tests each. 2,073,600 tiled camera rays on 1,004,000 triangles, generation included: 0.522 ms with
+// binary nodes and IEEE divisions, 0.472 ms with wide nodes and the fast reciprocal. Packets whose rays
+// part do not stay packets: see k_packet.
 
 constexpr uint32_t kPacketBlock = 256;
+// A packet ends after kPacketSteps steps that fewer than kPacketLanes of its rays take part in, and its
+// rays go on one per lane (k_packet).
+constexpr int kPacketSteps = 8, kPacketLanes = 24;
 
 __device__ __forceinline__ uint32_t lane_get(uint32_t v, int l)
 {
@@ -629,14 +633,15 @@ __device__ __forceinline__ void packet_leaf(const float4* __restrict__ tris, uin
 // leaf slot that was pushed is decided again when it is taken, from its box in the node (closest
 // hit; entry word 1 names node and slot). Any hit does not depend on order: all its leaf slots are
 // tested at once.
-template <bool kAnyHit>
+template <bool kAnyHit, class Leave>
 __device__ __forceinline__ void packet_wide(const float4* __restrict__ wide,
                                             const float4* __restrict__ tris, const dev::Ray& r,
-                                            bool active, Closest& c, bool& occluded)
+                                            bool active, Closest& c, bool& occluded,
+                                            Leave leave)
 {
 	const uint32_t lane = __lane_id();
 	uint32_t sR = 0u, sB = 0u, sL = 0u, sH = 0u;  // reference, node and slot, mask
-	int sp = 0;
+	int sp = 0, steps = 0;
 	uint32_t cur = 0u;
 	uint64_t mask = __ballot(active);
 	while (true) {
@@ -726,36 +731,24 @@ __device__ __forceinline__ void packet_wide(const float4* __restrict__ wide,
 			if (__ballot(on2) != 0ull) packet_leaf<false>(tris, ref2 & kWideIndex, r, on2, c, occluded);
 		}
 		if (mask == 0ull) break;
-	}
-}
-
-template <bool kAnyHit>
-__global__ __launch_bounds__(kPacketBlock) void k_packet(const float4* __restrict__ wide,
-                                                         const float4* __restrict__ nodes,
-                                                         const float4* __restrict__ tris,
-                                                         const float4* __restrict__ rays,
-                                                         void* __restrict__ out, uint32_t n)
-{
-	const uint32_t lane = __lane_id();
-	const uint32_t first = blockIdx.x * kPacketBlock + (threadIdx.x & ~63u);
-	if (first >= n) return;  // whole wave
-	const uint32_t i = first + lane;
-	const bool active = i < n;
-	const uint32_t ri = active ? i : first;  // lanes past the end read a valid ray, never used
-	const dev::Ray r = dev::make_ray(rays[2 * size_t(ri)], rays[2 * size_t(ri) + 1]);
-	Closest c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
-	bool occluded = false;
-	// The wide nodes only when every active lane may walk them (the decision is uniform).
-	if (wide && __ballot(active && !r.nanFree) == 0ull)
-		packet_wide<kAnyHit>(wide, tris, r, active, c, occluded);
-	else
-		packet_binary<kAnyHit>(nodes, tris, r, active, c, occluded);
-	if (active) {
-		if (kAnyHit)
-			static_cast<uint8_t*>(out)[i] = occluded ? 0 : 1;
-		else
-			static_cast<uint4*>(out)[i] = make_uint4(c.tri, __float_as_uint(c.t),
-			                                         __float_as_uint(c.u), __float_as_uint(c.v));
+		if (__popcll(mask) < kPacketLanes && ++steps == kPacketSteps) {
+			// Each lane goes on by itself with its part of the stack, bottom entry first, and the node.
+			int n = 0;
+			for (int e = 0; e < sp; e++) {
+				const uint64_t who = (uint64_t(lane_get(sH, e)) << 32) | lane_get(sL, e);
+				const uint64_t below = e > 0 ? (uint64_t(lane_get(sH, e - 1)) << 32) | lane_get(sL, e - 1) : 0ull;
+				uint32_t ref = lane_get(sR, e);
+				float tIn = -INFINITY;
+				if (!kAnyHit && (ref & kWideLeaf)) {
+					const float4* b = wide + 2u * size_t(lane_get(sB, e));
+					decide_slot(r, b[0], b[1], 0.0f, tIn);
+				}
+				if (((below >> lane) & 1ull) == 0ull) ref &= ~kWidePair;
+				if (((who & ~done) >> lane) & 1ull) leave.push(n++, ref, tIn);
+			}
+			leave(n, cur, ((mask >> lane) & 1ull) != 0);
+			break;
+		}
 	}
 }
 
@@ -1376,6 +1369,28 @@ struct LaneWalk {
 	}
 };
 
+// A lane's stack column: kRows entries in LDS, the deeper ones in private memory. (The LDS part through
+// an LDS pointer and read in any case: a choice between the two would be made of flat loads.)
+template <int kRows, int kEntries>
+struct PrivateStack {
+	LdsU2* col;
+	U32x2 (&deep)[kEntries - kRows];
+	__device__ __forceinline__ void put2(int at, uint32_t ref, float tIn)
+	{
+		const U32x2 e = {ref, __float_as_uint(tIn)};
+		if (__builtin_expect(at < kRows, 1)) col[at * kBlock] = e;
+		else deep[at - kRows] = e;
+	}
+	__device__ __forceinline__ void get2(int at, uint32_t& ref, float& tIn) const
+	{
+		U32x2 e = col[(at < kRows ? at : 0) * kBlock];
+		if (__builtin_expect(ballot(at >= kRows) != 0ull, 0))
+			if (at >= kRows) e = deep[at - kRows];
+		ref = e.x;
+		tIn = __uint_as_float(e.y);
+	}
+};
+
 // A lane's stack column: entries in LDS, the deeper ones spilled.
 struct SpillStack {
 	LdsU2* stacks;
@@ -1546,6 +1561,81 @@ __host__ __device__ __forceinline__ uint32_t lane_lds_words(uint32_t waves)
 	return waves * 2u * wave_stack_entries<kLaneRows, 64u>();
 }
 
+// ---- packets, then one ray per lane ----------------------------------------------------------------
+//
+// A packet whose rays part (a tile of grazing rays expands hundreds of nodes, most of them for a few of
+// its rays) takes as many steps as the union of its rays: of 32,400 tiles of a 1080p view of 1,004,000
+// triangles, half were done after 12 us and 90% after 78 us, but the longest took 351 us and set the
+// launch's 0.43 ms. Such a packet ends and its lanes go on by themselves, each with its part of the
+// shared stack: the longest now takes 250 us. The cast with ray generation: 0.468 -> 0.36 ms; a 1080p
+// frame with 8 lights, whose shadow rays are packets too: 1.77 -> 1.62 ms. (The limits matter little:
+// 0.377 to 0.383 ms for 4 or 8 steps and 12 to 48 rays; 16 steps of 24 rays 0.390, any 64 steps 0.419.
+// Four lanes per ray instead, 16 rays at a time: slower than not leaving, 0.59 ms.)
+
+constexpr int kPacketRows = 10;  // stack entries of a lane in LDS (20 KB a block, 7 blocks a CU)
+
+// Takes over a packet's lane: its stack entries, and whether the packet's next node is its own.
+struct PacketLeave {
+	PrivateStack<kPacketRows, kMaxPending>& stack;
+	LaneWalk& t;
+	bool& on;
+	__device__ __forceinline__ void push(int at, uint32_t ref, float tIn) { stack.put2(at, ref, tIn); }
+	__device__ __forceinline__ void operator()(int n, uint32_t node, bool at)
+	{
+		t.ref = node;
+		t.sp = n;
+		on = at;
+	}
+};
+
+template <bool kAnyHit>
+__global__ __launch_bounds__(kPacketBlock) void k_packet(const float4* __restrict__ wide,
+                                                         const float4* __restrict__ nodes,
+                                                         const float4* __restrict__ tris,
+                                                         const float4* __restrict__ rays,
+                                                         void* __restrict__ out, uint32_t n)
+{
+	__shared__ U32x2 stackLds[kPacketRows * kPacketBlock];
+	const uint32_t lane = __lane_id();
+	const uint32_t first = blockIdx.x * kPacketBlock + (threadIdx.x & ~63u);
+	if (first >= n) return;  // whole wave
+	const uint32_t i = first + lane;
+	const bool active = i < n;
+	const uint32_t ri = active ? i : first;  // lanes past the end read a valid ray, never used
+	LaneWalk t;
+	t.r = dev::make_ray(rays[2 * size_t(ri)], rays[2 * size_t(ri) + 1]);
+	bool occluded = false;
+	// The wide nodes only when every active lane may walk them (the decision is uniform).
+	if (wide && __ballot(active && !t.r.nanFree) == 0ull) {
+		U32x2 deep[kMaxPending - kPacketRows];
+		PrivateStack<kPacketRows, kMaxPending> stack = {(LdsU2*)(stackLds) + threadIdx.x, deep};
+		bool on = false;
+		t.ref = kWideLeaf;
+		packet_wide<kAnyHit>(wide, tris, t.r, active, t.c, occluded, PacketLeave{stack, t, on});
+		if (ballot(on || t.sp > 0) != 0ull) {
+			auto lim = [&] { return kAnyHit ? t.r.tMax : dev::min_first(t.r.tMax, t.c.t); };
+			if (!on && t.sp > 0) {
+				on = t.take(lim(), kAnyHit, stack);
+				if (on && !kAnyHit) t.decide_sibling(lim(), stack);
+			}
+			while (ballot(on) != 0ull) {
+				float4 w[8];
+				t.load(on, wide, tris, w);
+				if (on) on = !t.template advance<kAnyHit ? 1 : 0>(w, nodes, kAnyHit, stack, occluded);
+			}
+		}
+	} else {
+		packet_binary<kAnyHit>(nodes, tris, t.r, active, t.c, occluded);
+	}
+	if (active) {
+		if (kAnyHit)
+			static_cast<uint8_t*>(out)[i] = occluded ? 0 : 1;
+		else
+			static_cast<uint4*>(out)[i] = make_uint4(t.c.tri, __float_as_uint(t.c.t),
+			                                         __float_as_uint(t.c.u), __float_as_uint(t.c.v));
+	}
+}
+
 // ---- instances (two-level traversal) ------------------------------------------------------------
 //
 // A top tree over the instances' world boxes (one instance per leaf, PhxBVHNode layout) is walked
@@ -1595,29 +1685,7 @@ __device__ __forceinline__ bool object_ray(const DevInstance& in, const float4 a
 
 constexpr uint32_t kInstanceRefill = 8;  // idle lanes of a wave before it takes new rays
 constexpr uint32_t kInstanceWaves = 20;  // per CU: 5 per SIMD (96 registers)
-
-// A lane's stack column: 14 entries in LDS (28 KB a block, 5 blocks a CU), the deeper ones in private
-// memory. (The LDS part through an LDS pointer and read in any case: a choice between the two would be
-// made of flat loads.)
-struct InstanceStack {
-	static constexpr int kRows = 14;
-	LdsU2* col;
-	U32x2 (&deep)[2 * kMaxPending - kRows];
-	__device__ __forceinline__ void put2(int at, uint32_t ref, float tIn)
-	{
-		const U32x2 e = {ref, __float_as_uint(tIn)};
-		if (__builtin_expect(at < kRows, 1)) col[at * kBlock] = e;
-		else deep[at - kRows] = e;
-	}
-	__device__ __forceinline__ void get2(int at, uint32_t& ref, float& tIn) const
-	{
-		U32x2 e = col[(at < kRows ? at : 0) * kBlock];
-		if (__builtin_expect(ballot(at >= kRows) != 0ull, 0))
-			if (at >= kRows) e = deep[at - kRows];
-		ref = e.x;
-		tIn = __uint_as_float(e.y);
-	}
-};
+constexpr int kInstanceRows = 14;        // stack entries of a lane in LDS (28 KB a block, 5 blocks a CU)
 
 // The next float above x, so that t < next_up(x) is t <= x.
 __device__ __forceinline__ float next_up(float x)
@@ -1634,9 +1702,10 @@ __global__ __launch_bounds__(kBlock, 5) void k_trace_instances(
 	uint4* __restrict__ hits, uint32_t* __restrict__ instOut, uint8_t* __restrict__ inLight,
 	uint32_t n, uint32_t seeded, uint32_t* __restrict__ work)
 {
-	__shared__ U32x2 stackLds[InstanceStack::kRows * kBlock];
-	U32x2 deep[2 * kMaxPending - InstanceStack::kRows];
-	InstanceStack stack = {(LdsU2*)(stackLds) + threadIdx.x, deep};  // the top tree's entries, an instance's above
+	__shared__ U32x2 stackLds[kInstanceRows * kBlock];
+	U32x2 deep[2 * kMaxPending - kInstanceRows];
+	// The top tree's entries, an instance's above.
+	PrivateStack<kInstanceRows, 2 * kMaxPending> stack = {(LdsU2*)(stackLds) + threadIdx.x, deep};
 	QuadArgs P = {};
 	P.n = n;
 	P.window = 64u;

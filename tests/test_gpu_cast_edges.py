@@ -155,3 +155,24 @@ def test_spilled_stacks(ctx, depth):
                   True)
     finally:
         s.release()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 257, 4097, 32769])
+@pytest.mark.parametrize("which", ["random", "overlapping", "deep18", "deep60"])
+def test_packets_that_part(ctx, scenes, which, n):
+    """Packets of rays with nothing in common: they end, and their lanes go on with their parts of the
+    shared stack, some of it beyond the LDS rows."""
+    if which.startswith("deep"):
+        nodes, tris = caterpillar(int(which[4:]))
+        s, rays = ctx.upload_scene(nodes, tris), aimed(tris, n, 19, 2.0)
+    else:
+        s, b, rays = scenes[which == "overlapping"]
+        nodes, tris, rays = b.nodes, b.tris, rays[:n]
+    rays = rays[(rays["d"] != 0).all(axis=1)]  # (a zero component keeps its packet on binary nodes)
+    try:
+        assert ctx.cast_closest(s, rays, phx.KERNEL_PACKET).tobytes() == \
+            O.cast_closest(nodes, tris, rays).tobytes()
+        assert (ctx.cast_anyhit(s, rays, phx.KERNEL_PACKET) == O.cast_anyhit(nodes, tris, rays)).all()
+    finally:
+        if which.startswith("deep"):
+            s.release()
