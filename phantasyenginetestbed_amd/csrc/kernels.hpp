@@ -142,6 +142,19 @@ struct BatchClock {
 
 constexpr uint32_t kMaxFusedBatches = 1024;
 
+// Copies between pinned host memory and the device by a kernel, up to kCopyRanges ranges a launch; both
+// ends of a range are 16-byte aligned device addresses.
+constexpr uint32_t kCopyRanges = 64;
+struct CopyRange {
+	const void* src;
+	void* dst;
+	uint64_t bytes;
+};
+hipError_t launchCopies(const CopyRange* ranges, uint32_t count, hipStream_t stream);
+// The device address of `bytes` bytes at p if they are pinned host memory (one allocation) and 16-byte
+// aligned, else null.
+void* deviceAddress(const void* p, size_t bytes);
+
 // One persistent launch over `numBatches` batches; offsets[b] = first ray of batch b in the fused
 // index space, offsets[numBatches] = total. `clock` may be null (no completion tracking).
 hipError_t launchBatches(const BatchDesc* descs, const uint32_t* offsets, uint32_t numBatches,

@@ -75,6 +75,8 @@ struct PhxContext {
 	uint32_t window = 64;     // rays per fetch
 	uint32_t spillLanes = 0;  // lanes the device can hold: the limit of grid x block
 	// Staging buffers for calls that pass host pointers, grown on demand.
+	char* pinned = nullptr;   // rays and results of small casts on host buffers, read in place
+	char* pinnedDev = nullptr;  // its device address
 	void* stageIn = nullptr;
 	size_t stageInBytes = 0;
 	void* stageOut = nullptr;

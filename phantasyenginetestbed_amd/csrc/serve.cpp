@@ -35,11 +35,11 @@ double msSince(Clock::time_point t0) { return std::chrono::duration<double, std:
 constexpr size_t kAlign = 256;
 
 // Rays per fused launch before further admitted requests wait for the next launch. A backlog
-// coalesced into one or two launches runs its host-to-device copies, traversal and copies back
-// one after the other (the 143 M-ray saturated request mix: ~340 ms); in launches of a few million
-// rays the slot streams overlap one launch's copies with another's traversal (~175 ms). Each
-// launch of this size still fills the device many times over (4 M rays on ~1 k blocks).
-constexpr uint64_t kLaunchRays = 4u << 20;
+// coalesced into one or two launches runs its copies to the device, traversal and copies back one after
+// the other; in launches of about a million rays (0.7 ms of the link, 0.6 ms of traversal) the slot
+// streams overlap one launch's copies with another's traversal. 48 requests of 3.2 million rays in 3
+// slots: 3.34 ms at 4 million rays a launch, 3.12 at one million and at half, 3.79 at a quarter.
+constexpr uint64_t kLaunchRays = 1u << 20;
 size_t alignUp(size_t b) { return (b + kAlign - 1) / kAlign * kAlign; }
 
 // First-fit allocator over [0, size) with coalescing of neighbouring free ranges.
@@ -102,6 +102,9 @@ struct Request {
 	size_t outOff = 0, outBytes = 0;
 	const PhxRayIn* devRays = nullptr;
 	void* devOut = nullptr;
+	// Where kernels reach the caller's pinned rays and output; null: copied by copy calls.
+	const void* mappedRays = nullptr;
+	void* mappedOut = nullptr;
 	ReqState state = ReqState::Queued;
 	Clock::time_point submitted;
 	double latencyMs = 0.0;
@@ -116,7 +119,11 @@ struct Slot {
 	uint32_t* offsets = nullptr;
 	BatchDesc* hostDescs = nullptr;   // pinned
 	uint32_t* hostOffsets = nullptr;  // pinned
+	void* mappedDescs = nullptr;      // their device addresses
+	void* mappedOffsets = nullptr;
+	std::vector<CopyRange> copies;    // of the launch being formed
 	hipEvent_t done = nullptr;
+	hipEvent_t loaded = nullptr;      // its launch's rays are on the device
 	std::vector<Request*> reqs;
 	bool busy = false;
 };
@@ -135,6 +142,7 @@ struct PhxServer {
 	std::unordered_set<const PhxScene*> scenes;
 	std::vector<Slot> slots;
 	TraceLaunch shape;
+	hipEvent_t lastLoaded = nullptr;  // of the launch formed last
 
 	std::mutex mu;
 	std::condition_variable cvWork;  // dispatcher: new submissions
@@ -203,18 +211,34 @@ hipError_t launchSlot(PhxServer* s, Slot& slot)
 	hipError_t e = hipSuccess;
 	const uint32_t nb = uint32_t(slot.reqs.size());
 	uint32_t off = 0;
+	slot.copies.clear();
+	// One launch's rays at a time: on a shared link all would arrive late together.
+	if (s->lastLoaded && s->lastLoaded != slot.loaded)
+		e = hipStreamWaitEvent(slot.stream, s->lastLoaded, 0);
 	for (uint32_t b = 0; b < nb && e == hipSuccess; b++) {
 		Request* r = slot.reqs[b];
 		r->state = ReqState::InFlight;
-		if (!(r->req.flags & PHX_MEM_DEVICE) && r->req.numRays)
-			e = hipMemcpyAsync(const_cast<PhxRayIn*>(r->devRays), r->req.rays, r->rayBytes,
-			                   hipMemcpyHostToDevice, slot.stream);
+		if (!(r->req.flags & PHX_MEM_DEVICE) && r->req.numRays) {
+			if (r->mappedRays)
+				slot.copies.push_back({r->mappedRays, const_cast<PhxRayIn*>(r->devRays), r->rayBytes});
+			else
+				e = hipMemcpyAsync(const_cast<PhxRayIn*>(r->devRays), r->req.rays, r->rayBytes,
+				                   hipMemcpyHostToDevice, slot.stream);
+		}
 		slot.hostDescs[b] = batchDesc(r->req.scene, r->devRays, r->devOut, r->req.numRays, r->req.kind);
 		slot.hostOffsets[b] = off;
 		off += r->req.numRays;
 	}
 	slot.hostOffsets[nb] = off;
 	if (e != hipSuccess) return e;
+	if (!(s->flags & PHX_SERVE_PLAIN)) {
+		slot.copies.push_back({slot.mappedDescs, slot.descs, sizeof(BatchDesc) * nb});
+		slot.copies.push_back({slot.mappedOffsets, slot.offsets, sizeof(uint32_t) * (nb + 1)});
+	}
+	e = launchCopies(slot.copies.data(), uint32_t(slot.copies.size()), slot.stream);
+	if (e == hipSuccess) e = hipEventRecord(slot.loaded, slot.stream);
+	if (e != hipSuccess) return e;
+	s->lastLoaded = slot.loaded;
 	if (s->flags & PHX_SERVE_PLAIN) {
 		Request* r = slot.reqs[0];
 		TraceLaunch L = s->shape;
@@ -228,23 +252,21 @@ hipError_t launchSlot(PhxServer* s, Slot& slot)
 			e = launchClosest(sv, r->devRays, r->req.numRays, static_cast<PhxRayHit*>(r->devOut),
 			                  L, nullptr, slot.stream);
 	} else {
-		e = hipMemcpyAsync(slot.descs, slot.hostDescs, sizeof(BatchDesc) * nb,
-		                   hipMemcpyHostToDevice, slot.stream);
-		if (e == hipSuccess)
-			e = hipMemcpyAsync(slot.offsets, slot.hostOffsets, sizeof(uint32_t) * (nb + 1),
-			                   hipMemcpyHostToDevice, slot.stream);
 		TraceLaunch L = s->shape;
 		L.work = slot.work;
 		L.spill = slot.spill;
-		if (e == hipSuccess)
-			e = launchBatches(slot.descs, slot.offsets, nb, off, L, nullptr, slot.stream);
+		e = launchBatches(slot.descs, slot.offsets, nb, off, L, nullptr, slot.stream);
 	}
+	slot.copies.clear();
 	for (uint32_t b = 0; b < nb && e == hipSuccess; b++) {
 		Request* r = slot.reqs[b];
-		if (!(r->req.flags & PHX_MEM_DEVICE) && r->req.numRays)
-			e = hipMemcpyAsync(r->req.out, r->devOut, r->outBytes, hipMemcpyDeviceToHost,
-			                   slot.stream);
+		if ((r->req.flags & PHX_MEM_DEVICE) || !r->req.numRays) continue;
+		if (r->mappedOut)
+			slot.copies.push_back({r->devOut, r->mappedOut, r->outBytes});
+		else
+			e = hipMemcpyAsync(r->req.out, r->devOut, r->outBytes, hipMemcpyDeviceToHost, slot.stream);
 	}
+	if (e == hipSuccess) e = launchCopies(slot.copies.data(), uint32_t(slot.copies.size()), slot.stream);
 	if (e == hipSuccess) e = hipEventRecord(slot.done, slot.stream);
 	if (e == hipSuccess) {
 		slot.busy = true;
@@ -331,6 +353,7 @@ void destroyServer(PhxServer* s)
 		if (slot.hostDescs) hipHostFree(slot.hostDescs);
 		if (slot.hostOffsets) hipHostFree(slot.hostOffsets);
 		if (slot.done) hipEventDestroy(slot.done);
+		if (slot.loaded) hipEventDestroy(slot.loaded);
 		if (slot.stream && slot.ownStream) hipStreamDestroy(slot.stream);
 	}
 	hipFree(s->pool);
@@ -395,7 +418,13 @@ static phx_status phx_server_create_impl(PhxContext* ctx, uint64_t budgetBytes, 
 		if (e == hipSuccess)
 			e = hipHostMalloc(reinterpret_cast<void**>(&slot.hostOffsets),
 			                  4u * (kMaxFusedBatches + 1), hipHostMallocDefault);
+		if (e == hipSuccess) {
+			slot.mappedDescs = deviceAddress(slot.hostDescs, sizeof(BatchDesc) * kMaxFusedBatches);
+			slot.mappedOffsets = deviceAddress(slot.hostOffsets, 4u * (kMaxFusedBatches + 1));
+			if (!slot.mappedDescs || !slot.mappedOffsets) e = hipErrorInvalidDevicePointer;
+		}
 		if (e == hipSuccess) e = hipEventCreateWithFlags(&slot.done, hipEventDisableTiming);
+		if (e == hipSuccess) e = hipEventCreateWithFlags(&slot.loaded, hipEventDisableTiming);
 	}
 	if (e != hipSuccess) {
 		destroyServer(s);
@@ -498,6 +527,10 @@ static phx_status phx_server_submit_impl(PhxServer* s, const PhxRequest* req, ui
 	r->submitted = Clock::now();
 	r->rayBytes = size_t(req->numRays) * sizeof(PhxRayIn);
 	r->outBytes = size_t(req->numRays) * outBytesPerRay(req->kind);
+	if (!(req->flags & PHX_MEM_DEVICE) && req->numRays) {
+		r->mappedRays = deviceAddress(req->rays, r->rayBytes);
+		r->mappedOut = deviceAddress(req->out, r->outBytes);
+	}
 	std::lock_guard<std::mutex> g(s->mu);
 	if (!s->error.empty()) {
 		delete r;
