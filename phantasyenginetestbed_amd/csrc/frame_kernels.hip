@@ -8,31 +8,14 @@
 
 #include <cfloat>
 
-#include "kernels.hpp"
-#include "rng.hpp"
-#include "shading.hpp"
+#include "frame_device.hpp"
 
 namespace phx {
 namespace {
 
-using namespace shading;
+using namespace frame;
 
 constexpr uint32_t kBlock1D = 256;
-
-__device__ __forceinline__ uint32_t pixel_id(uint32_t x, uint32_t y, uint32_t w, uint32_t h)
-{
-	if ((w % 8u) == 0u && (h % 8u) == 0u) {
-		const uint32_t tile = (y / 8u) * (w / 8u) + (x / 8u);
-		return tile * 64u + (y % 8u) * 8u + (x % 8u);
-	}
-	return y * w + x;
-}
-
-__device__ __forceinline__ Pcg32 frame_rng(uint64_t seed, uint32_t frame, uint32_t purpose,
-                                           uint32_t id)
-{
-	return Pcg32::seeded(seed ^ (uint64_t(frame) << 32), (uint64_t(purpose) << 32) | id);
-}
 
 __device__ __forceinline__ void store_ray(float4* rays, size_t i, V3 o, float tMin, V3 d,
                                           float tMax)
@@ -47,8 +30,6 @@ __device__ __forceinline__ void store_dummy(float4* rays, size_t i)
 	rays[2 * i] = make_float4(1000000.0f, 1000000.0f, 1000000.0f, 0.001f);
 	rays[2 * i + 1] = make_float4(0.0f, 1.0f, 0.0f, 0.001f);
 }
-
-__device__ __forceinline__ V3 xyz(float4 a) { return v3(a.x, a.y, a.z); }
 
 // Texel coordinate along one axis of a wrapping, nearest-texel lookup
 // (CPURayTracerRenderer::sampleImage, CPUTracerRenderer.cpp:160-180):
@@ -165,12 +146,10 @@ __global__ __launch_bounds__(kBlock1D) void k_interpret(const float4* __restrict
 	info[3 * size_t(i) + 2] = make_float4(alb.x, alb.y, alb.z, fabsf(alb.w));
 }
 
-// shadeHit (MaterialKernel.cu:49-114) of every record: per light the contribution
-// mask * falloff * shade and a shadow ray towards a point on the light's disc (soft shadows,
-// radius 0 = point light), or the dummy ray when the light has no static shadows or contributes
-// nothing (every channel <= 1e-4). Primary records (rays == nullptr) view towards camPos with
-// mask 1 (gBufferMaterialKernel, :119-140); bounce records view along -ray.dir with their path
-// throughput (materialKernel, :145-184). Records without a hit get dummy rays and zero.
+// Every light's contribution and shadow ray (sample_light) of every record; where there is no ray, the
+// dummy one. Primary records (rays == nullptr) view towards camPos with mask 1 (gBufferMaterialKernel,
+// MaterialKernel.cu:119-140); bounce records view along -ray.dir with their path throughput
+// (materialKernel, :145-184). Records without a hit get dummy rays and zero.
 __global__ __launch_bounds__(kBlock1D) void k_shade(const float4* __restrict__ info,
                                                     const float4* __restrict__ rays,
                                                     const float4* __restrict__ throughput,
@@ -209,34 +188,13 @@ __global__ __launch_bounds__(kBlock1D) void k_shade(const float4* __restrict__ i
 	}
 	Pcg32 rng = frame_rng(seed, frame, purpose, id);
 	for (uint32_t i = 0; i < numLights; i++) {
-		const PhxSphereLight& L = lights[i];
-		const V3 lp = v3(L.pos[0], L.pos[1], L.pos[2]);
-		const V3 toL = sub(lp, p);
-		const float dist = length(toL);
-		const V3 l = divs(toL, dist);
-		const float fo = falloff(dist, L.range);
-		const V3 sh = shade(n, view, albedo, rough, metal, l, dist,
-		                    v3(L.strength[0], L.strength[1], L.strength[2]), L.range);
-		const V3 c = mul(scale(mask, fo), sh);
+		const LightSample sample = sample_light(lights[i], p, n, view, albedo, rough, metal, mask, rng);
 		const size_t s = size_t(id) + size_t(i) * count;
-		contrib[s] = make_float4(c.x, c.y, c.z, 0.0f);
-		const float eps = 0.0001f;
-		const bool lit = c.x > eps || c.y > eps || c.z > eps;
-		if (L.staticShadows && lit) {
-			const V3 cu = fabsf(n.z) > 0.01f ? normalize(v3(0.0f, -n.z, n.y))
-			                                 : normalize(v3(-n.y, n.x, 0.0f));
-			const V3 cv = cross(cu, l);
-			const float r1 = rng.uniform();
-			const float r2 = rng.uniform();
-			const float cd = L.radius * (2.0f * r2 - 1.0f);
-			float sn, cs;
-			turn_sincos(r1, sn, cs);
-			const V3 off = add(scale(scale(cu, cs), cd), scale(scale(cv, sn), cd));
-			const V3 diff = sub(add(lp, off), p);
-			store_ray(shadow, s, p, 0.001f, normalize(diff), length(diff));
-		} else {
+		contrib[s] = make_float4(sample.c.x, sample.c.y, sample.c.z, 0.0f);
+		if (sample.ray)
+			store_ray(shadow, s, p, 0.001f, sample.dir, sample.len);
+		else
 			store_dummy(shadow, s);
-		}
 	}
 }
 

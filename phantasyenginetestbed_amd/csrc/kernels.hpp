@@ -36,9 +36,8 @@ struct TexSet {
 	uint32_t count = 0;
 };
 
-// Persistent: four lanes per ray. Lane: also persistent, one ray per lane, the last ones four lanes
-// each. Simple: one ray per lane, no persistence. Packet: 64 rays walk together.
-enum class TraceKernel { Persistent, Lane, Simple, Packet };
+// Persistent: four lanes per ray. Simple: one ray per lane. Packet: 64 rays walk together.
+enum class TraceKernel { Persistent, Simple, Packet };
 
 // Words of a launch's ray counters, and words of stack spill per ray in flight.
 constexpr uint32_t kRayCounterWords = 1024;
@@ -184,6 +183,12 @@ hipError_t launchSetFrameParams(FrameParams* dst, const FrameParams& value, hipS
 hipError_t launchGenPrimaryRays(const PhxCameraDef& cam, uint32_t w, uint32_t h, float jx,
                                 float jy, float tMin, float tMax, uint32_t order, PhxRayIn* rays,
                                 hipStream_t stream, const FrameParams* fp = nullptr);
+
+// The primary records' colours: launchShade of `info` (primary), an any-hit cast against `s` of its
+// shadow rays and launchShadowLogic at full resolution, in one pass over the records.
+hipError_t launchShadeTrace(const SceneView& s, const float4* info, const PhxSphereLight* lights,
+                            uint32_t numLights, uint32_t w, uint32_t h, const FrameParams* fp,
+                            uint32_t purpose, float4* img, hipStream_t stream);
 
 // Wavefront frame kernels (frame_kernels.hip). Hit records are 3 float4 each:
 // (position, roughness) (normal, metallic) (albedo, alpha; alpha < 0 = no hit).

@@ -130,19 +130,14 @@ phx_status enqueueFrame(PhxContext* ctx, PhxRenderer* r, const PhxScene* scene,
 	const TraceLaunch closest = traceLaunch(ctx, 0, false);
 	// Shadow rays are coherent -- a pixel tile's rays towards one light, tiles in order -- so they
 	// are traced as packets, each wave expanding the union of 64 rays' nodes. So are camera rays in
-	// 8x8-tile order (a wave's 64 rays are one tile): 0.50 ms instead of 0.77 ms for a 1080p
-	// frame's closest hits; in row-major order a wave's rays span a 64-pixel row segment and
-	// packets gain nothing, so those go to the persistent kernel.
+	// 8x8-tile order (a wave's 64 rays are one tile): 0.33 ms for a 1080p frame's closest hits, where
+	// the persistent kernel takes 0.47 ms for half of them; in row-major order a wave's rays span a
+	// 64-pixel row segment and packets gain nothing, so those go to the persistent kernel.
 	TraceLaunch shadows = traceLaunch(ctx, 0, true);
 	shadows.kernel = TraceKernel::Packet;
 	// The bounce hits' shadow rays start at scattered points (neighbouring half-resolution pixels'
 	// bounce rays go anywhere), so a packet's union of nodes is large: the persistent kernel.
 	const TraceLaunch bounceShadows = traceLaunch(ctx, 0, true);
-	// The bounce rays are traced beside the shadow packets, which the kernel of four lanes per ray
-	// would slow down more than it gains: 1080p with 8 lights takes 1.87 ms with it, 1.74 ms with one
-	// ray per lane.
-	TraceLaunch bounce = closest;
-	bounce.kernel = TraceKernel::Lane;
 	TraceLaunch primary = closest;
 	if (order == PHX_RAYS_TILED_8X8) primary.kernel = TraceKernel::Packet;
 	const char* what = "phx_render_frame";
@@ -162,39 +157,44 @@ phx_status enqueueFrame(PhxContext* ctx, PhxRenderer* r, const PhxScene* scene,
 	        what);
 	PHX_HIP(launchClosest(sv, r->prim, r->n, r->primHits, primary, nullptr, s), what);
 	if (inst)
-		PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst, r->prim, r->n,
-		                        r->primHits, r->primInst, nullptr, true, onMain, s),
+		PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst,
+		                        r->prim, r->n, r->primHits, r->primInst, nullptr, true, onMain, s),
 		        what);
 	PHX_HIP(launchInterpret(r->prim, r->primHits, r->n, scene->datas, scene->numTris,
 	                        scene->materials, scene->numMaterials, scene->tex, r->gbuf, s,
 	                        inst ? r->primInst : nullptr, instByIndex, numInst),
 	        what);
-	PHX_HIP(launchShade(r->gbuf, nullptr, nullptr, scene->lights, L, r->n, r->params, 1u,
-	                    r->contrib, r->shadow, s),
-	        what);
-	// Bounce rays (they need only the hit records): incoherent, traced by the persistent kernel.
+	// Bounce rays (they need only the hit records, so they start before the shading): incoherent, traced
+	// by the persistent kernel.
 	PHX_HIP(launchGenSecondary(r->gbuf, r->w, r->h, r->params, r->bounce, r->throughput, s),
 	        what);
 	// The bounce rays' closest hits (the persistent kernel, whose last rays take long) overlap the
-	// primary shadow rays and their shadow logic; the bounce records need the shading buffers back,
-	// so the streams join before them. No other persistent launch runs meanwhile, so the two
+	// primary shading and shadow rays; the bounce records need the shading buffers back, so the
+	// streams join before them. No other persistent launch runs meanwhile, so the two
 	// streams never share the context's ray counter or spill area.
 	if (r->m) {
 		PHX_HIP(hipEventRecord(r->fork, s), what);
 		PHX_HIP(hipStreamWaitEvent(r->side, r->fork, 0), what);
-		PHX_HIP(launchClosest(sv, r->bounce, r->m, r->bounceHits, bounce, nullptr, r->side), what);
+		PHX_HIP(launchClosest(sv, r->bounce, r->m, r->bounceHits, closest, nullptr, r->side), what);
 		if (inst)
-			PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst, r->bounce,
-			                        r->m, r->bounceHits, r->bounceInst, nullptr, true, closest, r->side),
+			PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst,
+			                        r->bounce, r->m, r->bounceHits, r->bounceInst, nullptr, true, closest, r->side),
 			        what);
 		PHX_HIP(hipEventRecord(r->join, r->side), what);
 	}
-	PHX_HIP(launchAnyHit(sv, r->shadow, r->n * L, r->inLight, shadows, s), what);
-	if (inst)
-		PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst, r->shadow,
-		                        r->n * L, nullptr, nullptr, r->inLight, true, onMain, s),
+	if (!inst) {
+		PHX_HIP(launchShadeTrace(sv, r->gbuf, scene->lights, L, r->w, r->h, r->params, 1u, r->color, s),
 		        what);
-	PHX_HIP(launchShadowLogic(r->color, r->w, r->h, 1u, false, r->inLight, r->contrib, L, s), what);
+	} else {  // the instances occlude too: a pass of their own over the stored shadow rays
+		PHX_HIP(launchShade(r->gbuf, nullptr, nullptr, scene->lights, L, r->n, r->params, 1u,
+		                    r->contrib, r->shadow, s),
+		        what);
+		PHX_HIP(launchAnyHit(sv, r->shadow, r->n * L, r->inLight, shadows, s), what);
+		PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst,
+		                        r->shadow, r->n * L, nullptr, nullptr, r->inLight, true, onMain, s),
+		        what);
+		PHX_HIP(launchShadowLogic(r->color, r->w, r->h, 1u, false, r->inLight, r->contrib, L, s), what);
+	}
 
 	// Bounce hits: records, shading x throughput with shadow rays, any hit, added at half res.
 	if (r->m) {
@@ -208,8 +208,8 @@ phx_status enqueueFrame(PhxContext* ctx, PhxRenderer* r, const PhxScene* scene,
 		        what);
 		PHX_HIP(launchAnyHit(sv, r->shadow, r->m * L, r->inLight, bounceShadows, s), what);
 		if (inst)
-			PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst, r->shadow,
-			                        r->m * L, nullptr, nullptr, r->inLight, true, onMain, s),
+			PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst,
+			                        r->shadow, r->m * L, nullptr, nullptr, r->inLight, true, onMain, s),
 			        what);
 		PHX_HIP(launchShadowLogic(r->color, r->w, r->h, 2u, true, r->inLight, r->contrib, L, s),
 		        what);
