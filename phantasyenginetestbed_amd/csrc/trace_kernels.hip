@@ -31,8 +31,11 @@ constexpr int kBlock = 256;
 // and which wait on both the vector-memory and LDS counters.
 typedef uint32_t U32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t U32x4 __attribute__((ext_vector_type(4)));
+typedef float F32x4 __attribute__((ext_vector_type(4)));
 #if defined(__HIP_DEVICE_COMPILE__)
 typedef const float4 __attribute__((address_space(1))) GlobalF4;
+typedef const F32x4 __attribute__((address_space(1))) GlobalV4;
+typedef F32x4 __attribute__((address_space(3))) LdsF4;
 typedef U32x2 __attribute__((address_space(1))) GlobalU2;
 typedef U32x4 __attribute__((address_space(1))) GlobalU4;
 typedef uint8_t __attribute__((address_space(1))) GlobalU8;
@@ -40,6 +43,8 @@ typedef U32x2 __attribute__((address_space(3))) LdsU2;
 typedef uint32_t __attribute__((address_space(3))) LdsU1;
 #else  // the host pass only needs the declarations to parse
 typedef const float4 GlobalF4;
+typedef const F32x4 GlobalV4;
+typedef F32x4 LdsF4;
 typedef U32x2 GlobalU2;
 typedef U32x4 GlobalU4;
 typedef uint8_t GlobalU8;
@@ -781,11 +786,14 @@ __device__ __forceinline__ uint32_t find_batch(const uint32_t* offsets, uint32_t
 // pipeline and a one-ray-per-wave mode for a wave's last rays) a launch was bound by its chains of
 // steps: 25 a bounce ray on 1,004,000 triangles, half of the time spent on the last 1% of the rays,
 // and 15,600 fetches from and 2,048 retirements to one address at 10 ns each. Before and now:
-//   998,029 bounce rays, closest hit   0.567 ms   0.466 ms
+//   998,029 bounce rays, closest hit   0.567 ms   0.438 ms
 //   their 998,029 shadow rays, any hit  0.254 ms   0.122 ms
-//   65,536 random rays, 100,000 random triangles  0.243 ms   0.125 ms
+//   65,536 random rays, 100,000 random triangles  0.243 ms   0.120 ms
 // Many rays at once are bound by VALU issue (a wave instruction serves 16 rays), the rest by the
-// chain of the costliest rays: about 450 iterations of 0.9 us, the time a wave takes to issue one.
+// chain of the costliest rays: about 450 iterations of 0.9 us, the time a wave takes to issue one. So
+// instructions count: flags between bytes, selects and compares to make a ballot, minima that first
+// canonicalise, a multiplication by 48 and the binary walk's checks cost 5% (bounce 0.467 -> 0.442).
+// Selects in place of the branches of what comes next cost more than they save (0.488).
 
 constexpr uint32_t kQuadBlock = 512;  // largest block of the persistent kernels
 constexpr uint32_t kQuadWavesPerSimd = 7;  // (72 registers)
@@ -794,9 +802,9 @@ constexpr uint32_t kQuadWavesPerSimd = 7;  // (72 registers)
 // that the top three can be read at any depth. Deeper entries spill to memory, kSpillEntries a
 // column, one after another.
 constexpr int kQuadRows = 20;  // (pending stacks of 20 are rare)
-constexpr int kLaneRows = 16;  // (9.5 KB a wave: 16 waves per CU)
+constexpr int kLaneRows = 12;  // (9.5 KB a wave with 2 KB of rays: 16 waves per CU)
 // Idle lanes of a one-ray-per-lane wave before it takes new rays: 64 batches of 3.2 million rays take
-// 1.79 ms with 4, 1.73 with 8 and 32, 1.70 with 16.
+// 1.66 ms with 4, 1.65 with 8 and 16, 1.68 with 24.
 constexpr uint32_t kLaneRefill = 16;
 constexpr uint32_t kSpillEntries = kSpillWordsPerRay / 2u;
 static_assert(kLaneRows + int(kSpillEntries) >= kMaxPending, "stack entries of a ray");
@@ -827,7 +835,7 @@ constexpr uint32_t kCounterStride = 32;
 
 __host__ __device__ __forceinline__ uint32_t quad_lds_words(uint32_t waves)
 {
-	return waves * 2u * wave_stack_entries<kQuadRows, 16u>();
+	return waves * (2u * wave_stack_entries<kQuadRows, 16u>() + 512u);  // stacks, staged rays
 }
 
 // (__ballot takes an int: a select and a compare more.)
@@ -890,20 +898,21 @@ struct Quad {
 	uint32_t ray = kInvalid;     // index in the launch
 	uint32_t node = kInvalid;    // node to expand next, entered at nodeIn
 	float nodeIn = 0.0f;
-	bool leaf = false;           // triangles to test before it: this lane's is tri
 	uint32_t tri = 0u, triNext = 0u;  // triNext: lane 0's next one if the leaf goes on
 	uint32_t skip = 0u;          // lanes whose end marker is the first leaf's of a pair
 	int sp = 0;
 	uint32_t base = 0u;          // its stack column: LDS entry of the bottom row
 	float best = FLT_MAX, u = FLT_MAX, v = FLT_MAX;  // closest hit; u, v, hit in the lane it is `mine`
 	uint32_t hit = kInvalid;
-	bool mine = false;
-	bool exact = false;          // walks the binary nodes
+	// (4-byte flags: between the others' bytes, hit was kept in four registers.)
+	uint32_t mine = 0u;          // holds the closest hit
+	uint32_t exact = 0u;         // walks the binary nodes
+	uint32_t any = 0u;
+	bool leaf = false;           // triangles to test before node: this lane's is tri
 	// batches
 	const float4* wide = nullptr;
 	const float4* tris = nullptr;
 	uint32_t batch = 0u;
-	bool any = false;
 };
 
 // Writes a ray's result: its closest hit, or 0 if occluded and 1 if not.
@@ -969,14 +978,13 @@ struct QuadTracer {
 	const QuadArgs& P;
 	LdsU2* stacks;       // the block's stack columns
 	uint32_t lane, l;
+	bool someExact = false;  // (uniform) a ray of the wave may walk the binary nodes
 	Quad q;
 
 	__device__ __forceinline__ bool isAny() const { return kAny == 1 || (kAny == 2 && q.any); }
-	__device__ __forceinline__ uint32_t nibble(bool p) const
-	{
-		const uint64_t b = ballot(p);
-		return uint32_t(b >> (lane & 60u)) & 15u;
-	}
+	// The quad's four bits of a ballot. (Ballots of single comparisons, combined as masks: of a
+	// combined condition, a ballot takes a select and a compare more.)
+	__device__ __forceinline__ uint32_t nibble(uint64_t b) const { return uint32_t(b >> (lane & 60u)) & 15u; }
 	// Entry `at` of the stack column: in LDS, or spilled (at >= kRows).
 	__device__ __forceinline__ LdsU2* row(int at) const { return stacks + (q.base + uint32_t(at) * kCols); }
 	__device__ __forceinline__ GlobalU2* spilled(int at) const
@@ -991,14 +999,36 @@ struct QuadTracer {
 		return e;
 	}
 
-	// Sets this quad up for ray `ray`: its record, and if it is new its traversal.
-	__device__ __forceinline__ void start(uint32_t ray, bool fresh)
+	// Sets this quad up for ray `ray` with the record (a, b).
+	__device__ __forceinline__ void set(uint32_t ray, const float4 a, const float4 b, bool hasWide)
+	{
+		q.exact = !(quad_ray(a, b, q.r) && hasWide);
+		if (__builtin_expect(ballot(q.exact) != 0ull, 0)) {
+			q.r.ix = 1.0f / b.x;
+			q.r.iy = 1.0f / b.y;
+			q.r.iz = 1.0f / b.z;
+		}
+		q.ray = ray;
+	}
+	// Starts a ray of a single cast.
+	__device__ __forceinline__ void start(uint32_t ray, const float4 a, const float4 b)
+	{
+		set(ray, a, b, P.wide != P.tris);
+		q.node = 0u;
+		q.nodeIn = -INFINITY;
+		q.leaf = false;
+		q.sp = 0;
+		q.best = q.u = q.v = FLT_MAX;
+		q.hit = kInvalid;
+		q.mine = l == 0u;
+	}
+	// Takes over a ray that is being traced (its batch is set; its traversal is the caller's).
+	__device__ __forceinline__ void take_over(uint32_t ray)
 	{
 		const float4* rays = P.rays;
 		uint32_t at = ray;
 		bool hasWide = P.wide != P.tris;
 		if (kBatch) {
-			if (fresh) q.batch = find_batch(P.offsets, P.numBatches, ray);
 			at = ray - P.offsets[q.batch];
 			const BatchDesc d = P.descs[q.batch];
 			rays = d.rays;
@@ -1007,23 +1037,7 @@ struct QuadTracer {
 			q.any = d.kind != 0u;
 			hasWide = d.wide != d.tris;
 		}
-		const float4 a = as_global(rays)[2 * size_t(at)], b = as_global(rays)[2 * size_t(at) + 1];
-		q.exact = !(quad_ray(a, b, q.r) && hasWide);
-		if (__builtin_expect(ballot(q.exact) != 0ull, 0)) {
-			q.r.ix = 1.0f / b.x;
-			q.r.iy = 1.0f / b.y;
-			q.r.iz = 1.0f / b.z;
-		}
-		q.ray = ray;
-		if (fresh) {
-			q.node = 0u;
-			q.nodeIn = -INFINITY;
-			q.leaf = false;
-			q.sp = 0;
-			q.best = q.u = q.v = FLT_MAX;
-			q.hit = kInvalid;
-			q.mine = l == 0u;
-		}
+		set(ray, as_global(rays)[2 * size_t(at)], as_global(rays)[2 * size_t(at) + 1], hasWide);
 	}
 
 	// Expands a binary node: lanes 0 and 1 decide its children as castRay does, and what is visited is
@@ -1038,8 +1052,8 @@ struct QuadTracer {
 		float tIn, tOut;
 		dev::slab(q.r, box[0], box[1], box[2], box[3], box[4], box[5], tIn, tOut);
 		const bool pass = l < 2u && (tOut >= tIn) && tOut > q.r.tMin && tIn < lim;
-		const uint32_t m = nibble(pass);
-		const bool leftFirst = (nibble(pass && isLeaf) & 1u) != 0u;
+		const uint32_t m = nibble(ballot(pass));
+		const bool leftFirst = (nibble(ballot(pass && isLeaf)) & 1u) != 0u;
 		const int at = q.sp + (m == 3u && (l == 0u) == leftFirst ? 1 : 0);
 		const U32x2 e = {child_index(child) | (isLeaf ? kWideLeaf : 0u), __float_as_uint(-INFINITY)};
 		if (pass) {
@@ -1060,14 +1074,17 @@ struct QuadTracer {
 		// compiler waits for the first to test its end marker); quads without one read the array's
 		// first line. Offsets in bytes: 48 per triangle, 128 per wide node.
 		const uint32_t tri = q.leaf ? q.tri : 0u;
-		const uint32_t node = q.node != kInvalid && !q.exact ? q.node : 0u;
+		uint32_t node = q.node != kInvalid ? q.node : 0u;
+		if (someExact) node = q.exact ? 0u : node;
 		const float4* pl;
 		const float4* pn;
 		if (kBig) {
 			pl = tris + 3u * size_t(tri);
 			pn = wide + 8u * size_t(node) + 2u * l;
 		} else {
-			pl = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(tris) + ((tri + 2u * tri) << 4));
+			uint32_t tri3;
+			asm("v_lshl_add_u32 %0, %1, 1, %1" : "=v"(tri3) : "v"(tri));  // (a 32-bit multiply takes four times as long)
+			pl = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(tris) + (tri3 << 4));
 			pn = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(wide) + ((node << 7) + (l << 5)));
 		}
 		const float4 p0 = as_global(pl)[0], e1 = as_global(pl)[1], e2 = as_global(pl)[2];
@@ -1076,23 +1093,23 @@ struct QuadTracer {
 		if (q.leaf) {
 			// The leaf's triangles up to its end marker; candidates are accepted in lane order, which
 			// is castRay's: the smallest t, the lowest lane on equal t.
-			const uint32_t ends = nibble(p0.w < 0.0f) & ~q.skip;
+			const uint32_t ends = nibble(ballot(p0.w < 0.0f)) & ~q.skip;
 			const bool inLeaf = (ends & ((1u << l) - 1u)) == 0u;
 			const dev::TriDet d = dev::tri_det(q.r, e1, e2);
 			const float f = recip_wave(d.a);
 			float t, u, v;
 			const bool hit = dev::tri_finish(q.r, d, f, p0, e1, e2, t, u, v) && inLeaf && q.r.tMin <= t;
-			if (kAny != 0) occluded = nibble(hit && t < q.r.tMax) != 0u && any;
+			if (kAny != 0) occluded = nibble(ballot(hit) & ballot(t < q.r.tMax)) != 0u && any;
 			if (kAny != 1 && !any) {
 				const bool cand = hit && t < q.best && t <= q.r.tMax;
 				float tm = cand ? t : INFINITY;
-				tm = fminf(tm, quad_perm<0xB1>(tm));  // lanes 1 0 3 2
-				tm = fminf(tm, quad_perm<0x4E>(tm));  // lanes 2 3 0 1
+				tm = dev::vmin(tm, quad_perm<0xB1>(tm));  // lanes 1 0 3 2
+				tm = dev::vmin(tm, quad_perm<0x4E>(tm));  // lanes 2 3 0 1
 				const bool least = cand && t == tm;
-				const uint32_t win = nibble(least);
+				const uint32_t win = nibble(ballot(cand) & ballot(t == tm));
 				const bool me = least && (win & ((1u << l) - 1u)) == 0u;
-				q.best = me ? t : fminf(q.best, tm);  // (its own t: a zero's sign)
-				q.mine = win != 0u ? me : q.mine;
+				q.best = me ? t : dev::vmin(q.best, tm);  // (its own t: a zero's sign)
+				q.mine = win != 0u ? uint32_t(me) : q.mine;
 				q.u = me ? u : q.u;
 				q.v = me ? v : q.v;
 				q.hit = me ? q.tri : q.hit;
@@ -1103,15 +1120,19 @@ struct QuadTracer {
 			q.skip = 0u;
 		}
 		const float lim = any ? q.r.tMax : dev::min_first(q.r.tMax, q.best);
-		if (__builtin_expect(q.exact && q.node != kInvalid && !more, 0)) {
-			expand_binary(lim);
-			q.node = kInvalid;
-		}
+		if (__builtin_expect(someExact, 0))
+			if (q.exact && q.node != kInvalid && !more) {
+				expand_binary(lim);
+				q.node = kInvalid;
+			}
 		if (q.node != kInvalid && !more) {
 			// The passing slots are pushed, last slot first; a leaf pair stays one only if both pass.
 			float tIn;
-			const bool pass = decide_slot(q.r, lo, hi, lim, tIn) && (any || q.nodeIn < lim);
-			const uint32_t m = nibble(pass);
+			float tOut;
+			dev::slab_fast(q.r, lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, tIn, tOut);
+			const bool enters = any || q.nodeIn < lim;
+			const bool pass = (tOut >= tIn) && tOut > q.r.tMin && tIn < lim && enters;
+			const uint32_t m = nibble(ballot(tOut >= tIn) & ballot(tOut > q.r.tMin) & ballot(tIn < lim) & ballot(enters));
 			const uint32_t after = m >> (l + 1u);
 			uint32_t ref = __float_as_uint(lo.w);
 			ref = (after & 1u) ? ref : ref & ~kWidePair;
@@ -1197,28 +1218,51 @@ struct QuadTracer {
 	}
 };
 
-template <int kAny, bool kBatch, bool kTrack, bool kClock, bool kBig>
+// A window's rays are loaded when it is claimed, one per lane, and handed out of LDS: a ray that started
+// with loads of its own held up the wave's other 15 (with 2 of 16 rays taking new ones at a time, every
+// other step). With it 998,029 any-hit shadow rays take 0.122 ms instead of 0.127, bounce rays 0.438
+// instead of 0.449.
+template <int kAny, bool kClock, bool kBig>
 __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 {
 	const uint32_t waveInBlock = uniform(threadIdx.x >> 6), blockWaves = blockDim.x / 64u;
-	QuadTracer<kAny, kBatch, kTrack, kClock, kBig, kQuadRows, 16u> T{P};
+	QuadTracer<kAny, false, false, kClock, kBig, kQuadRows, 16u> T{P};
 	T.stacks = (LdsU2*)(reinterpret_cast<U32x2*>(lds));
 	T.lane = __lane_id();
 	T.l = T.lane & 3u;
 	T.q.base = stack_base<kQuadRows, 16u>(waveInBlock, T.lane >> 2);
+	LdsF4* const staged =
+		(LdsF4*)(lds + blockWaves * 2u * wave_stack_entries<kQuadRows, 16u>()) + waveInBlock * 128u;
 	if (kClock && threadIdx.x == 0u) atomicMin(&P.clock[P.n], wall_clock64());
 	RayWindows W(P, waveInBlock);
+	uint32_t first = W.next;  // the staged window's first ray
+	auto stage = [&] {
+		first = W.next;
+		if (W.next + T.lane < W.end) {
+			GlobalV4* p = (GlobalV4*)(P.rays) + 2u * size_t(W.next + T.lane);
+			staged[T.lane] = p[0];
+			staged[64u + T.lane] = p[1];
+		}
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+	};
+	stage();
 	while (true) {
 		const uint64_t idle = ballot(T.q.ray == kInvalid);
 		if (idle != 0ull) {
 			if (W.next >= W.end) {
 				if (!W.claim(P)) break;
-							if (W.next >= W.end) continue;
+				stage();
 			}
 			const uint32_t room = uint32_t(__popcll(idle)) / 4u;
 			if (room >= P.refill) {
 				const uint32_t ray = W.next + uint32_t(__popcll(idle & __lanemask_lt())) / 4u;
-				if (T.q.ray == kInvalid && ray < W.end) T.start(ray, true);
+				if (T.q.ray == kInvalid && ray < W.end) {
+					const F32x4 a = staged[ray - first], b = staged[64u + ray - first];
+					T.start(ray, make_float4(a.x, a.y, a.z, a.w), make_float4(b.x, b.y, b.z, b.w));
+				}
+				T.someExact = ballot(T.q.exact != 0u) != 0ull;
 				W.next = W.end - W.next < room ? W.end : W.next + room;
 			}
 		}
@@ -1232,13 +1276,13 @@ __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 
 // ---- one ray per lane, then four lanes per ray -----------------------------------------------------
 //
-// Fused launches: a wave traces 64 rays, one a lane, and once no rays are left to take and at most 16 are busy, those four lanes each, on the
-// stack columns that they have. A step of one ray per lane issues fewer instructions a ray (a wave
+// Fused launches: a wave traces 64 rays, one a lane, and once no rays are left to take and at most 16
+// are busy, those four lanes each, on the stack columns that they have. A step of one ray per lane issues fewer instructions a ray (a wave
 // instruction serves 64 rays, not 16) but reads 64 lines with each load, takes a leaf and a node in
 // steps of their own and is as slow as its costliest lane, so four lanes per ray are the faster way
 // for a launch by itself (1,048,576 random rays, 4 waves per SIMD: 0.485 ms against 0.468 ms) and one
-// lane is where the device is full: 64 batches of 3.2 million rays on two scenes take 1.66 ms (2.3 ms
-// four lanes each; 1.80 ms with the binary nodes). There the texture data path is busy 85% of the
+// lane is where the device is full: 64 batches of 3.2 million rays on two scenes take 1.65 ms (2.3 ms
+// four lanes each; 1.79 ms with the binary nodes). There the texture data path is busy 85% of the
 // time, the VALUs 63%. Handing the records over in LDS, four lanes to a line, took it to 1.60 ms and
 // single casts from 0.106 to 0.123 ms, so each lane loads its own.
 
@@ -1423,22 +1467,55 @@ struct LaneTracer {
 	const float4* tris = nullptr;
 
 	__device__ __forceinline__ bool isAny() const { return kAny == 1 || (kAny == 2 && any); }
+
+	// A window whose rays are staged in LDS, a lane's each. Its batch and that one's scene, if it has
+	// only one.
+	LdsF4* staged;
+	uint32_t first = 0u, windowBatch = 0u;
+	bool single = true;
+	BatchDesc desc = {};
+	__device__ __forceinline__ void stage(const RayWindows& W)
+	{
+		const uint32_t lane = __lane_id();
+		first = W.next;
+		const float4* rays = P.rays;
+		uint32_t at = first + lane;
+		if (kBatch && W.next < W.end) {
+			windowBatch = uniform(find_batch(P.offsets, P.numBatches, first));
+			single = uniform(P.offsets[windowBatch + 1u]) >= W.end;
+			desc = P.descs[windowBatch];
+			if (at < W.end) {
+				const uint32_t b = single ? windowBatch : find_batch(P.offsets, P.numBatches, at);
+				rays = single ? desc.rays : P.descs[b].rays;
+				at -= P.offsets[b];
+			}
+		}
+		if (first + lane < W.end) {
+			GlobalV4* p = (GlobalV4*)(rays) + 2u * size_t(at);
+			staged[lane] = p[0];
+			staged[64u + lane] = p[1];
+		}
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+	}
 	__device__ __forceinline__ void start(uint32_t index)
 	{
-		const float4* rays = P.rays;
-		uint32_t at = index;
 		bool hasWide = P.wide != P.tris;
 		if (kBatch) {
-			batch = find_batch(P.offsets, P.numBatches, index);
-			at = index - P.offsets[batch];
-			const BatchDesc d = P.descs[batch];
-			rays = d.rays;
+			batch = windowBatch;
+			BatchDesc d = desc;
+			if (!single) {
+				batch = find_batch(P.offsets, P.numBatches, index);
+				d = P.descs[batch];
+			}
 			wide = d.wide;
 			tris = d.tris;
 			any = d.kind != 0u;
 			hasWide = d.wide != d.tris;
 		}
-		const float4 a = as_global(rays)[2 * size_t(at)], b = as_global(rays)[2 * size_t(at) + 1];
+		const F32x4 sa = staged[index - first], sb = staged[64u + index - first];
+		const float4 a = make_float4(sa.x, sa.y, sa.z, sa.w), b = make_float4(sb.x, sb.y, sb.z, sb.w);
 		t.exact = !(quad_ray(a, b, t.r) && hasWide);
 		if (__builtin_expect(t.exact, 0)) {
 			t.r.ix = 1.0f / b.x;
@@ -1477,13 +1554,15 @@ __device__ __forceinline__ void lane_trace(const QuadArgs& P, uint32_t* lds)
 		T.wide = P.descs[0].wide;
 		T.tris = P.descs[0].tris;
 	}
+	T.staged = (LdsF4*)(lds + blockDim.x / 64u * 2u * wave_stack_entries<kLaneRows, 64u>()) + waveInBlock * 128u;
 	RayWindows W(P, waveInBlock);
+	T.stage(W);
 	while (true) {
 		const uint64_t idle = ballot(T.ray == kInvalid);
 		if (idle != 0ull) {
 			if (W.next >= W.end) {
 				if (!W.claim(P)) break;
-							if (W.next >= W.end) continue;
+				T.stage(W);
 			}
 			const uint32_t room = uint32_t(__popcll(idle));
 			if (room >= P.refill) {
@@ -1523,7 +1602,7 @@ __device__ __forceinline__ void lane_trace(const QuadArgs& P, uint32_t* lds)
 	const uint32_t hit = move(T.t.c.tri), batch = kBatch ? move(T.batch) : 0u;
 	if (lane / 4u < uint32_t(__popcll(busy))) {
 		Q.q.batch = batch;
-		Q.start(ray, false);
+		Q.take_over(ray);
 		Q.q.best = best;
 		Q.q.u = u;
 		Q.q.v = v;
@@ -1539,6 +1618,7 @@ __device__ __forceinline__ void lane_trace(const QuadArgs& P, uint32_t* lds)
 		Q.q.wide = P.descs[0].wide;
 		Q.q.tris = P.descs[0].tris;
 	}
+	Q.someExact = ballot(Q.q.exact != 0u) != 0ull;
 	while (ballot(Q.q.ray != kInvalid) != 0ull) Q.step();
 }
 
@@ -1558,7 +1638,7 @@ __device__ __forceinline__ bool retire_block(uint32_t* work)
 
 __host__ __device__ __forceinline__ uint32_t lane_lds_words(uint32_t waves)
 {
-	return waves * 2u * wave_stack_entries<kLaneRows, 64u>();
+	return waves * (2u * wave_stack_entries<kLaneRows, 64u>() + 512u);  // stacks, staged rays
 }
 
 // ---- packets, then one ray per lane ----------------------------------------------------------------
@@ -1900,7 +1980,7 @@ __global__ __launch_bounds__(kQuadBlock, kQuadWavesPerSimd) void k_quad(
 	extern __shared__ uint32_t lds[];
 	const QuadArgs P = {wide, nodes, tris, rays, out, n, window, refill, work, spill, clock,
 	                    nullptr, nullptr, 0u, nullptr, nullptr};
-	quad_trace<kAnyHit ? 1 : 0, false, false, kClock, kBig>(P, lds);
+	quad_trace<kAnyHit ? 1 : 0, kClock, kBig>(P, lds);
 	if (threadIdx.x == 0u) retire_block(work);
 }
 
