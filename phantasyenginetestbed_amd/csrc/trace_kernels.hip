@@ -796,6 +796,7 @@ __device__ __forceinline__ uint32_t find_batch(const uint32_t* offsets, uint32_t
 // Selects in place of the branches of what comes next cost more than they save (0.488).
 
 constexpr uint32_t kQuadBlock = 512;  // largest block of the persistent kernels
+constexpr uint32_t kStageWords = 512u + 64u;  // of a wave: a window's rays and their indices
 constexpr uint32_t kQuadWavesPerSimd = 7;  // (72 registers)
 
 // Stacks of a wave: kCols columns of kRows entries (8 B) in LDS, with three rows below the bottom, so
@@ -835,7 +836,7 @@ constexpr uint32_t kCounterStride = 32;
 
 __host__ __device__ __forceinline__ uint32_t quad_lds_words(uint32_t waves)
 {
-	return waves * (2u * wave_stack_entries<kQuadRows, 16u>() + 512u);  // stacks, staged rays
+	return waves * (2u * wave_stack_entries<kQuadRows, 16u>() + kStageWords);
 }
 
 // (__ballot takes an int: a select and a compare more.)
@@ -1221,7 +1222,7 @@ struct QuadTracer {
 // A window's rays are loaded when it is claimed, one per lane, and handed out of LDS: a ray that started
 // with loads of its own held up the wave's other 15 (with 2 of 16 rays taking new ones at a time, every
 // other step). With it 998,029 any-hit shadow rays take 0.122 ms instead of 0.127, bounce rays 0.438
-// instead of 0.449.
+// instead of 0.449. An any-hit ray with an empty interval (what stands for none) is answered there.
 template <int kAny, bool kClock, bool kBig>
 __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 {
@@ -1231,18 +1232,34 @@ __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 	T.lane = __lane_id();
 	T.l = T.lane & 3u;
 	T.q.base = stack_base<kQuadRows, 16u>(waveInBlock, T.lane >> 2);
-	LdsF4* const staged =
-		(LdsF4*)(lds + blockWaves * 2u * wave_stack_entries<kQuadRows, 16u>()) + waveInBlock * 128u;
+	LdsU1* const area = (LdsU1*)(lds) + blockWaves * 2u * wave_stack_entries<kQuadRows, 16u>() + waveInBlock * kStageWords;
+	LdsF4* const staged = (LdsF4*)(area);  // ray records: first words, then second ones
+	LdsU1* const index = area + 512u;      // any hit: the rays that they are of
 	if (kClock && threadIdx.x == 0u) atomicMin(&P.clock[P.n], wall_clock64());
 	RayWindows W(P, waveInBlock);
-	uint32_t first = W.next;  // the staged window's first ray
+	uint32_t taken = 0u, count = 0u;  // of the staged rays
 	auto stage = [&] {
-		first = W.next;
-		if (W.next + T.lane < W.end) {
-			GlobalV4* p = (GlobalV4*)(P.rays) + 2u * size_t(W.next + T.lane);
-			staged[T.lane] = p[0];
-			staged[64u + T.lane] = p[1];
+		const uint32_t ray = W.next + T.lane;
+		bool mine = W.next < W.end && ray < W.end;
+		F32x4 a = {}, b = {};
+		if (mine) {
+			GlobalV4* p = (GlobalV4*)(P.rays) + 2u * size_t(ray);
+			a = p[0];
+			b = p[1];
+			if (kAny == 1 && !(a.w < b.w)) {
+				quad_result<false, false, kClock>(P, ray, 0u, Closest{}, true, false);
+				mine = false;
+			}
 		}
+		const uint64_t all = ballot(mine);
+		const uint32_t at = uint32_t(__popcll(all & __lanemask_lt()));
+		if (mine) {
+			staged[at] = a;
+			staged[64u + at] = b;
+			if (kAny == 1) index[at] = ray;
+		}
+		taken = 0u;
+		count = uint32_t(__popcll(all));
 		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 		__builtin_amdgcn_wave_barrier();
 		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -1251,19 +1268,21 @@ __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 	while (true) {
 		const uint64_t idle = ballot(T.q.ray == kInvalid);
 		if (idle != 0ull) {
-			if (W.next >= W.end) {
+			if (taken >= count) {
 				if (!W.claim(P)) break;
 				stage();
+				if (count == 0u) continue;
 			}
 			const uint32_t room = uint32_t(__popcll(idle)) / 4u;
 			if (room >= P.refill) {
-				const uint32_t ray = W.next + uint32_t(__popcll(idle & __lanemask_lt())) / 4u;
-				if (T.q.ray == kInvalid && ray < W.end) {
-					const F32x4 a = staged[ray - first], b = staged[64u + ray - first];
-					T.start(ray, make_float4(a.x, a.y, a.z, a.w), make_float4(b.x, b.y, b.z, b.w));
+				const uint32_t at = taken + uint32_t(__popcll(idle & __lanemask_lt())) / 4u;
+				if (T.q.ray == kInvalid && at < count) {
+					const F32x4 a = staged[at], b = staged[64u + at];
+					T.start(kAny == 1 ? index[at] : W.next + at, make_float4(a.x, a.y, a.z, a.w),
+					        make_float4(b.x, b.y, b.z, b.w));
 				}
 				T.someExact = ballot(T.q.exact != 0u) != 0ull;
-				W.next = W.end - W.next < room ? W.end : W.next + room;
+				taken += room;
 			}
 		}
 		T.step();
@@ -1717,8 +1736,11 @@ __global__ __launch_bounds__(kPacketBlock) void k_packet(const float4* __restric
 	const uint32_t ri = active ? i : first;  // lanes past the end read a valid ray, never used
 	LaneWalk t;
 	t.r = dev::make_ray(rays[2 * size_t(ri)], rays[2 * size_t(ri) + 1]);
+	// (An any-hit ray with an empty interval hits nothing; the one that stands for none would keep its
+	// packet on the binary nodes.)
+	const bool traced = active && (!kAnyHit || t.r.tMin < t.r.tMax);
 	const bool occluded =
-		packet_trace<kAnyHit>(wide, nodes, tris, t, active, (LdsU2*)(stackLds) + threadIdx.x);
+		packet_trace<kAnyHit>(wide, nodes, tris, t, traced, (LdsU2*)(stackLds) + threadIdx.x);
 	if (active) {
 		if (kAnyHit)
 			static_cast<uint8_t*>(out)[i] = occluded ? 0 : 1;

@@ -176,3 +176,25 @@ def test_packets_that_part(ctx, scenes, which, n):
     finally:
         if which.startswith("deep"):
             s.release()
+
+
+@pytest.mark.parametrize("kernel", [0, phx.KERNEL_ONE_RAY_PER_LANE, phx.KERNEL_PACKET])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 130, 5000])
+@pytest.mark.parametrize("share", [0.3, 0.95, 1.0])
+def test_empty_intervals(ctx, scenes, n, share, kernel):
+    """Any-hit rays with an empty interval among others (all of a window's, some, none): tMin equal to
+    or above tMax, NaN at either end, and the ray that stands for none."""
+    s, b, rays = scenes[0]
+    r = rays[:n].copy()
+    rng = np.random.default_rng(n)
+    empty = np.flatnonzero(rng.random(n) < share)
+    kinds = [(0.5, 0.5), (2.0, 1.0), (np.nan, 1.0), (0.0, np.nan), (np.inf, np.inf)]
+    for i, k in zip(empty, rng.integers(0, len(kinds) + 1, len(empty))):
+        if k == len(kinds):
+            r[i]["o"], r[i]["d"] = 1.0e6, (0.0, 1.0, 0.0)
+            r[i]["tmin"] = r[i]["tmax"] = 0.001
+        else:
+            r[i]["tmin"], r[i]["tmax"] = kinds[k]
+    with np.errstate(all="ignore"):
+        assert (ctx.cast_anyhit(s, r, kernel) == O.cast_anyhit(b.nodes, b.tris, r)).all()
+        assert ctx.cast_closest(s, r, kernel).tobytes() == O.cast_closest(b.nodes, b.tris, r).tobytes()
