@@ -168,18 +168,39 @@ phx_status enqueueFrame(PhxContext* ctx, PhxRenderer* r, const PhxScene* scene,
 	// by the persistent kernel.
 	PHX_HIP(launchGenSecondary(r->gbuf, r->w, r->h, r->params, r->bounce, r->throughput, s),
 	        what);
-	// The bounce rays' closest hits (the persistent kernel, whose last rays take long) overlap the
-	// primary shading and shadow rays; the bounce records need the shading buffers back, so the
-	// streams join before them. No other persistent launch runs meanwhile, so the two
-	// streams never share the context's ray counter or spill area.
+	// The bounce rays' hits, their records, shading and shadow rays run on the side stream beside the
+	// primary shading, each filling the other's last waves; only adding the bounce light waits for both
+	// (1080p, 8 lights: 1.35 ms, with a join after the closest hits 1.38). With instances, whose primary
+	// shadow rays are stored where the bounce shading's are, the streams join after the closest hits.
+	// No other persistent launch of the context's ray counters and spill area runs meanwhile.
+	hipStream_t q = inst ? s : r->side;
+	auto bounceRecords = [&]() -> phx_status {  // records, shading x throughput with shadow rays, any hit
+		PHX_HIP(launchInterpret(r->bounce, r->bounceHits, r->m, scene->datas, scene->numTris,
+		                        scene->materials, scene->numMaterials, scene->tex, r->bounceInfo, q,
+		                        inst ? r->bounceInst : nullptr, instByIndex, numInst),
+		        what);
+		PHX_HIP(launchShade(r->bounceInfo, r->bounce, r->throughput, scene->lights, L, r->m, r->params,
+		                    3u, r->contrib, r->shadow, q),
+		        what);
+		PHX_HIP(launchAnyHit(sv, r->shadow, r->m * L, r->inLight, bounceShadows, q), what);
+		if (inst)
+			PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst,
+			                        r->shadow, r->m * L, nullptr, nullptr, r->inLight, true, onMain, q),
+			        what);
+		return PHX_OK;
+	};
 	if (r->m) {
 		PHX_HIP(hipEventRecord(r->fork, s), what);
 		PHX_HIP(hipStreamWaitEvent(r->side, r->fork, 0), what);
 		PHX_HIP(launchClosest(sv, r->bounce, r->m, r->bounceHits, closest, nullptr, r->side), what);
-		if (inst)
+		if (inst) {
 			PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst,
 			                        r->bounce, r->m, r->bounceHits, r->bounceInst, nullptr, true, closest, r->side),
 			        what);
+		} else {
+			const phx_status st = bounceRecords();
+			if (st != PHX_OK) return st;
+		}
 		PHX_HIP(hipEventRecord(r->join, r->side), what);
 	}
 	if (!inst) {
@@ -196,21 +217,13 @@ phx_status enqueueFrame(PhxContext* ctx, PhxRenderer* r, const PhxScene* scene,
 		PHX_HIP(launchShadowLogic(r->color, r->w, r->h, 1u, false, r->inLight, r->contrib, L, s), what);
 	}
 
-	// Bounce hits: records, shading x throughput with shadow rays, any hit, added at half res.
+	// The bounce light, added at half resolution.
 	if (r->m) {
 		PHX_HIP(hipStreamWaitEvent(s, r->join, 0), what);
-		PHX_HIP(launchInterpret(r->bounce, r->bounceHits, r->m, scene->datas, scene->numTris,
-		                        scene->materials, scene->numMaterials, scene->tex, r->bounceInfo,
-		                        s, inst ? r->bounceInst : nullptr, instByIndex, numInst),
-		        what);
-		PHX_HIP(launchShade(r->bounceInfo, r->bounce, r->throughput, scene->lights, L, r->m,
-		                    r->params, 3u, r->contrib, r->shadow, s),
-		        what);
-		PHX_HIP(launchAnyHit(sv, r->shadow, r->m * L, r->inLight, bounceShadows, s), what);
-		if (inst)
-			PHX_HIP(launchInstances(instanceTop(inst), instanceTopWide(inst), instanceArray(inst), numInst,
-			                        r->shadow, r->m * L, nullptr, nullptr, r->inLight, true, onMain, s),
-			        what);
+		if (inst) {
+			const phx_status st = bounceRecords();
+			if (st != PHX_OK) return st;
+		}
 		PHX_HIP(launchShadowLogic(r->color, r->w, r->h, 2u, true, r->inLight, r->contrib, L, s),
 		        what);
 	}
