@@ -41,7 +41,7 @@ enum class TraceKernel { Persistent, Simple, Packet };
 
 // Words of a launch's ray counters, and words of stack spill per ray in flight.
 constexpr uint32_t kRayCounterWords = 1024;
-constexpr uint32_t kSpillWordsPerRay = 108;
+constexpr uint32_t kSpillWordsPerRay = 112;
 // Most rays in flight per CU: 16 waves of 64 rays, one per lane (28 of 16 rays, four lanes each).
 constexpr uint32_t kRaysPerCu = 1024;
 
@@ -60,7 +60,7 @@ struct TraceLaunch {
 };
 
 // Scratch of the allocation-free closest-hit cast: a static device array per GPU holding the
-// launch's ray counters (first kNoAllocCounterBytes) and its stack spill area (40.5 MiB: 98,304 rays).
+// launch's ray counters (first kNoAllocCounterBytes) and its stack spill area (42 MiB: 98,304 rays).
 constexpr size_t kNoAllocCounterBytes = kRayCounterWords * 4u;
 constexpr uint32_t kNoAllocSpillWords = 98304u * kSpillWordsPerRay;
 constexpr int kNoAllocMaxDevices = 64;

@@ -3,7 +3,7 @@
 // Requests (ray batches against resident scenes) are admitted in arrival order while their
 // buffers fit the HBM budget (a first-fit arena over one device allocation, so admission never
 // calls hipMalloc), and admitted requests are coalesced into the next fused persistent launch, up
-// to kLaunchRays rays per launch (at least one request).
+// to a quarter of the waiting rays per launch (launchSlot; at least one request).
 // Launches run on `slots` streams, each with its own work counter and stack spill area, so a
 // launch formed from requests that arrived while another one runs starts on the next stream and
 // fills the running launch's tail. A dispatcher thread forms launches and retires them (outputs
@@ -34,12 +34,14 @@ double msSince(Clock::time_point t0) { return std::chrono::duration<double, std:
 
 constexpr size_t kAlign = 256;
 
-// Rays per fused launch before further admitted requests wait for the next launch. A backlog
-// coalesced into one or two launches runs its copies to the device, traversal and copies back one after
-// the other; in launches of about a million rays (0.7 ms of the link, 0.6 ms of traversal) the slot
-// streams overlap one launch's copies with another's traversal. 48 requests of 3.2 million rays in 3
-// slots: 3.34 ms at 4 million rays a launch, 3.12 at one million and at half, 3.79 at a quarter.
-constexpr uint64_t kLaunchRays = 1u << 20;
+// Rays per fused launch before further admitted requests wait for the next launch: a quarter of what is
+// waiting, between one and four million; four million for requests whose rays are on the device. A
+// backlog coalesced into one or two launches runs its copies to the device, traversal and copies back
+// one after the other; split, the slot streams overlap one launch's copies with another's traversal. A
+// launch that is too small spends its time on its last rays.
+//   48 requests, 3.2 million rays, 3 slots: 3.34 ms at 4 million, 3.12 at 1 million, 3.79 at 1/4 million
+//   1,500 requests, 143 million rays: 105 ms at 4 million, 126 at 1 million (on the device: 37 and 50)
+constexpr uint64_t kLeastLaunchRays = 1u << 20, kMostLaunchRays = 4u << 20;
 size_t alignUp(size_t b) { return (b + kAlign - 1) / kAlign * kAlign; }
 
 // First-fit allocator over [0, size) with coalescing of neighbouring free ranges.
@@ -197,11 +199,15 @@ void admit(PhxServer* s)
 hipError_t launchSlot(PhxServer* s, Slot& slot)
 {
 	slot.reqs.clear();
-	uint64_t total = 0;
+	uint64_t total = 0, waiting = 0;
+	for (const Request* r : s->admitted) waiting += r->req.numRays;
+	for (const Request* r : s->queue) waiting += r->req.numRays;
+	const uint64_t hostRays = std::min(std::max(waiting / 4u, kLeastLaunchRays), kMostLaunchRays);
 	while (!s->admitted.empty() && slot.reqs.size() < kMaxFusedBatches) {
 		Request* r = s->admitted.front();
 		if (total + r->req.numRays > 0x7FFFFFFFull) break;
-		if (!slot.reqs.empty() && total + r->req.numRays > kLaunchRays) break;
+		const uint64_t most = (r->req.flags & PHX_MEM_DEVICE) ? kMostLaunchRays : hostRays;
+		if (!slot.reqs.empty() && total + r->req.numRays > most) break;
 		total += r->req.numRays;
 		slot.reqs.push_back(r);
 		s->admitted.pop_front();

@@ -796,6 +796,8 @@ __device__ __forceinline__ uint32_t find_batch(const uint32_t* offsets, uint32_t
 // Selects in place of the branches of what comes next cost more than they save (0.488).
 
 constexpr uint32_t kQuadBlock = 512;  // largest block of the persistent kernels
+constexpr uint32_t kLaneBlock = 1024;  // (of fused launches)
+constexpr uint32_t kLdsBytes = 160u * 1024u;  // of a CU
 constexpr uint32_t kStageWords = 512u + 64u;  // of a wave: a window's rays and their indices
 constexpr uint32_t kQuadWavesPerSimd = 7;  // (72 registers)
 
@@ -803,7 +805,7 @@ constexpr uint32_t kQuadWavesPerSimd = 7;  // (72 registers)
 // that the top three can be read at any depth. Deeper entries spill to memory, kSpillEntries a
 // column, one after another.
 constexpr int kQuadRows = 20;  // (pending stacks of 20 are rare)
-constexpr int kLaneRows = 12;  // (9.5 KB a wave with 2 KB of rays: 16 waves per CU)
+constexpr int kLaneRows = 10;  // (8.5 KB a wave with 2 KB of rays: 16 waves per CU beside the batch tables)
 // Idle lanes of a one-ray-per-lane wave before it takes new rays: 64 batches of 3.2 million rays take
 // 1.66 ms with 4, 1.65 with 8 and 16, 1.68 with 24.
 constexpr uint32_t kLaneRefill = 16;
@@ -2025,7 +2027,7 @@ __host__ __device__ __forceinline__ uint32_t batch_lds_words(uint32_t waves, uin
 }
 
 template <bool kTrack>
-__global__ __launch_bounds__(kQuadBlock, 4) void k_trace_batches(
+__global__ __launch_bounds__(kLaneBlock, 4) void k_trace_batches(
 	const BatchDesc* __restrict__ descs, const uint32_t* __restrict__ offsetsGlobal,
 	uint32_t numBatches, uint32_t total, uint32_t window, uint32_t refill,
 	uint32_t* __restrict__ work, U32x2* __restrict__ spill, BatchClock* __restrict__ clock)
@@ -2127,13 +2129,20 @@ Shape quadShape(const TraceLaunch& L, uint32_t n)
 	return s;
 }
 
-// One ray per lane: windows of 64 rays; blocks small enough that every CU has one.
-Shape laneShape(const TraceLaunch& L, uint32_t n)
+// One ray per lane: windows of 64 rays; blocks small enough that every CU has one, and of 1,024 threads
+// where `tableWords` of LDS beside the waves' (the batch tables) would halve the waves of a CU in blocks
+// of 512 (256 tracked batches of 29.6 million rays: 7.4 ms with 8 waves per CU, 4.7 with 16). No more waves
+// than are resident: the others' first windows would wait for a block to end.
+Shape laneShape(const TraceLaunch& L, uint32_t n, uint32_t tableWords)
 {
-	const uint32_t most =
-		std::max(1u, std::min(std::min(L.raysInFlight, L.spillColumns) / 64u, L.cus * 16u));
+	auto resident = [&](uint32_t block) {
+		const uint32_t perBlock = block / 64u, lds = (lane_lds_words(perBlock) + tableWords) * 4u;
+		return std::min(16u, kLdsBytes / lds * perBlock);
+	};
+	uint32_t block = resident(kLaneBlock) > resident(kQuadBlock) ? kLaneBlock : kQuadBlock;
+	const uint32_t most = std::max(1u, std::min(std::min(L.raysInFlight, L.spillColumns) / 64u,
+	                                            L.cus * std::max(1u, resident(block))));
 	const uint32_t waves = std::min(most, gridFor(n, 64u));
-	uint32_t block = kQuadBlock;
 	while (block > 64u && waves / (block / 64u) < L.cus) block /= 2u;
 	Shape s = shapeOf(waves, most, block);
 	s.window = 64u;
@@ -2325,7 +2334,7 @@ hipError_t launchBatches(const BatchDesc* descs, const uint32_t* offsets, uint32
                          uint32_t total, const TraceLaunch& L, BatchClock* clock, hipStream_t stream)
 {
 	if (total == 0) return hipSuccess;
-	const Shape q = laneShape(L, total);
+	const Shape q = laneShape(L, total, batch_lds_words(0u, numBatches, clock != nullptr));
 	hipLaunchKernelGGL(clock ? k_trace_batches<true> : k_trace_batches<false>, dim3(q.grid),
 	                   dim3(q.block), batch_lds_words(q.block / 64u, numBatches, clock != nullptr) * 4u,
 	                   stream, descs, offsets, numBatches, total, 64u, q.refill, L.work,

@@ -198,3 +198,16 @@ def test_empty_intervals(ctx, scenes, n, share, kernel):
     with np.errstate(all="ignore"):
         assert (ctx.cast_anyhit(s, r, kernel) == O.cast_anyhit(b.nodes, b.tris, r)).all()
         assert ctx.cast_closest(s, r, kernel).tobytes() == O.cast_closest(b.nodes, b.tris, r).tobytes()
+
+
+@pytest.mark.parametrize("track", [False, True])
+@pytest.mark.parametrize("batches", [200, 520, 1024])
+def test_many_batches(ctx, scenes, batches, track):
+    """Batch tables that leave a CU two blocks of 512 threads, one of 1,024, or the least room."""
+    parts = []
+    for i in range(batches):
+        s, b, rays = scenes[i % 2]
+        n = 900 if i % 7 == 0 else i % 90
+        parts.append((s, b.nodes, b.tris, np.ascontiguousarray(rays[i:i + n]),
+                      phx.BATCH_ANYHIT if i % 3 == 2 else phx.BATCH_CLOSEST))
+    run_fused(ctx, parts, track)
