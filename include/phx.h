@@ -216,16 +216,14 @@ void* phx_context_stream(PhxContext* ctx);
 uint32_t phx_context_num_cus(PhxContext* ctx);
 
 /* Launch shape of the persistent traversal kernels on this context: grid size in blocks for
- * closest-hit and any-hit, block size (lane-mode threads, a multiple of 64 up to 1024), the number
- * of top tree nodes each block keeps in LDS (0..2048; the upload lays out the top of the tree
- * breadth first), the refill threshold (a wave refills its idle lanes once at least `refillMin` of
- * its 64 lanes are idle; 1..64), and helper waves: extra waves per block that trace no ray of
- * their own and take over, one wave per ray, the last rays the block's lane-mode waves hand out
- * (blockThreads + 64 * helperWaves <= 1024), rays per fetch (the rays a wave claims from the
- * launch's shared counter with one atomic; 8..4096) and the stack split (the traversal stack
- * entries per lane kept in LDS, 4..32; deeper entries live in HBM). phx_create's defaults: one
- * block of 512 threads per CU, no treelet, refill 8, no helper waves, 64 rays per fetch, 16 LDS
- * stack entries; phx_autotune picks them per scene and ray mix. In phx_set_launch_params a zero
+ * closest-hit and any-hit and block size (a multiple of 64 up to 1024), which together bound the
+ * rays in flight; the refill threshold (1..64: how many of a wave's ray places are idle before it
+ * takes new rays); rays per fetch (8..4096: an upper bound on the rays a wave claims from a shared
+ * counter with one atomic). topNodes (0..2048), helperWaves (blockThreads + 64 * helperWaves <=
+ * 1024) and stackLdsEntries (4..32) do not change how the kernels run; they are checked, kept and
+ * reported. phx_create's defaults: one block of 512 threads per CU, topNodes 0, refill 8,
+ * helperWaves 0, 64 rays per fetch, 16 stack entries; phx_autotune picks the grid, refill threshold
+ * and rays per fetch per scene and ray mix. In phx_set_launch_params a zero
  * field (0xFFFFFFFF for topNodes and helperWaves) keeps the current value; combinations that do
  * not fit a CU are rejected. In phx_plan_set_launch_params 0xFFFFFFFF helper waves means none and
  * a zero raysPerFetch or stackLdsEntries the default. Results do not depend on these parameters. */
@@ -245,11 +243,10 @@ phx_status phx_get_launch_params(PhxContext* ctx, PhxLaunchParams* out);
 phx_status phx_set_launch_params(PhxContext* ctx, const PhxLaunchParams* params);
 
 /* Autotuner for single-batch casts: times phx_cast_closest (or, with PHX_AUTOTUNE_ANYHIT,
- * phx_cast_anyhit) on the given device rays under candidate launch shapes -- block 256/512,
- * treelet 0/512/1024 nodes, 1/4, 1/2 or all of the resident grid, refill 8/32, 0 or 4 helper
- * waves, the one-ray-per-lane kernel and the packet kernel -- with HIP events; if a persistent
- * shape wins it then refines rays per fetch (16..256) and the stack split (8..32 LDS entries) one
- * at a time around it, and applies the fastest persistent shape to the context. `chosen` (may be NULL) receives it; residentGridBlocks
+ * phx_cast_anyhit) on the given device rays under candidate launch shapes -- 1/4, 1/2 or
+ * all of the resident grid, refill 8/32, the one-ray-per-lane kernel and the packet kernel -- with
+ * HIP events; if a persistent shape wins it then tries 16 and 32 rays per fetch with it, and applies
+ * the fastest persistent shape to the context. `chosen` (may be NULL) receives it; residentGridBlocks
  * = 0xFFFFFFFF there means the one-ray-per-lane kernel won (pass PHX_KERNEL_ONE_RAY_PER_LANE to
  * the casts) and 0xFFFFFFFE the packet kernel (pass PHX_KERNEL_PACKET). `rays` must be device
  * memory (PHX_MEM_DEVICE). */
@@ -494,12 +491,12 @@ phx_status phx_plan_launch(PhxContext* ctx, PhxPlan* plan, uint32_t flags);
 phx_status phx_plan_batch_times(PhxContext* ctx, PhxPlan* plan, float* msSinceStart);
 
 /* Launch shape of one plan (a fused launch is throughput bound, so plans default to the resident
- * grid without a treelet). gridBlocksClosest is the grid; gridBlocksAnyhit is ignored. */
+ * grid). gridBlocksClosest is the grid; gridBlocksAnyhit is ignored. */
 phx_status phx_plan_set_launch_params(PhxContext* ctx, PhxPlan* plan,
                                       const PhxLaunchParams* params);
 
-/* Times the plan under a set of candidate shapes (block 256/512, treelet 0/512/1024 nodes, 1/4,
- * 1/2 or all of the resident grid, refill 8/32) and keeps the fastest. Runs the plan's batches
+/* Times the plan under a set of candidate shapes (1/4, 1/2 or all of the resident
+ * grid, refill 8/32, 16 and 32 rays per fetch) and keeps the fastest. Runs the plan's batches
  * several times (outputs are overwritten with the same values). */
 phx_status phx_plan_autotune(PhxContext* ctx, PhxPlan* plan, PhxLaunchParams* chosen);
 
@@ -594,15 +591,15 @@ typedef struct PhxServerStats {
 /* A server on ctx's device with an HBM budget (resident scenes + request buffers) and `slots`
  * (1..4) launch streams. Requests are admitted in arrival order while their buffers fit, and
  * admitted requests are coalesced, in order, into the next fused persistent launch on an idle
- * slot, up to 4M rays per launch (a larger request gets a launch of its own), so a backlog spreads
+ * slot, a quarter of the waiting rays per launch but one to four million (four million where the
+ * rays are on the device; a larger request gets a launch of its own), so a backlog spreads
  * over the slots and one launch's copies overlap another's traversal; a launch formed while
  * another runs fills that launch's tail. Slot 0 launches on the context's stream (other work on
  * that stream runs in order with it); each further slot has a stream of its own. HIP spreads a
  * process's streams over a few hardware queues (4 by default) and slots that share a queue
  * serialise, so more than 3 slots only pay where more queues exist. A dispatcher thread owns the
  * device work. The server
- * launches with the default stack split and rays per fetch and no treelet or helper waves; it
- * takes the block size and refill threshold from the context. */
+ * launches with the default rays per fetch; it takes the refill threshold from the context. */
 phx_status phx_server_create(PhxContext* ctx, uint64_t budgetBytes, uint32_t slots,
                              uint32_t flags, PhxServer** outServer);
 /* Waits for every submitted request, then frees the server. */
@@ -670,8 +667,8 @@ void phx_renderer_release(PhxRenderer* renderer);
  * as taa.frag does, and clamped to the 3x3 neighbourhood. The primary hits' shadow rays
  * (coherent: a pixel tile's rays towards one light) and, when width and height are multiples of 8
  * (camera rays in 8x8-tile order), camera rays are traced as packets (PHX_KERNEL_PACKET); bounce
- * rays, and camera rays in row-major order, by the persistent kernel; the bounce hits' shadow
- * rays (scattered origins) one ray per lane (PHX_KERNEL_ONE_RAY_PER_LANE). `rgba`
+ * rays, their hits' shadow rays (scattered origins) and camera rays in row-major order by the
+ * persistent kernel. `rgba`
  * (width*height*4 floats, row-major; host or device with PHX_MEM_DEVICE; may be NULL) receives
  * the output. Random numbers: PCG32 streams keyed by (seed, frameIndex, pass, record). The
  * frame's kernels read the per-frame values (camera, previous camera, jitter, frame index, seed,
