@@ -38,11 +38,12 @@ struct PhxRenderer {
 	const PhxInstanceSet* instances = nullptr;
 	uint32_t* primInst = nullptr;
 	uint32_t* bounceInst = nullptr;
-	uint32_t* instWork = nullptr;  // ray counters of the instance casts on the frame's stream
+	uint32_t* instWork = nullptr;  // ray counters of the instance casts on the frame's stream (if any)
 	float4* lastOut = nullptr;
 	FrameParams* params = nullptr;  // per-frame values the frame kernels read (device)
-	// The bounce rays' closest hits run on a side stream beside the primary shadow rays (fork
-	// after the bounce rays are generated, join before the bounce records).
+	// The bounce rays' hits, records, shading and shadow rays run on a side stream beside the primary
+	// shading (fork after the bounce rays are generated, join before their light is added; with
+	// instances the join comes before the bounce records).
 	hipStream_t side = nullptr;
 	hipEvent_t fork = nullptr, join = nullptr;
 	// The captured frame (PHX_FRAME_GRAPH) and what it was captured for. The cameras, jitter and
@@ -116,6 +117,23 @@ phx_status growLights(PhxRenderer* r, uint32_t lights)
 	if (st == PHX_OK) st = devAlloc(r->inLight, k, "phx_render_frame");
 	if (st == PHX_OK) r->lightCap = lights;
 	return st;
+}
+
+// The ray counters of the instance casts, made for the first frame that has some: two small calls that
+// a renderer without instances would pay for when it is created.
+phx_status makeInstWork(PhxRenderer* r)
+{
+	if (!r->instances || r->instWork) return PHX_OK;
+	const char* what = "phx_render_frame";
+	uint32_t* work = nullptr;
+	const phx_status st = devAlloc(work, kRayCounterWords, what);
+	if (st != PHX_OK) return st;
+	if (launchZeroWords(work, kRayCounterWords, r->ctx->stream) != hipSuccess) {
+		hipFree(work);
+		return fail(PHX_ERR_HIP, "%s: clearing the ray counters failed", what);
+	}
+	r->instWork = work;
+	return PHX_OK;
 }
 
 // The frame's launches, all on stream s; per-frame values come from r->params, so this sequence is
@@ -282,15 +300,12 @@ phx_status phx_renderer_create(PhxContext* ctx, uint32_t width, uint32_t height,
 	if (st == PHX_OK) st = devAlloc(r->color, r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->hist[0], r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->hist[1], r->n, what);
-	if (st == PHX_OK) st = devAlloc(r->instWork, kRayCounterWords, what);
 	if (st == PHX_OK) st = devAlloc(r->primInst, r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->bounceInst, std::max(r->m, 1u), what);
 	if (st == PHX_OK) st = devAlloc(r->vel[0], r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->vel[1], r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->out, r->n, what);
 	if (st == PHX_OK) st = devAlloc(r->params, 1, what);
-	if (st == PHX_OK && launchZeroWords(r->instWork, kRayCounterWords, ctx->stream) != hipSuccess)
-		st = fail(PHX_ERR_HIP, "%s: clearing the ray counters failed", what);
 	if (st == PHX_OK && (hipStreamCreateWithFlags(&r->side, hipStreamNonBlocking) != hipSuccess ||
 	                     hipEventCreateWithFlags(&r->fork, hipEventDisableTiming) != hipSuccess ||
 	                     hipEventCreateWithFlags(&r->join, hipEventDisableTiming) != hipSuccess))
@@ -367,6 +382,8 @@ phx_status phx_render_frame(PhxContext* ctx, PhxRenderer* r, const PhxScene* sce
 	if (async && rgba && !device)
 		return fail(PHX_ERR_INVALID_ARGUMENT, "phx_render_frame: PHX_ASYNC needs PHX_MEM_DEVICE");
 	st = growLights(r, scene->numLights);
+	if (st != PHX_OK) return st;
+	st = makeInstWork(r);
 	if (st != PHX_OK) return st;
 
 	hipStream_t s = ctx->stream;
