@@ -289,7 +289,7 @@ __device__ __forceinline__ bool anyhit_one(const float4* __restrict__ nodes,
 // 9.8 wide node visits where it takes 21.6 binary ones (random triangles: 32 for 65).
 
 struct WideWords {
-	float4 w[8];  // slot i: (min.xyz, reference) in word 2i, (max.xyz, -) in word 2i + 1
+	float4 w[8];  // slot i: (min.xyz, reference) in word 2i, (max.xyz, lastMax) in word 2i + 1
 };
 
 __device__ __forceinline__ WideWords load_wide(const float4* __restrict__ wide, uint32_t i)
@@ -1302,7 +1302,7 @@ __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 // instruction serves 64 rays, not 16) but reads 64 lines with each load, takes a leaf and a node in
 // steps of their own and is as slow as its costliest lane, so four lanes per ray are the faster way
 // for a launch by itself (1,048,576 random rays, 4 waves per SIMD: 0.485 ms against 0.468 ms) and one
-// lane is where the device is full: 64 batches of 3.2 million rays on two scenes take 1.65 ms (2.3 ms
+// lane is where the device is full: 64 batches of 3.2 million rays on two scenes take 1.56 ms (2.3 ms
 // four lanes each; 1.79 ms with the binary nodes). There the texture data path is busy 85% of the
 // time, the VALUs 63%. Handing the records over in LDS, four lanes to a line, took it to 1.60 ms and
 // single casts from 0.106 to 0.123 ms, so each lane loads its own.
@@ -1334,20 +1334,23 @@ struct LaneWalk {
 	__device__ __forceinline__ bool at_leaf() const { return (ref & kWideLeaf) != 0u; }
 	// The record that advance() consumes: a wide node, or a leaf's next two triangles (the words past
 	// a leaf's last one are the next triangle's or the array's padding). Lanes without one (`on`
-	// false) and exact nodes read the array's first line.
+	// false) and exact nodes read the array's first line. Seven words: slot 3's max.xyz is in the last
+	// components of words 1, 3 and 5 too, and these loads are bound by the 16 B a lane that the texture
+	// data path returns a cycle (eight words: 64 fused batches 1.635 ms, now 1.563; 1,048,576 rays into
+	// 300 instances 3.235 ms, now 3.137).
 	__device__ __forceinline__ void load(bool on, const float4* wide, const float4* tris,
-	                                     float4 w[8]) const
+	                                     float4 w[7]) const
 	{
 		const float4* rec = on && at_leaf() ? tris + 3u * size_t(ref & kWideIndex)
 		                                    : wide + 8u * size_t(on && !exact ? ref : 0u);
 #pragma unroll
-		for (int i = 0; i < 8; i++) w[i] = as_global(rec)[i];
+		for (int i = 0; i < 7; i++) w[i] = as_global(rec)[i];
 	}
 
 	// Expands a node or tests up to two triangles of a leaf, and picks what the lane takes next. True
 	// if the traversal has ended (`occluded`: with an any-hit ray's hit).
 	template <int kAny, class Stack>
-	__device__ __forceinline__ bool advance(const float4 w[8], const float4* nodes, bool any, Stack& st,
+	__device__ __forceinline__ bool advance(const float4 w[7], const float4* nodes, bool any, Stack& st,
 	                                        bool& occluded)
 	{
 		const bool leaf = at_leaf(), node = !leaf && !exact;
@@ -1383,7 +1386,8 @@ struct LaneWalk {
 		if (node) {
 			WideWords n;
 #pragma unroll
-			for (int i = 0; i < 8; i++) n.w[i] = w[i];
+			for (int i = 0; i < 7; i++) n.w[i] = w[i];
+			n.w[7] = make_float4(w[1].w, w[3].w, w[5].w, 0.0f);
 			const WideVisit v = decide_wide(r, n, lim);
 			const bool p0 = v.pass[0], p1 = v.pass[1], p2 = v.pass[2], p3 = v.pass[3];
 			uint32_t r0 = __float_as_uint(w[0].w), r1 = __float_as_uint(w[2].w);
@@ -1552,7 +1556,7 @@ struct LaneTracer {
 	__device__ __forceinline__ void step()
 	{
 		const bool active = ray != kInvalid;
-		float4 w[8];
+		float4 w[7];
 		t.load(active, kBatch ? wide : P.wide, kBatch ? tris : P.tris, w);
 		if (!active) return;
 		bool occluded;
@@ -1715,7 +1719,7 @@ __device__ __forceinline__ bool packet_trace(const float4* __restrict__ wide,
 		if (on && !kAnyHit) t.decide_sibling(lim, stack);
 	}
 	while (ballot(on) != 0ull) {
-		float4 w[8];
+		float4 w[7];
 		t.load(on, wide, tris, w);
 		if (on) on = !t.template advance<kAnyHit ? 1 : 0>(w, nodes, kAnyHit, stack, occluded);
 	}
@@ -1849,7 +1853,7 @@ __device__ __forceinline__ bool object_ray(const DevInstance& in, const float4 a
 // (65%, with 17 of 64 lanes active on average). On the binary nodes, with exact slabs and divisions, a
 // top-tree step in every iteration and a fixed range of rays per wave, 1,048,576 rays into 300
 // instances took 4.92 ms (closest) and 262,147 any-hit rays into 120 instances and a scene 0.71 ms;
-// now 3.17 and 0.44 ms. (Wide nodes inside the instances alone: 4.14 and 0.49 ms.)
+// now 3.14 and 0.41 ms. (Wide nodes inside the instances alone: 4.14 and 0.49 ms.)
 
 constexpr uint32_t kInstanceRefill = 8;  // idle lanes of a wave before it takes new rays
 constexpr uint32_t kInstanceWaves = 20;  // per CU: 5 per SIMD (96 registers)
@@ -1978,7 +1982,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_trace_instances(
 		}
 		const bool walks = ray != kInvalid && !leave && (inside || !t.at_leaf());
 		if (ballot(walks) == 0ull) continue;
-		float4 w[8];
+		float4 w[7];
 		t.load(walks, wide, tris, w);
 		bool occluded;
 		if (walks && t.template advance<kAnyHit ? 1 : 0>(w, nodes, kAnyHit, stack, occluded)) {

@@ -88,7 +88,7 @@ WideNode emptyNode()
 {
 	WideNode w;
 	const float nan = std::numeric_limits<float>::quiet_NaN();
-	for (WideNode::Slot& s : w.slot) s = WideNode::Slot{{nan, nan, nan}, 0u, {nan, nan, nan}, 0u};
+	for (WideNode::Slot& s : w.slot) s = WideNode::Slot{{nan, nan, nan}, 0u, {nan, nan, nan}, nan};
 	return w;
 }
 
@@ -183,6 +183,8 @@ std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint
 		stack.insert(stack.end(), kids.rbegin(), kids.rend());
 	}
 	if (maxPending > kWideMaxPending || out.size() > kWideIndex) out.clear();
+	for (WideNode& n : out)
+		for (int i = 0; i < 3; i++) n.slot[i].lastMax = n.slot[3].max[i];
 	return out;
 }
 

@@ -36,14 +36,15 @@ constexpr uint32_t kWideCountShift = 28u;
 // Pending slots a traversal may hold (the kernels' stacks hold this many 8-byte entries).
 constexpr uint32_t kWideMaxPending = 60u;
 
-// 128 B, one cache line: a 32-B record per slot, so that four lanes read one slot each and one lane
-// reads a slot in two 16-B words. Empty slots have NaN boxes, which no ray passes.
+// 128 B, one cache line: a 32-B record per slot, so that four lanes read one slot each. Slots 0 to 2
+// repeat slot 3's max.xyz in their last words, so that one lane reads the whole node in its first seven
+// 16-B words. Empty slots have NaN boxes, which no ray passes.
 struct WideNode {
 	struct Slot {
 		float min[3];
 		uint32_t ref;
 		float max[3];
-		uint32_t pad;
+		float lastMax;  // slot i < 3: slot[3].max[i]
 	} slot[4];
 };
 static_assert(sizeof(WideNode) == 128, "WideNode is one 128-B line");

@@ -87,6 +87,10 @@ extern "C" uint32_t wide_check(const PhxBVHNode* nodes, uint32_t numNodes, const
 	// The root's slots refer to nodes 1, 2, ... in order.
 	for (uint32_t i = 0; i < 4; i++)
 		if (wide[0].slot[i].min[0] == wide[0].slot[i].min[0] && wide[0].slot[i].ref != i + 1u) return 0;
+	// Slots 0 to 2 repeat slot 3's max.xyz.
+	for (const WideNode& w : wide)
+		for (int i = 0; i < 3; i++)
+			if (std::memcmp(&w.slot[i].lastMax, &w.slot[3].max[i], 4) != 0) return 0;
 	OrHit unused;
 	for (uint32_t i = 0; i < n; i++) {
 		walk(wide, tris, rays[i], false, hits[i], *deepest);
