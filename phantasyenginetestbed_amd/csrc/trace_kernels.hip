@@ -1303,8 +1303,8 @@ __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 // steps of their own and is as slow as its costliest lane, so four lanes per ray are the faster way
 // for a launch by itself (1,048,576 random rays, 4 waves per SIMD: 0.485 ms against 0.468 ms) and one
 // lane is where the device is full: 64 batches of 3.2 million rays on two scenes take 1.56 ms (2.3 ms
-// four lanes each; 1.79 ms with the binary nodes). There the texture data path is busy 85% of the
-// time, the VALUs 63%. Handing the records over in LDS, four lanes to a line, took it to 1.60 ms and
+// four lanes each; 1.79 ms with the binary nodes). There the texture data path was busy 85% of
+// the time, the VALUs 63% (with eight words a node). Handing the records over in LDS, four lanes to a line, took it to 1.60 ms and
 // single casts from 0.106 to 0.123 ms, so each lane loads its own.
 
 // One lane's castRay over the wide nodes, or the binary ones (exact), one record at a time.
@@ -1333,12 +1333,13 @@ struct LaneWalk {
 
 	__device__ __forceinline__ bool at_leaf() const { return (ref & kWideLeaf) != 0u; }
 	// The record that advance() consumes: a wide node, or a leaf's next two triangles (the words past
-	// a leaf's last one are the next triangle's or the array's padding). Exact nodes read
-	// the array's first line, lanes without a record (`on` false) nothing: with 17 of 64 lanes active on
-	// average, the instance kernel takes 2.98 ms so, 3.04 where they read the first line too. Seven words: slot 3's max.xyz is in the last
-	// components of words 1, 3 and 5 too, and these loads are bound by the 16 B a lane that the texture
-	// data path returns a cycle (eight words: 64 fused batches 1.635 ms, now 1.563; 1,048,576 rays into
-	// 300 instances 3.235 ms, now 3.137).
+	// a leaf's last one are the next triangle's or the array's padding). Exact nodes read the array's
+	// first line. The loads are bound by the 16 B a lane that the texture data path returns a cycle, so
+	//   - a node is read in seven words: slot 3's max.xyz is in the last components of words 1, 3 and 5
+	//     too (with eight, 64 fused batches took 1.635 ms, with seven 1.563; 1,048,576 rays into 300
+	//     instances 3.235 and 3.137 ms);
+	//   - lanes without a record (`on` false) read nothing: 17 of 64 lanes are active on average in the
+	//     instance kernel, which took 3.036 ms where they read the first line, and 2.977 so.
 	__device__ __forceinline__ void load(bool on, const float4* wide, const float4* tris,
 	                                     float4 w[7]) const
 	{
