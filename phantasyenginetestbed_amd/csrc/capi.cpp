@@ -110,7 +110,9 @@ bool pinnedStage(PhxContext* ctx)
 	return ctx->pinnedDev != nullptr;
 }
 
-// Runs `launch(raysDev, outDev)` with host/device handling of the ray and output arrays.
+// Runs `launch(raysDev, outDev)` with host/device handling of the ray and output arrays. A launch that
+// writes none of `out` (outBytesPerRay 0: its results stay on the device) gets no output to write to, and
+// nothing is copied back.
 template <class Launch>
 phx_status castCommon(PhxContext* ctx, const PhxRayIn* rays, uint32_t n, void* out,
                       size_t outBytesPerRay, uint32_t flags, Launch launch, const char* what)
@@ -120,7 +122,8 @@ phx_status castCommon(PhxContext* ctx, const PhxRayIn* rays, uint32_t n, void* o
 	if (async && !device)
 		return fail(PHX_ERR_INVALID_ARGUMENT, "%s: PHX_ASYNC needs PHX_MEM_DEVICE", what);
 	if (n == 0) return ok();
-	if (!rays || !out) return fail(PHX_ERR_INVALID_ARGUMENT, "%s: null ray/output pointer", what);
+	if (!rays || (!out && outBytesPerRay))
+		return fail(PHX_ERR_INVALID_ARGUMENT, "%s: null ray/output pointer", what);
 	if (device) {
 		PHX_HIP(launch(rays, out), what);
 		if (!async) PHX_HIP(hipStreamSynchronize(ctx->stream), what);
@@ -132,7 +135,7 @@ phx_status castCommon(PhxContext* ctx, const PhxRayIn* rays, uint32_t n, void* o
 		std::memcpy(ctx->pinned, rays, inBytes);
 		PHX_HIP(launch(reinterpret_cast<const PhxRayIn*>(ctx->pinnedDev), ctx->pinnedDev + kPinnedIn), what);
 		PHX_HIP(hipStreamSynchronize(ctx->stream), what);
-		std::memcpy(out, ctx->pinned + kPinnedIn, outBytes);
+		if (outBytes) std::memcpy(out, ctx->pinned + kPinnedIn, outBytes);
 		return ok();
 	}
 	phx_status st = growStage(ctx->stageIn, ctx->stageInBytes, inBytes);
@@ -141,7 +144,8 @@ phx_status castCommon(PhxContext* ctx, const PhxRayIn* rays, uint32_t n, void* o
 	if (st != PHX_OK) return st;
 	PHX_HIP(hipMemcpyAsync(ctx->stageIn, rays, inBytes, hipMemcpyHostToDevice, ctx->stream), what);
 	PHX_HIP(launch(static_cast<const PhxRayIn*>(ctx->stageIn), ctx->stageOut), what);
-	PHX_HIP(hipMemcpyAsync(out, ctx->stageOut, outBytes, hipMemcpyDeviceToHost, ctx->stream), what);
+	if (outBytes)
+		PHX_HIP(hipMemcpyAsync(out, ctx->stageOut, outBytes, hipMemcpyDeviceToHost, ctx->stream), what);
 	PHX_HIP(hipStreamSynchronize(ctx->stream), what);
 	return ok();
 }
@@ -868,7 +872,7 @@ phx_status phx_traversal_stats(PhxContext* ctx, const PhxScene* scene, const Phx
 	const TraceLaunch L = traceLaunch(ctx, flags & ~PHX_STATS_ANYHIT, false);
 	if (e == hipSuccess) {
 		st = castCommon(
-			ctx, rays, numRays, dHits, sizeof(PhxRayHit), (flags & PHX_MEM_DEVICE),
+			ctx, rays, numRays, nullptr, 0, (flags & PHX_MEM_DEVICE),
 			[&](const PhxRayIn* r, void*) {
 				return anyhit ? launchAnyHitCounted(sv, r, numRays, reinterpret_cast<uint8_t*>(dHits),
 				                                    dCounters, ctx->stream)

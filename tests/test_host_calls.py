@@ -1,0 +1,91 @@
+"""The library's host code without a GPU: its objects linked with a HIP runtime that logs launches,
+copies, waits and allocations, and whose device memory the CPU cannot touch (tests/cpp/fake_hip.cpp).
+Kernels do not run, so results are not looked at here."""
+import ctypes as C
+import multiprocessing
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+from phantasyenginetestbed_amd import build as pkg_build
+from phantasyenginetestbed_amd import phx
+
+ROOT = Path(__file__).resolve().parents[1]
+
+
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    sources = [p for p in pkg_build.CSRC.iterdir() if p.suffix in (".cpp", ".hip")]
+    objects = [pkg_build.BUILD / (p.name + ".o") for p in sources]
+    if not all(o.exists() and o.stat().st_mtime >= p.stat().st_mtime
+               for o, p in zip(objects, sources)):
+        pkg_build.build()
+    so = tmp_path_factory.mktemp("host") / "libphx_host.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__",
+                    f"-I{pkg_build.ROCM}/include", str(ROOT / "tests" / "cpp" / "fake_hip.cpp"),
+                    *map(str, objects), "-Wl,-Bsymbolic", "-lpthread", "-o", str(so)], check=True)
+    return so
+
+
+def _child(so, test, args, pipe):
+    phx.LIB_PATH = Path(so)
+    try:
+        pipe.send((None, test(phx.lib(), *args)))
+    except BaseException as e:  # reported by the parent
+        pipe.send((f"{type(e).__name__}: {e}", None))
+
+
+def run(so, test, *args):
+    """test(lib, *args) in a process of its own, with the library at `so`; a crash fails the test."""
+    spawn = multiprocessing.get_context("spawn")
+    mine, theirs = spawn.Pipe()
+    p = spawn.Process(target=_child, args=(str(so), test, args, theirs))
+    p.start()
+    theirs.close()
+    try:
+        error, result = mine.recv()
+    except EOFError:
+        p.join()
+        pytest.fail(f"the process ended with {p.exitcode}")
+    p.join()
+    assert error is None, error
+    return result
+
+
+def log(lib) -> list:
+    lib.fake_log.restype = C.c_size_t
+    out = C.create_string_buffer(1 << 22)
+    n = lib.fake_log(out, C.c_size_t(len(out)))
+    assert n <= len(out)
+    return out.raw[:n].decode().splitlines()
+
+
+def upload(ctx, n=50, seed=1):
+    t, d = phx.random_triangles(n, seed, 0.1, 0.5)
+    b = phx.BVH(t, d)
+    return ctx.upload_scene(b.nodes, b.tris, b.datas)
+
+
+def some_rays(n):
+    rays = np.zeros(n, phx.RAY)
+    rays["d"], rays["tmax"] = 1, 1
+    return rays
+
+
+def traversal_stats(lib, n, mode):
+    ctx = phx.Context(0)
+    s = upload(ctx)
+    ctx.cast_closest(s, some_rays(5))
+    log(lib)
+    ctx.traversal_stats(s, some_rays(n), mode)
+    return log(lib)
+
+
+@pytest.mark.parametrize("mode", [0, phx.STATS_ANYHIT])
+@pytest.mark.parametrize("n", [1, 8192, 8193, 20000])
+def test_traversal_stats_of_host_rays_keeps_its_results_on_the_device(library, n, mode):
+    """Its hits are device memory: nothing is copied there, by a store or by a call."""
+    copies = [x for x in run(library, traversal_stats, n, mode) if x.startswith("copy")]
+    assert copies == ([] if n <= 8192 else [f"copy {32 * n} kind=1 {copies[0].split()[-1]}"])
