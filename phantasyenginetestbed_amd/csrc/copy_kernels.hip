@@ -61,18 +61,22 @@ __global__ __launch_bounds__(256) void k_copy_ranges(Ranges R)
 void* deviceAddress(const void* p, size_t bytes)
 {
 	if (!p || bytes == 0) return nullptr;
-	hipPointerAttribute_t first{}, last{};
-	const char* c = static_cast<const char*>(p);
-	if (hipPointerGetAttributes(&first, c) != hipSuccess ||
-	    hipPointerGetAttributes(&last, c + bytes - 1) != hipSuccess) {
+	hipPointerAttribute_t at{};
+	if (hipPointerGetAttributes(&at, p) != hipSuccess) {
 		(void)hipGetLastError();  // not known to the runtime: pageable
 		return nullptr;
 	}
-	if (first.type != hipMemoryTypeHost || last.type != hipMemoryTypeHost || !first.devicePointer ||
-	    static_cast<char*>(last.devicePointer) - static_cast<char*>(first.devicePointer) !=
-	        ptrdiff_t(bytes - 1))
+	if (at.type != hipMemoryTypeHost || !at.devicePointer) return nullptr;
+	// All of it in the allocation of its first byte: between two allocations there may be pageable memory.
+	hipDeviceptr_t base = nullptr;
+	size_t size = 0;
+	if (hipMemGetAddressRange(&base, &size, at.devicePointer) != hipSuccess) {
+		(void)hipGetLastError();
 		return nullptr;
-	return reinterpret_cast<uintptr_t>(first.devicePointer) % 16u == 0u ? first.devicePointer : nullptr;
+	}
+	const uintptr_t first = reinterpret_cast<uintptr_t>(at.devicePointer), start = reinterpret_cast<uintptr_t>(base);
+	if (first < start || first - start > size || bytes > size - (first - start)) return nullptr;
+	return first % 16u == 0u ? at.devicePointer : nullptr;
 }
 
 hipError_t launchCopies(const CopyRange* ranges, uint32_t count, hipStream_t stream)

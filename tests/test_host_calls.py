@@ -42,9 +42,11 @@ def run(so, test, *args):
     spawn = multiprocessing.get_context("spawn")
     mine, theirs = spawn.Pipe()
     p = spawn.Process(target=_child, args=(str(so), test, args, theirs))
+    p.daemon = True
     p.start()
     theirs.close()
     try:
+        assert mine.poll(120), "no answer"
         error, result = mine.recv()
     except EOFError:
         p.join()
@@ -89,3 +91,43 @@ def test_traversal_stats_of_host_rays_keeps_its_results_on_the_device(library, n
     """Its hits are device memory: nothing is copied there, by a store or by a call."""
     copies = [x for x in run(library, traversal_stats, n, mode) if x.startswith("copy")]
     assert copies == ([] if n <= 8192 else [f"copy {32 * n} kind=1 {copies[0].split()[-1]}"])
+
+
+def serve(lib, rays, n, out):
+    ctx = phx.Context(0)
+    s = upload(ctx)
+    server = phx.Server(ctx, 1 << 28)
+    server.add_scene(s)
+    log(lib)
+    try:
+        server.wait(server.submit(phx.Server.request(s, rays, out, n, phx.BATCH_CLOSEST)))
+        return log(lib)
+    finally:
+        server.destroy()
+
+
+def serve_pinned(lib, pins, at, n):
+    """A request whose n rays start `at` bytes into memory of which the ranges `pins` are pinned."""
+    mem = np.zeros(1 << 20, np.uint8)
+    first = mem.ctypes.data + -mem.ctypes.data % 4096
+    for lo, hi in pins:
+        lib.fake_pin(C.c_void_p(first + lo), C.c_size_t(hi - lo))
+    out = np.zeros(n, phx.HIT)
+    return serve(lib, first + at, n, out.ctypes.data)
+
+
+K = 1024
+
+
+@pytest.mark.parametrize("pins, at, n, in_place", [
+    ([(0, 64 * K)], 0, 2048, True),
+    ([(0, 64 * K)], 32 * K, 1024, True),
+    ([(0, 64 * K)], 32 * K, 1025, False),                     # one ray past the end
+    ([(0, 64 * K), (128 * K, 192 * K)], 0, 6144, False),      # pageable memory between two allocations
+    ([(0, 64 * K), (64 * K, 128 * K)], 0, 4096, False),       # two allocations side by side
+    ([(64 * K, 128 * K)], 64 * K - 32, 2, False),
+    ([(0, 64 * K)], 8, 16, False),                            # misaligned
+    ([], 0, 64, False)])
+def test_only_rays_inside_one_pinned_allocation_are_read_in_place(library, pins, at, n, in_place):
+    copies = [x for x in run(library, serve_pinned, pins, at, n) if x.startswith(f"copy {32 * n} kind=1")]
+    assert len(copies) == (0 if in_place else 1)
