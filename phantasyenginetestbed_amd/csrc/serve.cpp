@@ -144,7 +144,7 @@ struct PhxServer {
 	std::unordered_set<const PhxScene*> scenes;
 	std::vector<Slot> slots;
 	TraceLaunch shape;
-	hipEvent_t lastLoaded = nullptr;  // of the launch formed last
+	hipEvent_t lastLoaded = nullptr;  // of the last launch that brought rays from the host
 
 	std::mutex mu;
 	std::condition_variable cvWork;  // dispatcher: new submissions
@@ -218,8 +218,12 @@ hipError_t launchSlot(PhxServer* s, Slot& slot)
 	const uint32_t nb = uint32_t(slot.reqs.size());
 	uint32_t off = 0;
 	slot.copies.clear();
-	// One launch's rays at a time: on a shared link all would arrive late together.
-	if (s->lastLoaded && s->lastLoaded != slot.loaded)
+	// One launch's rays at a time: on a shared link all would arrive late together. A launch that brings
+	// none over the link waits for nobody's.
+	const bool brings = std::any_of(slot.reqs.begin(), slot.reqs.end(), [](const Request* r) {
+		return !(r->req.flags & PHX_MEM_DEVICE) && r->req.numRays;
+	});
+	if (brings && s->lastLoaded && s->lastLoaded != slot.loaded)
 		e = hipStreamWaitEvent(slot.stream, s->lastLoaded, 0);
 	for (uint32_t b = 0; b < nb && e == hipSuccess; b++) {
 		Request* r = slot.reqs[b];
@@ -242,9 +246,11 @@ hipError_t launchSlot(PhxServer* s, Slot& slot)
 		slot.copies.push_back({slot.mappedOffsets, slot.offsets, sizeof(uint32_t) * (nb + 1)});
 	}
 	e = launchCopies(slot.copies.data(), uint32_t(slot.copies.size()), slot.stream);
-	if (e == hipSuccess) e = hipEventRecord(slot.loaded, slot.stream);
+	if (e == hipSuccess && brings) {
+		e = hipEventRecord(slot.loaded, slot.stream);
+		if (e == hipSuccess) s->lastLoaded = slot.loaded;
+	}
 	if (e != hipSuccess) return e;
-	s->lastLoaded = slot.loaded;
 	if (s->flags & PHX_SERVE_PLAIN) {
 		Request* r = slot.reqs[0];
 		TraceLaunch L = s->shape;

@@ -131,3 +131,54 @@ K = 1024
 def test_only_rays_inside_one_pinned_allocation_are_read_in_place(library, pins, at, n, in_place):
     copies = [x for x in run(library, serve_pinned, pins, at, n) if x.startswith(f"copy {32 * n} kind=1")]
     assert len(copies) == (0 if in_place else 1)
+
+
+def served_backlog(lib, where):
+    """One launch per request: 4 million rays each (2 million: a mixed launch's two requests)."""
+    ctx = phx.Context(0)
+    s = upload(ctx)
+    server = phx.Server(ctx, 1 << 31, slots=4)
+    server.add_scene(s)
+    n = 4 << 20
+    rays, out = phx.HostBuffer(np.uint8, 32 * n), phx.HostBuffer(np.uint8, 16 * n)
+    try:
+        server.pause()
+        tickets = []
+        for w in where:
+            for part, flags in {"host": [(n, 0)], "device": [(n, phx.MEM_DEVICE)], "empty": [(0, 0), (n, phx.MEM_DEVICE)],
+                                "mixed": [(n // 4, 0), (3 * n // 4, phx.MEM_DEVICE)]}[w]:
+                tickets.append(server.submit(phx.Server.request(
+                    s, rays.array.ctypes.data, out.array.ctypes.data, part, phx.BATCH_ANYHIT, flags)))
+        log(lib)
+        server.pause(False)
+        for t in tickets:
+            server.wait(t)
+        return log(lib)
+    finally:
+        server.destroy()
+
+
+@pytest.mark.parametrize("where, waits", [
+    (["host", "host", "host"], [None, 0, 1]),
+    (["host", "device", "device"], [None, None, None]),
+    (["host", "device", "host"], [None, None, 0]),
+    (["device", "host", "host"], [None, None, 1]),
+    (["host", "mixed", "empty"], [None, 0, None])])
+def test_launches_that_bring_no_rays_wait_for_nobodys(library, where, waits):
+    """waits: per launch, the earlier launch whose rays' arrival it waits for."""
+    lines = run(library, served_backlog, where)
+    launches = [{}]  # per launch, what comes before its traversal: (wait's event, event recorded)
+    for x in lines:
+        words = dict(w.split("=") for w in x.split() if "=" in w)
+        if x.startswith("wait"):
+            launches[-1]["waits"] = words["event"]
+        elif x.startswith("record") and "traced" not in launches[-1]:
+            launches[-1]["loaded"] = words["event"]
+        elif "k_trace_batches" in x:
+            launches[-1]["traced"] = True
+        elif x.startswith("record"):
+            launches.append({})
+    launches.pop()
+    assert len(launches) == len(where)
+    loaded = [k.get("loaded") for k in launches]
+    assert [k.get("waits") for k in launches] == [None if w is None else loaded[w] for w in waits]
