@@ -149,7 +149,7 @@ struct CopyRange {
 	void* dst;
 	uint64_t bytes;
 };
-hipError_t launchCopies(const CopyRange* ranges, uint32_t count, hipStream_t stream);
+hipError_t launchCopies(const CopyRange* ranges, uint32_t count, bool toHost, hipStream_t stream);
 // The device address of `bytes` bytes at p if they are pinned host memory (one allocation) and 16-byte
 // aligned, else null.
 void* deviceAddress(const void* p, size_t bytes);

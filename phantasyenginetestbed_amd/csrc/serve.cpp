@@ -245,7 +245,7 @@ hipError_t launchSlot(PhxServer* s, Slot& slot)
 		slot.copies.push_back({slot.mappedDescs, slot.descs, sizeof(BatchDesc) * nb});
 		slot.copies.push_back({slot.mappedOffsets, slot.offsets, sizeof(uint32_t) * (nb + 1)});
 	}
-	e = launchCopies(slot.copies.data(), uint32_t(slot.copies.size()), slot.stream);
+	e = launchCopies(slot.copies.data(), uint32_t(slot.copies.size()), false, slot.stream);
 	if (e == hipSuccess && brings) {
 		e = hipEventRecord(slot.loaded, slot.stream);
 		if (e == hipSuccess) s->lastLoaded = slot.loaded;
@@ -278,7 +278,7 @@ hipError_t launchSlot(PhxServer* s, Slot& slot)
 		else
 			e = hipMemcpyAsync(r->req.out, r->devOut, r->outBytes, hipMemcpyDeviceToHost, slot.stream);
 	}
-	if (e == hipSuccess) e = launchCopies(slot.copies.data(), uint32_t(slot.copies.size()), slot.stream);
+	if (e == hipSuccess) e = launchCopies(slot.copies.data(), uint32_t(slot.copies.size()), true, slot.stream);
 	if (e == hipSuccess) e = hipEventRecord(slot.done, slot.stream);
 	if (e == hipSuccess) {
 		slot.busy = true;

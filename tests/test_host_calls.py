@@ -182,3 +182,10 @@ def test_launches_that_bring_no_rays_wait_for_nobodys(library, where, waits):
     assert len(launches) == len(where)
     loaded = [k.get("loaded") for k in launches]
     assert [k.get("waits") for k in launches] == [None if w is None else loaded[w] for w in waits]
+
+
+def test_copies_leave_the_link_to_others(library):
+    """The reads of a copy kernel that are in flight hold up every other read over the link."""
+    lines = run(library, served_backlog, ["host", "device"])
+    grids = [int(w[5:]) for x in lines if "k_copy_ranges" in x for w in x.split() if w.startswith("grid=")]
+    assert grids == [32, 16, 2]  # rays in, flags out; the device-resident launch's table
