@@ -1155,12 +1155,27 @@ struct Candidate {
 	float ms = 0.0f;
 };
 
+// Drops the persistent candidates that come to the same launch as an earlier one (of few rays, say).
+template <class ShapeOf>
+void dropSame(std::vector<Candidate>& cands, ShapeOf shapeOf)
+{
+	std::vector<Candidate> kept;
+	for (const Candidate& c : cands) {
+		const bool same = std::any_of(kept.begin(), kept.end(), [&](const Candidate& k) {
+			return c.launch.kernel == TraceKernel::Persistent && k.launch.kernel == TraceKernel::Persistent &&
+			       shapeOf(k.launch) == shapeOf(c.launch);
+		});
+		if (!same) kept.push_back(c);
+	}
+	cands.swap(kept);
+}
+
 // Candidate shapes: a quarter, half or all of the rays in flight that the device holds, refill
 // threshold 8 or 32 -- plus the one-ray-per-lane and packet kernels for single batches.
 std::vector<Candidate> candidates(PhxContext* ctx, const PhxPlan* plan)
 {
 	std::vector<Candidate> out;
-	const uint32_t block = 512u, resident = ctx->numCUs * kRaysPerCu / block;
+	const uint32_t block = 512u, resident = ctx->numCUs * (plan ? kRaysPerCu : kCastRaysPerCu) / block;
 	for (uint32_t div : {4u, 2u, 1u})
 		for (uint32_t refill : {8u, 32u}) {
 			Candidate c;
@@ -1185,10 +1200,11 @@ std::vector<Candidate> candidates(PhxContext* ctx, const PhxPlan* plan)
 // time is its median round (single launches vary by a few percent, and a minimum would reward
 // the candidate with the luckiest draw). Interleaving the rounds spreads clock and cache drift
 // over all candidates instead of favouring those timed last.
-template <class Launch>
+template <class Launch, class ShapeOf>
 phx_status tune(PhxContext* ctx, std::vector<Candidate>& cands, int reps, Launch launch,
-                Candidate& best)
+                ShapeOf shapeOf, Candidate& best)
 {
+	dropSame(cands, shapeOf);
 	hipEvent_t a = nullptr, b = nullptr;
 	PHX_HIP(hipEventCreate(&a), "autotune");
 	hipError_t e = hipEventCreate(&b);
@@ -1224,8 +1240,9 @@ phx_status tune(PhxContext* ctx, std::vector<Candidate>& cands, int reps, Launch
 
 // Second stage for a persistent winner: rays per fetch around `best` (the current value stays a
 // candidate, so `best` only improves).
-template <class Launch>
-phx_status refine(PhxContext* ctx, const PhxPlan* plan, int reps, Launch launch, Candidate& best)
+template <class Launch, class ShapeOf>
+phx_status refine(PhxContext* ctx, const PhxPlan* plan, int reps, Launch launch, ShapeOf shapeOf,
+                  Candidate& best)
 {
 	if (best.launch.kernel != TraceKernel::Persistent) return PHX_OK;
 	std::vector<Candidate> cands{best};
@@ -1234,7 +1251,7 @@ phx_status refine(PhxContext* ctx, const PhxPlan* plan, int reps, Launch launch,
 		c.params.raysPerFetch = v;
 		if (shapeFor(ctx, c.params, c.launch, plan) == PHX_OK) cands.push_back(c);
 	}
-	return tune(ctx, cands, reps, launch, best);
+	return tune(ctx, cands, reps, launch, shapeOf, best);
 }
 
 }  // namespace
@@ -1261,8 +1278,9 @@ static phx_status phx_autotune_impl(PhxContext* ctx, const PhxScene* scene, cons
 		              : launchClosest(sv, rays, numRays, static_cast<PhxRayHit*>(out), L, nullptr,
 		                              ctx->stream);
 	};
-	st = tune(ctx, cands, 13, cast, best);
-	if (st == PHX_OK) st = refine(ctx, nullptr, 15, cast, best);
+	auto shapeOf = [&](const TraceLaunch& L) { return castShape(L, numRays); };
+	st = tune(ctx, cands, 13, cast, shapeOf, best);
+	if (st == PHX_OK) st = refine(ctx, nullptr, 15, cast, shapeOf, best);
 	hipStreamSynchronize(ctx->stream);
 	hipFree(out);
 	if (st != PHX_OK) return st;
@@ -1330,8 +1348,11 @@ static phx_status phx_plan_autotune_impl(PhxContext* ctx, PhxPlan* plan, PhxLaun
 		return launchBatches(plan->descs, plan->offsets, plan->numBatches, plan->total, L,
 		                     plan->clock, ctx->stream);
 	};
-	st = tune(ctx, cands, 3, run, best);
-	if (st == PHX_OK) st = refine(ctx, plan, 5, run, best);
+	auto shapeOf = [&](const TraceLaunch& L) {
+		return batchShape(L, plan->total, plan->numBatches, plan->clock != nullptr);
+	};
+	st = tune(ctx, cands, 3, run, shapeOf, best);
+	if (st == PHX_OK) st = refine(ctx, plan, 5, run, shapeOf, best);
 	if (st != PHX_OK) return st;
 	st = phx_plan_set_launch_params(ctx, plan, &best.params);
 	if (st != PHX_OK) return st;

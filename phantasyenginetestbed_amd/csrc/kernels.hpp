@@ -42,8 +42,9 @@ enum class TraceKernel { Persistent, Simple, Packet };
 // Words of a launch's ray counters, and words of stack spill per ray in flight.
 constexpr uint32_t kRayCounterWords = 1024;
 constexpr uint32_t kSpillWordsPerRay = 112;
-// Most rays in flight per CU: 16 waves of 64 rays, one per lane (28 of 16 rays, four lanes each).
-constexpr uint32_t kRaysPerCu = 1024;
+// Most rays in flight per CU: 16 waves of 64 rays, one per lane (fused launches), or 28 of 16 rays,
+// four lanes each (single casts).
+constexpr uint32_t kRaysPerCu = 1024, kCastRaysPerCu = 448;
 
 // Launch parameters of the traversal kernels. `work` points at kRayCounterWords zeroed words owned
 // by the launching stream (the persistent kernels leave them zeroed); `spill` holds
@@ -53,11 +54,23 @@ struct TraceLaunch {
 	uint32_t raysInFlight = 0;
 	uint32_t cus = 0;
 	uint32_t spillColumns = 0;
-	uint32_t refillMin = 8;      // refill a wave once this many of its lanes are idle
+	uint32_t refillMin = 8;      // refill a wave once this many of its lanes are idle (fused: 8 and 16 the
+	                             // same, 4 and 24 up to 2% slower)
 	uint32_t window = 64;        // most rays a wave claims per fetch from a ray counter
 	uint32_t* work = nullptr;
 	uint32_t* spill = nullptr;
 };
+
+// What a persistent launch of n rays comes to under `launch`: a single cast, or a fused launch.
+struct LaunchShape {
+	uint32_t grid, block, window, refill;
+	bool operator==(const LaunchShape& o) const
+	{
+		return grid == o.grid && block == o.block && window == o.window && refill == o.refill;
+	}
+};
+LaunchShape castShape(const TraceLaunch& launch, uint32_t n);
+LaunchShape batchShape(const TraceLaunch& launch, uint32_t total, uint32_t numBatches, bool tracked);
 
 // Scratch of the allocation-free closest-hit cast: a static device array per GPU holding the
 // launch's ray counters (first kNoAllocCounterBytes) and its stack spill area (42 MiB: 98,304 rays).

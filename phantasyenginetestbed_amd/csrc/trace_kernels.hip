@@ -800,15 +800,13 @@ constexpr uint32_t kLaneBlock = 1024;  // (of fused launches)
 constexpr uint32_t kLdsBytes = 160u * 1024u;  // of a CU
 constexpr uint32_t kStageWords = 512u + 64u;  // of a wave: a window's rays and their indices
 constexpr uint32_t kQuadWavesPerSimd = 7;  // (72 registers)
+static_assert(kCastRaysPerCu == kQuadWavesPerSimd * 4u * 16u, "rays in flight per CU of a single cast");
 
 // Stacks of a wave: kCols columns of kRows entries (8 B) in LDS, with three rows below the bottom, so
 // that the top three can be read at any depth. Deeper entries spill to memory, kSpillEntries a
 // column, one after another.
 constexpr int kQuadRows = 20;  // (pending stacks of 20 are rare)
 constexpr int kLaneRows = 10;  // (8.5 KB a wave with 2 KB of rays: 16 waves per CU beside the batch tables)
-// Idle lanes of a one-ray-per-lane wave before it takes new rays: 64 batches of 3.2 million rays take
-// 1.66 ms with 4, 1.65 with 8 and 16, 1.68 with 24.
-constexpr uint32_t kLaneRefill = 16;
 constexpr uint32_t kSpillEntries = kSpillWordsPerRay / 2u;
 static_assert(kLaneRows + int(kSpillEntries) >= kMaxPending, "stack entries of a ray");
 static_assert(kQuadRows + int(kSpillEntries) >= kMaxPending, "stack entries of a ray");
@@ -2104,10 +2102,9 @@ bool bigScene(const SceneView& s)
 }
 
 // Launch shapes of the persistent kernels for n rays. A launch keeps at most L.raysInFlight rays in
-// flight, each on a column of the spill area.
-struct Shape {
-	uint32_t grid, block, window, refill;
-};
+// flight, each on a column of the spill area, takes at most L.window of them at a time and new ones when
+// a share of L.refillMin / 64 of a wave's places is idle.
+using Shape = LaunchShape;
 
 Shape shapeOf(uint32_t waves, uint32_t most, uint32_t block)
 {
@@ -2127,8 +2124,9 @@ Shape quadShape(const TraceLaunch& L, uint32_t n)
 	const uint32_t most = std::max(
 		1u, std::min(std::min(L.raysInFlight, L.spillColumns) / 16u, L.cus * kQuadWavesPerSimd * 4u));
 	const uint32_t window =
-		n / 16u >= most ? std::min(std::max(16u, n / (2u * most)), std::min(64u, std::max(16u, L.window)))
-		                : std::min(16u, std::max(gridFor(n, 2048u), gridFor(n, most)));
+		std::min(std::min(64u, L.window),
+		         n / 16u >= most ? std::max(16u, n / (2u * most))
+		                         : std::min(16u, std::max(gridFor(n, 2048u), gridFor(n, most))));
 	const uint32_t waves = std::min(most, gridFor(n, window));
 	Shape s = shapeOf(waves, most, 256u);  // (four waves: a CU holds seven such blocks)
 	s.window = window;
@@ -2136,7 +2134,7 @@ Shape quadShape(const TraceLaunch& L, uint32_t n)
 	return s;
 }
 
-// One ray per lane: windows of 64 rays; blocks small enough that every CU has one, and of 1,024 threads
+// One ray per lane: windows of 64 rays, or what L says; blocks small enough that every CU has one, and of 1,024 threads
 // where `tableWords` of LDS beside the waves' (the batch tables) would halve the waves of a CU in blocks
 // of 512 (256 tracked batches of 29.6 million rays: 7.4 ms with 8 waves per CU, 4.7 with 16). No more waves
 // than are resident: the others' first windows would wait for a block to end.
@@ -2149,11 +2147,11 @@ Shape laneShape(const TraceLaunch& L, uint32_t n, uint32_t tableWords)
 	uint32_t block = resident(kLaneBlock) > resident(kQuadBlock) ? kLaneBlock : kQuadBlock;
 	const uint32_t most = std::max(1u, std::min(std::min(L.raysInFlight, L.spillColumns) / 64u,
 	                                            L.cus * std::max(1u, resident(block))));
-	const uint32_t waves = std::min(most, gridFor(n, 64u));
+	const uint32_t window = std::min(64u, L.window), waves = std::min(most, gridFor(n, window));
 	while (block > 64u && waves / (block / 64u) < L.cus) block /= 2u;
 	Shape s = shapeOf(waves, most, block);
-	s.window = 64u;
-	s.refill = kLaneRefill;
+	s.window = window;
+	s.refill = std::min(64u, std::max(1u, L.refillMin));
 	return s;
 }
 
@@ -2337,14 +2335,21 @@ hipError_t launchShadeTrace(const SceneView& s, const float4* info, const PhxSph
 	return hipGetLastError();
 }
 
+LaunchShape castShape(const TraceLaunch& L, uint32_t n) { return quadShape(L, n); }
+
+LaunchShape batchShape(const TraceLaunch& L, uint32_t total, uint32_t numBatches, bool tracked)
+{
+	return laneShape(L, total, batch_lds_words(0u, numBatches, tracked));
+}
+
 hipError_t launchBatches(const BatchDesc* descs, const uint32_t* offsets, uint32_t numBatches,
                          uint32_t total, const TraceLaunch& L, BatchClock* clock, hipStream_t stream)
 {
 	if (total == 0) return hipSuccess;
-	const Shape q = laneShape(L, total, batch_lds_words(0u, numBatches, clock != nullptr));
+	const Shape q = batchShape(L, total, numBatches, clock != nullptr);
 	hipLaunchKernelGGL(clock ? k_trace_batches<true> : k_trace_batches<false>, dim3(q.grid),
 	                   dim3(q.block), batch_lds_words(q.block / 64u, numBatches, clock != nullptr) * 4u,
-	                   stream, descs, offsets, numBatches, total, 64u, q.refill, L.work,
+	                   stream, descs, offsets, numBatches, total, q.window, q.refill, L.work,
 	                   reinterpret_cast<U32x2*>(L.spill), clock);
 	return hipGetLastError();
 }

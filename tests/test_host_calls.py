@@ -189,3 +189,75 @@ def test_copies_leave_the_link_to_others(library):
     lines = run(library, served_backlog, ["host", "device"])
     grids = [int(w[5:]) for x in lines if "k_copy_ranges" in x for w in x.split() if w.startswith("grid=")]
     assert grids == [32, 16, 2]  # rays in, flags out; the device-resident launch's table
+
+
+def launches(lines, kernel):
+    """(grid, block, window, refill) of every launch of `kernel`, in order."""
+    out = []
+    for x in lines:
+        if x.startswith("kernel") and kernel in x:
+            w = dict(w.split("=") for w in x.split() if "=" in w)
+            out.append(tuple(int(w[k]) for k in ("grid", "block", "window", "refill")))
+    return out
+
+
+def fused(lib, n, refill, fetch, how):
+    ctx = phx.Context(0)
+    s = upload(ctx)
+    rays, out = ctx.alloc(32 * n), ctx.alloc(16 * n)
+    ctx.set_launch_params(refill_min=refill, rays_per_fetch=fetch)
+    if how == "server":
+        server = phx.Server(ctx, 1 << 28)
+        server.add_scene(s)
+        log(lib)
+        try:
+            server.wait(server.submit(phx.Server.request(s, rays.ptr, out.ptr, n, phx.BATCH_CLOSEST,
+                                                         phx.MEM_DEVICE)))
+        finally:
+            server.destroy()
+        return log(lib)
+    if how == "set":  # by hand, after the context's
+        ctx.set_launch_params(refill_min=8, rays_per_fetch=64)
+    plan = phx.Plan(ctx, [(s, rays.ptr, out.ptr, n, phx.BATCH_CLOSEST)])
+    if how == "set":
+        plan.set_launch_params(512, block_threads=512, refill_min=refill, rays_per_fetch=fetch)
+    log(lib)
+    plan.launch()
+    return log(lib)
+
+
+@pytest.mark.parametrize("how", ["context", "set", "server"])
+@pytest.mark.parametrize("refill, fetch", [(1, 8), (8, 64), (24, 16), (64, 256)])
+def test_fused_launches_take_refill_threshold_and_rays_per_fetch(library, how, refill, fetch):
+    """From the plan, or the context that it or the server was made with (the server's rays per fetch:
+    the default)."""
+    (_, _, window, took), = launches(run(library, fused, 200000, refill, fetch, how), "k_trace_batches")
+    assert took == refill and window == (64 if how == "server" else min(fetch, 64))
+
+
+def tuned(lib, n, plan):
+    ctx = phx.Context(0)
+    s = upload(ctx)
+    rays, out = ctx.alloc(32 * n), ctx.alloc(16 * n)
+    p = phx.Plan(ctx, [(s, rays.ptr, out.ptr, n, phx.BATCH_CLOSEST)]) if plan else None
+    log(lib)
+    p.autotune() if plan else ctx.autotune(s, rays.ptr, n)
+    return log(lib)
+
+
+@pytest.mark.parametrize("plan", [False, True], ids=["cast", "plan"])
+@pytest.mark.parametrize("n", [100, 3000, 60000, 4000000])
+def test_autotuners_time_no_launch_twice(library, plan, n):
+    """Both stages time each of their launch shapes once a round."""
+    lines = run(library, tuned, n, plan)
+    shapes = launches(lines, "k_trace_batches" if plan else "k_quad")
+    reps = (3, 5) if plan else (13, 15)
+    # A warm-up and reps rounds of the first stage, then of the second, which has its winner again.
+    k = next(i for i in range(1, len(shapes)) if shapes[i] == shapes[0])
+    assert len(set(shapes[:k])) == k
+    rest = shapes[k * (reps[0] + 1):]
+    assert shapes[:k * (reps[0] + 1)] == shapes[:k] * (reps[0] + 1)
+    m = len(rest) // (reps[1] + 1)
+    assert rest == rest[:m] * (reps[1] + 1) and len(set(rest[:m])) == m
+    if n == 4000000:
+        assert k == 6 and m == 3
