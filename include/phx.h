@@ -233,7 +233,7 @@ typedef struct PhxLaunchParams {
 	uint32_t refillMin;
 	uint32_t blockThreads;
 	uint32_t topNodes;
-	uint32_t residentGridBlocks; /* read only: blocks of this shape the device holds at once */
+	uint32_t residentGridBlocks; /* read only: blocks of this size whose rays the device holds at once */
 	uint32_t helperWaves;
 	uint32_t raysPerFetch;
 	uint32_t stackLdsEntries;

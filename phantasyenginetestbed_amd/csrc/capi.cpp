@@ -155,16 +155,24 @@ constexpr uint32_t kTopCap = 2048;
 // Wide nodes kept in breadth-first order.
 constexpr uint32_t kWideTop = 1024;
 
-// Blocks per CU of a launch shape, by the LDS and registers it stands for: a stack split of `depth`
-// words per lane, the treelet, 1,440 B a wave for handed-over rays, and, for a plan, its batch
-// table; 20 waves per CU for single casts, 16 for a plan. A shape that does not fit is refused.
-uint32_t shapeBlocksPerCU(const PhxPlan* plan, uint32_t block, uint32_t top, uint32_t helpers,
-                          uint32_t depth)
+// Whether a launch shape is one that the interface takes: topNodes, helperWaves and stackLdsEntries no
+// longer change how the kernels run, but what they stand for has to fit a CU's LDS as it always had to --
+// a stack of `depth` words per lane, the treelet, 1,440 B a wave and, for a plan, its batch table -- so
+// that the shapes accepted and refused stay the same. A plan's treelet is at most its one scene's nodes.
+bool shapeFits(const PhxPlan* plan, uint32_t block, uint32_t top, uint32_t depth)
 {
-	const uint32_t waves = block / 64u, all = waves + helpers;
+	const uint32_t waves = block / 64u;
+	if (plan) top = std::min(top, plan->treelet);
 	uint32_t lds = waves * (depth + 1u) * 256u + top * 64u + 16u + waves * 1440u;
 	if (plan) lds += (plan->numBatches + 1u) * 4u + (plan->clock ? plan->numBatches * 12u : 0u);
-	return std::min(163840u / lds, (plan ? 16u : 20u) / std::max(all, 1u));
+	return lds <= 160u * 1024u;
+}
+
+// Blocks of `block` rays that the device has in flight at once: more of them change nothing.
+uint32_t residentBlocks(const PhxContext* ctx, const PhxPlan* plan, uint32_t block)
+{
+	const uint32_t rays = ctx->numCUs * (plan ? kRaysPerCu : kCastRaysPerCu);
+	return (rays + block - 1u) / block;
 }
 
 // Triangles as (p0, e1 = p1 - p0, e2 = p2 - p0); p0.w keeps the end marker. The subtractions are
@@ -407,9 +415,7 @@ phx_status phx_get_launch_params(PhxContext* ctx, PhxLaunchParams* out)
 	out->refillMin = ctx->refillMin;
 	out->blockThreads = ctx->blockThreads;
 	out->topNodes = ctx->topNodes;
-	const uint32_t bpc =
-		shapeBlocksPerCU(nullptr, ctx->blockThreads, ctx->topNodes, ctx->helperWaves, ctx->ldsDepth);
-	out->residentGridBlocks = ctx->numCUs * bpc;
+	out->residentGridBlocks = residentBlocks(ctx, nullptr, ctx->blockThreads);
 	out->helperWaves = ctx->helperWaves;
 	out->raysPerFetch = ctx->window;
 	out->stackLdsEntries = ctx->ldsDepth;
@@ -440,8 +446,7 @@ phx_status phx_set_launch_params(PhxContext* ctx, const PhxLaunchParams* p)
 	if (window < 8u || window > 4096u)
 		return fail(PHX_ERR_INVALID_ARGUMENT, "phx_set_launch_params: raysPerFetch %u outside 8..4096",
 		            window);
-	const uint32_t bpc = shapeBlocksPerCU(nullptr, block, top, helpers, depth);
-	if (bpc == 0)
+	if (!shapeFits(nullptr, block, top, depth))
 		return fail(PHX_ERR_INVALID_ARGUMENT,
 		            "phx_set_launch_params: %u threads (+%u helper waves) with a %u-node treelet and "
 		            "%u LDS stack entries do not fit a CU", block, helpers, top, depth);
@@ -454,7 +459,7 @@ phx_status phx_set_launch_params(PhxContext* ctx, const PhxLaunchParams* p)
 	// A new block or treelet size without an explicit grid gets the resident grid of that shape.
 	const bool reshaped = block != ctx->blockThreads || top != ctx->topNodes ||
 	                      helpers != ctx->helperWaves || depth != ctx->ldsDepth;
-	const uint32_t resident = std::min(ctx->numCUs * bpc, maxGrid);
+	const uint32_t resident = residentBlocks(ctx, nullptr, block);
 	ctx->blockThreads = block;
 	ctx->topNodes = top;
 	ctx->helperWaves = helpers;
@@ -1038,6 +1043,7 @@ static phx_status phx_plan_create_impl(PhxContext* ctx, const PhxBatch* batches,
 			p->scenes.push_back(batches[b].scene);
 			holdScene(batches[b].scene);
 		}
+	if (p->scenes.size() == 1) p->treelet = std::min(p->scenes[0]->numNodes, kTopCap);
 	holdContext(ctx);
 	registry().add(p);
 	*outPlan = p;
@@ -1134,7 +1140,7 @@ phx_status shapeFor(PhxContext* ctx, const PhxLaunchParams& p, TraceLaunch& L,
 		return fail(PHX_ERR_INVALID_ARGUMENT, "launch params: stackLdsEntries %u outside 4..32", depth);
 	if (window < 8u || window > 4096u)
 		return fail(PHX_ERR_INVALID_ARGUMENT, "launch params: raysPerFetch %u outside 8..4096", window);
-	if (shapeBlocksPerCU(plan, block, p.topNodes, helpers, depth) == 0)
+	if (!shapeFits(plan, block, p.topNodes, depth))
 		return fail(PHX_ERR_INVALID_ARGUMENT, "launch params: shape does not fit a CU");
 	const uint32_t maxGrid = ctx->spillLanes / block;
 	const uint32_t grid = p.gridBlocksClosest;
@@ -1175,7 +1181,7 @@ void dropSame(std::vector<Candidate>& cands, ShapeOf shapeOf)
 std::vector<Candidate> candidates(PhxContext* ctx, const PhxPlan* plan)
 {
 	std::vector<Candidate> out;
-	const uint32_t block = 512u, resident = ctx->numCUs * (plan ? kRaysPerCu : kCastRaysPerCu) / block;
+	const uint32_t block = 512u, resident = residentBlocks(ctx, plan, block);
 	for (uint32_t div : {4u, 2u, 1u})
 		for (uint32_t refill : {8u, 32u}) {
 			Candidate c;

@@ -93,6 +93,7 @@ struct PhxPlan {
 	phx::TraceLaunch launch;  // launch shape of this plan (set at creation, tunable)
 	uint32_t numBatches = 0;
 	uint32_t total = 0;
+	uint32_t treelet = 0;     // most topNodes that count when a shape is checked: one scene's, or none
 	phx::BatchDesc* descs = nullptr;
 	uint32_t* offsets = nullptr;
 	phx::BatchClock* clock = nullptr;

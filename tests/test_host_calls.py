@@ -261,3 +261,61 @@ def test_autotuners_time_no_launch_twice(library, plan, n):
     assert rest == rest[:m] * (reps[1] + 1) and len(set(rest[:m])) == m
     if n == 4000000:
         assert k == 6 and m == 3
+
+
+def shapes(lib, scenes, track, tries):
+    """For each (block, topNodes, helpers, depth): whether the context and a plan over `scenes` take it."""
+    ctx = phx.Context(0)
+    up = [upload(ctx, n, i + 1) for i, n in enumerate(scenes)]
+    mem = ctx.alloc(1 << 16)
+    plan = phx.Plan(ctx, [(s, mem.ptr, mem.ptr, 64, phx.BATCH_CLOSEST) for s in up for _ in range(20)], track)
+
+    def takes(f, *a, **k):
+        try:
+            f(*a, **k)
+            return True
+        except phx.PhxError as e:
+            assert e.status == phx.ERR_INVALID_ARGUMENT
+            return False
+
+    return [(takes(ctx.set_launch_params, block_threads=b, top_nodes=top, helper_waves=h, stack_lds_entries=d),
+             takes(plan.set_launch_params, 8, block_threads=b, top_nodes=top, helper_waves=h, stack_lds_entries=d))
+            for b, top, h, d in tries]
+
+
+@pytest.mark.parametrize("track", [False, True])
+@pytest.mark.parametrize("scenes", [[50], [6000], [50, 60], [6000, 6001]])
+def test_shapes_taken_and_refused(library, scenes, track):
+    """What a shape stands for has to fit 160 KB of LDS: (depth + 1) x 256 B and 1,440 B a wave, 64 B a
+    treelet node, 16 B. In a plan only the nodes count that its one scene has, and its batch table."""
+    tries = [(b, top, h, d) for b in (64, 256, 512, 1024) for top in (0, 100, 1000, 1900, 2048)
+             for h in (0, 4) for d in (4, 16, 32) if b + 64 * h <= 1024]
+    got = run(library, shapes, scenes, track, tries)
+    nodes = [len(phx.BVH(*phx.random_triangles(n, i + 1, 0.1, 0.5)).nodes) for i, n in enumerate(scenes)]
+    table = 20 * len(scenes) * (16 if track else 4) + 4
+    for (b, top, h, d), (by_context, by_plan) in zip(tries, got):
+        lds = b // 64 * ((d + 1) * 256 + 1440) + 16
+        treelet = min(top, nodes[0]) if len(scenes) == 1 else 0
+        assert by_context == (lds + 64 * top <= 163840)
+        assert by_plan == (lds + 64 * treelet + table <= 163840), (b, top, h, d)
+
+
+def resident(lib, block, n):
+    ctx = phx.Context(0)
+    s = upload(ctx)
+    mem = ctx.alloc(32 * n)
+    ctx.set_launch_params(block_threads=block, top_nodes=0, helper_waves=0)
+    top = ctx.launch_params()["residentGridBlocks"]
+    out = []
+    for grid in (top // 2, top, top + 9):
+        ctx.set_launch_params(grid_closest=grid)
+        log(lib)
+        ctx.cast_closest_device(s, mem.ptr, n, mem.ptr)
+        out += launches(log(lib), "k_quad")
+    return out
+
+
+@pytest.mark.parametrize("block", [64, 256, 512, 1024])
+def test_resident_grid_is_where_more_blocks_change_nothing(library, block):
+    half, whole, more = run(library, resident, block, 4 << 20)
+    assert half[0] < whole[0] and whole == more
