@@ -283,8 +283,10 @@ __device__ __forceinline__ bool anyhit_one(const float4* __restrict__ nodes,
 // ---- four-wide nodes ---------------------------------------------------------------------------
 //
 // wide_nodes.hpp says what they are and why taking their slots in order, with each slot's entry
-// distance compared again when it is taken, gives castRay's hits bit for bit for every ray whose
-// slab values cannot be NaN (dev::Ray::nanFree). The other rays walk the binary nodes.
+// distance compared again when it is taken, gives castRay's hits bit for bit for every ray with an origin
+// within 2^126. Rays whose slab values may be NaN are decided with castRay's own min and max (dev::slab)
+// by the kernels that trace four lanes per ray or one ray per lane in persistent waves; the others trace
+// such rays on the binary nodes (dev::Ray::nanFree).
 // A traversal is bound by its chain of dependent steps; on 1,004,000 triangles a bounce ray takes
 // 9.8 wide node visits where it takes 21.6 binary ones (random triangles: 32 for 65).
 
@@ -322,6 +324,20 @@ __device__ __forceinline__ WideVisit decide_wide(const dev::Ray& r, const WideWo
 #pragma unroll
 	for (int i = 0; i < 4; i++)
 		v.pass[i] = decide_slot(r, n.w[2 * i], n.w[2 * i + 1], tCurrMax, v.tIn[i]);
+	return v;
+}
+
+// The same of rays whose slab values may be NaN.
+__device__ __forceinline__ WideVisit decide_wide_nan(const dev::Ray& r, const WideWords& n, float tCurrMax)
+{
+	WideVisit v;
+#pragma unroll
+	for (int i = 0; i < 4; i++) {
+		const float4 lo = n.w[2 * i], hi = n.w[2 * i + 1];
+		float tOut;
+		dev::slab(r, lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, v.tIn[i], tOut);
+		v.pass[i] = (tOut >= v.tIn[i]) && tOut > r.tMin && v.tIn[i] < tCurrMax;
+	}
 	return v;
 }
 
@@ -857,10 +873,16 @@ __device__ __forceinline__ float recip_wave(float a)
 	return f;
 }
 
-// Sets r up from its record; false if it walks the binary nodes instead: a direction component
-// outside the fast reciprocal's range (zero among them) or an origin beyond 2^126, with which slab
-// values could be NaN.
-__device__ __forceinline__ bool quad_ray(const float4 a, const float4 b, dev::Ray& r)
+// What a ray's boxes are decided with.
+constexpr uint32_t kFast = 0;    // slab_fast, on the wide nodes
+constexpr uint32_t kSlab = 1;    // slab, on the wide nodes
+constexpr uint32_t kBinary = 2;  // slab, on the binary nodes
+
+// Sets r up from its record. A direction component outside the fast reciprocal's range (zero among them)
+// takes the division and slab, with which NaN slab values come out as castRay's; an origin beyond 2^126
+// the binary nodes (wide_nodes.hpp). Rays with a zero component are ordinary ones (probes, a sun
+// overhead): on the binary nodes 1,048,576 of them straight up took 0.91 ms, on the wide ones 0.52 ms.
+__device__ __forceinline__ uint32_t quad_ray(const float4 a, const float4 b, bool hasWide, dev::Ray& r)
 {
 	r.ox = a.x, r.oy = a.y, r.oz = a.z, r.tMin = a.w;
 	r.dx = b.x, r.dy = b.y, r.dz = b.z, r.tMax = b.w;
@@ -868,8 +890,14 @@ __device__ __forceinline__ bool quad_ray(const float4 a, const float4 b, dev::Ra
 	r.iy = dev::recip_newton(b.y);
 	r.iz = dev::recip_newton(b.z);
 	auto within = [](float x) { return fabsf(x) >= 0x1p-126f && fabsf(x) < 0x1p126f; };
-	return within(b.x) && within(b.y) && within(b.z) && fabsf(a.x) <= 0x1p126f &&
-	       fabsf(a.y) <= 0x1p126f && fabsf(a.z) <= 0x1p126f;
+	const bool near = fabsf(a.x) <= 0x1p126f && fabsf(a.y) <= 0x1p126f && fabsf(a.z) <= 0x1p126f;
+	return !(near && hasWide) ? kBinary : within(b.x) && within(b.y) && within(b.z) ? kFast : kSlab;
+}
+__device__ __forceinline__ void divide(const float4 b, dev::Ray& r)
+{
+	r.ix = 1.0f / b.x;
+	r.iy = 1.0f / b.y;
+	r.iz = 1.0f / b.z;
 }
 
 // What a launch traces. Single casts: one scene, ray array and output. Batches: per ray through its
@@ -907,7 +935,7 @@ struct Quad {
 	uint32_t hit = kInvalid;
 	// (4-byte flags: between the others' bytes, hit was kept in four registers.)
 	uint32_t mine = 0u;          // holds the closest hit
-	uint32_t exact = 0u;         // walks the binary nodes
+	uint32_t with = kFast;       // kFast, kSlab or kBinary
 	uint32_t any = 0u;
 	bool leaf = false;           // triangles to test before node: this lane's is tri
 	// batches
@@ -979,7 +1007,7 @@ struct QuadTracer {
 	const QuadArgs& P;
 	LdsU2* stacks;       // the block's stack columns
 	uint32_t lane, l;
-	bool someExact = false;  // (uniform) a ray of the wave may walk the binary nodes
+	bool slow = false;  // (uniform) a ray of the wave may be decided with slab
 	Quad q;
 
 	__device__ __forceinline__ bool isAny() const { return kAny == 1 || (kAny == 2 && q.any); }
@@ -1003,12 +1031,8 @@ struct QuadTracer {
 	// Sets this quad up for ray `ray` with the record (a, b).
 	__device__ __forceinline__ void set(uint32_t ray, const float4 a, const float4 b, bool hasWide)
 	{
-		q.exact = !(quad_ray(a, b, q.r) && hasWide);
-		if (__builtin_expect(ballot(q.exact) != 0ull, 0)) {
-			q.r.ix = 1.0f / b.x;
-			q.r.iy = 1.0f / b.y;
-			q.r.iz = 1.0f / b.z;
-		}
+		q.with = quad_ray(a, b, hasWide, q.r);
+		if (__builtin_expect(ballot(q.with != kFast) != 0ull, 0)) divide(b, q.r);
 		q.ray = ray;
 	}
 	// Starts a ray of a single cast.
@@ -1076,7 +1100,7 @@ struct QuadTracer {
 		// first line. Offsets in bytes: 48 per triangle, 128 per wide node.
 		const uint32_t tri = q.leaf ? q.tri : 0u;
 		uint32_t node = q.node != kInvalid ? q.node : 0u;
-		if (someExact) node = q.exact ? 0u : node;
+		if (slow) node = q.with == kBinary ? 0u : node;
 		const float4* pl;
 		const float4* pn;
 		if (kBig) {
@@ -1121,16 +1145,17 @@ struct QuadTracer {
 			q.skip = 0u;
 		}
 		const float lim = any ? q.r.tMax : dev::min_first(q.r.tMax, q.best);
-		if (__builtin_expect(someExact, 0))
-			if (q.exact && q.node != kInvalid && !more) {
+		float tIn, tOut;
+		dev::slab_fast(q.r, lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, tIn, tOut);
+		if (__builtin_expect(slow, 0)) {  // (all of it in one branch that fast rays' waves do not take)
+			dev::slab(q.r, lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, tIn, tOut);
+			if (q.with == kBinary && q.node != kInvalid && !more) {
 				expand_binary(lim);
 				q.node = kInvalid;
 			}
+		}
 		if (q.node != kInvalid && !more) {
 			// The passing slots are pushed, last slot first; a leaf pair stays one only if both pass.
-			float tIn;
-			float tOut;
-			dev::slab_fast(q.r, lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, tIn, tOut);
 			const bool enters = any || q.nodeIn < lim;
 			const bool pass = (tOut >= tIn) && tOut > q.r.tMin && tIn < lim && enters;
 			const uint32_t m = nibble(ballot(tOut >= tIn) & ballot(tOut > q.r.tMin) & ballot(tIn < lim) & ballot(enters));
@@ -1281,7 +1306,7 @@ __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 					T.start(kAny == 1 ? index[at] : W.next + at, make_float4(a.x, a.y, a.z, a.w),
 					        make_float4(b.x, b.y, b.z, b.w));
 				}
-				T.someExact = ballot(T.q.exact != 0u) != 0ull;
+				T.slow = ballot(T.q.with != kFast) != 0ull;
 				taken += room;
 			}
 		}
@@ -1305,14 +1330,14 @@ __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 // the time, the VALUs 63% (with eight words a node). Handing the records over in LDS, four lanes to a line, took it to 1.60 ms and
 // single casts from 0.106 to 0.123 ms, so each lane loads its own.
 
-// One lane's castRay over the wide nodes, or the binary ones (exact), one record at a time.
+// One lane's castRay over the wide nodes, or the binary ones, one record at a time.
 struct LaneWalk {
 	dev::Ray r;
 	uint32_t ref = 0u;  // what the ray takes next: a node, or kWideLeaf and a triangle
 	int sp = 0;
 	int floor = 0;      // the stack's bottom for this walk
 	Closest c = {kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
-	bool exact = false;
+	uint32_t with = kFast;  // kFast, kSlab or kBinary
 
 	// Decides a binary node's children as castRay does and pushes what is visited in its order.
 	template <class Stack>
@@ -1331,7 +1356,7 @@ struct LaneWalk {
 
 	__device__ __forceinline__ bool at_leaf() const { return (ref & kWideLeaf) != 0u; }
 	// The record that advance() consumes: a wide node, or a leaf's next two triangles (the words past
-	// a leaf's last one are the next triangle's or the array's padding). Exact nodes read the array's
+	// a leaf's last one are the next triangle's or the array's padding). Binary nodes read the array's
 	// first line. The loads are bound by the 16 B a lane that the texture data path returns a cycle, so
 	//   - a node is read in seven words: slot 3's max.xyz is in the last components of words 1, 3 and 5
 	//     too (with eight, 64 fused batches took 1.635 ms, with seven 1.563; 1,048,576 rays into 300
@@ -1343,18 +1368,18 @@ struct LaneWalk {
 	{
 		if (!on) return;
 		const float4* rec = at_leaf() ? tris + 3u * size_t(ref & kWideIndex)
-		                              : wide + 8u * size_t(!exact ? ref : 0u);
+		                              : wide + 8u * size_t(with != kBinary ? ref : 0u);
 #pragma unroll
 		for (int i = 0; i < 7; i++) w[i] = as_global(rec)[i];
 	}
 
 	// Expands a node or tests up to two triangles of a leaf, and picks what the lane takes next. True
 	// if the traversal has ended (`occluded`: with an any-hit ray's hit).
-	template <int kAny, class Stack>
+	template <int kAny, bool kSlow, class Stack>
 	__device__ __forceinline__ bool advance(const float4 w[7], const float4* nodes, bool any, Stack& st,
 	                                        bool& occluded)
 	{
-		const bool leaf = at_leaf(), node = !leaf && !exact;
+		const bool leaf = at_leaf(), node = !leaf && !(kSlow && with == kBinary);
 		bool pop = true;
 		occluded = false;
 		if (leaf) {
@@ -1389,7 +1414,9 @@ struct LaneWalk {
 #pragma unroll
 			for (int i = 0; i < 7; i++) n.w[i] = w[i];
 			n.w[7] = make_float4(w[1].w, w[3].w, w[5].w, 0.0f);
-			const WideVisit v = decide_wide(r, n, lim);
+			WideVisit v;
+			if (kSlow) v = decide_wide_nan(r, n, lim);
+			else v = decide_wide(r, n, lim);
 			const bool p0 = v.pass[0], p1 = v.pass[1], p2 = v.pass[2], p3 = v.pass[3];
 			uint32_t r0 = __float_as_uint(w[0].w), r1 = __float_as_uint(w[2].w);
 			uint32_t r2 = __float_as_uint(w[4].w);
@@ -1406,7 +1433,7 @@ struct LaneWalk {
 			sp = pop ? sp : at1 + (p1 ? 1 : 0) + (p0 ? 1 : 0) - 1;
 			ref = p0 ? r0 : p1 ? r1 : p2 ? r2 : r3;
 		}
-		if (__builtin_expect(exact && !leaf, 0)) expand_binary(nodes, lim, st);
+		if (kSlow && with == kBinary && !leaf) expand_binary(nodes, lim, st);
 		if (occluded || (pop && !take(lim, any, st))) return true;
 		if (!any && (pop || node)) decide_sibling(lim, st);
 		return false;
@@ -1542,12 +1569,8 @@ struct LaneTracer {
 		}
 		const F32x4 sa = staged[index - first], sb = staged[64u + index - first];
 		const float4 a = make_float4(sa.x, sa.y, sa.z, sa.w), b = make_float4(sb.x, sb.y, sb.z, sb.w);
-		t.exact = !(quad_ray(a, b, t.r) && hasWide);
-		if (__builtin_expect(t.exact, 0)) {
-			t.r.ix = 1.0f / b.x;
-			t.r.iy = 1.0f / b.y;
-			t.r.iz = 1.0f / b.z;
-		}
+		t.with = quad_ray(a, b, hasWide, t.r);
+		if (__builtin_expect(t.with != kFast, 0)) divide(b, t.r);
 		ray = index;
 		t.ref = 0u;
 		t.sp = 0;
@@ -1561,7 +1584,11 @@ struct LaneTracer {
 		t.load(active, kBatch ? wide : P.wide, kBatch ? tris : P.tris, w);
 		if (!active) return;
 		bool occluded;
-		if (t.template advance<kAny>(w, kBatch ? P.descs[batch].nodes : P.nodes, isAny(), stack, occluded)) {
+		const float4* nodes = kBatch ? P.descs[batch].nodes : P.nodes;
+		const bool ended = __builtin_expect(ballot(t.with != kFast) != 0ull, 0)
+		                       ? t.template advance<kAny, true>(w, nodes, isAny(), stack, occluded)
+		                       : t.template advance<kAny, false>(w, nodes, isAny(), stack, occluded);
+		if (ended) {
 			quad_result<kBatch, kTrack, kClock>(P, ray, batch, t.c, isAny(), occluded);
 			ray = kInvalid;
 		}
@@ -1644,7 +1671,7 @@ __device__ __forceinline__ void lane_trace(const QuadArgs& P, uint32_t* lds)
 		Q.q.wide = P.descs[0].wide;
 		Q.q.tris = P.descs[0].tris;
 	}
-	Q.someExact = ballot(Q.q.exact != 0u) != 0ull;
+	Q.slow = ballot(Q.q.with != kFast) != 0ull;
 	while (ballot(Q.q.ray != kInvalid) != 0ull) Q.step();
 }
 
@@ -1722,7 +1749,7 @@ __device__ __forceinline__ bool packet_trace(const float4* __restrict__ wide,
 	while (ballot(on) != 0ull) {
 		float4 w[7];
 		t.load(on, wide, tris, w);
-		if (on) on = !t.template advance<kAnyHit ? 1 : 0>(w, nodes, kAnyHit, stack, occluded);
+		if (on) on = !t.template advance<kAnyHit ? 1 : 0, false>(w, nodes, kAnyHit, stack, occluded);
 	}
 	return occluded;
 }
@@ -1820,9 +1847,9 @@ __global__ __launch_bounds__(kPacketBlock, 5) void k_shade_trace(
 // results wins, the lower instance index on equal t. With `hits` holding a static-scene result on
 // entry (seeded), that result counts as instance -1: an instance must be strictly closer.
 
-// Ray (a, b) in an instance's object space; false if it walks the binary nodes (quad_ray).
-__device__ __forceinline__ bool object_ray(const DevInstance& in, const float4 a, const float4 b,
-                                           dev::Ray& r)
+// Ray (a, b) in an instance's object space; what its boxes are decided with.
+__device__ __forceinline__ uint32_t object_ray(const DevInstance& in, const float4 a, const float4 b,
+                                               dev::Ray& r)
 {
 	const float* A = in.worldToObject;
 	float o[3], d[3];
@@ -1833,13 +1860,10 @@ __device__ __forceinline__ bool object_ray(const DevInstance& in, const float4 a
 		float q = A[4 * k] * b.x + A[4 * k + 1] * b.y;
 		d[k] = q + A[4 * k + 2] * b.z;
 	}
-	const bool fast = quad_ray(make_float4(o[0], o[1], o[2], a.w), make_float4(d[0], d[1], d[2], b.w), r);
-	if (!fast) {
-		r.ix = 1.0f / d[0];
-		r.iy = 1.0f / d[1];
-		r.iz = 1.0f / d[2];
-	}
-	return fast;
+	const float4 dir = make_float4(d[0], d[1], d[2], b.w);
+	const uint32_t with = quad_ray(make_float4(o[0], o[1], o[2], a.w), dir, in.wide != in.tris, r);
+	if (with != kFast) divide(dir, r);
+	return with;
 }
 
 // The kernel is a per-lane state machine over persistent waves. The top tree has wide nodes too, so a
@@ -1937,12 +1961,8 @@ __global__ __launch_bounds__(kBlock, 5) void k_trace_instances(
 						seededHit = false;
 					}
 				}
-				t.exact = !(quad_ray(a, b, t.r) && topWide != top);
-				if (__builtin_expect(t.exact, 0)) {
-					t.r.ix = 1.0f / b.x;
-					t.r.iy = 1.0f / b.y;
-					t.r.iz = 1.0f / b.z;
-				}
+				t.with = quad_ray(a, b, topWide != top, t.r);
+				if (__builtin_expect(t.with != kFast, 0)) divide(b, t.r);
 				if (!kAnyHit) t.r.tMax = next_up(t.r.tMax);
 				t.c = Closest{kInvalid, kAnyHit ? FLT_MAX : next_up(best.t), FLT_MAX, FLT_MAX};
 				t.floor = 0;
@@ -1974,7 +1994,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_trace_instances(
 				nodes = in.nodes;
 				tris = in.tris;
 				wide = in.wide;
-				t.exact = !(object_ray(in, a, b, t.r) && wide != tris);
+				t.with = object_ray(in, a, b, t.r);
 				t.ref = 0u;
 				t.floor = t.sp;
 				t.c = Closest{kInvalid, FLT_MAX, FLT_MAX, FLT_MAX};
@@ -1986,7 +2006,13 @@ __global__ __launch_bounds__(kBlock, 5) void k_trace_instances(
 		float4 w[7];
 		t.load(walks, wide, tris, w);
 		bool occluded;
-		if (walks && t.template advance<kAnyHit ? 1 : 0>(w, nodes, kAnyHit, stack, occluded)) {
+		bool ended = false;
+		if (__builtin_expect(ballot(walks && t.with != kFast) != 0ull, 0)) {
+			if (walks) ended = t.template advance<kAnyHit ? 1 : 0, true>(w, nodes, kAnyHit, stack, occluded);
+		} else if (walks) {
+			ended = t.template advance<kAnyHit ? 1 : 0, false>(w, nodes, kAnyHit, stack, occluded);
+		}
+		if (ended) {
 			leave = true;
 			if (kAnyHit && occluded) {
 				inLight[ray] = 0;

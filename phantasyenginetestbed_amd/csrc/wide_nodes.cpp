@@ -35,13 +35,25 @@ struct Slot {
 	const float* box;
 	uint32_t ref;    // leaf: the finished reference; inner: the binary node's index
 	bool leaf;
-	float area;      // half surface area, of inner slots
+	float area;      // half surface area of an inner slot that may be opened, else negative
 };
 
 float halfArea(const float* b)
 {
 	const float x = b[3] - b[0], y = b[4] - b[1], z = b[5] - b[2];
 	return x * y + y * z + z * x;
+}
+
+// Whether a wide node may hold the children of binary node `nd` in place of it, whose box is `b`: no ray
+// passes a child's box that does not pass b (wide_nodes.hpp: flat boxes).
+bool mayOpen(const PhxBVHNode& nd, const float* b)
+{
+	for (int c = 0; c < 2; c++)
+		for (int k = 1; k < 3; k++) {
+			const float* f = nd.fData + 6 * c;
+			if (f[k] == f[k + 3] && f[k] == b[k + 3] && b[k] < b[k + 3]) return false;
+		}
+	return true;
 }
 
 // The slots of binary node `node` in castRay's order (see wide_nodes.hpp); returns how many (2).
@@ -59,7 +71,7 @@ int expand(const PhxBVHNode* nodes, uint32_t node, Slot out[2])
 	for (int c = 1; c >= 0; c--)
 		if (nd.iData[2 + c] == 0) {
 			const float* b = nd.fData + 6 * c;
-			out[k++] = Slot{b, uint32_t(nd.iData[c]), false, halfArea(b)};
+			out[k++] = Slot{b, uint32_t(nd.iData[c]), false, mayOpen(nodes[nd.iData[c]], b) ? halfArea(b) : -1.0f};
 		}
 	return k;
 }
@@ -72,7 +84,7 @@ int collapse(const PhxBVHNode* nodes, uint32_t root, Slot s[4])
 	while (k < 4) {
 		int best = -1;
 		for (int i = 0; i < k; i++)
-			if (!s[i].leaf && (best < 0 || s[i].area > s[best].area)) best = i;
+			if (!s[i].leaf && s[i].area >= 0.0f && (best < 0 || s[i].area > s[best].area)) best = i;
 		if (best < 0) break;
 		Slot two[2];
 		expand(nodes, s[best].ref, two);
@@ -135,7 +147,8 @@ std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint
 			const Slot& b = s[rs[j].first + 1];
 			for (int k = 0; k < 3; k++) {
 				out[0].slot[j].min[k] = std::min(a.box[k], b.box[k]);
-				out[0].slot[j].max[k] = std::max(a.box[k + 3], b.box[k + 3]);
+				// (A float more: flat at the maximum, a leaf may be passed by a ray that does not pass there.)
+				out[0].slot[j].max[k] = std::nextafter(std::max(a.box[k + 3], b.box[k + 3]), HUGE_VALF);
 			}
 		}
 		out.push_back(emptyNode());

@@ -6,16 +6,21 @@
 //   - castRay's order does not depend on the ray: at a node, the leaf children are tested (left,
 //     then right), then the right inner child's subtree, then the left one's. The slots of a wide
 //     node are kept in that order, so taking the slots in order is castRay's order;
-//   - every child box lies inside its parent's (checked here). For a ray without NaN slab values
-//     rounding is monotonic, so a child that passes the box predicate at some closest t implies
-//     that its ancestors passed theirs at the larger t of that earlier moment: the binary node
-//     decisions that a wide node leaves out can never have been negative;
+//   - every child box lies inside its parent's (checked here), and for a ray with an origin within 2^126
+//     a child that passes the box predicate at some closest t implies that its ancestors passed theirs at
+//     the larger t of that earlier moment: the binary node decisions that a wide node leaves out can never
+//     have been negative. Without NaN slab values, because rounding is monotonic. With them (0 * inf: a
+//     direction component of zero, the origin on a plane of the box) castRay's min and max, which return
+//     their first operand, reject the box where the axis is x, or the plane the maximum and the box not
+//     flat there, and ignore the axis otherwise. Inside a box that is rejected so, only a box that is flat
+//     at that maximum, in y or z, is not rejected too; a binary node with such a child is not left out.
+//     (A NaN component makes every box's values of its axis NaN.)
 //   - a leaf is decided with the closest t it would be decided with by castRay: its entry distance
 //     is kept with the pending slot and compared when the slot is taken. Two leaves of one parent
 //     are decided together, before either is tested (kWidePair).
 // Trees where this does not hold (bounds outside +-2^126 or NaN, child boxes that are inverted or
 // stick out of their parent, more than kWideMaxPending slots pending at once) get no wide nodes
-// and are traversed binary, as rays with NaN slab values are.
+// and are traversed binary, as rays with origins beyond 2^126 are.
 #pragma once
 
 #include <cstdint>

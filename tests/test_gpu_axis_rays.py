@@ -1,0 +1,145 @@
+"""Rays with zero, negative-zero, infinite and NaN direction components and origins on the boxes' planes:
+through every kind of cast equal to the oracle bit for bit, and not far slower than rays beside them."""
+import time
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from phantasyenginetestbed_amd import phx
+from test_wide_nodes import axis_rays, lattice, scene
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ["fixture hf32", "tiny 1", "tiny 3", "random 4000", "twice 500", "terrain 60"]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = phx.Context(0)
+    yield c
+    c.destroy()
+
+
+def mixed(nodes, n, seed, share):
+    """axis_rays, a share of them with all components of a camera's; some origins beyond 2^126."""
+    rays, rng = axis_rays(nodes, n, seed), np.random.default_rng(seed)
+    plain = rng.random(n) < share
+    d = rng.normal(size=(n, 3)).astype(np.float32)
+    rays["d"] = np.where(plain[:, None], d, rays["d"])
+    rays["o"][rng.random(n) < 0.002, 1] = np.float32(2e38)
+    return rays
+
+
+@pytest.mark.parametrize("share", [0.0, 0.5, 0.99])
+@pytest.mark.parametrize("flat", [False, True], ids=["", "lattice"])
+@pytest.mark.parametrize("name", NAMES)
+def test_casts(ctx, name, flat, share):
+    nodes, tris, _ = scene(name)
+    if flat:
+        nodes = lattice(nodes, 2)
+    rays = mixed(nodes, 30011, 7, share)
+    n = len(rays)
+    hits, lit = O.cast_closest(nodes, tris, rays), O.cast_anyhit(nodes, tris, rays)
+    s = ctx.upload_scene(nodes, tris)
+    rb, hb, lb = ctx.alloc(32 * n).upload(rays), ctx.alloc(16 * n), ctx.alloc(n)
+    plan = phx.Plan(ctx, [(s, rb.ptr, hb.ptr, n, phx.BATCH_CLOSEST), (s, rb.ptr, lb.ptr, n, phx.BATCH_ANYHIT)])
+    try:
+        for kernel in (0, phx.KERNEL_ONE_RAY_PER_LANE, phx.KERNEL_PACKET):
+            assert ctx.cast_closest(s, rays, kernel).tobytes() == hits.tobytes()
+            assert (ctx.cast_anyhit(s, rays, kernel) == lit).all()
+            assert ctx.cast_closest(s, rays[:999], kernel).tobytes() == hits[:999].tobytes()
+        ctx.cast_closest_noalloc(s, rb.ptr, n, hb.ptr)
+        assert hb.download(phx.HIT, n).tobytes() == hits.tobytes()
+        ctx.cast_closest_timeline(s, rb.ptr, n, hb.ptr)
+        assert hb.download(phx.HIT, n).tobytes() == hits.tobytes()
+        hb.upload(np.zeros(n, phx.HIT))
+        plan.launch()
+        assert hb.download(phx.HIT, n).tobytes() == hits.tobytes()
+        assert (lb.download(np.uint8, n) == lit).all()
+    finally:
+        plan.release()
+        for b in (rb, hb, lb):
+            b.free()
+        s.release()
+
+
+@pytest.mark.parametrize("static", [False, True])
+@pytest.mark.parametrize("flat", [False, True], ids=["", "lattice"])
+def test_instances(ctx, flat, static):
+    """Placed by axis-parallel transforms, so that rays keep their zero components in the meshes."""
+    rng = np.random.default_rng(5)
+    meshes, placed, prepared = [], [], []
+    for name in ("fixture hf32", "random 4000", "tiny 1"):
+        nodes, tris, _ = scene(name)
+        meshes.append((lattice(nodes, 2) if flat else nodes, tris))
+    scenes = [ctx.upload_scene(*m) for m in meshes]
+    for k in range(24):
+        m = np.zeros((3, 4), np.float32)
+        m[np.arange(3), rng.permutation(3)] = rng.choice([-1.0, 0.5, 2.0], 3)
+        m[:, 3] = rng.integers(-3, 4, 3)
+        placed.append((scenes[k % 3], m))
+        prepared.append((*meshes[k % 3], m))
+    rays = mixed(meshes[0][0], 20011, 9, 0.3)
+    rays["o"][::2] = np.round(rays["o"][::2] * 4) / 4
+    ground = scene("terrain 60")[:2] if static else None
+    g = ctx.upload_scene(*ground) if static else None
+    iset = phx.InstanceSet(ctx, placed)
+    try:
+        ref, ref_ids = O.cast_instances(prepared, rays, ground)[:2]
+        hits, ids = iset.cast_closest(rays, g)
+        assert hits.tobytes() == ref.tobytes() and (ids == ref_ids).all()
+        assert (iset.cast_anyhit(rays, g) == O.cast_instances(prepared, rays, ground, anyhit=True)).all()
+    finally:
+        iset.release()
+        for s in scenes + ([g] if g else []):
+            s.release()
+
+
+@pytest.mark.parametrize("kind", ["closest", "anyhit", "plan"])
+def test_rays_with_a_zero_component_cost_what_their_neighbours_do(ctx, kind):
+    """Against the same rays tilted by 1e-4: their steps are the same ones, with 12 instructions more each
+    (of over 100), so a third more time is allowed; on the binary nodes they took up to twice as long."""
+    t, _ = phx.heightfield_boxes(362, 500, 3)
+    b = phx.BVH(t)
+    n = 1 << 19
+    rng = np.random.default_rng(1)
+    rays = np.zeros(n, phx.RAY)
+    rays["o"] = rng.uniform((0, -0.1, 0), (1, 0.3, 1), (n, 3))
+    a = rng.uniform(0, 2 * np.pi, n)
+    rays["d"][:, 0], rays["d"][:, 2] = np.cos(a), np.sin(a)
+    rays["tmin"], rays["tmax"] = np.float32(1e-4), np.float32(phx.FLT_MAX)
+    tilted = rays.copy()
+    tilted["d"][:, 1] = np.where(rng.random(n) < 0.5, np.float32(1e-4), np.float32(-1e-4))
+    s = ctx.upload_scene(b.nodes, b.tris)
+    out = ctx.alloc(16 * n)
+    bufs, calls, plans = [], [], []
+    for r in (rays, tilted):
+        rb = ctx.alloc(32 * n).upload(r)
+        bufs.append(rb)
+        if kind == "closest":
+            calls.append(lambda rb=rb: ctx.cast_closest_device(s, rb.ptr, n, out.ptr, asynchronous=True))
+        elif kind == "anyhit":
+            calls.append(lambda rb=rb: ctx.cast_anyhit_device(s, rb.ptr, n, out.ptr, asynchronous=True))
+        else:
+            plans.append(phx.Plan(ctx, [(s, rb.ptr, out.ptr, n, phx.BATCH_CLOSEST)]))
+            calls.append(lambda p=plans[-1]: p.launch(asynchronous=True))
+    try:
+        best = [1e9, 1e9]
+        for _ in range(9):
+            for i, call in enumerate(calls):
+                call()
+                ctx.synchronize()
+                t0 = time.perf_counter()
+                for _ in range(5):
+                    call()
+                ctx.synchronize()
+                best[i] = min(best[i], (time.perf_counter() - t0) / 5)
+        print(f"[gpu] {kind}: {best[0] * 1e6:.0f} us, tilted {best[1] * 1e6:.0f} us")
+        assert best[0] <= best[1] * 4 / 3
+    finally:
+        for p in plans:
+            p.release()
+        for x in [*bufs, out]:
+            x.free()
+        s.release()

@@ -104,3 +104,61 @@ def test_trees_with_unfit_boxes_get_no_wide_nodes(lib, spoil):
     rays = random_rays(10, 1)
     assert walk(lib, fx["nodes"], fx["tris"], rays)[0] > 0
     assert walk(lib, nodes, fx["tris"], rays)[0] == 0
+
+
+# ---- rays with which slab values may be NaN -----------------------------------------------------
+
+def lattice(nodes, seed):
+    """The tree with its boxes widened to multiples of 1/8, so that many planes coincide, and every third
+    leaf's box flattened onto a face of the box around it."""
+    n, rng = nodes.copy(), np.random.default_rng(seed)
+    f = n["f"].reshape(-1, 2, 2, 3)
+    f[:, :, 0], f[:, :, 1] = np.floor(f[:, :, 0] * 8) / 8, np.ceil(f[:, :, 1] * 8) / 8
+    around = {0: np.array([f[0, :, 0].min(0), f[0, :, 1].max(0)])}
+    for i in range(len(n)):  # parents come first
+        for c in range(2):
+            if n["i"][i, 2 + c] == 0:
+                around[int(n["i"][i, c])] = f[i, c].copy()
+            elif rng.random() < 1 / 3:
+                k, side = rng.integers(0, 3), rng.integers(0, 2)
+                f[i, c, :, k] = around[i][side, k]
+    return n
+
+
+def axis_rays(nodes, n, seed):
+    """Directions with zero, negative-zero, NaN and infinite components; origins on the boxes' planes."""
+    rng = np.random.default_rng(seed)
+    planes = nodes["f"].reshape(-1, 3)
+    rays = np.zeros(n, phx.RAY)
+    lo, hi = planes.min(0), planes.max(0)
+    rays["o"] = rng.uniform(lo - 0.1, hi + 0.1, (n, 3))
+    on = rng.random((n, 3)) < 0.7
+    picked = np.stack([planes[rng.integers(0, len(planes), n), k] for k in range(3)], 1)
+    rays["o"] = np.where(on, picked, rays["o"])
+    d = rng.normal(size=(n, 3)).astype(np.float32)
+    zero = rng.random((n, 3)) < 0.5
+    d[zero] = np.where(rng.random(zero.sum()) < 0.5, np.float32(0), np.float32(-0.0))
+    odd = rng.random((n, 3)) < 0.01
+    d[odd] = rng.choice(np.array([np.nan, np.inf, -np.inf, 1e-41], np.float32), odd.sum())
+    rays["d"] = d
+    rays["tmin"] = np.where(rng.random(n) < 0.5, np.float32(0), np.float32(-1))
+    rays["tmax"] = np.where(rng.random(n) < 0.5, np.float32(phx.FLT_MAX), rng.uniform(0, 2, n))
+    return rays
+
+
+@pytest.mark.parametrize("seed", range(4))
+@pytest.mark.parametrize("flat", [False, True], ids=["", "lattice"])
+@pytest.mark.parametrize("name", ["fixture rand2k", "fixture hf32", "tiny 1", "tiny 2", "tiny 3", "tiny 5",
+                                  "random 4000", "long 600", "twice 500", "terrain 60"])
+def test_slot_order_gives_castray_hits_on_box_planes(lib, name, flat, seed):
+    """With the slab test as castRay computes it (first operands where values are NaN), the wide nodes give
+    castRay's hits for every ray with an origin within 2^126."""
+    nodes, tris, _ = scene(name)
+    if flat:
+        nodes = lattice(nodes, seed)
+    rays = axis_rays(nodes, 20000, seed)
+    k, hits, lit, deepest = walk(lib, nodes, tris, rays, 64)
+    assert 0 < k and deepest <= CAPACITY
+    ref = O.cast_closest(nodes, tris, rays)
+    assert hits.tobytes() == ref.tobytes(), int((hits["tri"] != ref["tri"]).sum())
+    assert (lit == O.cast_anyhit(nodes, tris, rays)).all()
