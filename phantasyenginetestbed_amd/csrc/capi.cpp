@@ -578,7 +578,7 @@ static phx_status phx_scene_upload_impl(PhxContext* ctx, const PhxBVHNode* nodes
 	}
 	st = uploadArray(ctx, s->nodes, nodes, numNodes, s->bytes);
 	if (st == PHX_OK) {
-		const std::vector<WideNode> wide = buildWide(nodes, numNodes, kWideTop);
+		const std::vector<WideNode> wide = buildWide(nodes, numNodes, kWideTop, &s->loose);
 		st = uploadArray(ctx, s->wide, wide.data(), wide.size(), s->bytes);
 		if (st == PHX_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
 			st = fail(PHX_ERR_HIP, "phx_scene_upload: wide node upload failed");

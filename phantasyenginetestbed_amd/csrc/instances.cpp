@@ -231,6 +231,7 @@ static phx_status phx_instances_build_impl(PhxContext* ctx, const PhxInstance* i
 			            "or non-finite transform", i);
 		d.wide = in.mesh->wide ? reinterpret_cast<const float4*>(in.mesh->wide)
 		                       : reinterpret_cast<const float4*>(in.mesh->tris);
+		d.with = sceneWith(in.mesh->wide, in.mesh->loose);
 		d.nodes = reinterpret_cast<const float4*>(in.mesh->nodes);
 		d.tris = reinterpret_cast<const float4*>(in.mesh->tris);
 		d.datas = in.mesh->datas;

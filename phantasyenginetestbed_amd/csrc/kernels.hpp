@@ -18,7 +18,13 @@ struct SceneView {
 	uint32_t numNodes;
 	uint32_t numTris;
 	const WideNode* wide;   // four-wide nodes (wide_nodes.hpp), or null: binary traversal only
+	bool loose;             // they have kWideLoose slots
 };
+
+// What a ray's boxes are decided with: slab_fast on the wide nodes, slab (trace_device.hpp) on them, or
+// slab on the binary ones. The rays of a scene take at least sceneWith.
+constexpr uint32_t kFast = 0, kSlab = 1, kBinary = 2;
+inline uint32_t sceneWith(const WideNode* wide, bool loose) { return !wide ? kBinary : loose ? kSlab : kFast; }
 
 // Material textures of a scene: one device arena holding the linearisation table, the
 // descriptors and the texels (rows packed to width * bpp bytes, each image 16-byte aligned).
@@ -93,6 +99,8 @@ struct DevInstance {
 	float worldToObject[12];
 	uint32_t index;    // the instance's position in the caller's list (ties: lower wins)
 	uint32_t numTris;  // triangles of the mesh (hit records check indices against it)
+	uint32_t with;     // the mesh's sceneWith
+	uint32_t pad;
 };
 
 // Closest hit (inLight == nullptr; hits and optionally instOut written) or any hit (inLight) of
@@ -140,7 +148,7 @@ struct BatchDesc {
 	const float4* rays;
 	void* out;                // PhxRayHit* (closest) or uint8_t* (any hit)
 	uint32_t count;
-	uint32_t kind;            // 0 closest hit, 1 any hit
+	uint32_t kind;            // 0 closest hit, 1 any hit; + 2 x the scene's sceneWith
 };
 static_assert(sizeof(BatchDesc) == 48, "BatchDesc layout");
 

@@ -107,6 +107,7 @@ struct PhxScene {
 	PhxContext* ctx = nullptr;
 	PhxBVHNode* nodes = nullptr;
 	phx::WideNode* wide = nullptr;  // four-wide nodes, null if the tree cannot have them
+	bool loose = false;             // they have kWideLoose slots
 	PhxTriangleVertices* tris = nullptr;
 	PhxTriangleData* datas = nullptr;
 	PhxMaterial* materials = nullptr;
@@ -167,7 +168,7 @@ void dropContext(PhxContext* ctx);
 
 inline SceneView view(const PhxScene* s)
 {
-	return SceneView{s->nodes, s->tris, s->numNodes, s->numTris, s->wide};
+	return SceneView{s->nodes, s->tris, s->numNodes, s->numTris, s->wide, s->loose};
 }
 
 // One batch of a fused launch on scene `s`.
@@ -177,7 +178,7 @@ inline BatchDesc batchDesc(const PhxScene* s, const PhxRayIn* rays, void* out, u
 	const float4* tris = reinterpret_cast<const float4*>(s->tris);
 	return BatchDesc{s->wide ? reinterpret_cast<const float4*>(s->wide) : tris,
 	                 reinterpret_cast<const float4*>(s->nodes), tris,
-	                 reinterpret_cast<const float4*>(rays), out, count, kind};
+	                 reinterpret_cast<const float4*>(rays), out, count, kind + 2u * sceneWith(s->wide, s->loose)};
 }
 
 inline TraceLaunch traceLaunch(const PhxContext* ctx, uint32_t flags, bool anyhit)

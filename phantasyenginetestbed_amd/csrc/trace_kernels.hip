@@ -655,7 +655,7 @@ __device__ __forceinline__ void packet_leaf(const float4* __restrict__ tris, uin
 // leaf slot that was pushed is decided again when it is taken, from its box in the node (closest
 // hit; entry word 1 names node and slot). Any hit does not depend on order: all its leaf slots are
 // tested at once.
-template <bool kAnyHit, class Leave>
+template <bool kAnyHit, bool kLoose, class Leave>
 __device__ __forceinline__ void packet_wide(const float4* __restrict__ wide,
                                             const float4* __restrict__ tris, const dev::Ray& r,
                                             bool active, Closest& c, bool& occluded,
@@ -668,7 +668,7 @@ __device__ __forceinline__ void packet_wide(const float4* __restrict__ wide,
 	uint64_t mask = __ballot(active);
 	while (true) {
 		const bool in = ((mask >> lane) & 1ull) != 0;
-		const WideWords n = load_wide(wide, cur);
+		const WideWords n = load_wide(wide, kLoose ? cur & kWideIndex : cur);
 		const float lim = kAnyHit ? r.tMax : dev::min_first(r.tMax, c.t);
 		WideVisit v = decide_wide(r, n, lim);
 		const uint32_t refs[4] = {
@@ -753,7 +753,8 @@ __device__ __forceinline__ void packet_wide(const float4* __restrict__ wide,
 			if (__ballot(on2) != 0ull) packet_leaf<false>(tris, ref2 & kWideIndex, r, on2, c, occluded);
 		}
 		if (mask == 0ull) break;
-		if (__popcll(mask) < kPacketLanes && ++steps == kPacketSteps) {
+		// (In loose trees packets do not part: lanes by themselves would need the slow steps of LaneWalk.)
+		if (!kLoose && __popcll(mask) < kPacketLanes && ++steps == kPacketSteps) {
 			// Each lane goes on by itself with its part of the stack, bottom entry first, and the node.
 			int n = 0;
 			for (int e = 0; e < sp; e++) {
@@ -873,16 +874,11 @@ __device__ __forceinline__ float recip_wave(float a)
 	return f;
 }
 
-// What a ray's boxes are decided with.
-constexpr uint32_t kFast = 0;    // slab_fast, on the wide nodes
-constexpr uint32_t kSlab = 1;    // slab, on the wide nodes
-constexpr uint32_t kBinary = 2;  // slab, on the binary nodes
-
 // Sets r up from its record. A direction component outside the fast reciprocal's range (zero among them)
 // takes the division and slab, with which NaN slab values come out as castRay's; an origin beyond 2^126
 // the binary nodes (wide_nodes.hpp). Rays with a zero component are ordinary ones (probes, a sun
 // overhead): on the binary nodes 1,048,576 of them straight up took 0.91 ms, on the wide ones 0.52 ms.
-__device__ __forceinline__ uint32_t quad_ray(const float4 a, const float4 b, bool hasWide, dev::Ray& r)
+__device__ __forceinline__ uint32_t quad_ray(const float4 a, const float4 b, uint32_t sceneWith, dev::Ray& r)
 {
 	r.ox = a.x, r.oy = a.y, r.oz = a.z, r.tMin = a.w;
 	r.dx = b.x, r.dy = b.y, r.dz = b.z, r.tMax = b.w;
@@ -891,7 +887,8 @@ __device__ __forceinline__ uint32_t quad_ray(const float4 a, const float4 b, boo
 	r.iz = dev::recip_newton(b.z);
 	auto within = [](float x) { return fabsf(x) >= 0x1p-126f && fabsf(x) < 0x1p126f; };
 	const bool near = fabsf(a.x) <= 0x1p126f && fabsf(a.y) <= 0x1p126f && fabsf(a.z) <= 0x1p126f;
-	return !(near && hasWide) ? kBinary : within(b.x) && within(b.y) && within(b.z) ? kFast : kSlab;
+	const uint32_t with = !near ? kBinary : within(b.x) && within(b.y) && within(b.z) ? kFast : kSlab;
+	return with > sceneWith ? with : sceneWith;
 }
 __device__ __forceinline__ void divide(const float4 b, dev::Ray& r)
 {
@@ -909,8 +906,9 @@ struct QuadArgs {
 	const float4* rays;
 	void* out;                  // uint4 hits or uint8_t inLight flags
 	uint32_t n;                 // rays of the launch
+	uint32_t with;              // what the scene's rays are decided with at least
 	uint32_t window;            // rays a wave claims at a time (at most 64)
-	uint32_t refill;       // idle rays of a wave before it takes new ones
+	uint32_t refill;            // idle rays of a wave before it takes new ones
 	uint32_t* work;             // kCounters window counters, then the retirement counters
 	U32x2* spill;
 	unsigned long long* clock;  // completion clock per ray, and the earliest block start in word n
@@ -1029,16 +1027,16 @@ struct QuadTracer {
 	}
 
 	// Sets this quad up for ray `ray` with the record (a, b).
-	__device__ __forceinline__ void set(uint32_t ray, const float4 a, const float4 b, bool hasWide)
+	__device__ __forceinline__ void set(uint32_t ray, const float4 a, const float4 b, uint32_t sceneWith)
 	{
-		q.with = quad_ray(a, b, hasWide, q.r);
+		q.with = quad_ray(a, b, sceneWith, q.r);
 		if (__builtin_expect(ballot(q.with != kFast) != 0ull, 0)) divide(b, q.r);
 		q.ray = ray;
 	}
 	// Starts a ray of a single cast.
 	__device__ __forceinline__ void start(uint32_t ray, const float4 a, const float4 b)
 	{
-		set(ray, a, b, P.wide != P.tris);
+		set(ray, a, b, P.with);
 		q.node = 0u;
 		q.nodeIn = -INFINITY;
 		q.leaf = false;
@@ -1052,17 +1050,17 @@ struct QuadTracer {
 	{
 		const float4* rays = P.rays;
 		uint32_t at = ray;
-		bool hasWide = P.wide != P.tris;
+		uint32_t with = P.with;
 		if (kBatch) {
 			at = ray - P.offsets[q.batch];
 			const BatchDesc d = P.descs[q.batch];
 			rays = d.rays;
 			q.wide = d.wide;
 			q.tris = d.tris;
-			q.any = d.kind != 0u;
-			hasWide = d.wide != d.tris;
+			q.any = d.kind & 1u;
+			with = d.kind >> 1;
 		}
-		set(ray, as_global(rays)[2 * size_t(at)], as_global(rays)[2 * size_t(at) + 1], hasWide);
+		set(ray, as_global(rays)[2 * size_t(at)], as_global(rays)[2 * size_t(at) + 1], with);
 	}
 
 	// Expands a binary node: lanes 0 and 1 decide its children as castRay does, and what is visited is
@@ -1105,11 +1103,12 @@ struct QuadTracer {
 		const float4* pn;
 		if (kBig) {
 			pl = tris + 3u * size_t(tri);
-			pn = wide + 8u * size_t(node) + 2u * l;
+			pn = wide + 8u * size_t(node & kWideIndex) + 2u * l;
 		} else {
 			uint32_t tri3;
 			asm("v_lshl_add_u32 %0, %1, 1, %1" : "=v"(tri3) : "v"(tri));  // (a 32-bit multiply takes four times as long)
 			pl = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(tris) + (tri3 << 4));
+			// (a kWideLoose in the reference is shifted out)
 			pn = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(wide) + ((node << 7) + (l << 5)));
 		}
 		const float4 p0 = as_global(pl)[0], e1 = as_global(pl)[1], e2 = as_global(pl)[2];
@@ -1149,6 +1148,8 @@ struct QuadTracer {
 		dev::slab_fast(q.r, lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, tIn, tOut);
 		if (__builtin_expect(slow, 0)) {  // (all of it in one branch that fast rays' waves do not take)
 			dev::slab(q.r, lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, tIn, tOut);
+			if (int32_t(__float_as_uint(lo.w)) >= int32_t(kWideLoose))  // decided now, and not to be again
+				tIn = tOut >= tIn && tIn < lim ? -INFINITY : INFINITY;
 			if (q.with == kBinary && q.node != kInvalid && !more) {
 				expand_binary(lim);
 				q.node = kInvalid;
@@ -1420,7 +1421,16 @@ struct LaneWalk {
 			const bool p0 = v.pass[0], p1 = v.pass[1], p2 = v.pass[2], p3 = v.pass[3];
 			uint32_t r0 = __float_as_uint(w[0].w), r1 = __float_as_uint(w[2].w);
 			uint32_t r2 = __float_as_uint(w[4].w);
-			const uint32_t r3 = __float_as_uint(w[6].w);
+			uint32_t r3 = __float_as_uint(w[6].w);
+			if (kSlow) {
+				auto inner = [](uint32_t& at, float& tIn) {
+					if (int32_t(at) >= int32_t(kWideLoose)) at &= kWideIndex, tIn = -INFINITY;
+				};
+				inner(r0, v.tIn[0]);
+				inner(r1, v.tIn[1]);
+				inner(r2, v.tIn[2]);
+				inner(r3, v.tIn[3]);
+			}
 			r0 = p1 ? r0 : r0 & ~kWidePair;
 			r1 = p2 ? r1 : r1 & ~kWidePair;
 			r2 = p3 ? r2 : r2 & ~kWidePair;
@@ -1554,7 +1564,7 @@ struct LaneTracer {
 	}
 	__device__ __forceinline__ void start(uint32_t index)
 	{
-		bool hasWide = P.wide != P.tris;
+		uint32_t with = P.with;
 		if (kBatch) {
 			batch = windowBatch;
 			BatchDesc d = desc;
@@ -1564,12 +1574,12 @@ struct LaneTracer {
 			}
 			wide = d.wide;
 			tris = d.tris;
-			any = d.kind != 0u;
-			hasWide = d.wide != d.tris;
+			any = (d.kind & 1u) != 0u;
+			with = d.kind >> 1;
 		}
 		const F32x4 sa = staged[index - first], sb = staged[64u + index - first];
 		const float4 a = make_float4(sa.x, sa.y, sa.z, sa.w), b = make_float4(sb.x, sb.y, sb.z, sb.w);
-		t.with = quad_ray(a, b, hasWide, t.r);
+		t.with = quad_ray(a, b, with, t.r);
 		if (__builtin_expect(t.with != kFast, 0)) divide(b, t.r);
 		ray = index;
 		t.ref = 0u;
@@ -1722,7 +1732,7 @@ struct PacketLeave {
 };
 
 // Traces the wave's rays t.r of the `active` lanes: t.c, or for any hit whether one was hit.
-template <bool kAnyHit>
+template <bool kAnyHit, bool kLoose>
 __device__ __forceinline__ bool packet_trace(const float4* __restrict__ wide,
                                              const float4* __restrict__ nodes,
                                              const float4* __restrict__ tris, LaneWalk& t, bool active,
@@ -1739,7 +1749,7 @@ __device__ __forceinline__ bool packet_trace(const float4* __restrict__ wide,
 	PrivateStack<kPacketRows, kMaxPending> stack = {column, deep};
 	bool on = false;
 	t.sp = 0;
-	packet_wide<kAnyHit>(wide, tris, t.r, active, t.c, occluded, PacketLeave{stack, t, on});
+	packet_wide<kAnyHit, kLoose>(wide, tris, t.r, active, t.c, occluded, PacketLeave{stack, t, on});
 	if (ballot(on || t.sp > 0) == 0ull) return occluded;
 	if (!on && t.sp > 0) {
 		const float lim = kAnyHit ? t.r.tMax : dev::min_first(t.r.tMax, t.c.t);
@@ -1754,7 +1764,7 @@ __device__ __forceinline__ bool packet_trace(const float4* __restrict__ wide,
 	return occluded;
 }
 
-template <bool kAnyHit>
+template <bool kAnyHit, bool kLoose>
 __global__ __launch_bounds__(kPacketBlock) void k_packet(const float4* __restrict__ wide,
                                                          const float4* __restrict__ nodes,
                                                          const float4* __restrict__ tris,
@@ -1774,7 +1784,7 @@ __global__ __launch_bounds__(kPacketBlock) void k_packet(const float4* __restric
 	// packet on the binary nodes.)
 	const bool traced = active && (!kAnyHit || t.r.tMin < t.r.tMax);
 	const bool occluded =
-		packet_trace<kAnyHit>(wide, nodes, tris, t, traced, (LdsU2*)(stackLds) + threadIdx.x);
+		packet_trace<kAnyHit, kLoose>(wide, nodes, tris, t, traced, (LdsU2*)(stackLds) + threadIdx.x);
 	if (active) {
 		if (kAnyHit)
 			static_cast<uint8_t*>(out)[i] = occluded ? 0 : 1;
@@ -1794,6 +1804,7 @@ __global__ __launch_bounds__(kPacketBlock) void k_packet(const float4* __restric
 // k_shadow_logic), and a lane without a ray had a dummy one whose zero direction components kept its
 // packet on the binary nodes. A 1080p frame with 8 lights, whose bounce cast runs beside this and now
 // starts before the shading: 1.61 -> 1.43 ms; 333x251 with 2 lights, in row order: 0.33 -> 0.28 ms.
+template <bool kLoose>
 __global__ __launch_bounds__(kPacketBlock, 5) void k_shade_trace(
 	const float4* __restrict__ wide, const float4* __restrict__ nodes,
 	const float4* __restrict__ tris, const float4* __restrict__ info,
@@ -1822,7 +1833,7 @@ __global__ __launch_bounds__(kPacketBlock, 5) void k_shade_trace(
 			LaneWalk t;
 			t.r = dev::make_ray(make_float4(p.x, p.y, p.z, 0.001f),
 			                    make_float4(s.dir.x, s.dir.y, s.dir.z, s.len));
-			occluded = packet_trace<true>(wide, nodes, tris, t, s.ray, (LdsU2*)(stackLds) + threadIdx.x);
+			occluded = packet_trace<true, kLoose>(wide, nodes, tris, t, s.ray, (LdsU2*)(stackLds) + threadIdx.x);
 		}
 		if (hit && !occluded) {
 			c0 = c0 + s.c.x;
@@ -1861,7 +1872,7 @@ __device__ __forceinline__ uint32_t object_ray(const DevInstance& in, const floa
 		d[k] = q + A[4 * k + 2] * b.z;
 	}
 	const float4 dir = make_float4(d[0], d[1], d[2], b.w);
-	const uint32_t with = quad_ray(make_float4(o[0], o[1], o[2], a.w), dir, in.wide != in.tris, r);
+	const uint32_t with = quad_ray(make_float4(o[0], o[1], o[2], a.w), dir, in.with, r);
 	if (with != kFast) divide(dir, r);
 	return with;
 }
@@ -1961,7 +1972,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_trace_instances(
 						seededHit = false;
 					}
 				}
-				t.with = quad_ray(a, b, topWide != top, t.r);
+				t.with = quad_ray(a, b, topWide != top ? kFast : kBinary, t.r);
 				if (__builtin_expect(t.with != kFast, 0)) divide(b, t.r);
 				if (!kAnyHit) t.r.tMax = next_up(t.r.tMax);
 				t.c = Closest{kInvalid, kAnyHit ? FLT_MAX : next_up(best.t), FLT_MAX, FLT_MAX};
@@ -2030,10 +2041,10 @@ __global__ __launch_bounds__(kQuadBlock, kQuadWavesPerSimd) void k_quad(
 	const float4* __restrict__ wide, const float4* __restrict__ nodes,
 	const float4* __restrict__ tris, const float4* __restrict__ rays, void* __restrict__ out,
 	uint32_t n, uint32_t window, uint32_t refill, uint32_t* __restrict__ work,
-	U32x2* __restrict__ spill, unsigned long long* __restrict__ clock)
+	U32x2* __restrict__ spill, unsigned long long* __restrict__ clock, uint32_t with)
 {
 	extern __shared__ uint32_t lds[];
-	const QuadArgs P = {wide, nodes, tris, rays, out, n, window, refill, work, spill, clock,
+	const QuadArgs P = {wide, nodes, tris, rays, out, n, with, window, refill, work, spill, clock,
 	                    nullptr, nullptr, 0u, nullptr, nullptr};
 	quad_trace<kAnyHit ? 1 : 0, kClock, kBig>(P, lds);
 	if (threadIdx.x == 0u) retire_block(work);
@@ -2077,7 +2088,7 @@ __global__ __launch_bounds__(kLaneBlock, 4) void k_trace_batches(
 			blockDone[i] = 0u;
 		}
 	__syncthreads();
-	const QuadArgs P = {nullptr, nullptr, nullptr, nullptr, nullptr, total, window, refill, work,
+	const QuadArgs P = {nullptr, nullptr, nullptr, nullptr, nullptr, total, 0u, window, refill, work,
 	                    spill, nullptr, descs, offsets, numBatches, blockFinish, blockDone};
 	lane_trace<2, true, kTrack, false>(P, lds);
 	__syncthreads();
@@ -2252,8 +2263,8 @@ hipError_t launchClosest(const SceneView& s, const PhxRayIn* rays, uint32_t n, P
 	const float4* r4 = reinterpret_cast<const float4*>(rays);
 	uint4* h4 = reinterpret_cast<uint4*>(hits);
 	if (L.kernel == TraceKernel::Packet && !counters) {
-		hipLaunchKernelGGL(k_packet<false>, dim3(gridFor(n, kPacketBlock)), dim3(kPacketBlock), 0,
-		                   stream, wide, nodes, tris, r4, static_cast<void*>(h4), n);
+		hipLaunchKernelGGL((s.loose ? k_packet<false, true> : k_packet<false, false>), dim3(gridFor(n, kPacketBlock)),
+		                   dim3(kPacketBlock), 0, stream, wide, nodes, tris, r4, static_cast<void*>(h4), n);
 		return hipGetLastError();
 	}
 	// Counters count binary node visits, which the one-ray-per-lane kernel makes.
@@ -2264,14 +2275,14 @@ hipError_t launchClosest(const SceneView& s, const PhxRayIn* rays, uint32_t n, P
 	}
 	if (L.kernel != TraceKernel::Persistent || n > 0x7FFFFFFFu) {
 		hipLaunchKernelGGL(k_closest_simple<false>, dim3(gridFor(n, kBlock)), dim3(kBlock), 0, stream,
-		                   wide, nodes, tris, r4, h4, n, nullptr);
+		                   s.loose ? nullptr : wide, nodes, tris, r4, h4, n, nullptr);
 		return hipGetLastError();
 	}
 	const Shape q = quadShape(L, n);
 	auto kernel = bigScene(s) ? k_quad<false, false, true> : k_quad<false, false, false>;
 	hipLaunchKernelGGL(kernel, dim3(q.grid), dim3(q.block), quad_lds_words(q.block / 64u) * 4u, stream,
 	                   wide ? wide : tris, nodes, tris, r4, static_cast<void*>(h4), n, q.window, q.refill,
-	                   L.work, reinterpret_cast<U32x2*>(L.spill), nullptr);
+	                   L.work, reinterpret_cast<U32x2*>(L.spill), nullptr, sceneWith(s.wide, s.loose));
 	return hipGetLastError();
 }
 
@@ -2288,7 +2299,8 @@ hipError_t launchClosestClock(const SceneView& s, const PhxRayIn* rays, uint32_t
 	hipLaunchKernelGGL(kernel, dim3(q.grid), dim3(q.block), quad_lds_words(q.block / 64u) * 4u, stream,
 	                   wide, nodes, tris, reinterpret_cast<const float4*>(rays),
 	                   static_cast<void*>(hits), n, q.window,
-	                   q.refill, L.work, reinterpret_cast<U32x2*>(L.spill), clock);
+	                   q.refill, L.work, reinterpret_cast<U32x2*>(L.spill), clock,
+	                   sceneWith(s.wide, s.loose));
 	return hipGetLastError();
 }
 
@@ -2332,20 +2344,20 @@ hipError_t launchAnyHit(const SceneView& s, const PhxRayIn* rays, uint32_t n, ui
 	const float4* tris = reinterpret_cast<const float4*>(s.trisPre);
 	const float4* r4 = reinterpret_cast<const float4*>(rays);
 	if (L.kernel == TraceKernel::Packet) {
-		hipLaunchKernelGGL(k_packet<true>, dim3(gridFor(n, kPacketBlock)), dim3(kPacketBlock), 0,
-		                   stream, wide, nodes, tris, r4, static_cast<void*>(inLight), n);
+		hipLaunchKernelGGL((s.loose ? k_packet<true, true> : k_packet<true, false>), dim3(gridFor(n, kPacketBlock)),
+		                   dim3(kPacketBlock), 0, stream, wide, nodes, tris, r4, static_cast<void*>(inLight), n);
 		return hipGetLastError();
 	}
 	if (L.kernel == TraceKernel::Simple || n > 0x7FFFFFFFu) {
 		hipLaunchKernelGGL(k_anyhit_simple<false>, dim3(gridFor(n, kBlock)), dim3(kBlock), 0,
-		                   stream, wide, nodes, tris, r4, inLight, n, nullptr);
+		                   stream, s.loose ? nullptr : wide, nodes, tris, r4, inLight, n, nullptr);
 		return hipGetLastError();
 	}
 	const Shape q = quadShape(L, n);
 	auto kernel = bigScene(s) ? k_quad<true, false, true> : k_quad<true, false, false>;
 	hipLaunchKernelGGL(kernel, dim3(q.grid), dim3(q.block), quad_lds_words(q.block / 64u) * 4u, stream,
 	                   wide ? wide : tris, nodes, tris, r4, static_cast<void*>(inLight), n, q.window, q.refill,
-	                   L.work, reinterpret_cast<U32x2*>(L.spill), nullptr);
+	                   L.work, reinterpret_cast<U32x2*>(L.spill), nullptr, sceneWith(s.wide, s.loose));
 	return hipGetLastError();
 }
 
@@ -2354,7 +2366,8 @@ hipError_t launchShadeTrace(const SceneView& s, const float4* info, const PhxSph
                             uint32_t purpose, float4* img, hipStream_t stream)
 {
 	if (w == 0 || h == 0) return hipSuccess;
-	hipLaunchKernelGGL(k_shade_trace, dim3(gridFor(w * h, kPacketBlock)), dim3(kPacketBlock), 0, stream,
+	hipLaunchKernelGGL((s.loose ? k_shade_trace<true> : k_shade_trace<false>), dim3(gridFor(w * h, kPacketBlock)),
+	                   dim3(kPacketBlock), 0, stream,
 	                   reinterpret_cast<const float4*>(s.wide), reinterpret_cast<const float4*>(s.nodes),
 	                   reinterpret_cast<const float4*>(s.trisPre), info, lights, numLights, w, h, fp,
 	                   purpose, img);

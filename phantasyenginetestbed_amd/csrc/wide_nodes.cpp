@@ -9,22 +9,25 @@
 namespace phx {
 namespace {
 
-// True if the conditions of wide_nodes.hpp on the boxes hold for every node.
-bool eligible(const PhxBVHNode* nodes, uint32_t n)
+// Whether every child box lies within +-2^126 and is not inverted (false for NaN too). `loose` gets a
+// flag per node whose child boxes stick out of its own, or stays empty if there are none.
+bool eligible(const PhxBVHNode* nodes, uint32_t n, std::vector<uint8_t>& loose)
 {
 	for (uint32_t i = 0; i < n; i++) {
 		const PhxBVHNode& nd = nodes[i];
 		for (int c = 0; c < 2; c++) {
 			const float* b = nd.fData + 6 * c;
-			bool good = true;  // false for NaN too
+			bool good = true, inside = true;
 			for (int k = 0; k < 3; k++)
 				good &= std::fabs(b[k]) <= 0x1p126f && std::fabs(b[k + 3]) <= 0x1p126f && b[k] <= b[k + 3];
-			if (good && nd.iData[2 + c] == 0) {
-				const float* f = nodes[nd.iData[c]].fData;
-				for (int k = 0; k < 3; k++)
-					good &= f[k] >= b[k] && f[k + 6] >= b[k] && f[k + 3] <= b[k + 3] && f[k + 9] <= b[k + 3];
-			}
 			if (!good) return false;
+			if (nd.iData[2 + c] != 0) continue;
+			const float* f = nodes[nd.iData[c]].fData;
+			for (int k = 0; k < 3; k++)
+				inside &= f[k] >= b[k] && f[k + 6] >= b[k] && f[k + 3] <= b[k + 3] && f[k + 9] <= b[k + 3];
+			if (inside) continue;
+			if (loose.empty()) loose.resize(n);
+			loose[nd.iData[c]] = 1;
 		}
 	}
 	return true;
@@ -35,6 +38,7 @@ struct Slot {
 	const float* box;
 	uint32_t ref;    // leaf: the finished reference; inner: the binary node's index
 	bool leaf;
+	bool loose;      // inner: kWideLoose
 	float area;      // half surface area of an inner slot that may be opened, else negative
 };
 
@@ -44,10 +48,22 @@ float halfArea(const float* b)
 	return x * y + y * z + z * x;
 }
 
-// Whether a wide node may hold the children of binary node `nd` in place of it, whose box is `b`: no ray
-// passes a child's box that does not pass b (wide_nodes.hpp: flat boxes).
-bool mayOpen(const PhxBVHNode& nd, const float* b)
+// A binary tree, and its loose nodes (none: empty).
+struct Tree {
+	const PhxBVHNode* nodes;
+	std::vector<uint8_t> loose;
+	bool isLoose(int32_t node) const { return !loose.empty() && loose[node]; }
+};
+
+// Whether a wide node may hold the children of binary node `node` in place of it, whose box is `b`: no ray
+// passes a child's box that does not pass b (wide_nodes.hpp: flat boxes), and no child is loose, which has
+// to be decided when this node is taken.
+bool mayOpen(const Tree& t, int32_t node, const float* b)
 {
+	const PhxBVHNode& nd = t.nodes[node];
+	if (!t.loose.empty())
+		for (int c = 0; c < 2; c++)
+			if (t.loose[node] || (nd.iData[2 + c] == 0 && t.loose[nd.iData[c]])) return false;
 	for (int c = 0; c < 2; c++)
 		for (int k = 1; k < 3; k++) {
 			const float* f = nd.fData + 6 * c;
@@ -57,37 +73,38 @@ bool mayOpen(const PhxBVHNode& nd, const float* b)
 }
 
 // The slots of binary node `node` in castRay's order (see wide_nodes.hpp); returns how many (2).
-int expand(const PhxBVHNode* nodes, uint32_t node, Slot out[2])
+int expand(const Tree& tree, uint32_t node, Slot out[2])
 {
-	const PhxBVHNode& nd = nodes[node];
+	const PhxBVHNode& nd = tree.nodes[node];
 	int k = 0;
 	for (int c = 0; c < 2; c++)
 		if (nd.iData[2 + c] != 0) {
 			const uint32_t cnt = uint32_t(nd.iData[2 + c]);
 			uint32_t ref = kWideLeaf | uint32_t(~nd.iData[c]) | ((cnt <= 3u ? cnt : 0u) << kWideCountShift);
 			if (c == 0 && nd.iData[3] != 0) ref |= kWidePair;
-			out[k++] = Slot{nd.fData + 6 * c, ref, true, 0.0f};
+			out[k++] = Slot{nd.fData + 6 * c, ref, true, false, 0.0f};
 		}
 	for (int c = 1; c >= 0; c--)
 		if (nd.iData[2 + c] == 0) {
 			const float* b = nd.fData + 6 * c;
-			out[k++] = Slot{b, uint32_t(nd.iData[c]), false, mayOpen(nodes[nd.iData[c]], b) ? halfArea(b) : -1.0f};
+			const int32_t at = nd.iData[c];
+			out[k++] = Slot{b, uint32_t(at), false, tree.isLoose(at), mayOpen(tree, at, b) ? halfArea(b) : -1.0f};
 		}
 	return k;
 }
 
 // A wide node's slots: binary node `root` with the inner slots of largest area opened in place
 // until four are used.
-int collapse(const PhxBVHNode* nodes, uint32_t root, Slot s[4])
+int collapse(const Tree& tree, uint32_t root, Slot s[4])
 {
-	int k = expand(nodes, root, s);
+	int k = expand(tree, root, s);
 	while (k < 4) {
 		int best = -1;
 		for (int i = 0; i < k; i++)
 			if (!s[i].leaf && s[i].area >= 0.0f && (best < 0 || s[i].area > s[best].area)) best = i;
 		if (best < 0) break;
 		Slot two[2];
-		expand(nodes, s[best].ref, two);
+		expand(tree, s[best].ref, two);
 		for (int i = k; i > best + 1; i--) s[i] = s[i - 1];
 		s[best] = two[0];
 		s[best + 1] = two[1];
@@ -113,10 +130,14 @@ void setSlot(WideNode::Slot& s, const float* box, uint32_t ref)
 
 }  // namespace
 
-std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint32_t topCap)
+std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint32_t topCap, bool* loose)
 {
 	std::vector<WideNode> out;
-	if (!eligible(nodes, numNodes)) return out;
+	Tree tree{nodes, {}};
+	const bool fits = eligible(nodes, numNodes, tree.loose);
+	if (loose) *loose = fits && !tree.loose.empty();
+	if (!fits || (!loose && !tree.loose.empty())) return out;
+	auto inner = [](uint32_t at, bool isLoose) { return at | (isLoose ? kWideLoose : 0u); };
 
 	// A node to fill: the binary node whose subtree it covers and the slots pending beside it.
 	struct Item {
@@ -129,7 +150,7 @@ std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint
 
 	// The root: its slots become nodes 1..k. Leaves get a node that holds just them.
 	Slot s[4];
-	const int rootSlots = collapse(nodes, 0, s);
+	const int rootSlots = collapse(tree, 0, s);
 	struct RootSlot {
 		int first, count;  // range of s
 	};
@@ -142,7 +163,7 @@ std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint
 	}
 	for (int j = 0; j < numRoot; j++) {
 		const Slot& a = s[rs[j].first];
-		setSlot(out[0].slot[j], a.box, uint32_t(j + 1));
+		setSlot(out[0].slot[j], a.box, inner(uint32_t(j + 1), a.loose));
 		if (rs[j].count == 2) {
 			const Slot& b = s[rs[j].first + 1];
 			for (int k = 0; k < 3; k++) {
@@ -166,14 +187,14 @@ std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint
 	// Fills node it.at; its inner slots get the next indices and are appended to `next`.
 	auto fill = [&](const Item& it, std::vector<Item>& next) {
 		Slot t[4];
-		const int k = collapse(nodes, it.node, t);
+		const int k = collapse(tree, it.node, t);
 		maxPending = std::max(maxPending, it.pending + uint32_t(k - 1));
 		for (int i = 0; i < k; i++) {
 			if (t[i].leaf) {
 				setSlot(out[it.at].slot[i], t[i].box, t[i].ref);
 			} else {
 				const uint32_t child = uint32_t(out.size());
-				setSlot(out[it.at].slot[i], t[i].box, child);
+				setSlot(out[it.at].slot[i], t[i].box, inner(child, t[i].loose));
 				out.push_back(emptyNode());
 				next.push_back(Item{child, t[i].ref, it.pending + uint32_t(k - 1 - i)});
 			}

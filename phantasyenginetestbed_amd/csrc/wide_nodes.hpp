@@ -6,7 +6,7 @@
 //   - castRay's order does not depend on the ray: at a node, the leaf children are tested (left,
 //     then right), then the right inner child's subtree, then the left one's. The slots of a wide
 //     node are kept in that order, so taking the slots in order is castRay's order;
-//   - every child box lies inside its parent's (checked here), and for a ray with an origin within 2^126
+//   - every child box lies inside its parent's (but see kWideLoose), and for a ray with an origin within 2^126
 //     a child that passes the box predicate at some closest t implies that its ancestors passed theirs at
 //     the larger t of that earlier moment: the binary node decisions that a wide node leaves out can never
 //     have been negative. Without NaN slab values, because rounding is monotonic. With them (0 * inf: a
@@ -18,9 +18,9 @@
 //   - a leaf is decided with the closest t it would be decided with by castRay: its entry distance
 //     is kept with the pending slot and compared when the slot is taken. Two leaves of one parent
 //     are decided together, before either is tested (kWidePair).
-// Trees where this does not hold (bounds outside +-2^126 or NaN, child boxes that are inverted or
-// stick out of their parent, more than kWideMaxPending slots pending at once) get no wide nodes
-// and are traversed binary, as rays with origins beyond 2^126 are.
+// Trees where this does not hold (bounds outside +-2^126 or NaN, inverted child boxes, more than
+// kWideMaxPending slots pending at once) get no wide nodes and are traversed binary, as rays with
+// origins beyond 2^126 are.
 #pragma once
 
 #include <cstdint>
@@ -35,6 +35,11 @@ namespace phx {
 // end marker of the triangle array ends it then. kWidePair: the next slot is the sibling leaf.
 constexpr uint32_t kWideLeaf = 0x80000000u;
 constexpr uint32_t kWidePair = 0x40000000u;
+// An inner slot whose node's child boxes stick out of its own (of a tree made elsewhere, by a rounding):
+// neither that node nor its parent is merged into another, so that it is decided when castRay decides it,
+// and it is taken whatever its entry distance and the closest t are by then, as castRay takes it; its
+// children are decided by themselves. Trees with such slots are loose ones.
+constexpr uint32_t kWideLoose = kWidePair;
 constexpr uint32_t kWideIndex = 0x0FFFFFFFu;
 constexpr uint32_t kWideCountShift = 28u;
 
@@ -57,7 +62,9 @@ static_assert(sizeof(WideNode) == 128, "WideNode is one 128-B line");
 // Wide nodes of a validated SBVH (validateBVH), or an empty vector if the tree cannot have them.
 // Node 0 is the root and all its slots are inner: slot i refers to node i + 1 (a leaf or leaf pair
 // of the root gets a node of its own), so a kernel needs only the root's boxes. The first
-// `topCap` nodes are in breadth-first order, the rest depth first in slot order.
-std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint32_t topCap);
+// `topCap` nodes are in breadth-first order, the rest depth first in slot order. Without `loose`, which
+// says whether the tree has loose slots, such a tree gets none.
+std::vector<WideNode> buildWide(const PhxBVHNode* nodes, uint32_t numNodes, uint32_t topCap,
+                                bool* loose = nullptr);
 
 }  // namespace phx

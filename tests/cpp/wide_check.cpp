@@ -44,6 +44,7 @@ bool walk(const std::vector<WideNode>& wide, const OrTri* tris, const OrRay& r, 
 				if (pass[i]) {
 					if (have) stack[sp++] = cur;
 					cur = {tIn[i], n.slot[i].ref};
+					if (!(cur.ref & kWideLeaf) && (cur.ref & kWideLoose)) cur = {-inf, cur.ref & ~kWideLoose};
 					if (cur.ref & kWidePair && !(i < 3 && pass[i + 1])) cur.ref &= ~kWidePair;
 					have = true;
 				}
@@ -76,17 +77,16 @@ bool walk(const std::vector<WideNode>& wide, const OrTri* tris, const OrRay& r, 
 
 }  // namespace
 
-// Returns the wide nodes' number (0: the tree has none) and writes closest hits and in-light flags.
-extern "C" uint32_t wide_check(const PhxBVHNode* nodes, uint32_t numNodes, const OrTri* tris,
-                               const OrRay* rays, uint32_t n, uint32_t topCap, OrHit* hits,
-                               uint8_t* inLight, uint32_t* deepest)
+namespace {
+
+uint32_t check(const std::vector<WideNode>& wide, const OrTri* tris, const OrRay* rays, uint32_t n, OrHit* hits,
+               uint8_t* inLight, uint32_t* deepest)
 {
-	const std::vector<WideNode> wide = buildWide(nodes, numNodes, topCap);
 	*deepest = 0;
 	if (wide.empty()) return 0;
 	// The root's slots refer to nodes 1, 2, ... in order.
 	for (uint32_t i = 0; i < 4; i++)
-		if (wide[0].slot[i].min[0] == wide[0].slot[i].min[0] && wide[0].slot[i].ref != i + 1u) return 0;
+		if (wide[0].slot[i].min[0] == wide[0].slot[i].min[0] && (wide[0].slot[i].ref & ~kWideLoose) != i + 1u) return 0;
 	// Slots 0 to 2 repeat slot 3's max.xyz.
 	for (const WideNode& w : wide)
 		for (int i = 0; i < 3; i++)
@@ -97,4 +97,29 @@ extern "C" uint32_t wide_check(const PhxBVHNode* nodes, uint32_t numNodes, const
 		inLight[i] = walk(wide, tris, rays[i], true, unused, *deepest) ? 0 : 1;
 	}
 	return uint32_t(wide.size());
+}
+
+}  // namespace
+
+// Returns the wide nodes' number (0: the tree has none) and writes closest hits and in-light flags.
+extern "C" uint32_t wide_check(const PhxBVHNode* nodes, uint32_t numNodes, const OrTri* tris,
+                               const OrRay* rays, uint32_t n, uint32_t topCap, OrHit* hits,
+                               uint8_t* inLight, uint32_t* deepest)
+{
+	return check(buildWide(nodes, numNodes, topCap), tris, rays, n, hits, inLight, deepest);
+}
+
+// The same with loose trees, and how many loose slots there are.
+extern "C" uint32_t wide_check_loose(const PhxBVHNode* nodes, uint32_t numNodes, const OrTri* tris,
+                                     const OrRay* rays, uint32_t n, uint32_t topCap, OrHit* hits,
+                                     uint8_t* inLight, uint32_t* deepest, uint32_t* looseSlots)
+{
+	bool loose = false;
+	const std::vector<WideNode> wide = buildWide(nodes, numNodes, topCap, &loose);
+	*looseSlots = 0;
+	for (const WideNode& w : wide)
+		for (const WideNode::Slot& s : w.slot)
+			*looseSlots += !(s.ref & kWideLeaf) && (s.ref & kWideLoose);
+	if (loose != (*looseSlots != 0)) return 0;
+	return check(wide, tris, rays, n, hits, inLight, deepest);
 }

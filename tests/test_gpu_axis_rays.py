@@ -21,6 +21,39 @@ def ctx():
     c.destroy()
 
 
+def timed(ctx, kind, jobs):
+    """Best time in us of casting each (scene, rays) of equal numbers, in turn."""
+    n = len(jobs[0][1])
+    out = ctx.alloc(16 * n)
+    bufs, calls, plans = [out], [], []
+    for s, rays in jobs:
+        rb = ctx.alloc(32 * n).upload(rays)
+        bufs.append(rb)
+        if kind == "plan":
+            plans.append(phx.Plan(ctx, [(s, rb.ptr, out.ptr, n, phx.BATCH_CLOSEST)]))
+            calls.append(lambda p=plans[-1]: p.launch(asynchronous=True))
+        else:
+            cast = ctx.cast_closest_device if kind == "closest" else ctx.cast_anyhit_device
+            calls.append(lambda s=s, rb=rb, cast=cast: cast(s, rb.ptr, n, out.ptr, asynchronous=True))
+    try:
+        best = [1e9] * len(jobs)
+        for _ in range(9):
+            for i, call in enumerate(calls):
+                call()
+                ctx.synchronize()
+                t0 = time.perf_counter()
+                for _ in range(5):
+                    call()
+                ctx.synchronize()
+                best[i] = min(best[i], (time.perf_counter() - t0) / 5 * 1e6)
+        return best
+    finally:
+        for p in plans:
+            p.release()
+        for b in bufs:
+            b.free()
+
+
 def mixed(nodes, n, seed, share):
     """axis_rays, a share of them with all components of a camera's; some origins beyond 2^126."""
     rays, rng = axis_rays(nodes, n, seed), np.random.default_rng(seed)
@@ -31,14 +64,8 @@ def mixed(nodes, n, seed, share):
     return rays
 
 
-@pytest.mark.parametrize("share", [0.0, 0.5, 0.99])
-@pytest.mark.parametrize("flat", [False, True], ids=["", "lattice"])
-@pytest.mark.parametrize("name", NAMES)
-def test_casts(ctx, name, flat, share):
-    nodes, tris, _ = scene(name)
-    if flat:
-        nodes = lattice(nodes, 2)
-    rays = mixed(nodes, 30011, 7, share)
+def compare_casts(ctx, nodes, tris, rays):
+    """Every kind of cast of `rays` against the oracle."""
     n = len(rays)
     hits, lit = O.cast_closest(nodes, tris, rays), O.cast_anyhit(nodes, tris, rays)
     s = ctx.upload_scene(nodes, tris)
@@ -62,6 +89,16 @@ def test_casts(ctx, name, flat, share):
         for b in (rb, hb, lb):
             b.free()
         s.release()
+
+
+@pytest.mark.parametrize("share", [0.0, 0.5, 0.99])
+@pytest.mark.parametrize("flat", [False, True], ids=["", "lattice"])
+@pytest.mark.parametrize("name", NAMES)
+def test_casts(ctx, name, flat, share):
+    nodes, tris, _ = scene(name)
+    if flat:
+        nodes = lattice(nodes, 2)
+    compare_casts(ctx, nodes, tris, mixed(nodes, 30011, 7, share))
 
 
 @pytest.mark.parametrize("static", [False, True])
@@ -112,34 +149,7 @@ def test_rays_with_a_zero_component_cost_what_their_neighbours_do(ctx, kind):
     tilted = rays.copy()
     tilted["d"][:, 1] = np.where(rng.random(n) < 0.5, np.float32(1e-4), np.float32(-1e-4))
     s = ctx.upload_scene(b.nodes, b.tris)
-    out = ctx.alloc(16 * n)
-    bufs, calls, plans = [], [], []
-    for r in (rays, tilted):
-        rb = ctx.alloc(32 * n).upload(r)
-        bufs.append(rb)
-        if kind == "closest":
-            calls.append(lambda rb=rb: ctx.cast_closest_device(s, rb.ptr, n, out.ptr, asynchronous=True))
-        elif kind == "anyhit":
-            calls.append(lambda rb=rb: ctx.cast_anyhit_device(s, rb.ptr, n, out.ptr, asynchronous=True))
-        else:
-            plans.append(phx.Plan(ctx, [(s, rb.ptr, out.ptr, n, phx.BATCH_CLOSEST)]))
-            calls.append(lambda p=plans[-1]: p.launch(asynchronous=True))
-    try:
-        best = [1e9, 1e9]
-        for _ in range(9):
-            for i, call in enumerate(calls):
-                call()
-                ctx.synchronize()
-                t0 = time.perf_counter()
-                for _ in range(5):
-                    call()
-                ctx.synchronize()
-                best[i] = min(best[i], (time.perf_counter() - t0) / 5)
-        print(f"[gpu] {kind}: {best[0] * 1e6:.0f} us, tilted {best[1] * 1e6:.0f} us")
-        assert best[0] <= best[1] * 4 / 3
-    finally:
-        for p in plans:
-            p.release()
-        for x in [*bufs, out]:
-            x.free()
-        s.release()
+    (took, beside) = timed(ctx, kind, [(s, rays), (s, tilted)])
+    s.release()
+    print(f"[gpu] {kind}: {took:.0f} us, tilted {beside:.0f} us")
+    assert took <= beside * 4 / 3

@@ -162,3 +162,46 @@ def test_slot_order_gives_castray_hits_on_box_planes(lib, name, flat, seed):
     ref = O.cast_closest(nodes, tris, rays)
     assert hits.tobytes() == ref.tobytes(), int((hits["tri"] != ref["tri"]).sum())
     assert (lit == O.cast_anyhit(nodes, tris, rays)).all()
+
+
+# ---- trees whose boxes stick out of the boxes around them ----------------------------------------
+
+def sticking_out(nodes, seed, how):
+    """The tree with a share of its boxes moved: by a float ("ulp"), or by up to a tenth of their size."""
+    n, rng = nodes.copy(), np.random.default_rng(seed)
+    f = n["f"].reshape(-1, 2, 2, 3)
+    pick = rng.random(f.shape) < (0.1 if how == "ulp" else 0.2)
+    if how == "ulp":
+        moved = np.nextafter(f, rng.choice(np.array([-np.inf, np.inf], np.float32), f.shape))
+    else:
+        size = (f[:, :, 1] - f[:, :, 0])[:, :, None, :]
+        moved = (f + size * rng.uniform(-0.1, 0.1, f.shape)).astype(np.float32)
+    f[...] = np.where(pick, moved, f)
+    f[...] = np.sort(f, axis=2)
+    return n
+
+
+@pytest.mark.parametrize("seed", range(3))
+@pytest.mark.parametrize("how", ["none", "ulp", "tenth", "tenth lattice"])
+@pytest.mark.parametrize("name", ["fixture rand2k", "fixture hf32", "tiny 1", "tiny 2", "tiny 3", "tiny 5",
+                                  "random 4000", "long 600", "twice 500", "terrain 60"])
+def test_loose_trees_give_castray_hits(lib, name, how, seed):
+    nodes, tris, _ = scene(name)
+    if "lattice" in how:
+        nodes = lattice(nodes, seed)
+    if how != "none":
+        nodes = sticking_out(nodes, seed, how.split()[0])
+    rays = axis_rays(nodes, 20000, seed)
+    rays["d"][::2] = np.random.default_rng(seed).normal(size=rays["d"][::2].shape)
+    hits, lit = np.zeros(len(rays), phx.HIT), np.zeros(len(rays), np.uint8)
+    deepest, loose = C.c_uint32(), C.c_uint32()
+    p = [C.c_void_p(np.ascontiguousarray(a).ctypes.data) for a in (nodes, tris, rays)]
+    k = lib.wide_check_loose(p[0], len(nodes), p[1], p[2], len(rays), 64, C.c_void_p(hits.ctypes.data),
+                             C.c_void_p(lit.ctypes.data), C.byref(deepest), C.byref(loose))
+    assert 0 < k and deepest.value <= CAPACITY
+    assert hits.tobytes() == O.cast_closest(nodes, tris, rays).tobytes()
+    assert (lit == O.cast_anyhit(nodes, tris, rays)).all()
+    if how == "none":
+        assert loose.value == 0
+    elif len(nodes) > 50:
+        assert loose.value > 0
