@@ -5,9 +5,11 @@
 #include <atomic>
 #include <cmath>
 #include <cstring>
+#include <future>
 #include <memory>
 #include <mutex>
 #include <new>
+#include <system_error>
 #include <unordered_set>
 
 #include "runtime.hpp"
@@ -154,6 +156,8 @@ phx_status castCommon(PhxContext* ctx, const PhxRayIn* rays, uint32_t n, void* o
 constexpr uint32_t kTopCap = 2048;
 // Wide nodes kept in breadth-first order.
 constexpr uint32_t kWideTop = 1024;
+// Nodes of a tree from which on its wide nodes are made beside the upload.
+constexpr uint32_t kWideThreadNodes = 16384;
 
 // Whether a launch shape is one that the interface takes: topNodes, helperWaves and stackLdsEntries no
 // longer change how the kernels run, but what they stand for has to fit a CU's LDS as it always had to --
@@ -576,22 +580,32 @@ static phx_status phx_scene_upload_impl(PhxContext* ctx, const PhxBVHNode* nodes
 		s->rootMin[k] = std::min(lmn[k], rmn[k]);
 		s->rootMax[k] = std::max(lmx[k], rmx[k]);
 	}
+	// The wide nodes of a large tree are made beside the uploads, by several threads (1,004,000 triangles
+	// took 60 ms to upload with one, and 48 without wide nodes; so they take 45).
+	bool loose = false;
+	auto makeWide = [&] { return buildWide(nodes, numNodes, kWideTop, &loose); };
+	std::future<std::vector<WideNode>> making;
+	if (numNodes >= kWideThreadNodes) {
+		try {
+			making = std::async(std::launch::async, makeWide);
+		} catch (const std::system_error&) {  // no thread to be had: below
+		}
+	}
+	std::vector<PhxTriangleVertices> pre;  // (kept, as `wide`, until the copies have ended)
+	std::vector<WideNode> wide;
 	st = uploadArray(ctx, s->nodes, nodes, numNodes, s->bytes);
 	if (st == PHX_OK) {
-		const std::vector<WideNode> wide = buildWide(nodes, numNodes, kWideTop, &s->loose);
-		st = uploadArray(ctx, s->wide, wide.data(), wide.size(), s->bytes);
-		if (st == PHX_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
-			st = fail(PHX_ERR_HIP, "phx_scene_upload: wide node upload failed");
-	}
-	if (st == PHX_OK) {
-		std::vector<PhxTriangleVertices> pre = pretransform(triangles, numTriangles);
+		pre = pretransform(triangles, numTriangles);
 		st = uploadArray(ctx, s->tris, pre.data(), numTriangles, s->bytes, kTrianglePad);
-		if (st == PHX_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
-			st = fail(PHX_ERR_HIP, "phx_scene_upload: triangle upload failed");
 	}
 	if (st == PHX_OK && datas) st = uploadArray(ctx, s->datas, datas, numTriangles, s->bytes);
 	if (st == PHX_OK) st = uploadArray(ctx, s->materials, materials, numMaterials, s->bytes);
 	if (st == PHX_OK) st = uploadArray(ctx, s->lights, lights, numLights, s->bytes);
+	if (st == PHX_OK) {
+		wide = making.valid() ? making.get() : makeWide();
+		s->loose = loose;
+		st = uploadArray(ctx, s->wide, wide.data(), wide.size(), s->bytes);
+	}
 	if (st == PHX_OK) {
 		hipError_t e = hipStreamSynchronize(ctx->stream);
 		if (e != hipSuccess) st = hipFail(e, "phx_scene_upload");

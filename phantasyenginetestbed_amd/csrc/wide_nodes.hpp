@@ -56,6 +56,7 @@ struct WideNode {
 		float max[3];
 		float lastMax;  // slot i < 3: slot[3].max[i]
 	} slot[4];
+	WideNode() {}  // left unset: an array of them is touched first by the threads that fill it
 };
 static_assert(sizeof(WideNode) == 128, "WideNode is one 128-B line");
 

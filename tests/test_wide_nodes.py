@@ -205,3 +205,23 @@ def test_loose_trees_give_castray_hits(lib, name, how, seed):
         assert loose.value == 0
     elif len(nodes) > 50:
         assert loose.value > 0
+
+
+@pytest.mark.parametrize("top_cap", [0, 1024, 1 << 30])
+@pytest.mark.parametrize("how", ["none", "ulp"])
+def test_trees_merged_by_several_threads(lib, how, top_cap):
+    """Trees large enough for several threads (more than 16,384 nodes)."""
+    t, _ = phx.heightfield_boxes(200, 160, 5)
+    b = phx.BVH(t)
+    nodes = b.nodes if how == "none" else sticking_out(b.nodes, 1, how)
+    assert len(nodes) > 24576
+    rays = np.concatenate([axis_rays(nodes, 2000, 1), random_rays(4000, 3)])
+    hits, lit = np.zeros(len(rays), phx.HIT), np.zeros(len(rays), np.uint8)
+    deepest, loose = C.c_uint32(), C.c_uint32()
+    p = [C.c_void_p(np.ascontiguousarray(a).ctypes.data) for a in (nodes, b.tris, rays)]
+    for _ in range(5):
+        k = lib.wide_check_loose(p[0], len(nodes), p[1], p[2], len(rays), top_cap, C.c_void_p(hits.ctypes.data),
+                                 C.c_void_p(lit.ctypes.data), C.byref(deepest), C.byref(loose))
+        assert 0 < k
+        assert hits.tobytes() == O.cast_closest(nodes, b.tris, rays).tobytes()
+        assert (lit == O.cast_anyhit(nodes, b.tris, rays)).all()
