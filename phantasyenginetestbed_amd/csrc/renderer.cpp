@@ -14,7 +14,7 @@ struct PhxRenderer {
 	PhxContext* ctx = nullptr;
 	uint32_t w = 0, h = 0, n = 0;    // full resolution
 	uint32_t hw = 0, hh = 0, m = 0;  // half resolution (bounce records)
-	uint32_t lightCap = 0;           // lights the per-light buffers hold
+	size_t lightCap = 0;             // records x lights that the per-light buffers hold
 	PhxRayIn* prim = nullptr;
 	PhxRayHit* primHits = nullptr;
 	float4* gbuf = nullptr;
@@ -22,9 +22,9 @@ struct PhxRenderer {
 	float4* throughput = nullptr;
 	PhxRayHit* bounceHits = nullptr;
 	float4* bounceInfo = nullptr;
-	float4* contrib = nullptr;  // n * lightCap
-	PhxRayIn* shadow = nullptr;  // n * lightCap
-	uint8_t* inLight = nullptr;  // n * lightCap
+	float4* contrib = nullptr;  // lightCap of each
+	PhxRayIn* shadow = nullptr;
+	uint8_t* inLight = nullptr;
 	float4* color = nullptr;
 	float4* hist[2] = {nullptr, nullptr};
 	float2* vel[2] = {nullptr, nullptr};  // TAA: velocity of the frame that wrote hist[i]
@@ -99,9 +99,13 @@ phx_status devAlloc(T*& p, size_t count, const char* what)
 	return PHX_OK;
 }
 
+// Buffers for the lights of the bounce records, and with instances of the primary ones, which are shaded
+// without them otherwise (launchShadeTrace): a quarter of the memory.
 phx_status growLights(PhxRenderer* r, uint32_t lights)
 {
-	if (lights <= r->lightCap) return PHX_OK;
+	const bool instances = r->instances && instanceCount(r->instances);
+	const size_t k = size_t(instances ? r->n : r->m) * lights;
+	if (k <= r->lightCap) return PHX_OK;
 	hipStreamSynchronize(r->ctx->stream);  // earlier frames may still use the buffers
 	dropGraph(r);                           // a captured frame uses them too
 	hipFree(r->contrib);
@@ -111,11 +115,10 @@ phx_status growLights(PhxRenderer* r, uint32_t lights)
 	r->shadow = nullptr;
 	r->inLight = nullptr;
 	r->lightCap = 0;
-	const size_t k = size_t(r->n) * lights;
 	phx_status st = devAlloc(r->contrib, k, "phx_render_frame");
 	if (st == PHX_OK) st = devAlloc(r->shadow, k, "phx_render_frame");
 	if (st == PHX_OK) st = devAlloc(r->inLight, k, "phx_render_frame");
-	if (st == PHX_OK) r->lightCap = lights;
+	if (st == PHX_OK) r->lightCap = k;
 	return st;
 }
 

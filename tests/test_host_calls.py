@@ -319,3 +319,32 @@ def resident(lib, block, n):
 def test_resident_grid_is_where_more_blocks_change_nothing(library, block):
     half, whole, more = run(library, resident, block, 4 << 20)
     assert half[0] < whole[0] and whole == more
+
+
+def frame_memory(lib, w, h, lights, instances, graph):
+    """Device bytes allocated by a frame, with `instances` by those after one without too."""
+    ctx = phx.Context(0)
+    t, d = phx.random_triangles(50, 1, 0.1, 0.5)
+    b = phx.BVH(t, d)
+    s = ctx.upload_scene(b.nodes, b.tris, b.datas, phx.materials_random(4, 1), phx.lights_random(lights, 2))
+    r = ctx.renderer(w, h)
+    cam = phx.camera_look_at((0.5, 0.5, -1.5), (0.5, 0.5, 0), (0, 1, 0), 1.0, w, h)
+    image = ctx.alloc(16 * w * h)
+    iset = phx.InstanceSet(ctx, [(s, np.eye(3, 4, dtype=np.float32))])
+    out = []
+    for has in [False, True, False] if instances else [False, False]:
+        r.set_instances(iset if has else None)
+        log(lib)
+        for f in range(2):
+            r.render(s, cam, f, 1, phx.FRAME_GRAPH if graph else 0, out_ptr=image.ptr)
+        out.append(sum(int(x.split()[1]) for x in log(lib) if x.startswith("malloc")))
+    return out
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("w,h,lights", [(64, 32, 8), (33, 17, 3), (1, 9, 2)])
+def test_frames_allocate_light_buffers_for_the_records_that_use_them(library, w, h, lights, graph):
+    """49 bytes a record and light: the bounce records', and with instances the primary ones'."""
+    bounce, primary = (w // 2) * (h // 2) * lights * 49, w * h * lights * 49
+    assert run(library, frame_memory, w, h, lights, False, graph) == [bounce, 0]
+    assert run(library, frame_memory, w, h, lights, True, graph) == [bounce, primary + 4096, 0]
