@@ -1298,7 +1298,7 @@ static phx_status phx_autotune_impl(PhxContext* ctx, const PhxScene* scene, cons
 		              : launchClosest(sv, rays, numRays, static_cast<PhxRayHit*>(out), L, nullptr,
 		                              ctx->stream);
 	};
-	auto shapeOf = [&](const TraceLaunch& L) { return castShape(L, numRays); };
+	auto shapeOf = [&](const TraceLaunch& L) { return castShape(L, numRays, anyhit); };
 	st = tune(ctx, cands, 13, cast, shapeOf, best);
 	if (st == PHX_OK) st = refine(ctx, nullptr, 15, cast, shapeOf, best);
 	hipStreamSynchronize(ctx->stream);

@@ -75,7 +75,7 @@ struct LaunchShape {
 		return grid == o.grid && block == o.block && window == o.window && refill == o.refill;
 	}
 };
-LaunchShape castShape(const TraceLaunch& launch, uint32_t n);
+LaunchShape castShape(const TraceLaunch& launch, uint32_t n, bool anyHit);
 LaunchShape batchShape(const TraceLaunch& launch, uint32_t total, uint32_t numBatches, bool tracked);
 
 // Scratch of the allocation-free closest-hit cast: a static device array per GPU holding the

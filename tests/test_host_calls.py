@@ -260,7 +260,7 @@ def test_autotuners_time_no_launch_twice(library, plan, n):
     m = len(rest) // (reps[1] + 1)
     assert rest == rest[:m] * (reps[1] + 1) and len(set(rest[:m])) == m
     if n == 4000000:
-        assert k == 6 and m == 3
+        assert k == 6 and m == (3 if plan else 1)
 
 
 def shapes(lib, scenes, track, tries):
@@ -348,3 +348,28 @@ def test_frames_allocate_light_buffers_for_the_records_that_use_them(library, w,
     bounce, primary = (w // 2) * (h // 2) * lights * 49, w * h * lights * 49
     assert run(library, frame_memory, w, h, lights, False, graph) == [bounce, 0]
     assert run(library, frame_memory, w, h, lights, True, graph) == [bounce, primary + 4096, 0]
+
+
+def cast_windows(lib, n, anyhit, timeline, fetch):
+    ctx = phx.Context(0)
+    s = upload(ctx)
+    ctx.set_launch_params(rays_per_fetch=fetch)
+    rays, out = ctx.alloc(32 * n), ctx.alloc(16 * n)
+    log(lib)
+    if timeline:
+        ctx.cast_closest_timeline(s, rays.ptr, n, out.ptr)
+    else:
+        (ctx.cast_anyhit_device if anyhit else ctx.cast_closest_device)(s, rays.ptr, n, out.ptr)
+    return launches(log(lib), "k_quad")
+
+
+@pytest.mark.parametrize("fetch", [8, 16, 64, 4096])
+@pytest.mark.parametrize("n", [1, 2048, 40000, 1 << 20, 16 << 20])
+@pytest.mark.parametrize("call", ["closest", "anyhit", "timeline"])
+def test_waves_take_no_more_closest_hit_rays_than_they_trace_at_a_time(library, call, n, fetch):
+    """A wave traces 16 at a time; rays beside costly ones are costly too, and what is left of a wide window
+    is traced by the same wave, one after another."""
+    (_, _, window, _), = run(library, cast_windows, n, call == "anyhit", call == "timeline", fetch)
+    assert 1 <= window <= min(fetch, 64 if call == "anyhit" else 16)
+    if n >= 16 << 20:
+        assert window == min(fetch, 64 if call == "anyhit" else 16)
