@@ -2179,10 +2179,13 @@ Shape quadShape(const TraceLaunch& L, uint32_t n, bool anyHit)
 	return s;
 }
 
-// One ray per lane: windows of 64 rays, or what L says; blocks small enough that every CU has one, and of 1,024 threads
-// where `tableWords` of LDS beside the waves' (the batch tables) would halve the waves of a CU in blocks
-// of 512 (256 tracked batches of 29.6 million rays: 7.4 ms with 8 waves per CU, 4.7 with 16). No more waves
-// than are resident: the others' first windows would wait for a block to end.
+// One ray per lane: windows of 64 rays, or fewer by L. A launch whose waves need 16 rays at most takes 16,
+// which they trace four lanes each from the start: 6,077 rays in 8 batches 160 us with 64 and 98 with 16,
+// 46,460 in 8 238 and 228; 85,813 in 64 (which would take 21) 247 and 267.
+// Blocks small enough that every CU has one, and of 1,024 threads where `tableWords` of LDS beside the waves'
+// (the batch tables) would halve the waves of a CU in blocks of 512 (256 tracked batches of 29.6 million
+// rays: 7.4 ms with 8 waves per CU, 4.7 with 16). No more waves than are resident: the others' first windows
+// would wait for a block to end.
 Shape laneShape(const TraceLaunch& L, uint32_t n, uint32_t tableWords)
 {
 	auto resident = [&](uint32_t block) {
@@ -2192,7 +2195,7 @@ Shape laneShape(const TraceLaunch& L, uint32_t n, uint32_t tableWords)
 	uint32_t block = resident(kLaneBlock) > resident(kQuadBlock) ? kLaneBlock : kQuadBlock;
 	const uint32_t most = std::max(1u, std::min(std::min(L.raysInFlight, L.spillColumns) / 64u,
 	                                            L.cus * std::max(1u, resident(block))));
-	const uint32_t window = std::min(64u, L.window), waves = std::min(most, gridFor(n, window));
+	const uint32_t window = std::min(n <= 16u * most ? 16u : 64u, L.window), waves = std::min(most, gridFor(n, window));
 	while (block > 64u && waves / (block / 64u) < L.cus) block /= 2u;
 	Shape s = shapeOf(waves, most, block);
 	s.window = window;

@@ -373,3 +373,25 @@ def test_waves_take_no_more_closest_hit_rays_than_they_trace_at_a_time(library, 
     assert 1 <= window <= min(fetch, 64 if call == "anyhit" else 16)
     if n >= 16 << 20:
         assert window == min(fetch, 64 if call == "anyhit" else 16)
+
+
+def plan_shapes(lib, sizes):
+    ctx = phx.Context(0)
+    s = upload(ctx)
+    mem = ctx.alloc(32 * max(sizes))
+    out = []
+    for n in sizes:
+        plan = phx.Plan(ctx, [(s, mem.ptr, mem.ptr, n, phx.BATCH_CLOSEST)])
+        log(lib)
+        plan.launch()
+        out += launches(log(lib), "k_trace_batches")
+        plan.release()
+    return out
+
+
+def test_small_fused_launches_give_waves_as_many_rays_as_they_trace_four_lanes_each(library):
+    sizes = [1, 15, 16, 17, 1000, 65535, 65536, 65537, 4 << 20]
+    for n, (grid, block, window, _) in zip(sizes, run(library, plan_shapes, sizes)):
+        waves = grid * (block // 64)
+        assert window == (16 if n <= 65536 else 64)  # 256 CUs of 16 waves
+        assert waves * window >= min(n, 4096 * window) and waves <= 4096
