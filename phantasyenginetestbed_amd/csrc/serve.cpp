@@ -3,7 +3,7 @@
 // Requests (ray batches against resident scenes) are admitted in arrival order while their
 // buffers fit the HBM budget (a first-fit arena over one device allocation, so admission never
 // calls hipMalloc), and admitted requests are coalesced into the next fused persistent launch, up
-// to a quarter of the waiting rays per launch (launchSlot; at least one request).
+// to a quarter of the waiting rays per launch (formLaunch; at least one request).
 // Launches run on `slots` streams, each with its own work counter and stack spill area, so a
 // launch formed from requests that arrived while another one runs starts on the next stream and
 // fills the running launch's tail. A dispatcher thread forms launches and retires them (outputs
@@ -34,13 +34,14 @@ double msSince(Clock::time_point t0) { return std::chrono::duration<double, std:
 
 constexpr size_t kAlign = 256;
 
-// Rays per fused launch before further admitted requests wait for the next launch: a quarter of what is
-// waiting, between one and four million; four million for requests whose rays are on the device. A
+// Rays per fused launch before further admitted requests wait for the next launch: for requests in pinned
+// memory a quarter of what is waiting, between one and four million; four million for the others. A
 // backlog coalesced into one or two launches runs its copies to the device, traversal and copies back
 // one after the other; split, the slot streams overlap one launch's copies with another's traversal. A
-// launch that is too small spends its time on its last rays.
-//   48 requests, 3.2 million rays, 3 slots: 3.34 ms at 4 million, 3.12 at 1 million, 3.79 at 1/4 million
+// launch that is too small spends its time on its last rays; copies of pageable memory overlap nothing.
+//   48 requests, 2.6 million rays, 3 slots: 3.34 ms at 4 million, 3.12 at 1 million, 3.79 at 1/4 million
 //   1,500 requests, 143 million rays: 105 ms at 4 million, 126 at 1 million (on the device: 37 and 50)
+//   48 requests, 2.6 million rays, in pageable memory: 10.1 ms split, 7.0 at 4 million
 constexpr uint64_t kLeastLaunchRays = 1u << 20, kMostLaunchRays = 4u << 20;
 size_t alignUp(size_t b) { return (b + kAlign - 1) / kAlign * kAlign; }
 
@@ -195,8 +196,8 @@ void admit(PhxServer* s)
 	}
 }
 
-// Forms one launch on `slot` from the admitted requests. Caller holds the lock.
-hipError_t launchSlot(PhxServer* s, Slot& slot)
+// Takes the requests of one launch on `slot` from the admitted ones. Caller holds the lock.
+void formLaunch(PhxServer* s, Slot& slot)
 {
 	slot.reqs.clear();
 	uint64_t total = 0, waiting = 0;
@@ -206,13 +207,21 @@ hipError_t launchSlot(PhxServer* s, Slot& slot)
 	while (!s->admitted.empty() && slot.reqs.size() < kMaxFusedBatches) {
 		Request* r = s->admitted.front();
 		if (total + r->req.numRays > 0x7FFFFFFFull) break;
-		const uint64_t most = (r->req.flags & PHX_MEM_DEVICE) ? kMostLaunchRays : hostRays;
+		const uint64_t most = r->mappedRays && r->mappedOut ? hostRays : kMostLaunchRays;
 		if (!slot.reqs.empty() && total + r->req.numRays > most) break;
 		total += r->req.numRays;
+		r->state = ReqState::InFlight;
 		slot.reqs.push_back(r);
 		s->admitted.pop_front();
 		if (s->flags & PHX_SERVE_PLAIN) break;  // one request per launch
 	}
+}
+
+// Launches what formLaunch took. The lock is not held: a copy call on pageable memory returns when the
+// stream has got to it, and requests that come meanwhile (submitters waited for it) make the next launch.
+// Only the dispatcher touches slots, lastLoaded and requests in flight.
+hipError_t launchSlot(PhxServer* s, Slot& slot)
+{
 	if (slot.reqs.empty()) return hipSuccess;
 	hipError_t e = hipSuccess;
 	const uint32_t nb = uint32_t(slot.reqs.size());
@@ -227,7 +236,6 @@ hipError_t launchSlot(PhxServer* s, Slot& slot)
 		e = hipStreamWaitEvent(slot.stream, s->lastLoaded, 0);
 	for (uint32_t b = 0; b < nb && e == hipSuccess; b++) {
 		Request* r = slot.reqs[b];
-		r->state = ReqState::InFlight;
 		if (!(r->req.flags & PHX_MEM_DEVICE) && r->req.numRays) {
 			if (r->mappedRays)
 				slot.copies.push_back({r->mappedRays, const_cast<PhxRayIn*>(r->devRays), r->rayBytes});
@@ -280,10 +288,6 @@ hipError_t launchSlot(PhxServer* s, Slot& slot)
 	}
 	if (e == hipSuccess) e = launchCopies(slot.copies.data(), uint32_t(slot.copies.size()), true, slot.stream);
 	if (e == hipSuccess) e = hipEventRecord(slot.done, slot.stream);
-	if (e == hipSuccess) {
-		slot.busy = true;
-		s->stats.launches++;
-	}
 	return e;
 }
 
@@ -332,7 +336,14 @@ void dispatchLoop(PhxServer* s)
 			if (s->admitted.empty() || s->paused) break;
 			if (slot.busy) continue;
 			if ((s->flags & PHX_SERVE_PLAIN) && anyBusy) break;
+			formLaunch(s, slot);
+			lk.unlock();
 			const hipError_t e = launchSlot(s, slot);
+			lk.lock();
+			if (e == hipSuccess && !slot.reqs.empty()) {
+				slot.busy = true;
+				s->stats.launches++;
+			}
 			if (e != hipSuccess) {
 				failServer(s, "server launch", e);
 				for (Request* r : slot.reqs) r->state = ReqState::Admitted;

@@ -7,6 +7,7 @@
 #include <sys/mman.h>
 #include <unistd.h>
 
+#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -27,6 +28,7 @@ std::map<const void*, std::string> kernels;
 std::map<const void*, void*> variables;
 std::string text;
 uintptr_t nextHandle = 1;
+std::atomic<bool> held{false};  // copies to the device wait
 
 template <class... A>
 void say(const char* format, A... a)
@@ -105,6 +107,9 @@ size_t fake_log(char* out, size_t room)
 	text.clear();
 	return n;
 }
+
+// Holds copies to the device up, as a stream that is busy does copies from pageable memory.
+void fake_hold(int on) { held = on != 0; }
 
 void** __hipRegisterFatBinary(const void*)
 {
@@ -242,6 +247,7 @@ hipError_t hipMemcpy(void* dst, const void* src, size_t n, hipMemcpyKind)
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind kind, hipStream_t stream)
 {
 	say("copy %zu kind=%d stream=%p", n, int(kind), static_cast<void*>(stream));
+	while (held && kind == hipMemcpyHostToDevice) usleep(1000);
 	return hipMemcpy(dst, src, n, kind);
 }
 hipError_t hipMemset(void* dst, int v, size_t n)

@@ -4,6 +4,7 @@ Kernels do not run, so results are not looked at here."""
 import ctypes as C
 import multiprocessing
 import subprocess
+import threading
 from pathlib import Path
 
 import numpy as np
@@ -395,3 +396,68 @@ def test_small_fused_launches_give_waves_as_many_rays_as_they_trace_four_lanes_e
         waves = grid * (block // 64)
         assert window == (16 if n <= 65536 else 64)  # 256 CUs of 16 waves
         assert waves * window >= min(n, 4096 * window) and waves <= 4096
+
+
+def submit_beside_a_copy(lib):
+    """Whether requests are taken while the dispatcher copies, and the launches of all of them."""
+    ctx = phx.Context(0)
+    s = upload(ctx)
+    server = phx.Server(ctx, 1 << 28)
+    server.add_scene(s)
+    rays, outs = some_rays(256), [np.zeros(256, phx.HIT) for _ in range(9)]
+    tickets = []
+
+    def submit(i):
+        tickets.append(server.submit(phx.Server.request(s, rays.ctypes.data, outs[i].ctypes.data, 256,
+                                                        phx.BATCH_CLOSEST)))
+
+    try:
+        lib.fake_hold(1)
+        log(lib)
+        submit(0)
+        while not any(x.startswith("copy") for x in log(lib)):
+            pass
+        others = threading.Thread(target=lambda: [submit(i) for i in range(1, 9)], daemon=True)
+        others.start()
+        others.join(5)
+        taken = not others.is_alive()
+        lib.fake_hold(0)
+        others.join()
+        for t in tickets:
+            server.wait(t)
+        return taken, len(launches(log(lib), "k_trace_batches"))
+    finally:
+        lib.fake_hold(0)
+        server.destroy()
+
+
+def test_requests_are_taken_while_the_dispatcher_copies(library):
+    """A copy from pageable memory returns late; what comes meanwhile makes one launch."""
+    assert run(library, submit_beside_a_copy) == (True, 2)
+
+
+def backlog_launches(lib, pinned, count, n):
+    ctx = phx.Context(0)
+    s = upload(ctx)
+    server = phx.Server(ctx, 1 << 30)
+    server.add_scene(s)
+    make = (lambda k: phx.HostBuffer(np.uint8, k).array) if pinned else (lambda k: np.zeros(k, np.uint8))
+    rays, out = make(32 * n), make(n)
+    try:
+        server.pause()
+        tickets = [server.submit(phx.Server.request(s, rays.ctypes.data, out.ctypes.data, n, phx.BATCH_ANYHIT))
+                   for _ in range(count)]
+        log(lib)
+        server.pause(False)
+        for t in tickets:
+            server.wait(t)
+        return launches(log(lib), "k_trace_batches")
+    finally:
+        server.destroy()
+
+
+def test_requests_in_pageable_memory_are_not_split(library):
+    """Their copy calls return one after another, so nothing overlaps them: launches of up to 4 million
+    rays; requests in pinned memory, of a quarter of what waits, a million at least."""
+    assert len(run(library, backlog_launches, False, 48, 55000)) == 1
+    assert len(run(library, backlog_launches, True, 48, 55000)) == 3
