@@ -882,9 +882,10 @@ phx_status phx_traversal_stats(PhxContext* ctx, const PhxScene* scene, const Phx
 	const bool anyhit = (flags & PHX_STATS_ANYHIT) != 0;
 	for (int k = 0; k < 5; k++) counters[k] = 0;
 	if (numRays == 0) return ok();
+	unsigned long long host[kCountStripes * kCountStride];
 	unsigned long long* dCounters = nullptr;
-	PHX_HIP(hipMalloc(&dCounters, 5 * sizeof(unsigned long long)), "phx_traversal_stats");
-	hipError_t e = hipMemsetAsync(dCounters, 0, 5 * sizeof(unsigned long long), ctx->stream);
+	PHX_HIP(hipMalloc(&dCounters, sizeof(host)), "phx_traversal_stats");
+	hipError_t e = hipMemsetAsync(dCounters, 0, sizeof(host), ctx->stream);
 	PhxRayHit* dHits = nullptr;
 	if (e == hipSuccess) e = hipMalloc(&dHits, size_t(numRays) * sizeof(PhxRayHit));
 	SceneView sv = view(scene);
@@ -894,19 +895,19 @@ phx_status phx_traversal_stats(PhxContext* ctx, const PhxScene* scene, const Phx
 			ctx, rays, numRays, nullptr, 0, (flags & PHX_MEM_DEVICE),
 			[&](const PhxRayIn* r, void*) {
 				return anyhit ? launchAnyHitCounted(sv, r, numRays, reinterpret_cast<uint8_t*>(dHits),
-				                                    dCounters, ctx->stream)
+				                                    L, dCounters, ctx->stream)
 				              : launchClosest(sv, r, numRays, dHits, L, dCounters, ctx->stream);
 			},
 			"phx_traversal_stats");
 	}
-	unsigned long long host[5] = {0, 0, 0, 0, 0};
 	if (e == hipSuccess && st == PHX_OK)
 		e = hipMemcpy(host, dCounters, sizeof(host), hipMemcpyDeviceToHost);
 	hipFree(dHits);
 	hipFree(dCounters);
 	if (e != hipSuccess) return hipFail(e, "phx_traversal_stats");
 	if (st != PHX_OK) return st;
-	for (int k = 0; k < 5; k++) counters[k] = host[k];
+	for (uint32_t stripe = 0; stripe < kCountStripes; stripe++)
+		for (uint32_t k = 0; k < 5u; k++) counters[k] += host[stripe * kCountStride + k];
 	return ok();
 }
 

@@ -112,13 +112,17 @@ hipError_t launchInstances(const PhxBVHNode* top, const WideNode* topWide, const
                            uint32_t numInst, const PhxRayIn* rays, uint32_t n, PhxRayHit* hits, uint32_t* instOut,
                            uint8_t* inLight, bool seeded, const TraceLaunch& L, hipStream_t stream);
 
+// Counters of a counting cast: kCountStripes lines of kCountStride words, whose sums are the counts.
+constexpr uint32_t kCountStripes = 64, kCountStride = 16;
+
 // Any hit of every ray (one ray per lane) adding castDebugRay-style counters of the any-hit
-// traversal (trianglesIntersected = rays occluded) to counters[0..4].
+// traversal (trianglesIntersected = rays occluded) to words 0 to 4 of a stripe of `counters`.
 hipError_t launchAnyHitCounted(const SceneView& s, const PhxRayIn* rays, uint32_t n,
-                               uint8_t* inLight, unsigned long long* counters, hipStream_t stream);
+                               uint8_t* inLight, const TraceLaunch& launch,
+                               unsigned long long* counters, hipStream_t stream);
 
 // Closest hit in the CPU castRay visiting order. If `counters` is not null the castDebugRay
-// counters of the batch are added to counters[0..4] (device memory).
+// counters of the batch are added to words 0 to 4 of its stripes (device memory).
 // Counts the floats a (exhaustive: all of 2^-126 <= |a| < 2^126; else every significand at four
 // exponents, both signs) whose fast reciprocal differs from IEEE 1/a; adds them to *mismatches.
 // Returns the number of inputs compared in *tested.

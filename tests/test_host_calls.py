@@ -461,3 +461,14 @@ def test_requests_in_pageable_memory_are_not_split(library):
     rays; requests in pinned memory, of a quarter of what waits, a million at least."""
     assert len(run(library, backlog_launches, False, 48, 55000)) == 1
     assert len(run(library, backlog_launches, True, 48, 55000)) == 3
+
+
+@pytest.mark.parametrize("mode", [0, phx.STATS_ANYHIT])
+@pytest.mark.parametrize("n", [1, 1000, 4096, 4097, 20000, 300000])
+def test_counting_casts_spread_few_rays_over_the_device(library, n, mode):
+    """A wave takes as long as its rays' different steps together: no more rays a wave than 24 waves a CU
+    need (256 CUs)."""
+    line, = [x for x in run(library, traversal_stats, n, mode) if "simple" in x]
+    grid, block = (int(w.split("=")[1]) for w in line.split() if w.startswith(("grid", "block")))
+    per_wave = min(64, -(-n // 6144))
+    assert -(-n // per_wave) <= grid * (block // 64) < -(-n // per_wave) + 4
