@@ -812,7 +812,7 @@ __device__ __forceinline__ uint32_t find_batch(const uint32_t* offsets, uint32_t
 //
 // Single casts of incoherent rays (k_quad). Four lanes trace a ray: one box of a wide node each, or one
 // triangle of a leaf each, combined across the four (DPP and 4 bits of a ballot). A wave holds 16
-// rays, its stacks are in LDS, and it runs at eight waves per SIMD. An iteration loads and consumes a
+// rays, its stacks are in LDS, and seven of them run on a SIMD. An iteration loads and consumes a
 // leaf and the node to be taken after it together: the node's slots are decided after the leaf's
 // triangles, with its entry distance compared again, so the order is castRay's. See wide_nodes.hpp
 // for why the hits are too.
@@ -1063,22 +1063,15 @@ struct QuadTracer {
 		q.hit = kInvalid;
 		q.mine = l == 0u;
 	}
-	// Takes over a ray that is being traced (its batch is set; its traversal is the caller's).
+	// Takes over a ray of a batch that is being traced (its batch is set; its traversal is the caller's).
 	__device__ __forceinline__ void take_over(uint32_t ray)
 	{
-		const float4* rays = P.rays;
-		uint32_t at = ray;
-		uint32_t with = P.with;
-		if (kBatch) {
-			at = ray - P.offsets[q.batch];
-			const BatchDesc d = P.descs[q.batch];
-			rays = d.rays;
-			q.wide = d.wide;
-			q.tris = d.tris;
-			q.any = d.kind & 1u;
-			with = d.kind >> 1;
-		}
-		set(ray, as_global(rays)[2 * size_t(at)], as_global(rays)[2 * size_t(at) + 1], with);
+		const uint32_t at = ray - P.offsets[q.batch];
+		const BatchDesc d = P.descs[q.batch];
+		q.wide = d.wide;
+		q.tris = d.tris;
+		q.any = d.kind & 1u;
+		set(ray, as_global(d.rays)[2 * size_t(at)], as_global(d.rays)[2 * size_t(at) + 1], d.kind >> 1);
 	}
 
 	// Expands a binary node: lanes 0 and 1 decide its children as castRay does, and what is visited is
@@ -1344,7 +1337,7 @@ __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 // instruction serves 64 rays, not 16) but reads 64 lines with each load, takes a leaf and a node in
 // steps of their own and is as slow as its costliest lane, so four lanes per ray are the faster way
 // for a launch by itself (1,048,576 random rays, 4 waves per SIMD: 0.485 ms against 0.468 ms) and one
-// lane is where the device is full: 64 batches of 3.2 million rays on two scenes take 1.56 ms (2.3 ms
+// lane is where the device is full: 64 batches of 4.4 million rays on two scenes take 1.56 ms (2.3 ms
 // four lanes each; 1.79 ms with the binary nodes). There the texture data path was busy 85% of
 // the time, the VALUs 63% (with eight words a node). Handing the records over in LDS, four lanes to a line, took it to 1.60 ms and
 // single casts from 0.106 to 0.123 ms, so each lane loads its own.
@@ -1536,7 +1529,7 @@ struct SpillStack {
 	}
 };
 
-template <int kAny, bool kBatch, bool kTrack, bool kClock>
+template <bool kTrack>
 struct LaneTracer {
 	const QuadArgs& P;
 	SpillStack stack;
@@ -1546,8 +1539,6 @@ struct LaneTracer {
 	uint32_t batch = 0u;
 	const float4* wide = nullptr;
 	const float4* tris = nullptr;
-
-	__device__ __forceinline__ bool isAny() const { return kAny == 1 || (kAny == 2 && any); }
 
 	// A window whose rays are staged in LDS, a lane's each. Its batch and that one's scene, if it has
 	// only one.
@@ -1559,22 +1550,18 @@ struct LaneTracer {
 	{
 		const uint32_t lane = __lane_id();
 		first = W.next;
-		const float4* rays = P.rays;
-		uint32_t at = first + lane;
-		if (kBatch && W.next < W.end) {
+		if (W.next < W.end) {
 			windowBatch = uniform(find_batch(P.offsets, P.numBatches, first));
 			single = uniform(P.offsets[windowBatch + 1u]) >= W.end;
 			desc = P.descs[windowBatch];
+			const uint32_t at = first + lane;
 			if (at < W.end) {
 				const uint32_t b = single ? windowBatch : find_batch(P.offsets, P.numBatches, at);
-				rays = single ? desc.rays : P.descs[b].rays;
-				at -= P.offsets[b];
+				const float4* rays = single ? desc.rays : P.descs[b].rays;
+				GlobalV4* p = (GlobalV4*)(rays) + 2u * size_t(at - P.offsets[b]);
+				staged[lane] = p[0];
+				staged[64u + lane] = p[1];
 			}
-		}
-		if (first + lane < W.end) {
-			GlobalV4* p = (GlobalV4*)(rays) + 2u * size_t(at);
-			staged[lane] = p[0];
-			staged[64u + lane] = p[1];
 		}
 		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 		__builtin_amdgcn_wave_barrier();
@@ -1582,22 +1569,18 @@ struct LaneTracer {
 	}
 	__device__ __forceinline__ void start(uint32_t index)
 	{
-		uint32_t with = P.with;
-		if (kBatch) {
-			batch = windowBatch;
-			BatchDesc d = desc;
-			if (!single) {
-				batch = find_batch(P.offsets, P.numBatches, index);
-				d = P.descs[batch];
-			}
-			wide = d.wide;
-			tris = d.tris;
-			any = (d.kind & 1u) != 0u;
-			with = d.kind >> 1;
+		batch = windowBatch;
+		BatchDesc d = desc;
+		if (!single) {
+			batch = find_batch(P.offsets, P.numBatches, index);
+			d = P.descs[batch];
 		}
+		wide = d.wide;
+		tris = d.tris;
+		any = (d.kind & 1u) != 0u;
 		const F32x4 sa = staged[index - first], sb = staged[64u + index - first];
 		const float4 a = make_float4(sa.x, sa.y, sa.z, sa.w), b = make_float4(sb.x, sb.y, sb.z, sb.w);
-		t.with = quad_ray(a, b, with, t.r);
+		t.with = quad_ray(a, b, d.kind >> 1, t.r);
 		if (__builtin_expect(t.with != kFast, 0)) divide(b, t.r);
 		ray = index;
 		t.ref = 0u;
@@ -1609,32 +1592,27 @@ struct LaneTracer {
 	{
 		const bool active = ray != kInvalid;
 		float4 w[7];
-		t.load(active, kBatch ? wide : P.wide, kBatch ? tris : P.tris, w);
+		t.load(active, wide, tris, w);
 		if (!active) return;
 		bool occluded;
-		const float4* nodes = kBatch ? P.descs[batch].nodes : P.nodes;
+		const float4* nodes = P.descs[batch].nodes;
 		const bool ended = __builtin_expect(ballot(t.with != kFast) != 0ull, 0)
-		                       ? t.template advance<kAny, true>(w, nodes, isAny(), stack, occluded)
-		                       : t.template advance<kAny, false>(w, nodes, isAny(), stack, occluded);
+		                       ? t.template advance<2, true>(w, nodes, any, stack, occluded)
+		                       : t.template advance<2, false>(w, nodes, any, stack, occluded);
 		if (ended) {
-			quad_result<kBatch, kTrack, kClock>(P, ray, batch, t.c, isAny(), occluded);
+			quad_result<true, kTrack, false>(P, ray, batch, t.c, any, occluded);
 			ray = kInvalid;
 		}
 	}
 };
 
-template <int kAny, bool kBatch, bool kTrack, bool kClock>
+template <bool kTrack>
 __device__ __forceinline__ void lane_trace(const QuadArgs& P, uint32_t* lds)
 {
 	const uint32_t waveInBlock = uniform(threadIdx.x >> 6), lane = __lane_id();
 	LdsU2* stacks = (LdsU2*)(reinterpret_cast<U32x2*>(lds));
-	if (kClock && threadIdx.x == 0u) atomicMin(&P.clock[P.n], wall_clock64());
-	LaneTracer<kAny, kBatch, kTrack, kClock> T{P, {stacks, P.spill, stack_base<kLaneRows, 64u>(waveInBlock, lane)}};
+	LaneTracer<kTrack> T{P, {stacks, P.spill, stack_base<kLaneRows, 64u>(waveInBlock, lane)}};
 	T.t.r = {};
-	if (kBatch) {  // read by lanes without a ray
-		T.wide = P.descs[0].wide;
-		T.tris = P.descs[0].tris;
-	}
 	T.staged = (LdsF4*)(lds + blockDim.x / 64u * 2u * wave_stack_entries<kLaneRows, 64u>()) + waveInBlock * 128u;
 	RayWindows W(P, waveInBlock);
 	T.stage(W);
@@ -1662,7 +1640,7 @@ __device__ __forceinline__ void lane_trace(const QuadArgs& P, uint32_t* lds)
 	}
 	if (busy == 0ull) return;
 	// The k-th busy lane's ray goes to lanes 4k to 4k + 3.
-	QuadTracer<kAny, kBatch, kTrack, kClock, true, kLaneRows, 64u> Q{P};
+	QuadTracer<2, true, kTrack, false, true, kLaneRows, 64u> Q{P};
 	Q.stacks = stacks;
 	Q.lane = lane;
 	Q.l = lane & 3u;
@@ -1680,7 +1658,7 @@ __device__ __forceinline__ void lane_trace(const QuadArgs& P, uint32_t* lds)
 	const float best = __uint_as_float(move(__float_as_uint(T.t.c.t)));
 	const float u = __uint_as_float(move(__float_as_uint(T.t.c.u)));
 	const float v = __uint_as_float(move(__float_as_uint(T.t.c.v)));
-	const uint32_t hit = move(T.t.c.tri), batch = kBatch ? move(T.batch) : 0u;
+	const uint32_t hit = move(T.t.c.tri), batch = move(T.batch);
 	if (lane / 4u < uint32_t(__popcll(busy))) {
 		Q.q.batch = batch;
 		Q.take_over(ray);
@@ -1695,7 +1673,7 @@ __device__ __forceinline__ void lane_trace(const QuadArgs& P, uint32_t* lds)
 		Q.q.node = Q.q.leaf ? kInvalid : ref;
 		Q.q.nodeIn = -INFINITY;
 	}
-	if (kBatch && Q.q.ray == kInvalid) {  // read by lanes without a ray
+	if (Q.q.ray == kInvalid) {  // read by lanes without a ray
 		Q.q.wide = P.descs[0].wide;
 		Q.q.tris = P.descs[0].tris;
 	}
@@ -2072,13 +2050,13 @@ __global__ __launch_bounds__(kQuadBlock, kQuadWavesPerSimd) void k_quad(
 //
 // One persistent launch over many ray batches (closest-hit or any-hit, on one or several scenes):
 // the batches' rays form one index space [0, total) handed out as above; a ray's index is mapped to
-// (batch, local index) by binary search over the batch offsets held in LDS, when its quad starts it.
-// With completion tracking on, the quads completing rays in the block count completions and the
+// (batch, local index) by binary search over the batch offsets held in LDS, when its lane starts it.
+// With completion tracking on, the lanes completing rays in the block count completions and the
 // latest completion time per batch in LDS, and every block adds them to the batch table with one
 // global atomic per batch when it ends, so each batch's latency inside the launch is known (the
 // clock only grows, so completion times need no reset between launches). The last block to end
 // resets the counters for the next launch.
-// Six waves per SIMD: a ray's scene, batch and kind take 70 registers.
+// Four waves per SIMD: a wave's stacks and rays take 8.5 KB of LDS, and four fill blocks of 1,024 threads.
 
 __host__ __device__ __forceinline__ uint32_t batch_lds_words(uint32_t waves, uint32_t numBatches,
                                                              bool tracked)
@@ -2108,7 +2086,7 @@ __global__ __launch_bounds__(kLaneBlock, 4) void k_trace_batches(
 	__syncthreads();
 	const QuadArgs P = {nullptr, nullptr, nullptr, nullptr, nullptr, total, 0u, window, refill, work,
 	                    spill, nullptr, descs, offsets, numBatches, blockFinish, blockDone};
-	lane_trace<2, true, kTrack, false>(P, lds);
+	lane_trace<kTrack>(P, lds);
 	__syncthreads();
 	if (kTrack) {
 		for (uint32_t b = threadIdx.x; b < numBatches; b += blockDim.x)
