@@ -218,14 +218,16 @@ uint32_t phx_context_num_cus(PhxContext* ctx);
 /* Launch shape of the persistent traversal kernels on this context: grid size in blocks for
  * closest-hit and any-hit and block size (a multiple of 64 up to 1024), which together bound the
  * rays in flight; the refill threshold (1..64: how many of a wave's ray places are idle before it
- * takes new rays); rays per fetch (8..4096: an upper bound on the rays a wave claims from a shared
- * counter with one atomic). topNodes (0..2048), helperWaves (blockThreads + 64 * helperWaves <=
- * 1024) and stackLdsEntries (4..32) do not change how the kernels run; they are checked, kept and
+ * takes new rays; single casts, whose waves have 16 places, use a quarter of it, at most 16); rays per
+ * fetch (8..4096: an upper bound on the rays a wave claims from a shared counter with one atomic; no
+ * wave claims more than 64, or 16 of a closest-hit cast or of a plan of few rays). topNodes (0..2048),
+ * helperWaves (blockThreads + 64 * helperWaves <= 1024) and stackLdsEntries (4..32) do not change how
+ * the kernels run; they are checked, kept and
  * reported. phx_create's defaults: one block of 512 threads per CU, topNodes 0, refill 8,
  * helperWaves 0, 64 rays per fetch, 16 stack entries; phx_autotune picks the grid, refill threshold
  * and rays per fetch per scene and ray mix. In phx_set_launch_params a zero
- * field (0xFFFFFFFF for topNodes and helperWaves) keeps the current value; combinations that do
- * not fit a CU are rejected. In phx_plan_set_launch_params 0xFFFFFFFF helper waves means none and
+ * field (0xFFFFFFFF for topNodes and helperWaves) keeps the current value; combinations whose
+ * topNodes and stackLdsEntries would not fit a CU's local memory are rejected. In phx_plan_set_launch_params 0xFFFFFFFF helper waves means none and
  * a zero raysPerFetch or stackLdsEntries the default. Results do not depend on these parameters. */
 typedef struct PhxLaunchParams {
 	uint32_t gridBlocksClosest;
@@ -245,7 +247,8 @@ phx_status phx_set_launch_params(PhxContext* ctx, const PhxLaunchParams* params)
 /* Autotuner for single-batch casts: times phx_cast_closest (or, with PHX_AUTOTUNE_ANYHIT,
  * phx_cast_anyhit) on the given device rays under candidate launch shapes -- 1/4, 1/2 or
  * all of the resident grid, refill 8/32, the one-ray-per-lane kernel and the packet kernel -- with
- * HIP events; if a persistent shape wins it then tries 16 and 32 rays per fetch with it, and applies
+ * HIP events; if a persistent shape wins it then tries 16 and 32 rays per fetch with it (shapes that
+ * come to the same launch are timed once), and applies
  * the fastest persistent shape to the context. `chosen` (may be NULL) receives it; residentGridBlocks
  * = 0xFFFFFFFF there means the one-ray-per-lane kernel won (pass PHX_KERNEL_ONE_RAY_PER_LANE to
  * the casts) and 0xFFFFFFFE the packet kernel (pass PHX_KERNEL_PACKET). `rays` must be device
@@ -590,14 +593,15 @@ typedef struct PhxServerStats {
 /* A server on ctx's device with an HBM budget (resident scenes + request buffers) and `slots`
  * (1..4) launch streams. Requests are admitted in arrival order while their buffers fit, and
  * admitted requests are coalesced, in order, into the next fused persistent launch on an idle
- * slot, a quarter of the waiting rays per launch but one to four million (four million where the
- * rays are on the device; a larger request gets a launch of its own), so a backlog spreads
+ * slot: four million rays per launch, or, of requests whose rays and outputs lie in pinned memory, a
+ * quarter of the waiting rays but one to four million (a larger request gets a launch of its own), so a
+ * backlog of those spreads
  * over the slots and one launch's copies overlap another's traversal; a launch formed while
  * another runs fills that launch's tail. Slot 0 launches on the context's stream (other work on
  * that stream runs in order with it); each further slot has a stream of its own. HIP spreads a
  * process's streams over a few hardware queues (4 by default) and slots that share a queue
  * serialise, so more than 3 slots only pay where more queues exist. A dispatcher thread owns the
- * device work. The server
+ * device work; submit, poll and cancel do not wait for it while it launches. The server
  * launches with the default rays per fetch; it takes the refill threshold from the context. */
 phx_status phx_server_create(PhxContext* ctx, uint64_t budgetBytes, uint32_t slots,
                              uint32_t flags, PhxServer** outServer);

@@ -151,8 +151,8 @@ phx_status enqueueFrame(PhxContext* ctx, PhxRenderer* r, const PhxScene* scene,
 	const TraceLaunch closest = traceLaunch(ctx, 0, false);
 	// Shadow rays are coherent -- a pixel tile's rays towards one light, tiles in order -- so they
 	// are traced as packets, each wave expanding the union of 64 rays' nodes. So are camera rays in
-	// 8x8-tile order (a wave's 64 rays are one tile): 0.33 ms for a 1080p frame's closest hits, where
-	// the persistent kernel takes 0.47 ms for half of them; in row-major order a wave's rays span a
+	// 8x8-tile order (a wave's 64 rays are one tile): 0.35 ms for a 1080p frame's closest hits, where
+	// the persistent kernel takes 0.47 ms; in row-major order a wave's rays span a
 	// 64-pixel row segment and packets gain nothing, so those go to the persistent kernel.
 	TraceLaunch shadows = traceLaunch(ctx, 0, true);
 	shadows.kernel = TraceKernel::Packet;
@@ -191,7 +191,7 @@ phx_status enqueueFrame(PhxContext* ctx, PhxRenderer* r, const PhxScene* scene,
 	        what);
 	// The bounce rays' hits, their records, shading and shadow rays run on the side stream beside the
 	// primary shading, each filling the other's last waves; only adding the bounce light waits for both
-	// (1080p, 8 lights: 1.35 ms, with a join after the closest hits 1.38). With instances, whose primary
+	// (1080p, 8 lights, when it was made so: 1.35 ms, with a join after the closest hits 1.38). With instances, whose primary
 	// shadow rays are stored where the bounce shading's are, the streams join after the closest hits.
 	// No other persistent launch of the context's ray counters and spill area runs meanwhile.
 	hipStream_t q = inst ? s : r->side;

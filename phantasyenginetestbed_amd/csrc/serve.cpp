@@ -2,8 +2,8 @@
 //
 // Requests (ray batches against resident scenes) are admitted in arrival order while their
 // buffers fit the HBM budget (a first-fit arena over one device allocation, so admission never
-// calls hipMalloc), and admitted requests are coalesced into the next fused persistent launch, up
-// to a quarter of the waiting rays per launch (formLaunch; at least one request).
+// calls hipMalloc), and admitted requests are coalesced into the next fused persistent launch
+// (kLeastLaunchRays; at least one request).
 // Launches run on `slots` streams, each with its own work counter and stack spill area, so a
 // launch formed from requests that arrived while another one runs starts on the next stream and
 // fills the running launch's tail. A dispatcher thread forms launches and retires them (outputs

@@ -821,8 +821,8 @@ __device__ __forceinline__ uint32_t find_batch(const uint32_t* offsets, uint32_t
 // pipeline and a one-ray-per-wave mode for a wave's last rays) a launch was bound by its chains of
 // steps: 25 a bounce ray on 1,004,000 triangles, half of the time spent on the last 1% of the rays,
 // and 15,600 fetches from and 2,048 retirements to one address at 10 ns each. Before and now:
-//   998,029 bounce rays, closest hit   0.567 ms   0.438 ms
-//   their 998,029 shadow rays, any hit  0.254 ms   0.122 ms
+//   998,029 bounce rays, closest hit   0.567 ms   0.428 ms
+//   their 998,029 shadow rays, any hit  0.254 ms   0.119 ms
 //   65,536 random rays, 100,000 random triangles  0.243 ms   0.120 ms
 // Many rays at once are bound by VALU issue (a wave instruction serves 16 rays), the rest by the
 // chain of the costliest rays: about 450 iterations of 0.9 us, the time a wave takes to issue one. So
@@ -1337,10 +1337,10 @@ __device__ __forceinline__ void quad_trace(const QuadArgs& P, uint32_t* lds)
 // instruction serves 64 rays, not 16) but reads 64 lines with each load, takes a leaf and a node in
 // steps of their own and is as slow as its costliest lane, so four lanes per ray are the faster way
 // for a launch by itself (1,048,576 random rays, 4 waves per SIMD: 0.485 ms against 0.468 ms) and one
-// lane is where the device is full: 64 batches of 4.4 million rays on two scenes take 1.56 ms (2.3 ms
-// four lanes each; 1.79 ms with the binary nodes). There the texture data path was busy 85% of
-// the time, the VALUs 63% (with eight words a node). Handing the records over in LDS, four lanes to a line, took it to 1.60 ms and
-// single casts from 0.106 to 0.123 ms, so each lane loads its own.
+// lane is where the device is full: 64 batches of 4.4 million rays on two scenes take 1.48 ms (2.3 ms
+// four lanes each; 1.79 ms with the binary nodes). There the texture data path is busy 83% of
+// the time, the VALUs 70%. Handing the records over in LDS, four lanes to a line, took it from 1.65 to
+// 1.60 ms and single casts from 0.106 to 0.123 ms, so each lane loads its own.
 
 // One lane's castRay over the wide nodes, or the binary ones, one record at a time.
 struct LaneWalk {
@@ -1881,11 +1881,11 @@ __device__ __forceinline__ uint32_t object_ray(const DevInstance& in, const floa
 // 3.6 ms instead of 3.0). Rays are handed out as in the other persistent kernels, so lanes do not wait
 // for the wave's costliest ray.
 //
-// Bound by the texture data path, which returns a lane's 16 B a cycle (75% busy), and by VALU issue
-// (65%, with 17 of 64 lanes active on average). On the binary nodes, with exact slabs and divisions, a
+// Bound by VALU issue (81% busy, with 18 of 64 lanes active on average) and by the texture data path,
+// which returns a lane's 16 B a cycle (76%). On the binary nodes, with exact slabs and divisions, a
 // top-tree step in every iteration and a fixed range of rays per wave, 1,048,576 rays into 300
 // instances took 4.92 ms (closest) and 262,147 any-hit rays into 120 instances and a scene 0.71 ms;
-// now 3.14 and 0.41 ms. (Wide nodes inside the instances alone: 4.14 and 0.49 ms.)
+// now 2.92 and 0.40 ms. (Wide nodes inside the instances alone: 4.14 and 0.49 ms.)
 
 constexpr uint32_t kInstanceRefill = 8;  // idle lanes of a wave before it takes new rays
 constexpr uint32_t kInstanceWaves = 20;  // per CU: 5 per SIMD (96 registers)
